@@ -1,18 +1,20 @@
-"""Builds flash_pop_amd/libflashpop_hip.so for gfx950 with hipcc (cross-compiles without a GPU)."""
+"""Builds flash_pop_amd/libflashpop_hip.so for gfx950 with hipcc (cross-compiles without a GPU) and, linked to it,
+flash_pop_amd/_native.so, the PyTorch ops (host code only)."""
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "flash_pop_amd", "libflashpop_hip.so")
+NATIVE_OUT = os.path.join(HERE, "flash_pop_amd", "_native.so")
 SOURCES = ["launch_hip.hip", "flashpop_api.cpp"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
-def build(verbose: bool = True) -> str:
-    cmd = ["hipcc", *FLAGS, *[os.path.join(CSRC, s) for s in SOURCES], "-o", OUT]
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -22,7 +24,24 @@ def build(verbose: bool = True) -> str:
     if err.strip() and (verbose or res.returncode):
         print(err, file=sys.stderr)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed with exit code {res.returncode}")
+        raise RuntimeError(f"{cmd[0]} failed with exit code {res.returncode}")
+
+
+def _native_command():
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    includes = [f"{root}/include", f"{root}/include/torch/csrc/api/include", f"{rocm}/include", sysconfig.get_paths()["include"]]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[a for i in includes for a in ("-isystem", i)],
+            os.path.join(CSRC, "torch_ops.cpp"), "-o", NATIVE_OUT,
+            "-L", os.path.dirname(OUT), "-l:" + os.path.basename(OUT), "-L", f"{root}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu",
+            "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{root}/lib"]
+
+
+def build(verbose: bool = True) -> str:
+    _run(["hipcc", *FLAGS, *[os.path.join(CSRC, s) for s in SOURCES], "-o", OUT], verbose)
+    _run(_native_command(), verbose)
     return OUT
 
 

@@ -1,4 +1,5 @@
-"""ctypes binding of libflashpop_hip.so (declarations: include/flashpop_hip.h)."""
+"""The two native libraries: libflashpop_hip.so, bound with ctypes (declarations: include/flashpop_hip.h), and _native.so, the
+ops with their autograd nodes over it (csrc/torch_ops.cpp)."""
 from __future__ import annotations
 
 import ctypes
@@ -38,6 +39,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_native = None
 
 
 def bind(path: str) -> ctypes.CDLL:
@@ -61,6 +63,20 @@ def load() -> ctypes.CDLL:
                 "__graft_entry__.build()). flash_pop_amd has no non-HIP execution path.")
         _lib = bind(LIB_PATH)
     return _lib
+
+
+def native():
+    """The extension module with the ops, built in-tree like the library it is linked to."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise RuntimeError(f"{_HERE}/_native.so cannot be loaded ({e}): build it first (python flash-pop_amd/build.py, or "
+                               "__graft_entry__.build())") from e
+        _native = module
+    return _native
 
 
 def decays_array(head_decays) -> ctypes.Array:

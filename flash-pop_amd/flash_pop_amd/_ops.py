@@ -1,4 +1,6 @@
-"""Tensor-level plumbing shared by the two autograd Functions: checks, allocation, raw calls."""
+"""Argument checks, with the exceptions they raise, and the C ABI called on tensors through ctypes, without autograd (what a
+program that binds the library by itself does).  The ops that the package exports run in csrc/torch_ops.cpp, which makes the
+same checks and leaves it to this module to say what was wrong."""
 from __future__ import annotations
 
 import ctypes
@@ -45,6 +47,11 @@ def prepare(q, k, v, s, head_decays):
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     s = None if s is None else s.contiguous()
     return q, k, v, s, (B, T, H, dk, dv)
+
+
+def rejected(op):
+    """The native op refused its arguments and the checks above found nothing to say about them."""
+    raise TypeError(f"{op}: unsupported arguments")
 
 
 def _workspace(lib, shape, device):

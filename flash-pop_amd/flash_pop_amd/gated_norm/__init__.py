@@ -7,26 +7,12 @@ with the reference's rounding points.  retention [..., H, dv] (the op's output),
 (the output of g_proj before the activation); returns [..., H*dv].  bfloat16 on the GPU;
 dv = 8 * 2^k <= 512.  Gradients flow to both inputs (one launch).
 """
-import torch
-
-from .. import _ops
-
-
-class GatedGroupNorm(torch.autograd.Function):
-
-    @staticmethod
-    def forward(ctx, retention, gate, eps):
-        retention, gate = retention.contiguous(), gate.contiguous()
-        ctx.save_for_backward(retention, gate)
-        ctx.eps = eps
-        return _ops.gated_norm_fwd(retention, gate, eps)
-
-    @staticmethod
-    def backward(ctx, d_out):
-        retention, gate = ctx.saved_tensors
-        d_r, d_g = _ops.gated_norm_bwd(retention, gate, d_out, ctx.eps)
-        return d_r, d_g, None
+from .. import _lib, _ops
 
 
 def gated_group_norm(retention, gate, eps: float = 1e-6):
-    return GatedGroupNorm.apply(retention, gate, eps)
+    out = _lib.native().gated_group_norm(retention, gate, eps)
+    if out is NotImplemented:
+        _ops.gated_norm_fwd(retention, gate, eps)   # raises
+        _ops.rejected("gated_group_norm")
+    return out

@@ -17,67 +17,41 @@ index fastest (N = T // block_size, any Ls >= 1); last_state is the state after 
 block, the reference's `states[:, -1]`.  Tokens after the last block boundary (T % block_size of
 them) are context like any others; no suffix follows them.
 """
-import torch
-
-from .. import _ops
+from .. import _lib, _ops
 
 
-class FlashPOPRetention(torch.autograd.Function):
+def _refused(q, k, v, s, head_decays, block_size):
+    """Raises for arguments that the native ops did not take; -> the shape if it is the suffixes' fault."""
+    block_size = int(block_size)
+    assert block_size >= 1, f"block_size must be positive, got {block_size}"
+    return _ops.prepare(q, k, v, s, head_decays)[4]
 
-    @staticmethod
-    def forward(ctx, q, k, v, s, head_decays, block_size):
-        block_size = int(block_size)
-        assert block_size >= 1, f"block_size must be positive, got {block_size}"
-        q, k, v, s, shape = _ops.prepare(q, k, v, s, head_decays)
-        o, states = _ops.pop_retention_fwd(q, k, v, s, head_decays, block_size, shape)
-        ctx.save_for_backward(q, k, v, s)
-        ctx.set_materialize_grads(False)   # an output nobody differentiates arrives as None, not as a tensor of zeros
-        ctx.head_decays = tuple(head_decays)
-        ctx.shape = shape
-        ctx.block_size = block_size
-        return o, states
+
+class FlashPOPRetention:
+    """Stands for the reference's autograd Function of this name: `apply` is the op (forward, backward and graph node native)."""
 
     @staticmethod
-    def backward(ctx, d_o, d_block_states):
-        q, k, v, s = ctx.saved_tensors
-        if d_o is None:
-            d_o = torch.zeros((*q.shape[:3], v.shape[3]), dtype=q.dtype, device=q.device)
-        want_ds0 = s is not None and ctx.needs_input_grad[3]
-        dq, dk, dv, d_s0 = _ops.retention_bwd(q, k, v, s, ctx.head_decays, ctx.shape, d_o, None, d_block_states,
-                                              ctx.block_size, want_ds0)
-        return dq, dk, dv, d_s0, None, None
+    def apply(q, k, v, s, head_decays, block_size):
+        out = _lib.native().flash_pop_retention(q, k, v, s, head_decays, block_size)
+        if out is NotImplemented:
+            _refused(q, k, v, s, head_decays, block_size)
+            _ops.rejected("flash_pop_retention")
+        return out
 
 
 flash_pop_retention = FlashPOPRetention.apply
 
 
-class FlashPOPRetentionWithSuffixes(torch.autograd.Function):
+class FlashPOPRetentionWithSuffixes:
 
     @staticmethod
-    def forward(ctx, q, k, v, s, head_decays, block_size, q_sfx, k_sfx, v_sfx):
-        block_size = int(block_size)
-        assert block_size >= 1, f"block_size must be positive, got {block_size}"
-        q, k, v, s, shape = _ops.prepare(q, k, v, s, head_decays)
-        sfx = _ops.prepare_suffixes(q_sfx, k_sfx, v_sfx, shape, block_size)
-        o, o_sfx, last_state = _ops.pop_fused_fwd(q, k, v, s, sfx, head_decays, block_size, shape)
-        ctx.save_for_backward(q, k, v, s, *sfx)
-        ctx.set_materialize_grads(False)   # an output nobody differentiates arrives as None, not as a tensor of zeros
-        ctx.head_decays = tuple(head_decays)
-        ctx.shape = shape
-        ctx.block_size = block_size
-        return o, o_sfx, last_state
-
-    @staticmethod
-    def backward(ctx, d_o, d_o_sfx, d_last_state):
-        q, k, v, s, *sfx = ctx.saved_tensors
-        if d_o is None:
-            d_o = torch.zeros((*q.shape[:3], v.shape[3]), dtype=q.dtype, device=q.device)
-        if d_o_sfx is None:
-            d_o_sfx = torch.zeros((*sfx[0].shape[:3], v.shape[3]), dtype=q.dtype, device=q.device)
-        want_ds0 = s is not None and ctx.needs_input_grad[3]
-        (dq, dk, dv, dq_s, dk_s, dv_s), d_s0 = _ops.pop_fused_bwd(q, k, v, s, sfx, ctx.head_decays, ctx.block_size,
-                                                                   ctx.shape, d_o, d_o_sfx, d_last_state, want_ds0)
-        return dq, dk, dv, d_s0, None, None, dq_s, dk_s, dv_s
+    def apply(q, k, v, s, head_decays, block_size, q_sfx, k_sfx, v_sfx):
+        out = _lib.native().flash_pop_retention_with_suffixes(q, k, v, s, head_decays, block_size, q_sfx, k_sfx, v_sfx)
+        if out is NotImplemented:
+            shape = _refused(q, k, v, s, head_decays, block_size)
+            _ops.prepare_suffixes(q_sfx, k_sfx, v_sfx, shape, int(block_size))
+            _ops.rejected("flash_pop_retention_with_suffixes")
+        return out
 
 
 flash_pop_retention_with_suffixes = FlashPOPRetentionWithSuffixes.apply

@@ -9,11 +9,14 @@ With in_place=True the new state overwrites prev_state (no second state buffer, 
 allocations of a decode loop)."""
 import torch
 
-from .. import _ops
+from .. import _lib, _ops
 
 
-@torch.no_grad()
 def retention_recurrent(query, key, value, head_decays, prev_state, in_place=False):
     if isinstance(head_decays, torch.Tensor):
         head_decays = tuple(head_decays.flatten().tolist())
-    return _ops.decode_step(query, key, value, prev_state, head_decays, in_place)
+    out = _lib.native().decode_step(query, key, value, prev_state, head_decays, in_place)
+    if out is NotImplemented:
+        _ops.decode_step(query, key, value, prev_state, head_decays, in_place)   # raises
+        _ops.rejected("retention_recurrent")
+    return out

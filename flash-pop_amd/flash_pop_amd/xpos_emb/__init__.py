@@ -11,25 +11,12 @@ cache to grow or invalidate.  Gradients flow to q and k (the rotation by the neg
 """
 import torch
 
-from .. import _ops
+from .. import _lib, _ops
 
 
 def position_thetas(head_dim: int, scale: float = 10000.0) -> torch.Tensor:
     """d/2 fp32 frequencies, one per rotation pair (flash_pop/xpos_emb.py:26-28 before the repeat)."""
     return 1 / (scale ** torch.linspace(0, 1, steps=head_dim // 2))
-
-
-class RotaryQK(torch.autograd.Function):
-
-    @staticmethod
-    def forward(ctx, q, k, theta, start_idx):
-        ctx.theta, ctx.start = theta, start_idx
-        return _ops.rotary_qk(q, k, theta, start_idx)
-
-    @staticmethod
-    def backward(ctx, d_q, d_k):
-        d_q, d_k = _ops.rotary_qk(d_q, d_k, ctx.theta, ctx.start, inverse=True)
-        return d_q, d_k, None, None
 
 
 class XPos:
@@ -48,4 +35,9 @@ class XPos:
 
     def __call__(self, q, k, start_idx, *args, **kwargs):
         assert q.shape[-1] == self.head_dim, f"built for head dimension {self.head_dim}, got {q.shape[-1]}"
-        return RotaryQK.apply(q, k, self._theta(q.device), start_idx)
+        theta = self._theta(q.device)
+        out = _lib.native().rotary_qk(q, k, theta, start_idx, False)
+        if out is NotImplemented:
+            _ops.rotary_qk(q, k, theta, start_idx)   # raises
+            _ops.rejected("XPos")
+        return out
