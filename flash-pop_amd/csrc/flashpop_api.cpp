@@ -81,6 +81,7 @@ void read_environment() {
 
 struct Shape {
   int B, T, H, dk, dv;
+  int segs = 0, total = 0;   // the B sequences are segments that do not divide theirs evenly (PassArgs)
 };
 
 int check_shape(const Shape& s, const double* decays) {
@@ -119,6 +120,8 @@ void fill_common(fpk::PassArgs& a, const Shape& s, const double* decays) {
   a.B = s.B;
   a.T = s.T;
   a.H = s.H;
+  a.segs = s.segs;
+  a.total = s.total;
   // log2(gamma) from the double, so gammas that round to 1.0f keep their decay
   for (int h = 0; h < s.H; ++h) a.log2g[h] = (float)std::log2(decays[h]);
 }
@@ -228,13 +231,13 @@ int forward_short(const Shape& s, const void* q, const void* k, const void* v, c
 }
 
 int forward(const Shape& s, const void* q, const void* k, const void* v, const void* s0, const double* decays, void* o,
-            void* s_out, void* block_states, int block, void* stream) {
-  if (!block_states && block == 0 && use_short_forward(s)) return forward_short(s, q, k, v, s0, decays, o, s_out, stream);
+            void* s_out, void* block_states, int block, void* stream, const uint16_t* s0_lo = nullptr) {
+  if (!block_states && block == 0 && !s0_lo && use_short_forward(s)) return forward_short(s, q, k, v, s0, decays, o, s_out, stream);
   fpk::PassArgs a;
   fill_common(a, s, decays);
   const float sc = 1.0f / std::sqrt((float)s.dk);
   a.X = in(q); a.W = in(k); a.Z = in(v); a.Y = out(o);
-  a.R0 = in(s0); a.Rout = out(s_out); a.Bout = out(block_states);
+  a.R0 = in(s0); a.R0lo = s0_lo; a.Rout = out(s_out); a.Bout = out(block_states);
   plain_state(a, s);
   a.block = block;
   a.nblk = block > 0 ? s.T / block : 0;
@@ -387,48 +390,89 @@ int backward(const Shape& s, const void* q, const void* k, const void* v, const 
 // ---- long sequences, few streams: cut every sequence into segments ---------------------------
 // One workgroup walks one (batch, head, column tile) stream from end to end, so B * H * tiles
 // workgroups is all the parallelism a pass has.  When that leaves most of the chip idle, each
-// sequence is cut into S equal segments that run as separate sequences:
+// sequence is cut into S segments of whole chunks that run as separate sequences (all equally long but the last, which
+// takes what is left):
 //   1. a state-only pass gives the state each segment contributes on its own,
 //   2. a scan over the S contributions gives the state at the start of every segment,
 //   3. the ordinary pass runs on B * S sequences from those states.
 // The backward does the same for S (needed by the dq pass; recomputed, not stored) and, walking
 // backward, for dS.  Segment states pass through bf16 like POP block states do.
 
-// Number of segments per sequence (1: do not cut) for a call whose narrowest pass has
-// `tiles` column tiles per stream.  Cutting costs an extra state-only pass per recurrence, so it
-// is done only when the uncut call would leave at least two thirds of the compute units idle.
-int plan_segments(const Shape& s, int tiles) {
-  constexpr int kMinChunks = 4;                 // shortest segment worth a workgroup of its own
-  if (s.T % fpk::CH != 0) return 1;
-  const int chunks = s.T / fpk::CH;
-  const long long streams = (long long)s.B * s.H * tiles;
-  const long long target = fpk_compute_units() / streams;   // segments that fill the chip once
-  if (target < 3) return 1;
-  int best = 1;
-  for (int n = 2; n <= target && n <= chunks; ++n) {
-    if (chunks % n == 0 && chunks / n >= kMinChunks) best = n;
-  }
-  return best;
+// Tokens per segment for at most `target` segments (or segments of kMinChunks, the shortest worth a workgroup).
+constexpr int kMinChunks = 4;
+int segment_tokens(const Shape& s, long long target) {
+  const long long chunks = (s.T + fpk::CH - 1LL) / fpk::CH, each = (chunks + target - 1) / target;
+  return (int)(each > kMinChunks ? each : kMinChunks) * fpk::CH;
 }
-// Forward and backward cut a sequence the same way (the backward's narrowest pass has the fewest
-// column tiles and decides), so that the states the forward leaves at the start of every segment
-// are the ones the backward's dq pass needs.
-int plan_split(const Shape& s) { return plan_segments(s, (s.dk < s.dv ? s.dk : s.dv) / fpk::BV); }
-int plan_forward(const Shape& s) { return plan_split(s); }
-int plan_backward(const Shape& s) { return plan_split(s); }
+int segment_count(const Shape& s, int tokens) { return (int)((s.T + tokens - 1LL) / tokens); }
+
+long long waves(long long workgroups) { return (workgroups + fpk_compute_units() - 1) / fpk_compute_units(); }
+
+// The segments that fill the chip once (1: do not cut), for a call that uncut would leave at least two thirds of the compute
+// units idle in its narrowest pass.  Equally long ones are taken where there are some that are at most a quarter longer
+// than the shortest possible (a chunk step or two against a longer scan and more segment states).
+int plan_segments(const Shape& s) {
+  const int tiles = (s.dk < s.dv ? s.dk : s.dv) / fpk::BV;
+  const long long target = fpk_compute_units() / ((long long)s.B * s.H * tiles);
+  if (target < 3) return 1;
+  const int chunks = (int)((s.T + fpk::CH - 1LL) / fpk::CH), tokens = segment_tokens(s, target);
+  int even = 1;
+  for (int n = 2; n <= target && n <= chunks; ++n) {
+    if (s.T % fpk::CH == 0 && chunks % n == 0 && chunks / n >= kMinChunks) even = n;
+  }
+  return even > 1 && 4 * (chunks / even) * fpk::CH <= 5 * tokens ? even : segment_count(s, tokens);
+}
+// Whether n segments shorten the chain of chunk steps by what the cut costs: its extra launches, and the segment states
+// that it moves.  Forward, measured at 1.1 us (64-wide keys) to 1.4 us (128) a step on the 256-unit device, uncut -> cut:
+//   64 x 64    H4 B1        18 chunks 23.5 -> 20.3 us, 13 chunks 18.2 -> 19.9
+//   64 x 128   H12 B1       79 chunks 90.7 -> 39.6,    18 chunks 23.9 -> 22.2,  13 chunks 18.5 -> 20.9
+//   128 x 128  H8 B3        28 chunks 44.1 -> 38.5,    18 chunks 30.0 -> 35.3
+//   128 x 256  H8 B2        40 chunks 61.1 -> 51.5,    28 chunks 44.2 -> 46.4
+// Backward (the uncut passes share launches, or are the fused kernel with its longer step; the cut has four launches):
+//   64 x 64    H4 B1        28 chunks 35.4 -> 30.6,    18 chunks 24.3 -> 29.6
+//   64 x 64    H12 B6       40 chunks 84.9 -> 81.8,    28 chunks 61.6 -> 64.9 (fused)
+//   64 x 128   H12 B1       18 chunks 53.7 -> 43.4,    13 chunks 41.3 -> 42.3
+//   128 x 128  H16 B1       79 chunks 119 -> 91,       40 chunks 62.4 -> 63.4,  28 chunks 45.6 -> 56.9
+//   128 x 256  H8 B2        28 chunks 121 -> 84,       18 chunks 81.0 -> 78.9
+bool cut_pays(const Shape& s, int n, bool backward) {
+  const int launch = fpk_launch_steps();   // what a launch costs, in chunk steps
+  if (launch <= 0) return true;
+  const long long chunks = (s.T + fpk::CH - 1LL) / fpk::CH, each = segment_tokens(s, n) / fpk::CH;
+  const long long streams = (long long)s.B * s.H * n, tk = s.dk / fpk::BV, tv = s.dv / fpk::BV;
+  const double matrix = s.dk * s.dv / 16384.;
+  if (!backward) return chunks - each * (1 + waves(streams * tv)) >= launch * (2 + 1.25 * matrix);
+  const long long dk_dv = s.dk == s.dv ? waves(2 * streams * tk) : waves(streams * tk) + waves(streams * tv);
+  const long long uncut = use_fused_backward(s, nullptr) ? 7 * chunks / 4 : s.dk == s.dv ? chunks : 2 * chunks;
+  return uncut - each * (1 + waves(streams * tk) + dk_dv) >= launch * (2.5 + 1.75 * matrix);
+}
+// Forward and backward cut a sequence the same way, so that the states the forward leaves at the start of every segment
+// are the ones the backward's dq pass needs; a backward is cut only if its forward is.
+int plan_forward(const Shape& s) {
+  const int n = plan_segments(s);
+  return n > 1 && cut_pays(s, n, false) ? n : 1;
+}
+int plan_backward(const Shape& s) {
+  const int n = plan_forward(s);
+  return n > 1 && cut_pays(s, n, true) ? n : 1;
+}
 
 size_t workspace_bytes(const Shape& s, int segments) {
   return segments > 1 ? 2 * sizeof(uint16_t) * (size_t)s.B * segments * s.H * s.dk * s.dv : 0;
 }
 
 struct Workspace {
-  uint16_t* contrib;   // [B, S, H, dk, dv]: what each segment adds on its own
-  uint16_t* start;     // [B, S, H, dk, dv]: state at the segment's first token (last, walking backward)
+  uint16_t* contrib;      // [B, S, H, dk, dv]: what each segment adds on its own
+  uint16_t* start;        // [B, S, H, dk, dv]: state at the segment's first token (last, walking backward)
+  // What bf16 leaves of the two (PassArgs::R0lo), nullptr: they are bf16 alone.  The scan then works in place, so the
+  // bytes are the same either way.  Equal segments keep bf16 states (those of a POP caller's blocks are bf16 too, and at
+  // B2 H8 T16384 128 x 256 the halves would be 5 % more traffic); sequences that are cut unevenly keep both halves.
+  uint16_t *contrib_lo, *start_lo;
 };
 
-Workspace carve(void* workspace, const Shape& s, int segments) {
-  uint16_t* base = static_cast<uint16_t*>(workspace);
-  return Workspace{base, base + (size_t)s.B * segments * s.H * s.dk * s.dv};
+Workspace carve(void* workspace, const Shape& s, const Shape& seg) {
+  uint16_t* const base = static_cast<uint16_t*>(workspace);
+  uint16_t* const second = base + (size_t)seg.B * s.H * s.dk * s.dv;
+  return seg.segs > 0 ? Workspace{base, base, second, second} : Workspace{base, second, nullptr, nullptr};
 }
 
 int scan(const Shape& s, int segments, const double* decays, const Workspace& w, const void* r0, void* fin, int reverse,
@@ -436,15 +480,22 @@ int scan(const Shape& s, int segments, const double* decays, const Workspace& w,
   fpk::ScanArgs a;
   std::memset(&a, 0, sizeof a);
   a.U = w.contrib; a.R0 = in(r0); a.init = w.start; a.fin = out(fin);
-  a.B = s.B; a.S = segments; a.H = s.H; a.M = s.dk * s.dv; a.Tseg = s.T / segments; a.reverse = reverse;
+  a.U_lo = w.contrib_lo; a.init_lo = w.start_lo;
+  a.B = s.B; a.S = segments; a.H = s.H; a.M = s.dk * s.dv; a.reverse = reverse;
+  a.Tseg = segment_tokens(s, segments);
+  a.Tlast = s.T - (segments - 1) * a.Tseg;
   for (int h = 0; h < s.H; ++h) a.log2g[h] = (float)std::log2(decays[h]);
   const char* msg = "";
   if (fpk_launch_scan(a, stream, &msg) != 0) return fail(FP_ERR_LAUNCH, "segment scan: %s", msg);
   return FP_OK;
 }
 
-// the B * S sequences of T / S tokens that the segments form (the same memory, reinterpreted)
-Shape segment_shape(const Shape& s, int segments) { return Shape{s.B * segments, s.T / segments, s.H, s.dk, s.dv}; }
+// the B * S sequences that the segments form (the same memory, reinterpreted)
+Shape segment_shape(const Shape& s, int segments) {
+  const int tokens = segment_tokens(s, segments);
+  const bool even = (long long)tokens * segments == s.T;
+  return Shape{s.B * segments, tokens, s.H, s.dk, s.dv, even ? 0 : segments, even ? 0 : s.T};
+}
 
 // State-only pass: contributions of the segments to S (forward walk over k, v) or to dS
 // (backward walk over q, dO).
@@ -454,8 +505,9 @@ int contributions(const Shape& seg, const double* decays, const void* w_rows, co
   if (seg.dk == fpk::FB_D && seg.dv % fpk::FB_D == 0) {   // the kernel that holds 128 x 128 of the state per workgroup
     fpk::ContribArgs c;
     std::memset(&c, 0, sizeof c);
-    c.W = in(w_rows); c.Z = in(z_rows); c.U = w.contrib;
+    c.W = in(w_rows); c.Z = in(z_rows); c.U = w.contrib; c.U_lo = w.contrib_lo;
     c.B = seg.B; c.T = seg.T; c.H = seg.H; c.dB = seg.dv; c.reverse = reverse;
+    c.segs = seg.segs; c.total = seg.total;
     c.s_update = reverse ? 1.f : sc;
     for (int h = 0; h < seg.H; ++h) c.log2g[h] = (float)std::log2(decays[h]);
     const char* msg = "";
@@ -466,7 +518,7 @@ int contributions(const Shape& seg, const double* decays, const void* w_rows, co
   fill_common(a, seg, decays);
   a.X = in(w_rows);   // never read
   a.W = in(w_rows); a.Z = in(z_rows);
-  a.Rout = w.contrib;
+  a.Rout = w.contrib; a.Rout_lo = w.contrib_lo;
   plain_state(a, seg);
   a.reverse = reverse;
   a.state_only = 1;
@@ -477,18 +529,18 @@ int contributions(const Shape& seg, const double* decays, const void* w_rows, co
 int forward_split(const Shape& s, int segments, const void* q, const void* k, const void* v, const void* s0,
                   const double* decays, void* o, void* s_out, void* workspace, void* stream) {
   const Shape seg = segment_shape(s, segments);
-  const Workspace w = carve(workspace, s, segments);
+  const Workspace w = carve(workspace, s, seg);
   int rc;
   if ((rc = contributions(seg, decays, k, v, 0, w, stream)) != FP_OK) return rc;
   if ((rc = scan(s, segments, decays, w, s0, s_out, 0, stream)) != FP_OK) return rc;
-  return forward(seg, q, k, v, w.start, decays, o, nullptr, nullptr, 0, stream);
+  return forward(seg, q, k, v, w.start, decays, o, nullptr, nullptr, 0, stream, w.start_lo);
 }
 
 int backward_split(const Shape& s, int segments, const void* q, const void* k, const void* v, const void* s0,
                    const double* decays, const void* d_o, const void* d_s_out, void* dq, void* dk_, void* dv_,
                    void* d_s0, void* workspace, bool states_kept, void* stream) {
   const Shape seg = segment_shape(s, segments);
-  const Workspace w = carve(workspace, s, segments);
+  const Workspace w = carve(workspace, s, seg);
   const float sc = 1.0f / std::sqrt((float)s.dk);
   fpk::PassArgs a;
   int rc;
@@ -500,7 +552,7 @@ int backward_split(const Shape& s, int segments, const void* q, const void* k, c
   }
   fill_common(a, seg, decays);
   a.X = in(d_o); a.W = in(v); a.Z = in(k); a.Y = out(dq);
-  a.R0 = w.start;
+  a.R0 = w.start; a.R0lo = w.start_lo;
   transposed_state(a, seg);
   a.reverse = 0;
   a.s_intra = sc; a.s_read = 1.f; a.s_update = sc;
@@ -511,7 +563,7 @@ int backward_split(const Shape& s, int segments, const void* q, const void* k, c
   if ((rc = scan(s, segments, decays, w, d_s_out, d_s0, 1, stream)) != FP_OK) return rc;
   fill_common(a, seg, decays);
   a.X = in(v); a.W = in(d_o); a.Z = in(q); a.Y = out(dk_);
-  a.R0 = w.start;
+  a.R0 = w.start; a.R0lo = w.start_lo;
   transposed_state(a, seg);
   a.reverse = 1;
   a.s_intra = sc; a.s_read = sc; a.s_update = 1.f;
@@ -519,7 +571,7 @@ int backward_split(const Shape& s, int segments, const void* q, const void* k, c
   fpk::PassArgs b;
   fill_common(b, seg, decays);
   b.X = in(k); b.W = in(q); b.Z = in(d_o); b.Y = out(dv_);
-  b.R0 = w.start;
+  b.R0 = w.start; b.R0lo = w.start_lo;
   plain_state(b, seg);
   b.reverse = 1;
   b.s_intra = sc; b.s_read = sc; b.s_update = 1.f;

@@ -26,6 +26,12 @@ FP_DEVICE float bf16_elem(u32x4 v, int e) {
   return __builtin_bit_cast(float, (e & 1) ? (d & 0xffff0000u) : (d << 16));
 }
 FP_DEVICE uint16_t float_to_bf16_bits(float x) { return (uint16_t)(fprt::pack_bf16x2(x, 0.f) & 0xffffu); }
+// What rounding x to bf16 leaves of it: bf16(x) + bf16(residual) is x to 2^-17.  0 where x or bf16(x) is not finite, so that
+// the sum of the two is bf16(x) there.
+FP_DEVICE float bf16_residual(float x) {
+  const float d = x - bf16_bits_to_float(float_to_bf16_bits(x));
+  return __builtin_fabsf(d) < __builtin_inff() ? d : 0.f;
+}
 
 // row of the 32x32 MFMA accumulator held in element r by a lane of half-wave g
 FP_DEVICE int acc_row(int r, int g) { return 8 * (r >> 2) + 4 * g + (r & 3); }

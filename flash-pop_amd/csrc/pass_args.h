@@ -31,6 +31,10 @@ struct PassArgs {
   uint16_t* Y;
   const uint16_t* R0;    // initial R per (b, h), nullable (zeros)
   uint16_t* Rout;        // final R per (b, h), nullable
+  // What bf16 leaves of the two above, as bf16 again (nullable; only for the walks without block states and suffixes):
+  // R = R0 + R0lo, Rout + Rout_lo = R to 2^-17, for states that one launch hands to the next as if it had carried them.
+  const uint16_t* R0lo;
+  uint16_t* Rout_lo;
   uint16_t* Bout;        // R after every full block, [B, nblk, H, dk*dv], nullable (forward only)
   const uint16_t* Bin;   // added to R before the chunk that ends each full block, nullable (reverse only)
   // Suffix tensors, [B, nblk + 1, Ls, H, d] in the roles of X, W, Z, Y (all four or none; Ls > 0
@@ -47,6 +51,9 @@ struct PassArgs {
   int reverse;
   int Ls;                // tokens per suffix (walked in parts of CH); 0: no suffixes
   int state_only;        // only R is wanted (Rout per sequence): X is not read, Y not written, no read-out
+  // Sequences that are segments of longer ones (0: they are not): sequence b is segment b % segs of sequence
+  // b / segs of `total` tokens, T tokens of it each but for the last one, which has what is left (1 .. T).
+  int segs, total;
   int slots;             // workgroups per (head, column tile); workgroup `slot` walks the batch entries
                          // slot, slot + slots, ... one after another.  0: the launcher chooses.
   float s_intra, s_read, s_update;
@@ -58,8 +65,8 @@ struct PassArgs {
 struct PassTensors {
   const uint16_t *X, *W, *Z;
   uint16_t* Y;
-  const uint16_t* R0;
-  uint16_t *Rout, *Bout;
+  const uint16_t *R0, *R0lo;
+  uint16_t *Rout, *Rout_lo, *Bout;
   const uint16_t *Bin, *Xs, *Ws, *Zs;
   uint16_t* Ys;
   long long rs_a, rs_n;
@@ -72,16 +79,16 @@ struct PassTensors {
 #define FPK_HOST_DEVICE
 #endif
 FPK_HOST_DEVICE inline PassTensors tensors_of(const PassArgs& a) {
-  return PassTensors{a.X,  a.W,  a.Z,  a.Y,    a.R0,   a.Rout,    a.Bout,    a.Bin,    a.Xs,
-                     a.Ws, a.Zs, a.Ys, a.rs_a, a.rs_n, a.reverse, a.s_intra, a.s_read, a.s_update};
+  return PassTensors{a.X,  a.W,  a.Z,  a.Y,    a.R0,   a.R0lo,    a.Rout,    a.Rout_lo, a.Bout,    a.Bin, a.Xs,
+                     a.Ws, a.Zs, a.Ys, a.rs_a, a.rs_n, a.reverse, a.s_intra, a.s_read,  a.s_update};
 }
 
 constexpr int MAX_PASSES_PER_LAUNCH = 3;
 
 // Arguments of the segment scan that stitches a sequence cut into S segments back together.
-// U[b][s] is the state a segment contributes on its own (zero initial state); with g = gamma^Tseg
-//   init[b][0] = R0[b] (zeros if null),  init[b][s] = g init[b][s-1] + U[b][s-1],
-//   fin[b] = g init[b][S-1] + U[b][S-1]
+// U[b][s] is the state a segment contributes on its own (zero initial state); with g_s = gamma^(tokens of segment s)
+//   init[b][0] = R0[b] (zeros if null),  init[b][s] = g_(s-1) init[b][s-1] + U[b][s-1],
+//   fin[b] = g_(S-1) init[b][S-1] + U[b][S-1]
 // `reverse` runs the same recurrence from the last segment to the first (state gradients).
 // All matrices are bf16, M = dk * dv elements each, laid out [B, S, H, M] (U, init) and [B, H, M].
 struct ScanArgs {
@@ -89,18 +96,26 @@ struct ScanArgs {
   const uint16_t* R0;   // nullable
   uint16_t* init;
   uint16_t* fin;        // nullable
+  // Low halves of U and init (both or neither): matrices are then hi + lo, exact to 2^-17, so that a cut sequence
+  // carries its state as an uncut one does.  init may be U and init_lo U_lo.
+  const uint16_t* U_lo;
+  uint16_t* init_lo;
   int B, S, H, M, Tseg, reverse;
+  int Tlast;             // tokens of the last segment (1 .. Tseg)
   float log2g[MAX_HEADS];
 };
 // State-only pass for states of 128 rows (segment_contrib.h): U[b][h] = what sequence b adds to a
 // zero state, sum_j weight(j) W[j]^T Z[j] with weight(j) = s_update gamma^(T - 1 - j) walking forward
 // (`reverse` = 0) and s_update gamma^(j + 1) walking backward.  W [B,T,H,128], Z [B,T,H,dB],
-// U [B,H,128,dB], bf16; T a multiple of CH, dB a multiple of 128.
+// U [B,H,128,dB], bf16; T a multiple of CH, dB a multiple of 128.  `segs`, `total` as in PassArgs: only the last
+// segment of a longer sequence may end inside a chunk.
 struct ContribArgs {
   const uint16_t* W;
   const uint16_t* Z;
   uint16_t* U;
+  uint16_t* U_lo;        // low half of U (see PassArgs::Rout_lo), nullable
   int B, T, H, dB, reverse;
+  int segs, total;
   float s_update;
   float log2g[MAX_HEADS];
 };
@@ -180,6 +195,7 @@ constexpr int decode_lds_bytes(int dv) { return (DECODE_THREADS / (dv / 8)) * dv
 
 constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_VEC = 8;   // elements per thread
+constexpr int SCAN_AHEAD = 8;   // contributions requested together
 
 // Rotary position embedding of q and k in one launch.  Pairs (x[2i], x[2i+1]) of every head are
 // rotated by the angle float(position) * theta[i], `sign` = -1 rotates back (the gradient).
@@ -255,6 +271,9 @@ int fpk_stream_is_capturing(void* stream);
 
 // Compute units of the current device (what the launcher sizes its grids against).
 int fpk_compute_units();
+
+// What one more launch in a chain of dependent ones costs, in chunk steps of the pass kernel (0: nothing).
+int fpk_launch_steps();
 
 // Launches the decode-step kernel.  Same conventions as fpk_launch_pass.
 int fpk_launch_decode(const fpk::DecodeArgs& args, void* stream, const char** err);

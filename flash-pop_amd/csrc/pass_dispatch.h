@@ -17,6 +17,11 @@ inline const char* plan_pass(PassArgs& a, int compute_units) {
   const bool blocks = a.block > 0 && (a.Bout || a.Bin);
   const bool narrow = a.dA == 64 || a.dA == 128;   // one visit per chunk
   const bool suffix = a.Ls > 0;
+  if (a.segs < 0 || (a.segs > 0 && (blocks || suffix || a.B % a.segs != 0 || a.total > (long long)a.segs * a.T ||
+                                    a.total <= (a.segs - 1LL) * a.T)))
+    return "segments that do not cover their sequence, or segments with block states or suffixes";
+  if ((a.R0lo && (!a.R0 || blocks || suffix)) || (a.Rout_lo && (!a.Rout || !a.state_only)))
+    return "low halves of states that this walk does not take";
   if (a.dA != 64 && a.dA != 128 && a.dA != 192 && a.dA != 256) return "unsupported contraction width (dA must be 64, 128, 192 or 256)";
   if (a.dB < BV || a.dB % BV != 0) return "dB must be a multiple of 64";
   if (suffix) {
@@ -68,6 +73,7 @@ FP_DEVICE WorkgroupId place_workgroup(int block, int nwg, int passes) {
 inline bool same_walk(const PassArgs& a, const PassArgs& b) {
   return a.B == b.B && a.T == b.T && a.H == b.H && a.dA == b.dA && a.dB == b.dB && a.nblk == b.nblk &&
          a.block == b.block && a.Ls == b.Ls && a.state_only == b.state_only && a.slots == b.slots &&
+         a.segs == b.segs && a.total == b.total &&
          (a.Bout != nullptr || a.Bin != nullptr) == (b.Bout != nullptr || b.Bin != nullptr) &&
          std::memcmp(a.log2g, b.log2g, sizeof a.log2g) == 0;
 }

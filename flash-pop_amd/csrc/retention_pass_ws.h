@@ -36,6 +36,8 @@
 // operands of a phase are requested first, the MFMAs that consume them follow back to back,
 // and the vector work of one phase sits in the shadow of the next phase's MFMAs.
 #pragma once
+#include <type_traits>
+
 #include "pass_args.h"
 #include "lds_access.h"
 
@@ -154,10 +156,13 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
   const bool rev = io.reverse != 0;
   const float lg = p.log2g[h];
 
-  // chunk [t0, t0 + L) that follows position `pos` in walking order; never straddles a block boundary
-  auto chunk_at = [&](int pos, int& t0, int& L) {
+  constexpr bool SEGS = MODE == WALK_PLAIN || MULTI;   // the walks whose sequences may be segments of longer ones
+
+  // chunk [t0, t0 + L) that follows position `pos` in walking order in a sequence of `len` tokens; never straddles a
+  // block boundary
+  auto chunk_at = [&](int pos, int len, int& t0, int& L) {
     if (!rev) {
-      int end = pos + CH < T ? pos + CH : T;
+      int end = pos + CH < len ? pos + CH : len;
       if (bs > 0) {
         const int nbnd = (pos / bs + 1) * bs;
         if (nbnd < end) end = nbnd;
@@ -175,7 +180,7 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     }
   };
   auto next_pos = [&](int t0, int L) { return rev ? t0 : t0 + L; };
-  auto has_more = [&](int pos) { return rev ? pos > 0 : pos < T; };
+  auto has_more = [&](int pos, int len) { return rev ? pos > 0 : pos < len; };
 
   // The walk: all chunks of batch entry `slot`, then of slot + slots, ... Both roles step
   // through the same list.
@@ -187,8 +192,9 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     int part;               // WALK_SUFFIX only: which CH tokens of a suffix longer than a chunk (0 otherwise)
     int h;                  // NH = 2 only: which half of the contraction this visit covers
     uint32_t row;           // index of the item's first row among all rows of its tensor
+    int len;                // tokens of its sequence, where sequences may differ (SEGS)
   };
-  const Chunk no_chunk = {0, 0, 0, false, false, false, false, 0, 0, 0, 0u};
+  const Chunk no_chunk = {0, 0, 0, false, false, false, false, 0, 0, 0, 0u, 0};
   // A suffix of more than CH tokens is walked in parts of CH tokens (the last one shorter), in
   // walking order; between its parts the state moves on as between context chunks, on a copy.
   const int sfx_parts = SFX_ANY ? (p.Ls + CH - 1) / CH : 1;
@@ -216,8 +222,15 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
       } else if (SFX) {   // the suffix at the first boundary met: position 0, or T walking backward
         enter_suffix(ck, rev ? p.nblk : 0, rev ? T : 0, false);
       } else {
-        chunk_at(rev ? T : 0, ck.t0, ck.L);
-        ck.last = !has_more(next_pos(ck.t0, ck.L));
+        const int seg = SEGS && p.segs > 0 ? b % p.segs : 0;
+        const int len = SEGS && p.segs > 0 && p.total - seg * T < T ? p.total - seg * T : T;
+        chunk_at(rev ? len : 0, len, ck.t0, ck.L);
+        ck.last = !has_more(next_pos(ck.t0, ck.L), len);
+        if (SEGS) {
+          ck.len = len;
+          ck.row = (p.segs > 0 ? (uint32_t)(b / p.segs) * p.total + (uint32_t)seg * T : (uint32_t)b * T) + ck.t0;
+          return ck;
+        }
       }
     }
     return with_row(ck);
@@ -265,8 +278,14 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
       }
       return with_row(n);
     }
-    chunk_at(next_pos(ck.t0, ck.L), n.t0, n.L);
-    n.last = !has_more(next_pos(n.t0, n.L));
+    const int len = SEGS ? ck.len : T;
+    chunk_at(next_pos(ck.t0, ck.L), len, n.t0, n.L);
+    n.last = !has_more(next_pos(n.t0, n.L), len);
+    if (SEGS) {
+      n.len = len;
+      n.row = ck.row + (uint32_t)(n.t0 - ck.t0);
+      return n;
+    }
     return with_row(n);
   };
 
@@ -669,21 +688,22 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     }
     fprt::wave_sync();   // the staging area is reused right after
   };
-  // bf16(R) -> global matrix at dst, through stage s
-  auto tile_store = [&](uint16_t* dst, int s, const f32x16 (&racc)[NNW], int hf) {
+  // bf16(R), or with `low` what that leaves of R, -> global matrix at dst, through stage s
+  auto tile_store = [&](uint16_t* dst, int s, const f32x16 (&racc)[NNW], int hf, auto low) {
+    auto part = [](float x) { return decltype(low)::value ? bf16_residual(x) : x; };
     uint16_t* st = RT + s * BV * RT_LD;
 #pragma unroll
     for (int nn = 0; nn < NNW; ++nn) {
       if (!tposed) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          reinterpret_cast<u16_m*>(st)[dl_plain(nn, r)] = float_to_bf16_bits(racc[nn][r]);
+          reinterpret_cast<u16_m*>(st)[dl_plain(nn, r)] = float_to_bf16_bits(part(racc[nn][r]));
       } else {
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
           u32x2 d;
-          d[0] = fprt::pack_bf16x2(racc[nn][4 * qd], racc[nn][4 * qd + 1]);
-          d[1] = fprt::pack_bf16x2(racc[nn][4 * qd + 2], racc[nn][4 * qd + 3]);
+          d[0] = fprt::pack_bf16x2(part(racc[nn][4 * qd]), part(racc[nn][4 * qd + 1]));
+          d[1] = fprt::pack_bf16x2(part(racc[nn][4 * qd + 2]), part(racc[nn][4 * qd + 3]));
           st64(st + dl_tposed(nn, qd), d);
         }
       }
@@ -766,6 +786,10 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     const bool inj = BLOCKS && io.Bin && ends_block(cur.t0 + cur.L);
     tile_load(t_inj, inj ? block_matrix(io.Bin, cur.b, cur.t0 + cur.L) : nullptr, inj, hf);
     if (r0_first) tile_accumulate(t_init, 0, false, racc[hf]);
+    if (SEGS && r0_first && io.R0lo) {
+      tile_load(t_init, state_matrix(io.R0lo, cur.b), true, hf);
+      tile_accumulate(t_init, 0, true, racc[hf]);
+    }
     if (inj) tile_accumulate(t_inj, 0, true, racc[hf]);
   }
   write_rt(0, racc[0]);
@@ -901,17 +925,22 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
 #pragma unroll
       for (int hf = 0; hf < NH; ++hf) {
         if (BLOCKS && io.Bout && ends_block(t1))
-          tile_store(const_cast<uint16_t*>(block_matrix(io.Bout, cur.b, t1)), s ^ 1, racc[hf], hf);
+          tile_store(const_cast<uint16_t*>(block_matrix(io.Bout, cur.b, t1)), s ^ 1, racc[hf], hf, std::false_type{});
         // the state that leaves: after the last item; walking forward with suffixes, the one that the
         // suffix at the last block boundary reads (tokens after that boundary are not in it)
         const bool leaves = (SFX && !rev) ? cur.sfx && cur.n == p.nblk && cur.part == sfx_parts - 1 : cur.last;
-        if (leaves && io.Rout) tile_store(const_cast<uint16_t*>(state_matrix(io.Rout, cur.b)), s ^ 1, racc[hf], hf);
+        if (leaves && io.Rout) tile_store(const_cast<uint16_t*>(state_matrix(io.Rout, cur.b)), s ^ 1, racc[hf], hf, std::false_type{});
+        if (STATE && leaves && io.Rout_lo) tile_store(const_cast<uint16_t*>(state_matrix(io.Rout_lo, cur.b)), s ^ 1, racc[hf], hf, std::true_type{});
       }
     }
     if (nxt.ok) {
       if (MULTI && fresh) {
         if (io.R0) {
           tile_accumulate(t_init, s ^ 1, false, racc[0]);
+          if (io.R0lo) {   // loaded here, once per sequence: held from the start of the visit it costs every visit registers
+            tile_load(t_init, state_matrix(io.R0lo, nxt.b), true, 0);
+            tile_accumulate(t_init, s ^ 1, true, racc[0]);
+          }
         } else {
 #pragma unroll
           for (int nq = 0; nq < NNW; ++nq) racc[0][nq] = f32x16{0};

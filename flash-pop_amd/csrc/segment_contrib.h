@@ -22,6 +22,29 @@ namespace fpk {
 constexpr int sc_lds_bytes() { return 2 * (4 * FB_TILE); }
 static_assert(4 * FB_TILE >= FB_D * FB_LD, "the state copy fits where the tiles were");
 
+// R (accumulator tiles of all waves) -> bf16, through the LDS tile Rt -> its 128 columns of matrix `stream` of dst
+FP_DEVICE void put_contribution(const ContribArgs& p, uint16_t* Rt, uint16_t* dst, int stream, int ct, int tid, int c, int g,
+                                int at_, int nt0, const f32x16 (&racc)[2]) {
+  using namespace fb;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) put_state(Rt, 32 * (nt0 + u) + c, 32 * at_, g, racc[u]);
+  fprt::block_sync();
+  char* const ubase = reinterpret_cast<char*>(dst) + ((size_t)stream * FB_D * p.dB + (size_t)ct * FB_D) * 2;
+  const fprt::BufView uv = fprt::make_buf(ubase, (uint32_t)(FB_D - 1) * p.dB * 2 + FB_D * 2);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int pc = tid + FB_THREADS * u, a = pc >> 4, n8 = (pc & 15) * 8;
+    u32x4 d;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t lo = reinterpret_cast<const u16_m*>(Rt)[at(n8 + 2 * w, a)];
+      const uint32_t hi = reinterpret_cast<const u16_m*>(Rt)[at(n8 + 2 * w + 1, a)];
+      d[w] = lo | (hi << 16);
+    }
+    fprt::buf_store128(uv, (uint32_t)a * p.dB * 2 + n8 * 2, d);
+  }
+}
+
 template <bool REV>
 FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   using namespace fb;
@@ -31,13 +54,18 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   const int streams = p.B * p.H;
   const int ct = fprt::block_index() / streams, stream = fprt::block_index() % streams;
   const int h = stream % p.H, b = stream / p.H;
-  const int nch = p.T / CH;
+  // tokens of this sequence and its first row; a segment that ends inside a chunk is walked from its far end in whole
+  // chunks (forward: the chunk met first, from a zero state, begins before the segment and reads zeros there)
+  const int seg = p.segs > 0 ? b % p.segs : 0;
+  const int len = p.segs > 0 && p.total - seg * p.T < p.T ? p.total - seg * p.T : p.T;
+  const size_t row0 = p.segs > 0 ? (size_t)(b / p.segs) * p.total + (size_t)seg * p.T : (size_t)b * p.T;
+  const int nch = (len + CH - 1) / CH;
   const float lg = p.log2g[h];
   const uint32_t roww = (uint32_t)p.H * FB_D * 2, rowz = (uint32_t)p.H * p.dB * 2;   // bytes between tokens
-  const char* const wbase = reinterpret_cast<const char*>(p.W) + ((size_t)b * p.T * p.H + h) * FB_D * 2;
-  const char* const zbase = reinterpret_cast<const char*>(p.Z) + ((size_t)b * p.T * p.H + h) * p.dB * 2 + (size_t)ct * FB_D * 2;
-  const fprt::BufView wv = fprt::make_buf(wbase, (uint32_t)(p.T - 1) * roww + FB_D * 2);
-  const fprt::BufView zv = fprt::make_buf(zbase, (uint32_t)(p.T - 1) * rowz + FB_D * 2);
+  const char* const wbase = reinterpret_cast<const char*>(p.W) + (row0 * p.H + h) * FB_D * 2;
+  const char* const zbase = reinterpret_cast<const char*>(p.Z) + (row0 * p.H + h) * p.dB * 2 + (size_t)ct * FB_D * 2;
+  const fprt::BufView wv = fprt::make_buf(wbase, (uint32_t)(len - 1) * roww + FB_D * 2);
+  const fprt::BufView zv = fprt::make_buf(zbase, (uint32_t)(len - 1) * rowz + FB_D * 2);
   const fprt::BufView none = fprt::make_buf(wbase, 0u);   // visits beyond the walk read zeros and move nothing
 
   uint16_t* const TL = reinterpret_cast<uint16_t*>(lds);   // stage s: W tile at 2 s, Z tile at 2 s + 1
@@ -46,11 +74,12 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   // registers <- the chunk visited it-th
   auto load = [&](int it, u32x4 (&pf)[4]) {
     const bool live = it < nch;
-    const uint32_t t0 = (uint32_t)(REV ? nch - 1 - it : it) * CH;
+    const int t0 = REV ? (nch - 1 - it) * CH : len - (nch - it) * CH;
     const fprt::BufView w = live ? wv : none, z = live ? zv : none;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const uint32_t row = live ? t0 + ld_row + 32 * u : 0u;
+      const int r = live ? t0 + ld_row + 32 * u : 0;
+      const uint32_t row = r >= 0 ? r : len;   // row `len` is the first one beyond the views
       pf[u] = fprt::buf_load128(w, row * roww + ld_piece * 16);
       pf[2 + u] = fprt::buf_load128(z, row * rowz + ld_piece * 16);
     }
@@ -135,30 +164,23 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     fprt::block_sync();
   }
 
-  // R -> bf16 -> its 128 columns of the rows of U[b][h] (element (a, n) at a * dB + n)
-  uint16_t* const Rt = TL;   // every read of the tiles is behind the last barrier
-#pragma unroll
-  for (int u = 0; u < 2; ++u) put_state(Rt, 32 * (nt0 + u) + c, 32 * at_, g, racc[u]);
+  // R -> its 128 columns of the rows of U[b][h] (element (a, n) at a * dB + n), as bf16 and what that leaves; every read of the tiles is behind the last barrier
+  put_contribution(p, TL, p.U, stream, ct, tid, c, g, at_, nt0, racc);
+  if (!p.U_lo) return;
   fprt::block_sync();
-  char* const ubase = reinterpret_cast<char*>(p.U) + ((size_t)stream * FB_D * p.dB + (size_t)ct * FB_D) * 2;
-  const fprt::BufView uv = fprt::make_buf(ubase, (uint32_t)(FB_D - 1) * p.dB * 2 + FB_D * 2);
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int pc = tid + FB_THREADS * u, a = pc >> 4, n8 = (pc & 15) * 8;
-    u32x4 d;
+  for (int u = 0; u < 2; ++u) {
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const uint32_t lo = reinterpret_cast<const u16_m*>(Rt)[at(n8 + 2 * w, a)];
-      const uint32_t hi = reinterpret_cast<const u16_m*>(Rt)[at(n8 + 2 * w + 1, a)];
-      d[w] = lo | (hi << 16);
-    }
-    fprt::buf_store128(uv, (uint32_t)a * p.dB * 2 + n8 * 2, d);
+    for (int r = 0; r < 16; ++r) racc[u][r] = bf16_residual(racc[u][r]);
   }
+  put_contribution(p, TL, p.U_lo, stream, ct, tid, c, g, at_, nt0, racc);
 }
 
 // Host side: argument check, shared by the GPU launcher and the CPU test harness.
 inline const char* check_contrib(const ContribArgs& a) {
   if (a.B < 1 || a.T < CH || a.T % CH != 0 || a.H < 1 || a.H > MAX_HEADS) return "state-only pass: whole chunks, B, H >= 1 expected";
+  if (a.segs < 0 || (a.segs > 0 && (a.B % a.segs != 0 || a.total > (long long)a.segs * a.T || a.total <= (a.segs - 1LL) * a.T)))
+    return "state-only pass: segments that do not cover their sequence";
   if (a.dB < FB_D || a.dB % FB_D != 0) return "state-only pass: Z must have a multiple of 128 columns";
   if (!a.W || !a.Z || !a.U) return "state-only pass: null pointer";
   if ((long long)a.B * a.H * (a.dB / FB_D) > 0x7fffffffLL) return "state-only pass: too many sequences";

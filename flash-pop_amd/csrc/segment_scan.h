@@ -1,5 +1,8 @@
 // Segment scan (see ScanArgs in pass_args.h): one thread carries SCAN_VEC elements of one
-// (batch, head) state matrix through the S segments in fp32.
+// (batch, head) state matrix through the S segments in fp32.  The chain over the segments is one
+// fma per element; what bounds the launch is the latency of its loads (a state of 64 x 128 has 1024
+// threads, so a few streams are a few dozen waves), and the contributions do not depend on the chain:
+// SCAN_AHEAD of them are requested together.
 #pragma once
 #include "pass_args.h"
 #include "lds_access.h"
@@ -13,7 +16,7 @@ FP_DEVICE void segment_scan(const ScanArgs& p) {
   const int piece = (int)(item % per_mat);
   const int h = (int)((item / per_mat) % p.H);
   const int b = (int)(item / ((long long)per_mat * p.H));
-  const float gseg = fprt::exp2_approx((float)p.Tseg * p.log2g[h]);
+  const float gseg = fprt::exp2_approx((float)p.Tseg * p.log2g[h]), glast = fprt::exp2_approx((float)p.Tlast * p.log2g[h]);
   const size_t in_mat = (size_t)piece * SCAN_VEC;
   float r[SCAN_VEC];
   if (p.R0) {
@@ -24,16 +27,35 @@ FP_DEVICE void segment_scan(const ScanArgs& p) {
 #pragma unroll
     for (int e = 0; e < SCAN_VEC; ++e) r[e] = 0.f;
   }
-  for (int i = 0; i < p.S; ++i) {
-    const int s = p.reverse ? p.S - 1 - i : i;
-    const size_t at = (((size_t)b * p.S + s) * p.H + h) * p.M + in_mat;
-    u32x4 o;
+  auto segment = [&](int i) { return p.reverse ? p.S - 1 - i : i; };
+  auto matrix = [&](int i) { return (((size_t)b * p.S + segment(i)) * p.H + h) * p.M + in_mat; };
+  for (int i0 = 0; i0 < p.S; i0 += SCAN_AHEAD) {
+    u32x4 u[SCAN_AHEAD], ulo[SCAN_AHEAD];
+    // (init may be U: a batch is read before its first element is written)
 #pragma unroll
-    for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = fprt::pack_bf16x2(r[2 * e], r[2 * e + 1]);
-    st128(p.init + at, o);
-    const u32x4 u = ld128(p.U + at);
+    for (int j = 0; j < SCAN_AHEAD; ++j) {
+      ulo[j] = u32x4{0, 0, 0, 0};
+      if (i0 + j < p.S) {
+        u[j] = ld128(p.U + matrix(i0 + j));
+        if (p.U_lo) ulo[j] = ld128(p.U_lo + matrix(i0 + j));
+      }
+    }
 #pragma unroll
-    for (int e = 0; e < SCAN_VEC; ++e) r[e] = gseg * r[e] + bf16_elem(u, e);
+    for (int j = 0; j < SCAN_AHEAD; ++j) {
+      if (i0 + j >= p.S) break;
+      u32x4 o;
+#pragma unroll
+      for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = fprt::pack_bf16x2(r[2 * e], r[2 * e + 1]);
+      st128(p.init + matrix(i0 + j), o);
+      if (p.init_lo) {
+#pragma unroll
+        for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = fprt::pack_bf16x2(bf16_residual(r[2 * e]), bf16_residual(r[2 * e + 1]));
+        st128(p.init_lo + matrix(i0 + j), o);
+      }
+      const float g = segment(i0 + j) == p.S - 1 ? glast : gseg;
+#pragma unroll
+      for (int e = 0; e < SCAN_VEC; ++e) r[e] = g * r[e] + (bf16_elem(u[j], e) + bf16_elem(ulo[j], e));
+    }
   }
   if (p.fin) {
     u32x4 o;

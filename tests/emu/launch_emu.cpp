@@ -70,6 +70,7 @@ int fpk_stream_is_capturing(void* /*stream*/) { return g_emu_capturing; }
 
 // Pretends the chip has 8 compute units, so that small test shapes take the paths that large
 // ones take on a real device (several sequences per workgroup, split sequences).
+int fpk_launch_steps() { return 0; }   // the harness cuts whatever can be cut
 int fpk_compute_units() { return 8; }
 
 // one translation unit per pair of head dimensions (fused_family.cpp)

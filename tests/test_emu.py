@@ -164,6 +164,36 @@ def test_split_sequences_fwd_bwd(emu_lib, B, T, H, dk, dv, state_std, segments):
     assert torch.equal(o2, o) and all(torch.equal(a, b) for a, b in zip(again, (dq, dk_, dv_, ds0)))
 
 
+@pytest.mark.parametrize("B,T,H,dk,dv,state_std,segments", [
+    (1, 257, 1, 64, 64, 0.5, 2),       # the last segment is one token
+    (1, 511, 1, 128, 128, 0.5, 2),     # one token short of two whole segments: the state-only kernel's chunk that begins before its segment
+    (1, 700, 1, 64, 128, None, 3),     # 11 chunks, the last one short, no initial state
+    (1, 704, 1, 64, 64, 0.5, 3),       # 11 whole chunks in segments of 4, 4 and 3
+    (2, 300, 1, 128, 128, 0.5, 1),     # too many streams for the harness's 8 units: not cut
+    (1, 300, 1, 128, 256, 0.3, 2),     # two workgroups per segment in the state-only kernel
+    (1, 330, 1, 256, 64, 0.3, 2),      # the state-only walk visits every chunk twice
+    (2, 330, 1, 64, 64, 0.5, 2),       # rows of the second sequence start inside a chunk
+])
+def test_split_sequences_uneven(emu_lib, B, T, H, dk, dv, state_std, segments):
+    """Sequences that do not fall into equal segments of whole chunks, every segment with a decay strong enough that a
+    state one token off would show."""
+    decays = (0.9,) * H
+    q, k, v, s = hp.make_inputs(B, T, H, dk, dv, seed=T, state_std=state_std)
+    d_o, d_s = hp.make_cotangents([(B, T, H, dv), (B, H, dk, dv)], seed=T + 1)
+    o, S, nbytes, ws = hp.raw_split_fwd(emu_lib, q, k, v, s, decays, keep_workspace=True)
+    assert nbytes == (2 * 2 * B * segments * H * dk * dv if segments > 1 else 0)
+    dq, dk_, dv_, ds0 = hp.raw_split_bwd(emu_lib, q, k, v, s, decays, d_o, d_s, forward_workspace=ws if segments > 1 else None)
+    o_ref, S_ref, (gq, gk, gv, gs) = hp.oracle_plain(q, k, v, s, decays, d_o, d_s)
+    _check_all([("o", o, o_ref), ("S", S, S_ref), ("dq", dq, gq), ("dk", dk_, gk), ("dv", dv_, gv), ("ds0", ds0, gs)])
+    # the states between the segments carry 16 bits more than bf16: not further from the oracle than the uncut call
+    o1, S1 = hp.raw_fwd(emu_lib, q, k, v, s, decays)
+    grads1 = hp.raw_bwd(emu_lib, q, k, v, s, decays, d_o, d_s)
+    for name, got, uncut, ref in zip(("o", "S", "dq", "dk", "dv", "ds0"), (o, S, dq, dk_, dv_, ds0), (o1, S1, *grads1),
+                                     (o_ref, S_ref, gq, gk, gv, gs)):
+        if ref is not None:
+            assert oracle.rms_error_ratio(got.float(), ref) <= 1.05 * oracle.rms_error_ratio(uncut.float(), ref), name
+
+
 @pytest.mark.parametrize("B,nblk,block,Ls,H,state_std,dk,dv", [
     (1, 2, 128, 16, 1, 0.5, 128, 128),     # two chunks per block
     (1, 4, 64, 64, 1, None, 128, 128),     # block == chunk, suffixes as long as a chunk, no initial state
