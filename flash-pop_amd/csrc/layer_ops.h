@@ -12,6 +12,12 @@
 
 namespace fpk {
 
+// Every tensor here passes through once and is larger than the caches where time counts: loads and stores that do not claim
+// room in them.  B8 T4096 H16 128 x 128 (2.15 GB for both stages in both directions): 410 -> 377 us, 5.2 -> 5.7 TB/s; a
+// decode step of one or 256 sequences is as fast either way.
+FP_DEVICE u32x4 ld128_once(const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_m*>(p)); }
+FP_DEVICE void st128_once(uint16_t* p, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4_m*>(p)); }
+
 // ------------------------------------------------------------------------------------------
 // One thread: 8 adjacent features (4 rotation pairs) of one token, for p.heads_per_thread heads of
 // q and k (all of them when there are plenty of tokens: the sines and cosines are then computed
@@ -44,7 +50,7 @@ FP_DEVICE void rotary_qk(const RotaryArgs& p) {
       u32x4 v[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        if (h0 + u < h_end) v[u] = ld128(src + at0 + (size_t)(h0 + u) * p.d);
+        if (h0 + u < h_end) v[u] = ld128_once(src + at0 + (size_t)(h0 + u) * p.d);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
@@ -55,7 +61,7 @@ FP_DEVICE void rotary_qk(const RotaryArgs& p) {
           const float e = bf16_elem(v[u], 2 * j), d = bf16_elem(v[u], 2 * j + 1);
           o[j] = fprt::pack_bf16x2(e * cs[j] - d * sn[j], d * cs[j] + e * sn[j]);
         }
-        st128(dst + at0 + (size_t)(h0 + u) * p.d, o);
+        st128_once(dst + at0 + (size_t)(h0 + u) * p.d, o);
       }
     }
   }
@@ -103,8 +109,8 @@ FP_DEVICE void gated_norm_fwd(const GatedNormArgs& p) {
   const bool live = unit / lanes < p.groups;
   const size_t at = (size_t)unit * 8;
   const u32x4 zero = {0, 0, 0, 0};
-  const u32x4 rv = live ? ld128(p.r + at) : zero;
-  const u32x4 gv = live ? ld128(p.g + at) : zero;
+  const u32x4 rv = live ? ld128_once(p.r + at) : zero;
+  const u32x4 gv = live ? ld128_once(p.g + at) : zero;
   const HeadStats st = head_stats(rv, lanes, p.dv, p.eps);
   float y[8];
 #pragma unroll
@@ -116,7 +122,7 @@ FP_DEVICE void gated_norm_fwd(const GatedNormArgs& p) {
   u32x4 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = fprt::pack_bf16x2(y[2 * e], y[2 * e + 1]);
-  if (live) st128(p.out + at, o);
+  if (live) st128_once(p.out + at, o);
 }
 
 // With n^ = (r - mean) rstd, s = swish(g), dn = d_out * s:
@@ -128,9 +134,9 @@ FP_DEVICE void gated_norm_bwd(const GatedNormArgs& p) {
   const bool live = unit / lanes < p.groups;
   const size_t at = (size_t)unit * 8;
   const u32x4 zero = {0, 0, 0, 0};
-  const u32x4 rv = live ? ld128(p.r + at) : zero;
-  const u32x4 gv = live ? ld128(p.g + at) : zero;
-  const u32x4 dv_ = live ? ld128(p.d_out + at) : zero;
+  const u32x4 rv = live ? ld128_once(p.r + at) : zero;
+  const u32x4 gv = live ? ld128_once(p.g + at) : zero;
+  const u32x4 dv_ = live ? ld128_once(p.d_out + at) : zero;
   const HeadStats st = head_stats(rv, lanes, p.dv, p.eps);
   float nh[8], dn[8], dg[8];
   float s1 = 0.f, s2 = 0.f;
@@ -154,8 +160,8 @@ FP_DEVICE void gated_norm_bwd(const GatedNormArgs& p) {
     o_g[e] = fprt::pack_bf16x2(dg[2 * e], dg[2 * e + 1]);
   }
   if (live) {
-    st128(p.d_r + at, o_r);
-    st128(p.d_g + at, o_g);
+    st128_once(p.d_r + at, o_r);
+    st128_once(p.d_g + at, o_g);
   }
 }
 
