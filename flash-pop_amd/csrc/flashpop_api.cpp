@@ -434,26 +434,45 @@ int plan_segments(const Shape& s) {
 //   64 x 128   H12 B1       18 chunks 53.7 -> 43.4,    13 chunks 41.3 -> 42.3
 //   128 x 128  H16 B1       79 chunks 119 -> 91,       40 chunks 62.4 -> 63.4,  28 chunks 45.6 -> 56.9
 //   128 x 256  H8 B2        28 chunks 121 -> 84,       18 chunks 81.0 -> 78.9
-bool cut_pays(const Shape& s, int n, bool backward) {
+// `block`: a POP call, whose chunks end at its blocks and whose gradient passes share fewer launches (64 x 128, B4 H4 T1440
+// in blocks of 144, 30 chunks, with the suffix call and the launches between the two: 200 -> 166 us).
+bool cut_pays(const Shape& s, int n, int tokens, bool backward, int block = 0) {
   const int launch = fpk_launch_steps();   // what a launch costs, in chunk steps
   if (launch <= 0) return true;
-  const long long chunks = (s.T + fpk::CH - 1LL) / fpk::CH, each = segment_tokens(s, n) / fpk::CH;
+  const long long each = (tokens + fpk::CH - 1) / fpk::CH, chunks = block > 0 ? n * each : (s.T + fpk::CH - 1LL) / fpk::CH;
   const long long streams = (long long)s.B * s.H * n, tk = s.dk / fpk::BV, tv = s.dv / fpk::BV;
   const double matrix = s.dk * s.dv / 16384.;
-  if (!backward) return chunks - each * (1 + waves(streams * tv)) >= launch * (2 + 1.25 * matrix);
+  const long long contrib = waves(streams * (s.dk == fpk::FB_D && s.dv % fpk::FB_D == 0 ? s.dv / fpk::FB_D : tv));
+  if (!backward) return chunks - each * (contrib + waves(streams * tv)) >= launch * (2 + 1.25 * matrix);
   const long long dk_dv = s.dk == s.dv ? waves(2 * streams * tk) : waves(streams * tk) + waves(streams * tv);
-  const long long uncut = use_fused_backward(s, nullptr) ? 7 * chunks / 4 : s.dk == s.dv ? chunks : 2 * chunks;
-  return uncut - each * (1 + waves(streams * tk) + dk_dv) >= launch * (2.5 + 1.75 * matrix);
+  const bool fused = use_fused_backward(s, nullptr) && block % fpk::CH == 0;
+  const long long uncut = fused ? 7 * chunks / 4 : ((s.dk == s.dv ? 1 : 2) + (block > 0 ? 1 : 0)) * chunks;
+  return uncut - each * (contrib + waves(streams * tk) + dk_dv) >= launch * (2.5 + 1.75 * matrix);
 }
 // Forward and backward cut a sequence the same way, so that the states the forward leaves at the start of every segment
 // are the ones the backward's dq pass needs; a backward is cut only if its forward is.
 int plan_forward(const Shape& s) {
   const int n = plan_segments(s);
-  return n > 1 && cut_pays(s, n, false) ? n : 1;
+  return n > 1 && cut_pays(s, n, segment_tokens(s, n), false) ? n : 1;
 }
 int plan_backward(const Shape& s) {
   const int n = plan_forward(s);
-  return n > 1 && cut_pays(s, n, true) ? n : 1;
+  return n > 1 && cut_pays(s, n, segment_tokens(s, n), true) ? n : 1;
+}
+
+// Segments per sequence of a POP call (1: not cut), one per block and one for the tokens after the last block: the scan over
+// the contributions then passes every block state, and the gradients of block states join in it, so that the passes are
+// those of a plain call.  For the streams that a plain call is cut for, and blocks of at least a chunk (a shorter block
+// has more state than tokens to move), where the chain gets shorter by what the cut costs.
+int plan_pop_forward(const Shape& s, int block) {
+  const long long streams = (long long)s.B * s.H * ((s.dk < s.dv ? s.dk : s.dv) / fpk::BV);
+  if (block < fpk::CH || s.T <= block || 3 * streams > fpk_compute_units()) return 1;
+  const int n = segment_count(s, block);
+  return cut_pays(s, n, block, false, block) ? n : 1;
+}
+int plan_pop_backward(const Shape& s, int block) {
+  const int n = plan_pop_forward(s, block);
+  return n > 1 && cut_pays(s, n, block, true, block) ? n : 1;
 }
 
 size_t workspace_bytes(const Shape& s, int segments) {
@@ -475,15 +494,24 @@ Workspace carve(void* workspace, const Shape& s, const Shape& seg) {
   return seg.segs > 0 ? Workspace{base, base, second, second} : Workspace{base, second, nullptr, nullptr};
 }
 
-int scan(const Shape& s, int segments, const double* decays, const Workspace& w, const void* r0, void* fin, int reverse,
-         void* stream) {
+// Block states of a POP call that is cut at its blocks: where the forward's scan leaves them, the gradients that the
+// backward's scan meets
+struct BlockStates {
+  uint16_t* out;
+  const uint16_t* in;
+  int n;
+};
+
+int scan(const Shape& s, const Shape& seg, const double* decays, const Workspace& w, const void* r0, void* fin, int reverse,
+         const BlockStates& blocks, void* stream) {
   fpk::ScanArgs a;
   std::memset(&a, 0, sizeof a);
   a.U = w.contrib; a.R0 = in(r0); a.init = w.start; a.fin = out(fin);
   a.U_lo = w.contrib_lo; a.init_lo = w.start_lo;
-  a.B = s.B; a.S = segments; a.H = s.H; a.M = s.dk * s.dv; a.reverse = reverse;
-  a.Tseg = segment_tokens(s, segments);
-  a.Tlast = s.T - (segments - 1) * a.Tseg;
+  a.blocks_out = blocks.out; a.blocks_in = blocks.in; a.nblk = blocks.n;
+  a.B = s.B; a.S = seg.B / s.B; a.H = s.H; a.M = s.dk * s.dv; a.reverse = reverse;
+  a.Tseg = seg.T;
+  a.Tlast = s.T - (a.S - 1) * seg.T;
   for (int h = 0; h < s.H; ++h) a.log2g[h] = (float)std::log2(decays[h]);
   const char* msg = "";
   if (fpk_launch_scan(a, stream, &msg) != 0) return fail(FP_ERR_LAUNCH, "segment scan: %s", msg);
@@ -495,6 +523,12 @@ Shape segment_shape(const Shape& s, int segments) {
   const int tokens = segment_tokens(s, segments);
   const bool even = (long long)tokens * segments == s.T;
   return Shape{s.B * segments, tokens, s.H, s.dk, s.dv, even ? 0 : segments, even ? 0 : s.T};
+}
+
+// A POP call cut at its blocks: every block, and the tokens after the last one, a segment with both halves of its states.
+Shape block_segments(const Shape& s, int block) {
+  const int segments = segment_count(s, block);
+  return Shape{s.B * segments, block, s.H, s.dk, s.dv, segments, s.T};
 }
 
 // State-only pass: contributions of the segments to S (forward walk over k, v) or to dS
@@ -526,20 +560,18 @@ int contributions(const Shape& seg, const double* decays, const void* w_rows, co
   return run(a, stream, reverse ? "dS contributions" : "S contributions");
 }
 
-int forward_split(const Shape& s, int segments, const void* q, const void* k, const void* v, const void* s0,
-                  const double* decays, void* o, void* s_out, void* workspace, void* stream) {
-  const Shape seg = segment_shape(s, segments);
+int forward_split(const Shape& s, const Shape& seg, const void* q, const void* k, const void* v, const void* s0,
+                  const double* decays, void* o, void* s_out, void* workspace, void* stream, const BlockStates& blocks = {}) {
   const Workspace w = carve(workspace, s, seg);
   int rc;
   if ((rc = contributions(seg, decays, k, v, 0, w, stream)) != FP_OK) return rc;
-  if ((rc = scan(s, segments, decays, w, s0, s_out, 0, stream)) != FP_OK) return rc;
+  if ((rc = scan(s, seg, decays, w, s0, s_out, 0, blocks, stream)) != FP_OK) return rc;
   return forward(seg, q, k, v, w.start, decays, o, nullptr, nullptr, 0, stream, w.start_lo);
 }
 
-int backward_split(const Shape& s, int segments, const void* q, const void* k, const void* v, const void* s0,
+int backward_split(const Shape& s, const Shape& seg, const void* q, const void* k, const void* v, const void* s0,
                    const double* decays, const void* d_o, const void* d_s_out, void* dq, void* dk_, void* dv_,
-                   void* d_s0, void* workspace, bool states_kept, void* stream) {
-  const Shape seg = segment_shape(s, segments);
+                   void* d_s0, void* workspace, bool states_kept, void* stream, const BlockStates& blocks = {}) {
   const Workspace w = carve(workspace, s, seg);
   const float sc = 1.0f / std::sqrt((float)s.dk);
   fpk::PassArgs a;
@@ -548,7 +580,7 @@ int backward_split(const Shape& s, int segments, const void* q, const void* k, c
   // S at the start of every segment (unless the forward's are still there), then dq
   if (!states_kept) {
     if ((rc = contributions(seg, decays, k, v, 0, w, stream)) != FP_OK) return rc;
-    if ((rc = scan(s, segments, decays, w, s0, nullptr, 0, stream)) != FP_OK) return rc;
+    if ((rc = scan(s, seg, decays, w, s0, nullptr, 0, {}, stream)) != FP_OK) return rc;
   }
   fill_common(a, seg, decays);
   a.X = in(d_o); a.W = in(v); a.Z = in(k); a.Y = out(dq);
@@ -560,7 +592,7 @@ int backward_split(const Shape& s, int segments, const void* q, const void* k, c
 
   // dS at the end of every segment (the workspace is free again: the stream orders the passes), then dk and dv
   if ((rc = contributions(seg, decays, q, d_o, 1, w, stream)) != FP_OK) return rc;
-  if ((rc = scan(s, segments, decays, w, d_s_out, d_s0, 1, stream)) != FP_OK) return rc;
+  if ((rc = scan(s, seg, decays, w, d_s_out, d_s0, 1, blocks, stream)) != FP_OK) return rc;
   fill_common(a, seg, decays);
   a.X = in(v); a.W = in(d_o); a.Z = in(q); a.Y = out(dk_);
   a.R0 = w.start; a.R0lo = w.start_lo;
@@ -735,7 +767,7 @@ int fp_retention_fwd_split(const void* q, const void* k, const void* v, const vo
   const int segments = plan_forward(s);
   if (int rc = check_workspace(s, segments, workspace, workspace_bytes_given)) return rc;
   if (segments <= 1) return forward(s, q, k, v, s0, head_decays, o, s_out, nullptr, 0, stream);
-  return forward_split(s, segments, q, k, v, s0, head_decays, o, s_out, workspace, stream);
+  return forward_split(s, segment_shape(s, segments), q, k, v, s0, head_decays, o, s_out, workspace, stream);
 }
 
 int fp_retention_fwd_split_static(const void* q, const void* k, const void* v, const void* s0,
@@ -758,7 +790,7 @@ int fp_retention_fwd_split_static(const void* q, const void* k, const void* v, c
   if (fpk_static_scratch(&scratch_ptr, &msg) != 0) return fail(FP_ERR_LAUNCH, "%s", msg);
   // nothing in the scratch has to start at zero: the state-only pass writes every segment's
   // contribution and the scan every starting state before anything reads them
-  return forward_split(s, segments, q, k, v, s0, head_decays, o, s_out, scratch_ptr, stream);
+  return forward_split(s, segment_shape(s, segments), q, k, v, s0, head_decays, o, s_out, scratch_ptr, stream);
 }
 
 int fp_retention_bwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
@@ -773,7 +805,7 @@ int fp_retention_bwd_split(const void* q, const void* k, const void* v, const vo
   const int segments = plan_backward(s);
   if (int rc = check_workspace(s, segments, workspace, workspace_bytes_given)) return rc;
   if (segments <= 1) return backward(s, q, k, v, s0, head_decays, d_o, d_s_out, nullptr, 0, dq, dk_, dv_, d_s0, stream);
-  return backward_split(s, segments, q, k, v, s0, head_decays, d_o, d_s_out, dq, dk_, dv_, d_s0, workspace,
+  return backward_split(s, segment_shape(s, segments), q, k, v, s0, head_decays, d_o, d_s_out, dq, dk_, dv_, d_s0, workspace,
                         forward_states_kept != 0, stream);
 }
 
@@ -788,6 +820,42 @@ int fp_pop_retention_fwd(const void* q, const void* k, const void* v, const void
   if (!block_states && T / block_size > 0)
     return fail(FP_ERR_NULL_POINTER, "block_states is NULL but T / block_size = %d", T / block_size);
   return forward(s, q, k, v, s0, head_decays, o, nullptr, block_states, block_size, stream);
+}
+
+size_t fp_pop_retention_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size) {
+  const Shape s{B, T, H, dk, dv};
+  if (B < 1 || T < 1 || H < 1 || H > fpk::MAX_HEADS || !dim_ok(dk) || !dim_ok(dv) || block_size < 1) return 0;
+  return workspace_bytes(s, plan_pop_forward(s, block_size));
+}
+
+int fp_pop_retention_fwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
+                               void* o, void* block_states, int B, int T, int H, int dk, int dv, int block_size,
+                               void* workspace, size_t workspace_bytes_given, void* stream) {
+  const Shape s{B, T, H, dk, dv};
+  const int segments = block_size >= 1 && check_shape(s, head_decays) == FP_OK ? plan_pop_forward(s, block_size) : 1;
+  if (segments <= 1)
+    return fp_pop_retention_fwd(q, k, v, s0, head_decays, o, block_states, B, T, H, dk, dv, block_size, stream);
+  if (int rc = check_stream(stream, "fp_pop_retention_fwd_split")) return rc;
+  if (!q || !k || !v || !o || !block_states) return fail(FP_ERR_NULL_POINTER, "q, k, v, o and block_states must not be NULL");
+  if (int rc = check_workspace(s, segments, workspace, workspace_bytes_given)) return rc;
+  return forward_split(s, block_segments(s, block_size), q, k, v, s0, head_decays, o, nullptr, workspace, stream,
+                       BlockStates{out(block_states), nullptr, T / block_size});
+}
+
+int fp_pop_retention_bwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
+                               const void* d_o, const void* d_block_states, void* dq, void* dk_, void* dv_, void* d_s0,
+                               int B, int T, int H, int dk, int dv, int block_size, void* workspace,
+                               size_t workspace_bytes_given, int forward_states_kept, void* stream) {
+  const Shape s{B, T, H, dk, dv};
+  const int segments = block_size >= 1 && check_shape(s, head_decays) == FP_OK ? plan_pop_backward(s, block_size) : 1;
+  if (segments <= 1)
+    return fp_pop_retention_bwd(q, k, v, s0, head_decays, d_o, d_block_states, dq, dk_, dv_, d_s0, B, T, H, dk, dv, block_size, stream);
+  if (int rc = check_stream(stream, "fp_pop_retention_bwd_split")) return rc;
+  if (!q || !k || !v || !d_o || !dq || !dk_ || !dv_)
+    return fail(FP_ERR_NULL_POINTER, "q, k, v, d_o, dq, dk and dv must not be NULL");
+  if (int rc = check_workspace(s, segments, workspace, workspace_bytes_given)) return rc;
+  return backward_split(s, block_segments(s, block_size), q, k, v, s0, head_decays, d_o, nullptr, dq, dk_, dv_, d_s0, workspace,
+                        forward_states_kept != 0, stream, BlockStates{nullptr, in(d_block_states), T / block_size});
 }
 
 int fp_pop_retention_bwd(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,

@@ -100,6 +100,12 @@ struct ScanArgs {
   // carries its state as an uncut one does.  init may be U and init_lo U_lo.
   const uint16_t* U_lo;
   uint16_t* init_lo;
+  // POP: every segment but a shorter last one is a block.  Walking forward the state after block m leaves as
+  // blocks_out[b][m]; walking backward blocks_in[b][m], the gradient of that state, joins before segment m is met.
+  // [B, nblk, H, M], nullable.
+  uint16_t* blocks_out;
+  const uint16_t* blocks_in;
+  int nblk;
   int B, S, H, M, Tseg, reverse;
   int Tlast;             // tokens of the last segment (1 .. Tseg)
   float log2g[MAX_HEADS];
@@ -107,8 +113,7 @@ struct ScanArgs {
 // State-only pass for states of 128 rows (segment_contrib.h): U[b][h] = what sequence b adds to a
 // zero state, sum_j weight(j) W[j]^T Z[j] with weight(j) = s_update gamma^(T - 1 - j) walking forward
 // (`reverse` = 0) and s_update gamma^(j + 1) walking backward.  W [B,T,H,128], Z [B,T,H,dB],
-// U [B,H,128,dB], bf16; T a multiple of CH, dB a multiple of 128.  `segs`, `total` as in PassArgs: only the last
-// segment of a longer sequence may end inside a chunk.
+// U [B,H,128,dB], bf16; dB a multiple of 128.  `segs`, `total` as in PassArgs.
 struct ContribArgs {
   const uint16_t* W;
   const uint16_t* Z;

@@ -28,22 +28,26 @@ FP_DEVICE void segment_scan(const ScanArgs& p) {
     for (int e = 0; e < SCAN_VEC; ++e) r[e] = 0.f;
   }
   auto segment = [&](int i) { return p.reverse ? p.S - 1 - i : i; };
+  auto block = [&](int m) { return (((size_t)b * p.nblk + m) * p.H + h) * p.M + in_mat; };
   auto matrix = [&](int i) { return (((size_t)b * p.S + segment(i)) * p.H + h) * p.M + in_mat; };
   for (int i0 = 0; i0 < p.S; i0 += SCAN_AHEAD) {
-    u32x4 u[SCAN_AHEAD], ulo[SCAN_AHEAD];
+    u32x4 u[SCAN_AHEAD], ulo[SCAN_AHEAD], add[SCAN_AHEAD];
     // (init may be U: a batch is read before its first element is written)
 #pragma unroll
     for (int j = 0; j < SCAN_AHEAD; ++j) {
-      ulo[j] = u32x4{0, 0, 0, 0};
+      ulo[j] = add[j] = u32x4{0, 0, 0, 0};
       if (i0 + j < p.S) {
         u[j] = ld128(p.U + matrix(i0 + j));
         if (p.U_lo) ulo[j] = ld128(p.U_lo + matrix(i0 + j));
+        if (p.blocks_in && segment(i0 + j) < p.nblk) add[j] = ld128(p.blocks_in + block(segment(i0 + j)));
       }
     }
 #pragma unroll
     for (int j = 0; j < SCAN_AHEAD; ++j) {
       if (i0 + j >= p.S) break;
       u32x4 o;
+#pragma unroll
+      for (int e = 0; e < SCAN_VEC; ++e) r[e] += bf16_elem(add[j], e);
 #pragma unroll
       for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = fprt::pack_bf16x2(r[2 * e], r[2 * e + 1]);
       st128(p.init + matrix(i0 + j), o);
@@ -55,6 +59,11 @@ FP_DEVICE void segment_scan(const ScanArgs& p) {
       const float g = segment(i0 + j) == p.S - 1 ? glast : gseg;
 #pragma unroll
       for (int e = 0; e < SCAN_VEC; ++e) r[e] = g * r[e] + (bf16_elem(u[j], e) + bf16_elem(ulo[j], e));
+      if (p.blocks_out && segment(i0 + j) < p.nblk) {
+#pragma unroll
+        for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = fprt::pack_bf16x2(r[2 * e], r[2 * e + 1]);
+        st128(p.blocks_out + block(segment(i0 + j)), o);
+      }
     }
   }
   if (p.fin) {

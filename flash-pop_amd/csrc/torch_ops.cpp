@@ -95,11 +95,18 @@ void retention_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
 }
 
 void pop_retention_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& s, const Decays& g, int block,
-                       const Shape& n, Tensor& o, Tensor& states) {
+                       const Shape& n, bool for_backward, Tensor& o, Tensor& states, Kept& kept) {
   c10::DeviceGuard guard(q.device());
   refuse_capture("pop_retention_fwd");
   o = values_like(q, n);
   states = at::empty({n.B, n.T / block, n.H, n.dk, n.dv}, q.options());
+  if (const size_t bytes = fp_pop_retention_workspace_bytes(n.B, n.T, n.H, n.dk, n.dv, block)) {
+    Tensor ws = bytes_like(bytes, q);
+    check(fp_pop_retention_fwd_split(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(o), ptr(states), n.B, n.T, n.H, n.dk, n.dv, block,
+                                     ptr(ws), bytes, stream()));
+    if (for_backward) kept.t = ws;
+    return;
+  }
   check(fp_pop_retention_fwd(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(o), states.numel() ? ptr(states) : nullptr, n.B, n.T,
                              n.H, n.dk, n.dv, block, stream()));
 }
@@ -116,9 +123,18 @@ Grads retention_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Ten
   refuse_capture("retention_bwd");
   Grads r{at::empty_like(q), at::empty_like(k), at::empty_like(v), want_ds0 ? state_like(q, n) : Tensor()};
   if (block > 0) {
-    check(fp_pop_retention_bwd(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(d_o),
-                               d_blocks.defined() && d_blocks.numel() ? ptr(d_blocks) : nullptr, ptr(r.dq), ptr(r.dk), ptr(r.dv),
-                               ptr(r.ds0), n.B, n.T, n.H, n.dk, n.dv, block, stream()));
+    const void* const d_states = d_blocks.defined() && d_blocks.numel() ? ptr(d_blocks) : nullptr;
+    Tensor ws = kept.t;
+    if (!ws.defined()) {
+      if (const size_t bytes = fp_pop_retention_workspace_bytes(n.B, n.T, n.H, n.dk, n.dv, block)) ws = bytes_like(bytes, q);
+    }
+    if (ws.defined())
+      check(fp_pop_retention_bwd_split(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(d_o), d_states, ptr(r.dq), ptr(r.dk), ptr(r.dv),
+                                       ptr(r.ds0), n.B, n.T, n.H, n.dk, n.dv, block, ptr(ws), (size_t)ws.numel(),
+                                       kept.t.defined() && states_kept, stream()));
+    else
+      check(fp_pop_retention_bwd(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(d_o), d_states, ptr(r.dq), ptr(r.dk), ptr(r.dv),
+                                 ptr(r.ds0), n.B, n.T, n.H, n.dk, n.dv, block, stream()));
     return r;
   }
   if (kept.t.defined() && kept.every > 0) {
@@ -252,13 +268,21 @@ struct PlainBackward : public RetentionNode {
 
 struct PopBackward : public RetentionNode {
   int block = 0;
+  Kept kept;
+  bool spent = false;   // as in PlainBackward
   std::string name() const override { return "FlashPOPRetentionBackward"; }
+  void release_variables() override {
+    RetentionNode::release_variables();
+    std::lock_guard<std::mutex> lock(mutex);
+    kept.t.reset();
+  }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex);
     at::AutoGradMode no_grad(false);
     const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), s_ = s.unpack();
     const Tensor d_o = incoming(grads[0], {n.B, n.T, n.H, n.dv}, q_), d_b = incoming(grads[1], {}, q_);
-    Grads r = retention_bwd(q_, k_, v_, s_, decays, n, d_o, Tensor(), d_b, block, s_.defined() && task_should_compute_output(3), Kept{}, false);
+    Grads r = retention_bwd(q_, k_, v_, s_, decays, n, d_o, Tensor(), d_b, block, s_.defined() && task_should_compute_output(3), kept, !spent);
+    spent = spent || kept.t.defined();
     return {r.dq, r.dk, r.dv, r.ds0};
   }
 };
@@ -468,6 +492,7 @@ PyObject* py_flash_pop_retention(PyObject*, PyObject* const* a, Py_ssize_t nargs
   HANDLE_TH_ERRORS
   if (!count(nargs, 6)) return nullptr;
   Tensor q, k, v, s, o, states;
+  Kept kept;
   Decays g;
   Shape n;
   const int64_t block = as_int(a[5]);
@@ -477,12 +502,13 @@ PyObject* py_flash_pop_retention(PyObject*, PyObject* const* a, Py_ssize_t nargs
     const bool grad = differentiates(q, k, v, s);
     {
       at::AutoGradMode no_grad(false);
-      pop_retention_fwd(q, k, v, s, g, (int)block, n, o, states);
+      pop_retention_fwd(q, k, v, s, g, (int)block, n, grad, o, states, kept);
     }
     if (grad) {
       auto node = make_node<PopBackward>(q, k, v, s);
       node->save(q, k, v, s, std::move(g), n);
       node->block = (int)block;
+      node->kept = std::move(kept);
       torch::autograd::set_history(o, node);
       torch::autograd::set_history(states, node);
     }

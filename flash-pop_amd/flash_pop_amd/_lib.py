@@ -27,6 +27,9 @@ SIGNATURES = {
     "fp_retention_bwd_split": [_P, _P, _P, _P, _D, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _Z, _I, _P],
     "fp_pop_retention_fwd": [_P, _P, _P, _P, _D, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "fp_pop_retention_bwd": [_P, _P, _P, _P, _D, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
+    "fp_pop_retention_workspace_bytes": [_I, _I, _I, _I, _I, _I],
+    "fp_pop_retention_fwd_split": [_P, _P, _P, _P, _D, _P, _P, _I, _I, _I, _I, _I, _I, _P, _Z, _P],
+    "fp_pop_retention_bwd_split": [_P, _P, _P, _P, _D, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _Z, _I, _P],
     "fp_pop_fused_fwd": [_P] * 7 + [_D] + [_P] * 3 + [_I] * 7 + [_P],
     "fp_pop_fused_bwd": [_P] * 7 + [_D] + [_P] * 10 + [_I] * 7 + [_P],
     "fp_retention_decode_step": [_P, _P, _P, _P, _D, _P, _P, _I, _I, _I, _I, _P],
@@ -49,7 +52,7 @@ def bind(path: str) -> ctypes.CDLL:
         fn = getattr(lib, name)          # AttributeError if the symbol is missing
         fn.argtypes = argtypes
         fn.restype = {"fp_last_error": c_char_p, "fp_retention_workspace_bytes": c_size_t,
-                      "fp_retention_checkpoint_bytes": c_size_t}.get(name, c_int)
+                      "fp_pop_retention_workspace_bytes": c_size_t, "fp_retention_checkpoint_bytes": c_size_t}.get(name, c_int)
     return lib
 
 

@@ -119,6 +119,18 @@ int fp_retention_fwd_split_static(const void* q, const void* k, const void* v, c
                                   const double* head_decays, void* o, void* s_out, int B, int T, int H, int dk, int dv,
                                   void* stream);
 
+/* The POP entry points below for few streams and long sequences, cut at the blocks the way fp_retention_*_split cuts at
+ * segments of its own choice; workspace and forward_states_kept as there.  0 bytes: the shape is not cut, and the calls are
+ * fp_pop_retention_fwd / _bwd. */
+size_t fp_pop_retention_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size);
+int fp_pop_retention_fwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
+                               void* o, void* block_states, int B, int T, int H, int dk, int dv, int block_size,
+                               void* workspace, size_t workspace_bytes, void* stream);
+int fp_pop_retention_bwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
+                               const void* d_o, const void* d_block_states, void* dq, void* dk_, void* dv_, void* d_s0,
+                               int B, int T, int H, int dk, int dv, int block_size, void* workspace,
+                               size_t workspace_bytes, int forward_states_kept, void* stream);
+
 /* Replaces the kernel call in FlashPOPRetention.forward
  * (flash_pop/pop_retention/__init__.py:14-31).
  *   block_states  out: state after every FULL block of block_size tokens,

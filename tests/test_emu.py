@@ -194,6 +194,45 @@ def test_split_sequences_uneven(emu_lib, B, T, H, dk, dv, state_std, segments):
             assert oracle.rms_error_ratio(got.float(), ref) <= 1.05 * oracle.rms_error_ratio(uncut.float(), ref), name
 
 
+@pytest.mark.parametrize("B,T,H,dk,dv,block,state_std,segments", [
+    (1, 256, 1, 128, 128, 64, 0.5, 4),     # whole chunks per block, the sequence ends on a boundary
+    (1, 287, 1, 64, 128, 144, 0.5, 2),     # blocks that end inside a chunk, tokens after the last one
+    (2, 211, 1, 64, 64, 70, None, 4),      # one token after the last block, no initial state, two sequences
+    (1, 200, 1, 128, 64, 100, 0.3, 2),
+    (1, 150, 1, 256, 64, 65, 0.3, 3),      # the state-only walk visits every chunk twice
+    (1, 200, 1, 64, 64, 32, 0.5, 1),       # blocks shorter than a chunk: not cut
+    (1, 64, 1, 64, 64, 64, 0.5, 1),        # a single block
+])
+def test_pop_split_at_blocks(emu_lib, B, T, H, dk, dv, block, state_std, segments):
+    decays = (0.97,) * H
+    q, k, v, s = hp.make_inputs(B, T, H, dk, dv, seed=T + block, state_std=state_std)
+    d_o, d_b = hp.make_cotangents([(B, T, H, dv), (B, T // block, H, dk, dv)], seed=T)
+    nbytes = emu_lib.fp_pop_retention_workspace_bytes(B, T, H, dk, dv, block)
+    assert nbytes == (2 * 2 * B * segments * H * dk * dv if segments > 1 else 0)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8)
+    p, dec = hp._p, hp._dec(decays)
+    nan = lambda *shape: torch.full(shape, float("nan"), dtype=hp.BF16)
+    o, states = nan(B, T, H, dv), nan(B, T // block, H, dk, dv)
+    assert emu_lib.fp_pop_retention_fwd_split(p(q), p(k), p(v), p(s), dec, p(o), p(states), B, T, H, dk, dv, block, p(ws), nbytes, None) == 0
+    o_ref, st_ref, refs = hp.oracle_pop(q, k, v, s, decays, block, d_o, d_b)
+    o1, states1 = hp.raw_pop_fwd(emu_lib, q, k, v, s, decays, block)
+    grads1 = hp.raw_pop_bwd(emu_lib, q, k, v, s, decays, block, d_o, d_b)
+    for kept in (1, 0):   # from the states that the forward left, and from recomputed ones
+        grads = [nan(*q.shape), nan(*k.shape), nan(*v.shape), nan(B, H, dk, dv)]
+        assert emu_lib.fp_pop_retention_bwd_split(p(q), p(k), p(v), p(s), dec, p(d_o), p(d_b), *[p(g) for g in grads], B, T, H, dk, dv,
+                                                  block, p(ws), nbytes, kept, None) == 0
+        names, got, uncut = ("o", "states", "dq", "dk", "dv", "ds0"), (o, states, *grads), (o1, states1, *grads1)
+        for name, g, u, ref in zip(names, got, uncut, (o_ref, st_ref, *refs)):
+            if ref is None:
+                continue
+            hp.assert_close(g, ref, name)
+            # both halves of the states between the blocks: not further from the oracle than the uncut call
+            assert oracle.rms_error_ratio(g.float(), ref) <= 1.05 * oracle.rms_error_ratio(u.float(), ref), name
+    if nbytes:   # argument checks come before any launch
+        rc = lambda w, n: emu_lib.fp_pop_retention_fwd_split(p(q), p(k), p(v), p(s), dec, p(o), p(states), B, T, H, dk, dv, block, w, n, None)
+        assert rc(None, 0) == -1 and rc(p(ws), nbytes - 16) == -2
+
+
 @pytest.mark.parametrize("B,nblk,block,Ls,H,state_std,dk,dv", [
     (1, 2, 128, 16, 1, 0.5, 128, 128),     # two chunks per block
     (1, 4, 64, 64, 1, None, 128, 128),     # block == chunk, suffixes as long as a chunk, no initial state
