@@ -22,6 +22,8 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 
+#include <algorithm>
+#include <initializer_list>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -244,20 +246,31 @@ struct RetentionNode : public torch::autograd::Node {
   }
 };
 
-struct PlainBackward : public RetentionNode {
-  Kept kept;
-  bool spent = false;   // the kept workspace has been overwritten by a backward
-  std::string name() const override { return "FusedChunkRetentionBackward"; }
+// What a forward left (Kept) goes through SavedVariable like the inputs, so that saved-tensor hooks see all that a node holds.
+struct KeepingNode : public RetentionNode {
+  SavedVariable kept_tensor;
+  int every = 0;
+
+  void keep(const Kept& kept) {
+    kept_tensor = SavedVariable(kept.t, false);
+    every = kept.every;
+  }
   void release_variables() override {
     RetentionNode::release_variables();
     std::lock_guard<std::mutex> lock(mutex);
-    kept.t.reset();
+    kept_tensor.reset_data();
   }
+};
+
+struct PlainBackward : public KeepingNode {
+  bool spent = false;   // the kept workspace has been overwritten by a backward
+  std::string name() const override { return "FusedChunkRetentionBackward"; }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex);
     at::AutoGradMode no_grad(false);
     const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), s_ = s.unpack();
     const Tensor d_o = incoming(grads[0], {n.B, n.T, n.H, n.dv}, q_), d_s = incoming(grads[1], {}, q_);
+    const Kept kept{kept_tensor.unpack(), every};
     // a forward that cut its sequences leaves its workspace: the first backward starts from the states in it and overwrites them,
     // a second one (retain_graph) recomputes them
     Grads r = retention_bwd(q_, k_, v_, s_, decays, n, d_o, d_s, Tensor(), 0, s_.defined() && task_should_compute_output(3), kept, !spent);
@@ -266,21 +279,16 @@ struct PlainBackward : public RetentionNode {
   }
 };
 
-struct PopBackward : public RetentionNode {
+struct PopBackward : public KeepingNode {
   int block = 0;
-  Kept kept;
   bool spent = false;   // as in PlainBackward
   std::string name() const override { return "FlashPOPRetentionBackward"; }
-  void release_variables() override {
-    RetentionNode::release_variables();
-    std::lock_guard<std::mutex> lock(mutex);
-    kept.t.reset();
-  }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex);
     at::AutoGradMode no_grad(false);
     const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), s_ = s.unpack();
     const Tensor d_o = incoming(grads[0], {n.B, n.T, n.H, n.dv}, q_), d_b = incoming(grads[1], {}, q_);
+    const Kept kept{kept_tensor.unpack(), 0};
     Grads r = retention_bwd(q_, k_, v_, s_, decays, n, d_o, Tensor(), d_b, block, s_.defined() && task_should_compute_output(3), kept, !spent);
     spent = spent || kept.t.defined();
     return {r.dq, r.dk, r.dv, r.ds0};
@@ -401,6 +409,15 @@ int64_t as_int(PyObject* o) {
 }
 int64_t as_index(PyObject* o) { return PyLong_CheckExact(o) ? PyLong_AsLongLong(o) : as_int(o); }
 
+// The ops have no forward-mode rule: a call with a tangent is refused, as an autograd Function without a jvp refuses it.
+void refuse_tangents(std::initializer_list<const Tensor*> inputs) {
+  for (const Tensor* t : inputs)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), "flash_pop_amd's ops do not support forward mode AD");
+}
+
+// a block size as the C ABI takes it, whose sums stay below 2^31; any size beyond the sequence means no block
+int64_t as_block(PyObject* o) { return std::min<int64_t>(as_int(o), 1 << 30); }
+
 bool is_bf16(const Tensor& t) { return !t.defined() || (t.scalar_type() == at::kBFloat16 && t.is_cuda()); }
 
 // q, k [B,T,H,dk], v [B,T,H,dv], s [B,H,dk,dv] or none, H decays: what _ops.prepare asks for; makes them contiguous
@@ -412,6 +429,7 @@ bool retention_args(PyObject* const* a, Tensor& q, Tensor& k, Tensor& v, Tensor&
   n = Shape{(int)q.size(0), (int)q.size(1), (int)q.size(2), (int)q.size(3), (int)v.size(3)};
   if ((int64_t)g.size() != n.H || !is_bf16(q) || !is_bf16(k) || !is_bf16(v) || !is_bf16(s)) return false;
   if (s.defined() && !s.sizes().equals({n.B, n.H, n.dk, n.dv})) return false;
+  refuse_tangents({&q, &k, &v, &s});
   q = q.contiguous();
   k = k.contiguous();
   v = v.contiguous();
@@ -426,6 +444,7 @@ bool suffix_args(PyObject* const* a, const Shape& n, int block, Suffixes& x) {
     return false;
   if (x.q.size(0) != (int64_t)n.B * (n.T / block + 1) || x.q.size(2) != n.H || x.q.size(3) != n.dk || x.v.size(3) != n.dv) return false;
   if (!is_bf16(x.q) || !is_bf16(x.k) || !is_bf16(x.v)) return false;
+  refuse_tangents({&x.q, &x.k, &x.v});
   x = Suffixes{x.q.contiguous(), x.k.contiguous(), x.v.contiguous()};
   return true;
 }
@@ -478,7 +497,7 @@ PyObject* py_fused_chunk_retention(PyObject*, PyObject* const* a, Py_ssize_t nar
     if (grad) {
       auto node = make_node<PlainBackward>(q, k, v, s);
       node->save(q, k, v, s, std::move(g), n);
-      node->kept = std::move(kept);
+      node->keep(kept);
       torch::autograd::set_history(o, node);
       torch::autograd::set_history(s_out, node);
     }
@@ -495,7 +514,7 @@ PyObject* py_flash_pop_retention(PyObject*, PyObject* const* a, Py_ssize_t nargs
   Kept kept;
   Decays g;
   Shape n;
-  const int64_t block = as_int(a[5]);
+  const int64_t block = as_block(a[5]);
   if (block < 1 || !retention_args(a, q, k, v, s, g, n)) return not_implemented();
   {
     NoGil free;
@@ -508,7 +527,7 @@ PyObject* py_flash_pop_retention(PyObject*, PyObject* const* a, Py_ssize_t nargs
       auto node = make_node<PopBackward>(q, k, v, s);
       node->save(q, k, v, s, std::move(g), n);
       node->block = (int)block;
-      node->kept = std::move(kept);
+      node->keep(kept);
       torch::autograd::set_history(o, node);
       torch::autograd::set_history(states, node);
     }
@@ -525,7 +544,7 @@ PyObject* py_pop_with_suffixes(PyObject*, PyObject* const* a, Py_ssize_t nargs) 
   Suffixes x;
   Decays g;
   Shape n;
-  const int64_t block = as_int(a[5]);
+  const int64_t block = as_block(a[5]);
   if (block < 1 || !retention_args(a, q, k, v, s, g, n) || !suffix_args(a + 6, n, (int)block, x)) return not_implemented();
   {
     NoGil free;
@@ -602,6 +621,7 @@ PyObject* py_rotary_qk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   }
   const int inverse = PyObject_IsTrue(a[4]);
   if (inverse < 0) throw python_error();
+  refuse_tangents({&q, &k});
   {
     NoGil free;
     q = q.contiguous();
@@ -636,6 +656,7 @@ PyObject* py_gated_group_norm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (r.dim() < 2 || g.dim() < 1 || g.numel() != r.numel() || g.size(-1) != r.size(-2) * r.size(-1)) return not_implemented();
   const double eps = PyFloat_AsDouble(a[2]);
   if (eps == -1.0 && PyErr_Occurred()) throw python_error();
+  refuse_tangents({&r, &g});
   {
     NoGil free;
     r = r.contiguous();

@@ -56,6 +56,31 @@ def test_no_grad_in_place_changes_and_reuse():
     assert torch.autograd.grad(gated_group_norm(q, gate).sum(), q)[0].shape == q.shape
 
 
+def test_saved_tensor_hooks_see_all_and_tangents_are_refused():
+    from flash_pop_amd import XPos, flash_pop_retention, fused_chunk_retention, gated_group_norm
+    decays = oracle.head_decays(2)
+    q, k, v, s = hp.make_inputs(1, 1600, 2, 64, 64, seed=8, state_std=0.3, device=DEV)
+    q.requires_grad_()
+    for op, args in ((fused_chunk_retention, ()), (flash_pop_retention, (160,))):     # both cut into segments
+        ref = torch.autograd.grad(op(q, k, v, s, decays, *args)[0].sum(), q)[0]
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.numel()) or t.cpu(), lambda t: t.to(DEV)):
+            o, _ = op(q, k, v, s, decays, *args)
+        assert len(packed) == 5                                                       # q, k, v, s and the segment states
+        for _ in range(2):
+            assert torch.equal(torch.autograd.grad(o.sum(), q, retain_graph=True)[0], ref)
+    # (a block beyond the sequence is no block, however large)
+    assert flash_pop_retention(q, k, v, s, decays, 2 ** 32)[1].shape[1] == 0
+    import torch.autograd.forward_ad as fwd
+    q = q.detach()
+    with fwd.dual_level():
+        dual = fwd.make_dual(q, torch.ones_like(q))
+        for call in (lambda: fused_chunk_retention(dual, k, v, s, decays), lambda: flash_pop_retention(dual, k, v, s, decays, 64),
+                     lambda: XPos(64)(dual, k, 0), lambda: gated_group_norm(dual, q.flatten(2))):
+            with pytest.raises(NotImplementedError, match="forward mode"):
+                call()
+
+
 def test_threads_with_streams_of_their_own():
     from flash_pop_amd import fused_chunk_retention
     decays = oracle.head_decays(4)
