@@ -432,7 +432,8 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* stream, const char** err
 }
 
 int fpk_launch_scan(const fpk::ScanArgs& a, void* stream, const char** err) {
-  if (a.M % fpk::SCAN_VEC != 0 || a.B < 1 || a.S < 1 || a.H < 1 || !a.U || !a.init) {
+  if (a.M % fpk::SCAN_VEC != 0 || a.B < 1 || a.S < 1 || a.H < 1 || !a.U || !a.init || !a.U_lo != !a.init_lo ||
+      (!a.U_lo && (a.blocks_in || a.blocks_out))) {
     *err = "segment scan: bad arguments";
     return 1;
   }
