@@ -395,8 +395,9 @@ int backward(const Shape& s, const void* q, const void* k, const void* v, const 
 //   1. a state-only pass gives the state each segment contributes on its own,
 //   2. a scan over the S contributions gives the state at the start of every segment,
 //   3. the ordinary pass runs on B * S sequences from those states.
-// The backward does the same for S (needed by the dq pass; recomputed, not stored) and, walking
-// backward, for dS.  Segment states pass through bf16 like POP block states do.
+// The backward does the same for S (needed by the dq pass; the forward's, or recomputed) and, walking
+// backward, for dS.  The states of equal segments pass through bf16 like POP block states do, those of uneven ones and of
+// POP blocks stay fp32 (Workspace).
 
 // Tokens per segment for at most `target` segments (or segments of kMinChunks, the shortest worth a workgroup).
 constexpr int kMinChunks = 4;
@@ -482,9 +483,9 @@ size_t workspace_bytes(const Shape& s, int segments) {
 struct Workspace {
   uint16_t* contrib;      // [B, S, H, dk, dv]: what each segment adds on its own
   uint16_t* start;        // [B, S, H, dk, dv]: state at the segment's first token (last, walking backward)
-  // What bf16 leaves of the two (PassArgs::R0lo), nullptr: they are bf16 alone.  The scan then works in place, so the
-  // bytes are the same either way.  Equal segments keep bf16 states (those of a POP caller's blocks are bf16 too, and at
-  // B2 H8 T16384 128 x 256 the halves would be 5 % more traffic); sequences that are cut unevenly keep both halves.
+  // The lower halves of the two where they are fp32 (PassArgs::R0lo), nullptr: they are bf16.  With them the scan works in
+  // place, so the bytes are the same either way.  Equal segments keep bf16 states (at B2 H8 T16384 128 x 256 fp32 ones would
+  // be 5 % more traffic); where a sequence is cut unevenly or at its blocks the states stay fp32, as one walk carries them.
   uint16_t *contrib_lo, *start_lo;
 };
 
@@ -525,7 +526,7 @@ Shape segment_shape(const Shape& s, int segments) {
   return Shape{s.B * segments, tokens, s.H, s.dk, s.dv, even ? 0 : segments, even ? 0 : s.T};
 }
 
-// A POP call cut at its blocks: every block, and the tokens after the last one, a segment with both halves of its states.
+// A POP call cut at its blocks: every block, and the tokens after the last one, a segment with fp32 states.
 Shape block_segments(const Shape& s, int block) {
   const int segments = segment_count(s, block);
   return Shape{s.B * segments, block, s.H, s.dk, s.dv, segments, s.T};

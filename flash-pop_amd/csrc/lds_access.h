@@ -26,11 +26,22 @@ FP_DEVICE float bf16_elem(u32x4 v, int e) {
   return __builtin_bit_cast(float, (e & 1) ? (d & 0xffff0000u) : (d << 16));
 }
 FP_DEVICE uint16_t float_to_bf16_bits(float x) { return (uint16_t)(fprt::pack_bf16x2(x, 0.f) & 0xffffu); }
-// What rounding x to bf16 leaves of it: bf16(x) + bf16(residual) is x to 2^-17.  0 where x or bf16(x) is not finite, so that
-// the sum of the two is bf16(x) there.
-FP_DEVICE float bf16_residual(float x) {
-  const float d = x - bf16_bits_to_float(float_to_bf16_bits(x));
-  return __builtin_fabsf(d) < __builtin_inff() ? d : 0.f;
+// A float as it is stored 16 bits at a time: rounded to bf16, or, where a matrix keeps its fp32 values in two planes of 16
+// bits, the upper or the lower half of its bits.
+struct AsBf16 {};
+struct UpperHalf {};
+struct LowerHalf {};
+FP_DEVICE uint32_t pack16(float lo, float hi, AsBf16) { return fprt::pack_bf16x2(lo, hi); }
+FP_DEVICE uint32_t pack16(float lo, float hi, UpperHalf) {
+  return (__builtin_bit_cast(uint32_t, lo) >> 16) | (__builtin_bit_cast(uint32_t, hi) & 0xffff0000u);
+}
+FP_DEVICE uint32_t pack16(float lo, float hi, LowerHalf) {
+  return (__builtin_bit_cast(uint32_t, lo) & 0xffffu) | (__builtin_bit_cast(uint32_t, hi) << 16);
+}
+// the float whose halves are element e of `upper` and of `lower`
+FP_DEVICE float joined_elem(u32x4 upper, u32x4 lower, int e) {
+  const uint32_t u = upper[e >> 1], l = lower[e >> 1];
+  return __builtin_bit_cast(float, (e & 1) ? (u & 0xffff0000u) | (l >> 16) : (u << 16) | (l & 0xffffu));
 }
 
 // row of the 32x32 MFMA accumulator held in element r by a lane of half-wave g

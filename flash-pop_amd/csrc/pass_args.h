@@ -31,8 +31,9 @@ struct PassArgs {
   uint16_t* Y;
   const uint16_t* R0;    // initial R per (b, h), nullable (zeros)
   uint16_t* Rout;        // final R per (b, h), nullable
-  // What bf16 leaves of the two above, as bf16 again (nullable; only for the walks without block states and suffixes):
-  // R = R0 + R0lo, Rout + Rout_lo = R to 2^-17, for states that one launch hands to the next as if it had carried them.
+  // Where given, the two above are not bf16: the matrices are fp32, the upper 16 bits of each element in R0 (Rout), the lower
+  // 16 in these (only for the walks without block states and suffixes).  States that one launch hands to the next are the
+  // ones it carried.
   const uint16_t* R0lo;
   uint16_t* Rout_lo;
   uint16_t* Bout;        // R after every full block, [B, nblk, H, dk*dv], nullable (forward only)
@@ -90,14 +91,14 @@ constexpr int MAX_PASSES_PER_LAUNCH = 3;
 //   init[b][0] = R0[b] (zeros if null),  init[b][s] = g_(s-1) init[b][s-1] + U[b][s-1],
 //   fin[b] = g_(S-1) init[b][S-1] + U[b][S-1]
 // `reverse` runs the same recurrence from the last segment to the first (state gradients).
-// All matrices are bf16, M = dk * dv elements each, laid out [B, S, H, M] (U, init) and [B, H, M].
+// All matrices are bf16 (but see U_lo), M = dk * dv elements each, laid out [B, S, H, M] (U, init) and [B, H, M].
 struct ScanArgs {
   const uint16_t* U;
   const uint16_t* R0;   // nullable
   uint16_t* init;
   uint16_t* fin;        // nullable
-  // Low halves of U and init (both or neither): matrices are then hi + lo, exact to 2^-17, so that a cut sequence
-  // carries its state as an uncut one does.  init may be U and init_lo U_lo.
+  // Given (both or neither): U and init are fp32 matrices, the upper 16 bits of each element in U (init), the lower 16 here
+  // (PassArgs::R0lo), so that a cut sequence carries its state in fp32 as an uncut one does.  init may be U and init_lo U_lo.
   const uint16_t* U_lo;
   uint16_t* init_lo;
   // POP: every segment but a shorter last one is a block.  Walking forward the state after block m leaves as
@@ -118,7 +119,7 @@ struct ContribArgs {
   const uint16_t* W;
   const uint16_t* Z;
   uint16_t* U;
-  uint16_t* U_lo;        // low half of U (see PassArgs::Rout_lo), nullable
+  uint16_t* U_lo;        // the lower halves if U is fp32 (see PassArgs::Rout_lo), nullable
   int B, T, H, dB, reverse;
   int segs, total;
   float s_update;

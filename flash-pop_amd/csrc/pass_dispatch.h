@@ -21,7 +21,7 @@ inline const char* plan_pass(PassArgs& a, int compute_units) {
                                     a.total <= (a.segs - 1LL) * a.T)))
     return "segments that do not cover their sequence, or segments with block states or suffixes";
   if ((a.R0lo && (!a.R0 || blocks || suffix)) || (a.Rout_lo && (!a.Rout || !a.state_only)))
-    return "low halves of states that this walk does not take";
+    return "fp32 states that this walk does not take";
   if (a.dA != 64 && a.dA != 128 && a.dA != 192 && a.dA != 256) return "unsupported contraction width (dA must be 64, 128, 192 or 256)";
   if (a.dB < BV || a.dB % BV != 0) return "dB must be a multiple of 64";
   if (suffix) {

@@ -36,8 +36,6 @@
 // operands of a phase are requested first, the MFMAs that consume them follow back to back,
 // and the vector work of one phase sits in the shadow of the next phase's MFMAs.
 #pragma once
-#include <type_traits>
-
 #include "pass_args.h"
 #include "lds_access.h"
 
@@ -659,8 +657,14 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
 #pragma unroll
     for (int u = 0; u < NP; ++u) tr.v[u] = fprt::buf_load128(view, tile_goff[u] + hf * half_stride);
   };
-  // R (+)= loaded tile, through stage s
-  auto tile_accumulate = [&](const TileRegs& tr, int s, bool add, f32x16 (&racc)[NNW]) {
+  // through stage s, the loaded tile becomes R, is added to R, or (R holding the upper halves of fp32 values) gives the lower halves
+  enum Taken { TAKEN_AS_R, ADDED_TO_R, LOWER_HALVES };
+  auto taken = [](float r, uint32_t bits16, Taken how) {
+    if (how == LOWER_HALVES) return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) | bits16);
+    const float x = bf16_bits_to_float(bits16);
+    return how == ADDED_TO_R ? r + x : x;
+  };
+  auto tile_accumulate = [&](const TileRegs& tr, int s, Taken how, f32x16 (&racc)[NNW]) {
     uint16_t* st = RT + s * BV * RT_LD;
 #pragma unroll
     for (int u = 0; u < NP; ++u) st128(st + tile_soff[u], tr.v[u]);
@@ -669,41 +673,35 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     for (int nn = 0; nn < NNW; ++nn) {
       if (!tposed) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float x = bf16_bits_to_float(reinterpret_cast<const u16_m*>(st)[dl_plain(nn, r)]);
-          racc[nn][r] = add ? racc[nn][r] + x : x;
-        }
+        for (int r = 0; r < 16; ++r) racc[nn][r] = taken(racc[nn][r], reinterpret_cast<const u16_m*>(st)[dl_plain(nn, r)], how);
       } else {
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
           const u32x2 d = ld64(st + dl_tposed(nn, qd));
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const uint32_t w = d[k >> 1];
-            const float x = __builtin_bit_cast(float, (k & 1) ? (w & 0xffff0000u) : (w << 16));
-            racc[nn][4 * qd + k] = add ? racc[nn][4 * qd + k] + x : x;
+            racc[nn][4 * qd + k] = taken(racc[nn][4 * qd + k], (k & 1) ? d[k >> 1] >> 16 : d[k >> 1] & 0xffffu, how);
           }
         }
       }
     }
     fprt::wave_sync();   // the staging area is reused right after
   };
-  // bf16(R), or with `low` what that leaves of R, -> global matrix at dst, through stage s
-  auto tile_store = [&](uint16_t* dst, int s, const f32x16 (&racc)[NNW], int hf, auto low) {
-    auto part = [](float x) { return decltype(low)::value ? bf16_residual(x) : x; };
+  // 16 bits of every element of R -> global matrix at dst, through stage s
+  auto tile_store = [&](uint16_t* dst, int s, const f32x16 (&racc)[NNW], int hf, auto part) {
     uint16_t* st = RT + s * BV * RT_LD;
 #pragma unroll
     for (int nn = 0; nn < NNW; ++nn) {
       if (!tposed) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          reinterpret_cast<u16_m*>(st)[dl_plain(nn, r)] = float_to_bf16_bits(part(racc[nn][r]));
+          reinterpret_cast<u16_m*>(st)[dl_plain(nn, r)] = (uint16_t)pack16(racc[nn][r], 0.f, part);
       } else {
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
           u32x2 d;
-          d[0] = fprt::pack_bf16x2(part(racc[nn][4 * qd]), part(racc[nn][4 * qd + 1]));
-          d[1] = fprt::pack_bf16x2(part(racc[nn][4 * qd + 2]), part(racc[nn][4 * qd + 3]));
+          d[0] = pack16(racc[nn][4 * qd], racc[nn][4 * qd + 1], part);
+          d[1] = pack16(racc[nn][4 * qd + 2], racc[nn][4 * qd + 3], part);
           st64(st + dl_tposed(nn, qd), d);
         }
       }
@@ -785,12 +783,12 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     tile_load(t_init, r0_first ? state_matrix(io.R0, cur.b) : nullptr, true, hf);
     const bool inj = BLOCKS && io.Bin && ends_block(cur.t0 + cur.L);
     tile_load(t_inj, inj ? block_matrix(io.Bin, cur.b, cur.t0 + cur.L) : nullptr, inj, hf);
-    if (r0_first) tile_accumulate(t_init, 0, false, racc[hf]);
+    if (r0_first) tile_accumulate(t_init, 0, TAKEN_AS_R, racc[hf]);
     if (SEGS && r0_first && io.R0lo) {
       tile_load(t_init, state_matrix(io.R0lo, cur.b), true, hf);
-      tile_accumulate(t_init, 0, true, racc[hf]);
+      tile_accumulate(t_init, 0, LOWER_HALVES, racc[hf]);
     }
-    if (inj) tile_accumulate(t_inj, 0, true, racc[hf]);
+    if (inj) tile_accumulate(t_inj, 0, ADDED_TO_R, racc[hf]);
   }
   write_rt(0, racc[0]);
   store_transposed(wregs, cur);
@@ -925,21 +923,25 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
 #pragma unroll
       for (int hf = 0; hf < NH; ++hf) {
         if (BLOCKS && io.Bout && ends_block(t1))
-          tile_store(const_cast<uint16_t*>(block_matrix(io.Bout, cur.b, t1)), s ^ 1, racc[hf], hf, std::false_type{});
+          tile_store(const_cast<uint16_t*>(block_matrix(io.Bout, cur.b, t1)), s ^ 1, racc[hf], hf, AsBf16{});
         // the state that leaves: after the last item; walking forward with suffixes, the one that the
         // suffix at the last block boundary reads (tokens after that boundary are not in it)
         const bool leaves = (SFX && !rev) ? cur.sfx && cur.n == p.nblk && cur.part == sfx_parts - 1 : cur.last;
-        if (leaves && io.Rout) tile_store(const_cast<uint16_t*>(state_matrix(io.Rout, cur.b)), s ^ 1, racc[hf], hf, std::false_type{});
-        if (STATE && leaves && io.Rout_lo) tile_store(const_cast<uint16_t*>(state_matrix(io.Rout_lo, cur.b)), s ^ 1, racc[hf], hf, std::true_type{});
+        if (STATE && leaves && io.Rout_lo) {
+          tile_store(const_cast<uint16_t*>(state_matrix(io.Rout, cur.b)), s ^ 1, racc[hf], hf, UpperHalf{});
+          tile_store(const_cast<uint16_t*>(state_matrix(io.Rout_lo, cur.b)), s ^ 1, racc[hf], hf, LowerHalf{});
+        } else if (leaves && io.Rout) {
+          tile_store(const_cast<uint16_t*>(state_matrix(io.Rout, cur.b)), s ^ 1, racc[hf], hf, AsBf16{});
+        }
       }
     }
     if (nxt.ok) {
       if (MULTI && fresh) {
         if (io.R0) {
-          tile_accumulate(t_init, s ^ 1, false, racc[0]);
+          tile_accumulate(t_init, s ^ 1, TAKEN_AS_R, racc[0]);
           if (io.R0lo) {   // loaded here, once per sequence: held from the start of the visit it costs every visit registers
             tile_load(t_init, state_matrix(io.R0lo, nxt.b), true, 0);
-            tile_accumulate(t_init, s ^ 1, true, racc[0]);
+            tile_accumulate(t_init, s ^ 1, LOWER_HALVES, racc[0]);
           }
         } else {
 #pragma unroll
@@ -948,7 +950,7 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
       }
       if ((BLOCKS || SFX_ANY) && closes && inj) {
 #pragma unroll
-        for (int hf = 0; hf < NH; ++hf) tile_accumulate(t_inj[hf], s ^ 1, true, racc[hf]);
+        for (int hf = 0; hf < NH; ++hf) tile_accumulate(t_inj[hf], s ^ 1, ADDED_TO_R, racc[hf]);
       }
       // the next visit reads the other half (NH = 2), which this visit did not touch
       if (!STATE) write_rt(s ^ 1, racc[(HF + 1) % NH]);

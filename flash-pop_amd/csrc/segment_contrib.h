@@ -1,4 +1,4 @@
-// State-only pass for states of 128 rows: what a sequence of whole chunks adds to the carried
+// State-only pass for states of 128 rows: what a sequence (of any length) adds to the carried
 // state when nothing else is wanted of the pass (the first step of the split-sequence path),
 //   U[a][n] = sum over the tokens j of  weight(j) W[j][a] Z[j][n],
 // chunk by chunk as R <- gamma^64 R + (wkey W)^T Z from R = 0, with wkey(j) = s_update gamma^(63 - j)
@@ -22,12 +22,21 @@ namespace fpk {
 constexpr int sc_lds_bytes() { return 2 * (4 * FB_TILE); }
 static_assert(4 * FB_TILE >= FB_D * FB_LD, "the state copy fits where the tiles were");
 
-// R (accumulator tiles of all waves) -> bf16, through the LDS tile Rt -> its 128 columns of matrix `stream` of dst
+// R (accumulator tiles of all waves), 16 bits of each element, through the LDS tile Rt -> its 128 columns of matrix `stream` of dst
+template <typename Part>
 FP_DEVICE void put_contribution(const ContribArgs& p, uint16_t* Rt, uint16_t* dst, int stream, int ct, int tid, int c, int g,
-                                int at_, int nt0, const f32x16 (&racc)[2]) {
+                                int at_, int nt0, const f32x16 (&racc)[2], Part part) {
   using namespace fb;
 #pragma unroll
-  for (int u = 0; u < 2; ++u) put_state(Rt, 32 * (nt0 + u) + c, 32 * at_, g, racc[u]);
+  for (int u = 0; u < 2; ++u) {
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) {
+      u32x2 d;
+      d[0] = pack16(racc[u][4 * qd], racc[u][4 * qd + 1], part);
+      d[1] = pack16(racc[u][4 * qd + 2], racc[u][4 * qd + 3], part);
+      st64(Rt + at(32 * (nt0 + u) + c, 32 * at_ + 8 * qd + 4 * g), d);
+    }
+  }
   fprt::block_sync();
   char* const ubase = reinterpret_cast<char*>(dst) + ((size_t)stream * FB_D * p.dB + (size_t)ct * FB_D) * 2;
   const fprt::BufView uv = fprt::make_buf(ubase, (uint32_t)(FB_D - 1) * p.dB * 2 + FB_D * 2);
@@ -164,16 +173,12 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     fprt::block_sync();
   }
 
-  // R -> its 128 columns of the rows of U[b][h] (element (a, n) at a * dB + n), as bf16 and what that leaves; every read of the tiles is behind the last barrier
-  put_contribution(p, TL, p.U, stream, ct, tid, c, g, at_, nt0, racc);
-  if (!p.U_lo) return;
+  // R -> its 128 columns of the rows of U[b][h] (element (a, n) at a * dB + n), as bf16 or in fp32 halves; every read of the
+  // tiles is behind the last barrier
+  if (!p.U_lo) return put_contribution(p, TL, p.U, stream, ct, tid, c, g, at_, nt0, racc, AsBf16{});
+  put_contribution(p, TL, p.U, stream, ct, tid, c, g, at_, nt0, racc, UpperHalf{});
   fprt::block_sync();
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) racc[u][r] = bf16_residual(racc[u][r]);
-  }
-  put_contribution(p, TL, p.U_lo, stream, ct, tid, c, g, at_, nt0, racc);
+  put_contribution(p, TL, p.U_lo, stream, ct, tid, c, g, at_, nt0, racc, LowerHalf{});
 }
 
 // Host side: argument check, shared by the GPU launcher and the CPU test harness.

@@ -2,7 +2,7 @@
 // (batch, head) state matrix through the S segments in fp32.  The chain over the segments is one
 // fma per element; what bounds the launch is the latency of its loads (a state of 64 x 128 has 1024
 // threads, so a few streams are a few dozen waves), and the contributions do not depend on the chain:
-// SCAN_AHEAD of them are requested together.  What a form does not have (low halves, block states) is not in its loop: as
+// SCAN_AHEAD of them are requested together.  What a form does not have (lower halves, block states) is not in its loop: as
 // tests at run time around every load they kept the loads apart, 8.0 us a launch at B2 H8 T16384 128 x 256 against
 // 6.9 us without them.
 #pragma once
@@ -11,7 +11,7 @@
 
 namespace fpk {
 
-// LO: U and init have low halves.  BLOCKS: block states leave or join (those of calls cut at their blocks, which keep both
+// LO: U and init are fp32 in two planes.  BLOCKS: block states leave or join (those of calls cut at their blocks, which keep both
 // halves).
 template <bool LO, bool BLOCKS>
 FP_DEVICE void segment_scan_form(const ScanArgs& p) {
@@ -51,26 +51,25 @@ FP_DEVICE void segment_scan_form(const ScanArgs& p) {
     for (int j = 0; j < SCAN_AHEAD; ++j) {
       if (i0 + j >= p.S) break;
       u32x4 o;
+      auto store = [&](uint16_t* dst, auto part) {
+#pragma unroll
+        for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = pack16(r[2 * e], r[2 * e + 1], part);
+        st128(dst, o);
+      };
 #pragma unroll
       for (int e = 0; e < SCAN_VEC; ++e) {
         if (BLOCKS) r[e] += bf16_elem(add[BLOCKS ? j : 0], e);
       }
-#pragma unroll
-      for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = fprt::pack_bf16x2(r[2 * e], r[2 * e + 1]);
-      st128(p.init + matrix(i0 + j), o);
-      if (LO) {
-#pragma unroll
-        for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = fprt::pack_bf16x2(bf16_residual(r[2 * e]), bf16_residual(r[2 * e + 1]));
-        st128(p.init_lo + matrix(i0 + j), o);
+      if constexpr (LO) {
+        store(p.init + matrix(i0 + j), UpperHalf{});
+        store(p.init_lo + matrix(i0 + j), LowerHalf{});
+      } else {
+        store(p.init + matrix(i0 + j), AsBf16{});
       }
       const float g = segment(i0 + j) == p.S - 1 ? glast : gseg;
 #pragma unroll
-      for (int e = 0; e < SCAN_VEC; ++e) r[e] = g * r[e] + (LO ? bf16_elem(u[j], e) + bf16_elem(ulo[LO ? j : 0], e) : bf16_elem(u[j], e));
-      if (BLOCKS && p.blocks_out && segment(i0 + j) < p.nblk) {
-#pragma unroll
-        for (int e = 0; e < SCAN_VEC / 2; ++e) o[e] = fprt::pack_bf16x2(r[2 * e], r[2 * e + 1]);
-        st128(p.blocks_out + block(segment(i0 + j)), o);
-      }
+      for (int e = 0; e < SCAN_VEC; ++e) r[e] = g * r[e] + (LO ? joined_elem(u[j], ulo[LO ? j : 0], e) : bf16_elem(u[j], e));
+      if (BLOCKS && p.blocks_out && segment(i0 + j) < p.nblk) store(p.blocks_out + block(segment(i0 + j)), AsBf16{});
     }
   }
   if (p.fin) {

@@ -233,6 +233,42 @@ def test_pop_split_at_blocks(emu_lib, B, T, H, dk, dv, block, state_std, segment
         assert rc(None, 0) == -1 and rc(p(ws), nbytes - 16) == -2
 
 
+@pytest.mark.parametrize("T,dk,dv,block", [
+    (256, 128, 128, 64),   # POP cut at its blocks, 128-wide keys
+    (150, 256, 64, 64),    # the same through the pass kernel's state-only walk, a tail after the last block
+    (330, 256, 64, 0),     # the plain op in uneven segments
+])
+def test_cut_calls_carry_fp32_states(emu_lib, choose_backward, T, dk, dv, block):
+    """A cut call hands its states from launch to launch as fp32, so that it differs from the uncut one by the order of
+    fp32 sums alone.  A state element that moved by a few 2^-24 rounds to another bf16 operand in about one case of 2^13;
+    an output reads dk of them (1.5 % to 3 % have one that moved), and one operand off by half a bf16 step moves a sum of dk
+    such terms across a rounding boundary in about one case of sqrt(dk): 2e-3 of the outputs.  States that keep 17 bits
+    give 3e-3 (the plain op) to 8e-3 here.  (Of the gradients only dv of a POP call with
+    whole chunks per block: there both sides weigh the same operand of the same chunks.)"""
+    choose_backward(PASSES)
+    decays = (0.97,)
+    q, k, v, s = hp.make_inputs(1, T, 1, dk, dv, seed=T + block, state_std=0.5)
+    if block:
+        d_o, d_b = hp.make_cotangents([(1, T, 1, dv), (1, T // block, 1, dk, dv)], seed=T)
+        n = emu_lib.fp_pop_retention_workspace_bytes(1, T, 1, dk, dv, block)
+        ws, p = torch.empty(n, dtype=torch.uint8), hp._p
+        o, states, (dq, dk_, dv_) = torch.empty_like(v), torch.empty_like(d_b), [torch.empty_like(t) for t in (q, k, v)]
+        assert n > 0 and emu_lib.fp_pop_retention_fwd_split(p(q), p(k), p(v), p(s), hp._dec(decays), p(o), p(states), 1, T, 1, dk, dv, block,
+                                                            p(ws), n, None) == 0
+        assert emu_lib.fp_pop_retention_bwd_split(p(q), p(k), p(v), p(s), hp._dec(decays), p(d_o), p(d_b), p(dq), p(dk_), p(dv_), None,
+                                                  1, T, 1, dk, dv, block, p(ws), n, 1, None) == 0
+        pairs = [("o", o, hp.raw_pop_fwd(emu_lib, q, k, v, s, decays, block)[0]),
+                 ("dv", dv_, hp.raw_pop_bwd(emu_lib, q, k, v, s, decays, block, d_o, d_b)[2])]
+    else:
+        o, _, n = hp.raw_split_fwd(emu_lib, q, k, v, s, decays)
+        assert n > 0
+        pairs = [("o", o, hp.raw_fwd(emu_lib, q, k, v, s, decays)[0])]
+    for name, cut, uncut in pairs:
+        share = (cut != uncut).float().mean().item()
+        print(name, share)
+        assert share <= 2e-3, (name, share)
+
+
 @pytest.mark.parametrize("B,nblk,block,Ls,H,state_std,dk,dv", [
     (1, 2, 128, 16, 1, 0.5, 128, 128),     # two chunks per block
     (1, 4, 64, 64, 1, None, 128, 128),     # block == chunk, suffixes as long as a chunk, no initial state
