@@ -2,7 +2,7 @@
 // state when nothing else is wanted of the pass (the first step of the split-sequence path),
 //   U[a][n] = sum over the tokens j of  weight(j) W[j][a] Z[j][n],
 // chunk by chunk as R <- gamma^64 R + (wkey W)^T Z from R = 0, with wkey(j) = s_update gamma^(63 - j)
-// walking forward and s_update gamma^(j + 1) walking backward, the weighted W rounded to bf16 as the
+// walking forward (gamma^(L - 1 - j) in a last chunk of L tokens) and s_update gamma^(j + 1) walking backward, the weighted W rounded to bf16 as the
 // pass kernel rounds it.
 //
 // One workgroup per (sequence, head, 128 columns of Z) holds its whole 128 x 128 tile of R in the
@@ -63,8 +63,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   const int streams = p.B * p.H;
   const int ct = fprt::block_index() / streams, stream = fprt::block_index() % streams;
   const int h = stream % p.H, b = stream / p.H;
-  // tokens of this sequence and its first row; a segment that ends inside a chunk is walked from its far end in whole
-  // chunks (forward: the chunk met first, from a zero state, begins before the segment and reads zeros there)
+  // tokens of this sequence and its first row
   const int seg = p.segs > 0 ? b % p.segs : 0;
   const int len = p.segs > 0 && p.total - seg * p.T < p.T ? p.total - seg * p.T : p.T;
   const size_t row0 = p.segs > 0 ? (size_t)(b / p.segs) * p.total + (size_t)seg * p.T : (size_t)b * p.T;
@@ -83,12 +82,12 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   // registers <- the chunk visited it-th
   auto load = [&](int it, u32x4 (&pf)[4]) {
     const bool live = it < nch;
-    const int t0 = REV ? (nch - 1 - it) * CH : len - (nch - it) * CH;
+    const int t0 = (REV ? nch - 1 - it : it) * CH;
     const fprt::BufView w = live ? wv : none, z = live ? zv : none;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int r = live ? t0 + ld_row + 32 * u : 0;
-      const uint32_t row = r >= 0 ? r : len;   // row `len` is the first one beyond the views
+      const uint32_t row = r < len ? r : len;   // beyond a short last chunk: row `len`, the first one beyond the views, reads as zero
       pf[u] = fprt::buf_load128(w, row * roww + ld_piece * 16);
       pf[2 + u] = fprt::buf_load128(z, row * rowz + ld_piece * 16);
     }
@@ -116,9 +115,14 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   racc[0] = f32x16{0};
   racc[1] = f32x16{0};
 
-  auto update = [&](int s) {
+  // `L` tokens of the chunk are there.  Walking forward a short chunk is the last one and its weights count from its last token (in
+  // the order of the walk that carries a sequence through, so that a cut call gives the state of the uncut one); walking
+  // backward it is the first one, met with R = 0, and its weights are those of any other.
+  auto update = [&](int s, int L) {
     const uint16_t* const Ws = TL + (2 * s) * FB_TILE;
     const uint16_t* const Zs = Ws + FB_TILE;
+    const bool whole = REV || L == CH;
+    const float decay = whole ? gL : fprt::exp2_approx((float)L * lg);
     u32x4 ua[4], ub0[4], ub1[4];
     auto request = [&](int tt) {
       const int t = REV ? tt : 3 - tt;
@@ -132,7 +136,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) racc[u][r] *= gL;
+      for (int r = 0; r < 16; ++r) racc[u][r] *= decay;
     }
     float wk[8];
 #pragma unroll
@@ -140,6 +144,13 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     fprt::sched_fence();
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
+      if (!whole) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int left = L - 1 - 16 * (3 - tt) - nat_token(g, e);
+          wk[e] = p.s_update * fprt::exp2_approx((float)(left > 0 ? left : 0) * lg);
+        }
+      }
       const u32x4 wa = weigh(ua[tt], wk);
       racc[0] = fprt::mfma_32x32x16_bf16(wa, ub0[tt], racc[0]);
       racc[1] = fprt::mfma_32x32x16_bf16(wa, ub1[tt], racc[1]);
@@ -155,6 +166,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   // Chunk it is multiplied from stage it & 1 while chunk it + 1 moves from registers into the
   // other stage and the loads of chunk it + 3 take its place; chunk it + 2 is on its way in the
   // second set of registers.
+  auto tokens = [&](int it) { return len - it * CH < CH ? len - it * CH : CH; };   // walking forward
   u32x4 pa[4], pb[4];
   load(0, pa);
   load(1, pb);
@@ -164,12 +176,12 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   for (int it = 0; it < nch; it += 2) {
     stage(1, pb);
     load(it + 3, pb);
-    update(0);
+    update(0, tokens(it));
     fprt::block_sync();
     if (it + 1 >= nch) break;
     stage(0, pa);
     load(it + 4, pa);
-    update(1);
+    update(1, tokens(it + 1));
     fprt::block_sync();
   }
 

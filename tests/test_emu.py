@@ -269,6 +269,21 @@ def test_cut_calls_carry_fp32_states(emu_lib, choose_backward, T, dk, dv, block)
         assert share <= 2e-3, (name, share)
 
 
+@pytest.mark.parametrize("T,dk,dv", [
+    (511, 128, 128),    # the 128-wide state-only kernel, a last chunk of 63 tokens
+    (257, 128, 256),    # of one token, two workgroups per segment
+    (330, 64, 128),     # the pass kernel's state-only walk
+])
+def test_cut_final_state_follows_the_uncut_walk(emu_lib, T, dk, dv):
+    """The state-only walk of a cut call takes the chunks of the uncut one, the short one last, and weighs the same keys the
+    same way, so that the final state (bf16 of an fp32 sum, see above: half a step in 2^13 or so) is the uncut one's."""
+    q, k, v, s = hp.make_inputs(1, T, 1, dk, dv, seed=T, state_std=0.5)
+    _, S, n = hp.raw_split_fwd(emu_lib, q, k, v, s, (0.97,))
+    _, S1 = hp.raw_fwd(emu_lib, q, k, v, s, (0.97,))
+    share = (S != S1).float().mean().item()
+    assert n > 0 and share <= 1e-3, share
+
+
 @pytest.mark.parametrize("B,nblk,block,Ls,H,state_std,dk,dv", [
     (1, 2, 128, 16, 1, 0.5, 128, 128),     # two chunks per block
     (1, 4, 64, 64, 1, None, 128, 128),     # block == chunk, suffixes as long as a chunk, no initial state
