@@ -27,21 +27,22 @@ def _run(cmd, verbose):
         raise RuntimeError(f"{cmd[0]} failed with exit code {res.returncode}")
 
 
-def _native_command():
+def native_command(out=NATIVE_OUT, library=OUT, device_dir=CSRC):
+    """`library`: the C-ABI library to link; `device_dir`: where torch_device.h is found (the CPU tests have one of their own)."""
     import torch
     root = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
-    includes = [f"{root}/include", f"{root}/include/torch/csrc/api/include", f"{rocm}/include", sysconfig.get_paths()["include"]]
+    includes = [device_dir, f"{root}/include", f"{root}/include/torch/csrc/api/include", f"{rocm}/include", sysconfig.get_paths()["include"]]
     return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[a for i in includes for a in ("-isystem", i)],
-            os.path.join(CSRC, "torch_ops.cpp"), "-o", NATIVE_OUT,
-            "-L", os.path.dirname(OUT), "-l:" + os.path.basename(OUT), "-L", f"{root}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu",
+            os.path.join(CSRC, "torch_ops.cpp"), "-o", out,
+            "-L", os.path.dirname(library), "-l:" + os.path.basename(library), "-L", f"{root}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu",
             "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{root}/lib"]
 
 
 def build(verbose: bool = True) -> str:
     _run(["hipcc", *FLAGS, *[os.path.join(CSRC, s) for s in SOURCES], "-o", OUT], verbose)
-    _run(_native_command(), verbose)
+    _run(native_command(), verbose)
     return OUT
 
 

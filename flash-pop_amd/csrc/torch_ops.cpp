@@ -4,17 +4,16 @@
 // after, per pass: decode layer step B1 H12 64 x 128 (three calls) 53 -> 20 us, forward B1 H4 T512 64 x 64 28 -> 17 us (now its
 // three launches), forward + backward B3 H8 T1777 128 x 128 166 -> 89 us and B32 H4 T2048 64 x 64 148 -> 118 us (now their kernels).
 //
-// Functions return NotImplemented when an argument is not what they take; the Python wrappers then raise the exception that
-// says what is wrong (flash_pop_amd/_ops.py).  Errors of the C ABI become RuntimeError.
+// Functions return NotImplemented when an argument is not what they take, or the call is being traced; the Python wrappers then
+// raise the exception that says what is wrong, or make the call one that can be traced (flash_pop_amd/_ops.py).  Errors of the C ABI become RuntimeError.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/TracerMode.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
 #include <ATen/ops/zeros.h>
 #include <c10/core/DeviceGuard.h>
-#include <c10/hip/HIPGraphsC10Utils.h>
-#include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -31,6 +30,7 @@
 #include <vector>
 
 #include "../../include/flashpop_hip.h"
+#include <torch_device.h>
 
 namespace {
 
@@ -45,12 +45,12 @@ void check(int rc) {
 }
 
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
-void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+using fpt::stream;
 
 // The pass kernels must not be recorded into a HIP graph: instantiating a graph that holds them has crashed the host process
 // (a segmentation fault inside the runtime, after every launch had been recorded without error).
 void refuse_capture(const char* what) {
-  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+  if (fpt::capturing())
     throw std::runtime_error(std::string(what) +
                              " cannot be captured into a HIP graph with this ROCm / PyTorch build (graph instantiation crashes "
                              "the process); call it eagerly, outside torch.cuda.graph");
@@ -418,7 +418,7 @@ void refuse_tangents(std::initializer_list<const Tensor*> inputs) {
 // a block size as the C ABI takes it, whose sums stay below 2^31; any size beyond the sequence means no block
 int64_t as_block(PyObject* o) { return std::min<int64_t>(as_int(o), 1 << 30); }
 
-bool is_bf16(const Tensor& t) { return !t.defined() || (t.scalar_type() == at::kBFloat16 && t.is_cuda()); }
+bool is_bf16(const Tensor& t) { return !t.defined() || (t.scalar_type() == at::kBFloat16 && fpt::on_device(t)); }
 
 // q, k [B,T,H,dk], v [B,T,H,dv], s [B,H,dk,dv] or none, H decays: what _ops.prepare asks for; makes them contiguous
 bool retention_args(PyObject* const* a, Tensor& q, Tensor& k, Tensor& v, Tensor& s, Decays& g, Shape& n) {
@@ -465,6 +465,9 @@ PyObject* tuple_of(const T&... t) {
 }
 
 PyObject* not_implemented() { Py_RETURN_NOTIMPLEMENTED; }
+// torch.jit.trace cannot see native ops and would keep their results as constants: the wrappers then call them through an autograd
+// Function (flash_pop_amd/_ops.py), which it records.
+bool traced() { return at::tracer::impl::is_dispatch_enabled(); }
 bool count(Py_ssize_t n, Py_ssize_t want) {
   if (n == want) return true;
   PyErr_Format(PyExc_TypeError, "%zd arguments expected, got %zd", want, n);
@@ -482,6 +485,7 @@ struct NoGil {
 PyObject* py_fused_chunk_retention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (!count(nargs, 5)) return nullptr;
+  if (traced()) return not_implemented();
   Tensor q, k, v, s, o, s_out;
   Decays g;
   Shape n;
@@ -510,6 +514,7 @@ PyObject* py_fused_chunk_retention(PyObject*, PyObject* const* a, Py_ssize_t nar
 PyObject* py_flash_pop_retention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (!count(nargs, 6)) return nullptr;
+  if (traced()) return not_implemented();
   Tensor q, k, v, s, o, states;
   Kept kept;
   Decays g;
@@ -540,6 +545,7 @@ PyObject* py_flash_pop_retention(PyObject*, PyObject* const* a, Py_ssize_t nargs
 PyObject* py_pop_with_suffixes(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (!count(nargs, 9)) return nullptr;
+  if (traced()) return not_implemented();
   Tensor q, k, v, s, o, o_sfx, last;
   Suffixes x;
   Decays g;
@@ -606,6 +612,7 @@ PyObject* py_decode_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 PyObject* py_rotary_qk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (!count(nargs, 5)) return nullptr;
+  if (traced()) return not_implemented();
   Tensor q, k, theta, start, q_out, k_out;
   int64_t start0 = 0;
   if (!as_tensor(a[0], q) || !as_tensor(a[1], k) || !as_tensor(a[2], theta) || !q.defined() || !theta.defined()) return not_implemented();
@@ -651,6 +658,7 @@ PyObject* py_rotary_qk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 PyObject* py_gated_group_norm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (!count(nargs, 3)) return nullptr;
+  if (traced()) return not_implemented();
   Tensor r, g, out;
   if (!as_tensor(a[0], r) || !as_tensor(a[1], g) || !r.defined() || !g.defined() || !is_bf16(r) || !is_bf16(g)) return not_implemented();
   if (r.dim() < 2 || g.dim() < 1 || g.numel() != r.numel() || g.size(-1) != r.size(-2) * r.size(-1)) return not_implemented();

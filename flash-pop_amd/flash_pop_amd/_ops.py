@@ -49,6 +49,37 @@ def prepare(q, k, v, s, head_decays):
     return q, k, v, s, (B, T, H, dk, dv)
 
 
+class Traced(torch.autograd.Function):
+    """An op as torch.jit.trace can record it: the tracer keeps calls of autograd Functions and runs them again, and does not see
+    native ones.  apply(op, *op's arguments)."""
+
+    @staticmethod
+    def forward(ctx, op, *args):
+        tracing = torch._C._get_tracing_state()
+        torch._C._set_tracing_state(None)
+        try:
+            with torch.enable_grad():
+                ctx.ins = [a.detach().requires_grad_(a.requires_grad) if isinstance(a, torch.Tensor) else a for a in args]
+                out = op(*ctx.ins)
+        finally:
+            torch._C._set_tracing_state(tracing)
+        ctx.set_materialize_grads(False)
+        ctx.outs = (out,) if isinstance(out, torch.Tensor) else out
+        detached = tuple(None if o is None else o.detach() for o in ctx.outs)
+        return detached[0] if isinstance(out, torch.Tensor) else detached
+
+    @staticmethod
+    def backward(ctx, *grads):
+        used = [(o, g) for o, g in zip(ctx.outs, grads) if g is not None]
+        leaves = [a for a in ctx.ins if isinstance(a, torch.Tensor) and a.requires_grad]
+        got = iter(torch.autograd.grad([o for o, _ in used], leaves, [g for _, g in used], retain_graph=True, allow_unused=True))
+        return (None, *[next(got) if isinstance(a, torch.Tensor) and a.requires_grad else None for a in ctx.ins])
+
+
+def tracing():
+    return torch._C._get_tracing_state() is not None
+
+
 def rejected(op):
     """The native op refused its arguments and the checks above found nothing to say about them."""
     raise TypeError(f"{op}: unsupported arguments")

@@ -18,6 +18,8 @@ class FusedChunkRetention:
     def apply(q, k, v, s, head_decays):
         out = _lib.native().fused_chunk_retention(q, k, v, s, head_decays)
         if out is NotImplemented:
+            if _ops.tracing():
+                return _ops.Traced.apply(FusedChunkRetention.apply, q, k, v, s, head_decays)
             _ops.prepare(q, k, v, s, head_decays)
             _ops.rejected("fused_chunk_retention")
         return out

@@ -13,6 +13,8 @@ from .. import _lib, _ops
 def gated_group_norm(retention, gate, eps: float = 1e-6):
     out = _lib.native().gated_group_norm(retention, gate, eps)
     if out is NotImplemented:
+        if _ops.tracing():
+            return _ops.Traced.apply(gated_group_norm, retention, gate, eps)
         _ops.gated_norm_fwd(retention, gate, eps)   # raises
         _ops.rejected("gated_group_norm")
     return out

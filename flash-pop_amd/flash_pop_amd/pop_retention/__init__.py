@@ -34,6 +34,8 @@ class FlashPOPRetention:
     def apply(q, k, v, s, head_decays, block_size):
         out = _lib.native().flash_pop_retention(q, k, v, s, head_decays, block_size)
         if out is NotImplemented:
+            if _ops.tracing():
+                return _ops.Traced.apply(FlashPOPRetention.apply, q, k, v, s, head_decays, block_size)
             _refused(q, k, v, s, head_decays, block_size)
             _ops.rejected("flash_pop_retention")
         return out
@@ -48,6 +50,8 @@ class FlashPOPRetentionWithSuffixes:
     def apply(q, k, v, s, head_decays, block_size, q_sfx, k_sfx, v_sfx):
         out = _lib.native().flash_pop_retention_with_suffixes(q, k, v, s, head_decays, block_size, q_sfx, k_sfx, v_sfx)
         if out is NotImplemented:
+            if _ops.tracing():
+                return _ops.Traced.apply(FlashPOPRetentionWithSuffixes.apply, q, k, v, s, head_decays, block_size, q_sfx, k_sfx, v_sfx)
             shape = _refused(q, k, v, s, head_decays, block_size)
             _ops.prepare_suffixes(q_sfx, k_sfx, v_sfx, shape, int(block_size))
             _ops.rejected("flash_pop_retention_with_suffixes")

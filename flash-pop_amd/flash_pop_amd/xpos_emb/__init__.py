@@ -38,6 +38,8 @@ class XPos:
         theta = self._theta(q.device)
         out = _lib.native().rotary_qk(q, k, theta, start_idx, False)
         if out is NotImplemented:
+            if _ops.tracing():
+                return _ops.Traced.apply(self, q, k, start_idx)
             _ops.rotary_qk(q, k, theta, start_idx)   # raises
             _ops.rejected("XPos")
         return out

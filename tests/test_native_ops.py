@@ -1,0 +1,83 @@
+"""The native ops (csrc/torch_ops.cpp) on the CPU: the same source, built over the CPU harness of the kernels, behind the
+package's Python wrappers."""
+import importlib.util
+import os
+import subprocess
+
+import pytest
+import torch
+
+import helpers as hp
+import oracle
+
+EMU_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "emu")
+PKG_DIR = os.path.join(os.path.dirname(os.path.dirname(EMU_DIR)), "flash-pop_amd")
+DEC = (0.97, 0.9)
+
+
+def _module(name, path):
+    spec = importlib.util.spec_from_file_location(name, path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+@pytest.fixture(scope="module")
+def emu(tmp_path_factory):
+    """(C-ABI library of the harness, the native ops over it)"""
+    from flash_pop_amd import _lib
+    lib = str(tmp_path_factory.mktemp("emu") / "libflashpop_emu.so")
+    native = os.path.join(os.path.dirname(lib), "_native.so")
+    build = _module("flash_pop_amd_build", os.path.join(PKG_DIR, "build.py"))
+    ops = subprocess.Popen([os.path.join(EMU_DIR, "build_emu.sh")], env=dict(os.environ, EMU_OUT=lib))
+    assert ops.wait() == 0
+    subprocess.run(build.native_command(native, lib, EMU_DIR), check=True)
+    return _lib.bind(lib), _module("_native", native)
+
+
+@pytest.fixture
+def ops(emu, monkeypatch):
+    """The package, its wrappers over the harness"""
+    import flash_pop_amd
+    monkeypatch.setattr(flash_pop_amd._lib, "_native", emu[1])
+    return flash_pop_amd
+
+
+def _inputs(seed, B=1, T=70, H=2, d=64, block=32, Ls=3):
+    q, k, v, s = hp.make_inputs(B, T, H, d, d, seed=seed, state_std=0.3)
+    sfx = hp.make_suffix_inputs(B, T // block, Ls, H, d, d, seed=seed + 1)
+    return q, k, v, s, sfx, torch.randn(B, T, H * d, generator=torch.Generator().manual_seed(seed)).to(hp.BF16)
+
+
+def _calls(ops):
+    """op -> (call of tensors alone, those tensors from a seed)"""
+    xpos = ops.XPos(64)
+    return {
+        "plain": (lambda q, k, v, s: ops.fused_chunk_retention(q, k, v, s, DEC), lambda n: _inputs(n)[:4]),
+        "pop": (lambda q, k, v, s: ops.flash_pop_retention(q, k, v, s, DEC, 32), lambda n: _inputs(n)[:4]),
+        "pop_sfx": (lambda q, k, v, s, *x: ops.flash_pop_retention_with_suffixes(q, k, v, s, DEC, 32, *x), lambda n: (*_inputs(n)[:4], *_inputs(n)[4])),
+        "rotary": (lambda q, k: xpos(q, k, 3), lambda n: _inputs(n)[:2]),
+        "norm": (lambda q, g: ops.gated_group_norm(q, g), lambda n: (_inputs(n)[0], _inputs(n)[5])),
+    }
+
+
+OPS = ["plain", "pop", "pop_sfx", "rotary", "norm"]
+
+
+def _tuple(out):
+    return (out,) if isinstance(out, torch.Tensor) else out
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.filterwarnings("ignore")
+def test_traced_programs_run_the_op_again(ops, op):
+    """A program traced on some inputs gives, on others, what the op gives on those, gradients included."""
+    call, inputs = _calls(ops)[op]
+    traced = torch.jit.trace(call, tuple(inputs(1)))
+    ins, ins2 = ([t.requires_grad_() for t in inputs(2)] for _ in range(2))
+    out, ref = _tuple(traced(*ins)), _tuple(call(*ins2))
+    assert all(torch.equal(a, b) for a, b in zip(out, ref))
+    grads, ref = (torch.autograd.grad(x[0].sum(), y, allow_unused=True) for x, y in ((out, ins), (ref, ins2)))
+    assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(grads, ref))
+    with pytest.raises((RuntimeError, ValueError)):
+        torch.jit.trace(call, (ins[0][:, :1], *ins[1:]))
