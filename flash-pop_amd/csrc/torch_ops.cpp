@@ -319,8 +319,11 @@ struct PopFusedBackward : public RetentionNode {
   }
 };
 
+// (This node and the next give an input whose output nobody differentiates a gradient of zeros, as the retention nodes do.)
 struct RotaryBackward : public torch::autograd::Node {
   Tensor theta, start;
+  std::vector<int64_t> shape;   // of q and of k
+  at::TensorOptions options;
   int64_t start0 = 0;
   bool inverse = false;
   std::string name() const override { return "RotaryQKBackward"; }
@@ -332,6 +335,9 @@ struct RotaryBackward : public torch::autograd::Node {
     }
     if (in[0].defined()) rotary(in[0], in[1], theta, start, start0, !inverse, out[0], out[1]);
     else if (in[1].defined()) rotary(in[1], none, theta, start, start0, !inverse, out[1], none);
+    for (int i = 0; i < 2; ++i) {
+      if (!out[i].defined() && task_should_compute_output(i)) out[i] = at::zeros(shape, options);
+    }
     return {out[0], out[1]};
   }
 };
@@ -349,8 +355,8 @@ struct GatedNormBackward : public torch::autograd::Node {
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex);
     at::AutoGradMode no_grad(false);
-    if (!grads[0].defined()) return {Tensor(), Tensor()};
     const Tensor r_ = r.unpack(), g_ = g.unpack();
+    if (!grads[0].defined()) return {at::zeros(r_.sizes(), r_.options()), at::zeros(g_.sizes(), g_.options())};
     Tensor d_r, d_g;
     gated_norm_bwd(r_, g_, grads[0].contiguous(), eps, d_r, d_g);
     return {d_r, d_g};
@@ -643,6 +649,8 @@ PyObject* py_rotary_qk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (grad) {
       auto node = make_node<RotaryBackward>(q, k);
       node->theta = theta;
+      node->shape = q.sizes().vec();
+      node->options = q.options();
       node->start = start;
       node->start0 = start0;
       node->inverse = inverse;

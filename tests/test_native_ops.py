@@ -81,3 +81,32 @@ def test_traced_programs_run_the_op_again(ops, op):
     assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(grads, ref))
     with pytest.raises((RuntimeError, ValueError)):
         torch.jit.trace(call, (ins[0][:, :1], *ins[1:]))
+
+
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_gradients_are_zeros_where_nothing_arrives(ops, op):
+    """Every input of an op gets a gradient: zeros where no output that depends on it is differentiated, or where what comes
+    after the op passes nothing on."""
+    call, inputs = _calls(ops)[op]
+    ins = [t.requires_grad_() for t in inputs(1)]
+    grads = torch.autograd.grad(_NoGradient.apply(_tuple(call(*ins))[0]).sum(), ins)
+    assert all(g.shape == t.shape and not g.any() for g, t in zip(grads, ins))
+    if op == "rotary":
+        for i in (0, 1):
+            grads = torch.autograd.grad(call(*ins)[i].sum(), ins)
+            assert grads[i].any() and not grads[1 - i].any()
+        call(*ins)[1].sum().backward()
+        assert not ins[0].grad.any() and ins[1].grad.any()
+        # an input that needs no gradient still gets none, and a lone q works
+        assert torch.autograd.grad(call(ins[0], ins[1].detach())[0].sum(), ins[0])[0].any()
+        assert torch.autograd.grad(ops.XPos(64)(ins[0], None, 0)[0].sum(), ins[0])[0].any()
