@@ -388,21 +388,28 @@ bool as_tensor(PyObject* o, Tensor& t) {
   return true;
 }
 
-bool as_decays(PyObject* o, Decays& g) {
+// what has a length and gives, item by item, something that float() takes
+void as_decays(PyObject* o, Decays& g) {
+  if (PyObject_Length(o) < 0) throw python_error();   // (an iterator would be spent by the first look at it)
   PyObject* fast = PySequence_Fast(o, "head decays: a sequence of numbers expected");
   if (!fast) throw python_error();
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(fast);
   g.resize((size_t)n);
   for (Py_ssize_t i = 0; i < n; ++i) {
     PyObject* item = PySequence_Fast_GET_ITEM(fast, i);
-    g[(size_t)i] = PyFloat_CheckExact(item) ? PyFloat_AS_DOUBLE(item) : PyFloat_AsDouble(item);
-    if (g[(size_t)i] == -1.0 && PyErr_Occurred()) {
+    if (PyFloat_CheckExact(item)) {
+      g[(size_t)i] = PyFloat_AS_DOUBLE(item);
+      continue;
+    }
+    PyObject* number = PyNumber_Float(item);
+    if (!number) {
       Py_DECREF(fast);
       throw python_error();
     }
+    g[(size_t)i] = PyFloat_AS_DOUBLE(number);
+    Py_DECREF(number);
   }
   Py_DECREF(fast);
-  return true;
 }
 
 int64_t as_int(PyObject* o) {

@@ -110,3 +110,14 @@ def test_gradients_are_zeros_where_nothing_arrives(ops, op):
         # an input that needs no gradient still gets none, and a lone q works
         assert torch.autograd.grad(call(ins[0], ins[1].detach())[0].sum(), ins[0])[0].any()
         assert torch.autograd.grad(ops.XPos(64)(ins[0], None, 0)[0].sum(), ins[0])[0].any()
+
+
+def test_head_decays_are_what_has_a_length_and_floats(ops):
+    q, k, v, s = _inputs(1)[:4]
+    ref = ops.fused_chunk_retention(q, k, v, s, DEC)[0]
+    for decays in (list(DEC), torch.tensor(DEC, dtype=torch.float64), [str(g) for g in DEC], dict.fromkeys(DEC)):
+        assert torch.equal(ops.fused_chunk_retention(q, k, v, s, decays)[0], ref)
+    for op in (lambda g: ops.fused_chunk_retention(q, k, v, s, g), lambda g: ops.retention_recurrent(q[:, 0], k[:, 0], v[:, 0], g, s)):
+        for bad, error in (((g for g in DEC), TypeError), (DEC[0], TypeError), (("x", 0.5), ValueError), (DEC + DEC, AssertionError)):
+            with pytest.raises(error):
+                op(bad)
