@@ -16,6 +16,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
@@ -217,6 +218,22 @@ void gated_norm_bwd(const Tensor& r, const Tensor& g, const Tensor& d_out, doubl
 
 // ---- autograd nodes -----------------------------------------------------------------------------------------------------
 
+// The gradients that a backward returns.  The ops have no second derivative: under create_graph, where gradients without a history
+// would count as constants, they get one that raises when it is differentiated.  `inputs`: what the gradients depend on.
+template <typename... Inputs>
+variable_list once_differentiable(variable_list&& gradients, bool create_graph, const Inputs&... inputs) {
+  at::AutoGradMode grad_mode(create_graph);
+  if (create_graph && torch::autograd::compute_requires_grad(inputs...)) {
+    std::shared_ptr<torch::autograd::Node> error(
+        new torch::autograd::Error("flash_pop_amd's ops can be differentiated once only", torch::autograd::collect_next_edges(inputs...)),
+        torch::autograd::deleteNode);
+    for (Tensor& g : gradients) {
+      if (g.defined()) torch::autograd::set_history(g, error);
+    }
+  }
+  return std::move(gradients);
+}
+
 // q, k, v, s and the decays of a retention op, saved for its backward
 struct RetentionNode : public torch::autograd::Node {
   SavedVariable q, k, v, s;
@@ -267,6 +284,7 @@ struct PlainBackward : public KeepingNode {
   std::string name() const override { return "FusedChunkRetentionBackward"; }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex);
+    const bool create_graph = at::GradMode::is_enabled();
     at::AutoGradMode no_grad(false);
     const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), s_ = s.unpack();
     const Tensor d_o = incoming(grads[0], {n.B, n.T, n.H, n.dv}, q_), d_s = incoming(grads[1], {}, q_);
@@ -275,7 +293,7 @@ struct PlainBackward : public KeepingNode {
     // a second one (retain_graph) recomputes them
     Grads r = retention_bwd(q_, k_, v_, s_, decays, n, d_o, d_s, Tensor(), 0, s_.defined() && task_should_compute_output(3), kept, !spent);
     spent = spent || (kept.t.defined() && kept.every == 0);
-    return {r.dq, r.dk, r.dv, r.ds0};
+    return once_differentiable({r.dq, r.dk, r.dv, r.ds0}, create_graph, grads, q_, k_, v_, s_);
   }
 };
 
@@ -285,13 +303,14 @@ struct PopBackward : public KeepingNode {
   std::string name() const override { return "FlashPOPRetentionBackward"; }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex);
+    const bool create_graph = at::GradMode::is_enabled();
     at::AutoGradMode no_grad(false);
     const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), s_ = s.unpack();
     const Tensor d_o = incoming(grads[0], {n.B, n.T, n.H, n.dv}, q_), d_b = incoming(grads[1], {}, q_);
     const Kept kept{kept_tensor.unpack(), 0};
     Grads r = retention_bwd(q_, k_, v_, s_, decays, n, d_o, Tensor(), d_b, block, s_.defined() && task_should_compute_output(3), kept, !spent);
     spent = spent || kept.t.defined();
-    return {r.dq, r.dk, r.dv, r.ds0};
+    return once_differentiable({r.dq, r.dk, r.dv, r.ds0}, create_graph, grads, q_, k_, v_, s_);
   }
 };
 
@@ -308,6 +327,7 @@ struct PopFusedBackward : public RetentionNode {
   }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex);
+    const bool create_graph = at::GradMode::is_enabled();
     at::AutoGradMode no_grad(false);
     const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), s_ = s.unpack();
     const Suffixes x{qs.unpack(), ks.unpack(), vs.unpack()};
@@ -315,7 +335,7 @@ struct PopFusedBackward : public RetentionNode {
                  d_s = incoming(grads[2], {}, q_);
     Suffixes dx;
     Grads r = pop_fused_bwd(q_, k_, v_, s_, x, decays, block, n, d_o, d_os, d_s, s_.defined() && task_should_compute_output(3), dx);
-    return {r.dq, r.dk, r.dv, r.ds0, dx.q, dx.k, dx.v};
+    return once_differentiable({r.dq, r.dk, r.dv, r.ds0, dx.q, dx.k, dx.v}, create_graph, grads, q_, k_, v_, s_, x.q, x.k, x.v);
   }
 };
 
@@ -328,6 +348,7 @@ struct RotaryBackward : public torch::autograd::Node {
   bool inverse = false;
   std::string name() const override { return "RotaryQKBackward"; }
   variable_list apply(variable_list&& grads) override {
+    const bool create_graph = at::GradMode::is_enabled();
     at::AutoGradMode no_grad(false);
     Tensor in[2], out[2], none;
     for (int i = 0; i < 2; ++i) {
@@ -338,7 +359,7 @@ struct RotaryBackward : public torch::autograd::Node {
     for (int i = 0; i < 2; ++i) {
       if (!out[i].defined() && task_should_compute_output(i)) out[i] = at::zeros(shape, options);
     }
-    return {out[0], out[1]};
+    return once_differentiable({out[0], out[1]}, create_graph, grads);
   }
 };
 
@@ -354,12 +375,13 @@ struct GatedNormBackward : public torch::autograd::Node {
   }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex);
+    const bool create_graph = at::GradMode::is_enabled();
     at::AutoGradMode no_grad(false);
     const Tensor r_ = r.unpack(), g_ = g.unpack();
     if (!grads[0].defined()) return {at::zeros(r_.sizes(), r_.options()), at::zeros(g_.sizes(), g_.options())};
     Tensor d_r, d_g;
     gated_norm_bwd(r_, g_, grads[0].contiguous(), eps, d_r, d_g);
-    return {d_r, d_g};
+    return once_differentiable({d_r, d_g}, create_graph, grads, r_, g_);
   }
 };
 

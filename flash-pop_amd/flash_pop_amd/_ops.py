@@ -69,6 +69,7 @@ class Traced(torch.autograd.Function):
         return detached[0] if isinstance(out, torch.Tensor) else detached
 
     @staticmethod
+    @torch.autograd.function.once_differentiable
     def backward(ctx, *grads):
         used = [(o, g) for o, g in zip(ctx.outs, grads) if g is not None]
         leaves = [a for a in ctx.ins if isinstance(a, torch.Tensor) and a.requires_grad]

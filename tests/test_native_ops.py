@@ -121,3 +121,17 @@ def test_head_decays_are_what_has_a_length_and_floats(ops):
         for bad, error in (((g for g in DEC), TypeError), (DEC[0], TypeError), (("x", 0.5), ValueError), (DEC + DEC, AssertionError)):
             with pytest.raises(error):
                 op(bad)
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_second_derivatives_raise(ops, op):
+    """create_graph gives the first derivative; what depends on it cannot be differentiated, and is not taken for a constant."""
+    call, inputs = _calls(ops)[op]
+    ins = [t.requires_grad_() for t in inputs(1)]
+    first = lambda **kw: torch.autograd.grad(_tuple(call(*ins))[0].float().square().sum(), ins, allow_unused=True, **kw)
+    grads = first(create_graph=True)
+    assert all(torch.equal(a, b) for a, b in zip(grads, first()))
+    penalty = ins[0].float().sum() + sum(g.float().square().sum() for g in grads)
+    for differentiate in (lambda: penalty.backward(retain_graph=True), lambda: torch.autograd.grad(penalty, ins[0])):
+        with pytest.raises(RuntimeError, match="once"):
+            differentiate()
