@@ -341,21 +341,29 @@ struct PopFusedBackward : public RetentionNode {
 
 // (This node and the next give an input whose output nobody differentiates a gradient of zeros, as the retention nodes do.)
 struct RotaryBackward : public torch::autograd::Node {
-  Tensor theta, start;
+  Tensor theta;          // a table of the module's own
+  SavedVariable start;   // a tensor of the caller's, which may advance it in place before the backward runs: that is an error then
+  std::mutex mutex;
   std::vector<int64_t> shape;   // of q and of k
   at::TensorOptions options;
   int64_t start0 = 0;
   bool inverse = false;
   std::string name() const override { return "RotaryQKBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex);
+    start.reset_data();
+  }
   variable_list apply(variable_list&& grads) override {
     const bool create_graph = at::GradMode::is_enabled();
     at::AutoGradMode no_grad(false);
+    std::lock_guard<std::mutex> lock(mutex);
+    const Tensor start_ = start.unpack();
     Tensor in[2], out[2], none;
     for (int i = 0; i < 2; ++i) {
       if (i < (int)grads.size() && grads[i].defined()) in[i] = grads[i].contiguous();
     }
-    if (in[0].defined()) rotary(in[0], in[1], theta, start, start0, !inverse, out[0], out[1]);
-    else if (in[1].defined()) rotary(in[1], none, theta, start, start0, !inverse, out[1], none);
+    if (in[0].defined()) rotary(in[0], in[1], theta, start_, start0, !inverse, out[0], out[1]);
+    else if (in[1].defined()) rotary(in[1], none, theta, start_, start0, !inverse, out[1], none);
     for (int i = 0; i < 2; ++i) {
       if (!out[i].defined() && task_should_compute_output(i)) out[i] = at::zeros(shape, options);
     }
@@ -680,7 +688,8 @@ PyObject* py_rotary_qk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
       node->theta = theta;
       node->shape = q.sizes().vec();
       node->options = q.options();
-      node->start = start;
+      if (start.defined() && start.is_inference()) start = start.clone();   // (cannot be saved as it is)
+      node->start = SavedVariable(start, false);
       node->start0 = start0;
       node->inverse = inverse;
       torch::autograd::set_history(q_out, node);

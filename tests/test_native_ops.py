@@ -135,3 +135,21 @@ def test_second_derivatives_raise(ops, op):
     for differentiate in (lambda: penalty.backward(retain_graph=True), lambda: torch.autograd.grad(penalty, ins[0])):
         with pytest.raises(RuntimeError, match="once"):
             differentiate()
+
+
+def test_positions_changed_before_the_backward_raise(ops):
+    q, k = (t.requires_grad_() for t in _inputs(1, B=2)[:2])
+    xpos, start = ops.XPos(64), torch.tensor([3, 5])
+    out = xpos(q, k, start)[0].sum()
+    ref = torch.autograd.grad(out, q, retain_graph=True)[0]
+    start += 1
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(out, q)
+    with torch.inference_mode():
+        start = torch.tensor([3, 5])
+    assert torch.equal(torch.autograd.grad(xpos(q, k, start)[0].sum(), q)[0], ref)
+    # (positions of another type are converted, and the conversion is the op's own)
+    start = torch.tensor([3, 5], dtype=torch.int32)
+    out = xpos(q, k, start)[0].sum()
+    start += 1
+    assert torch.equal(torch.autograd.grad(out, q)[0], ref)
