@@ -646,6 +646,7 @@ PyObject* py_decode_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     s_out = in_place ? s : at::empty({B, H, dk, dv}, q.options());
     o = at::empty({B, H, dv}, q.options());
     check(fp_retention_decode_step(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(o), ptr(s_out), B, H, dk, dv, stream()));
+    if (in_place && !s.is_inference()) s.unsafeGetTensorImpl()->bump_version();   // a graph node that saved this state must notice
   }
   return tuple_of(o, s_out);
   END_HANDLE_TH_ERRORS

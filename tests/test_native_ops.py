@@ -153,3 +153,18 @@ def test_positions_changed_before_the_backward_raise(ops):
     out = xpos(q, k, start)[0].sum()
     start += 1
     assert torch.equal(torch.autograd.grad(out, q)[0], ref)
+
+
+def test_in_place_steps_are_seen_by_the_graph(ops):
+    q, k, v, s = _inputs(1)[:4]
+    q.requires_grad_()
+    out = ops.fused_chunk_retention(q, k, v, s, DEC)[0].sum()   # its node saves s
+    step = lambda state, **kw: ops.retention_recurrent(q[:, 0], k[:, 0], v[:, 0], DEC, state, **kw)
+    _, new = step(s)
+    torch.autograd.grad(out, q, retain_graph=True)
+    assert step(s, in_place=True)[1].data_ptr() == s.data_ptr() and torch.equal(s, new)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(out, q)
+    with torch.inference_mode():
+        state = s.clone()
+    step(state, in_place=True)                                  # (has no version to advance)
