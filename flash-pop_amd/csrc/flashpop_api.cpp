@@ -461,15 +461,31 @@ int plan_backward(const Shape& s) {
   return n > 1 && cut_pays(s, n, segment_tokens(s, n), true) ? n : 1;
 }
 
+// Whether the bytes that a POP call cut at its blocks moves are worth the chain they replace: q, k, v, o, k and v a second time,
+// and per element of a block's state 18 bytes (fp32 written, read and written by the scan, read; bf16 out), where the uncut call
+// moves 2.  There are as many states as blocks, however many fill the chip, and the cut call streams them at 3.5 to 4.5 TB/s
+// while the uncut one walks, 1.4 to 2 us a chunk: 6.8 MB a step tell the two apart (three steps: the launches).  Uncut -> cut,
+// forward / backward, us:
+//   128 x 128  blocks of 64    B10 H4 T4096   132 -> 259 / 226 -> 399      B4 H4 T4096   131 -> 110 / 225 -> 161
+//   128 x 128  blocks of 144   B10 H4 T16384  593 -> 678 / 934 -> 1091     B4 H8 T4096   145 -> 137 / 237 -> 231
+//   64 x 128   blocks of 64    B6 H8 T4096     99 -> 131 / 216 -> 231      B6 H4 T2048    52 -> 47 / 162 -> 80
+//   64 x 64    blocks of 64    B10 H8 T4096    98 -> 120 / 174 -> 217      B6 H8 T16384  452 -> 377 / 672 -> 594
+bool block_states_pay(const Shape& s, int segments, int block) {
+  if (fpk_launch_steps() <= 0) return true;   // (a device whose launches cost nothing)
+  const double chunks = (double)segments * ((block + fpk::CH - 1) / fpk::CH);
+  const double bytes = 6.0 * s.B * s.T * s.H * (s.dk + s.dv) + 18.0 * s.B * segments * s.H * s.dk * s.dv;
+  return bytes <= 6.8e6 * (chunks - 3);
+}
+
 // Segments per sequence of a POP call (1: not cut), one per block and one for the tokens after the last block: the scan over
 // the contributions then passes every block state, and the gradients of block states join in it, so that the passes are
 // those of a plain call.  For the streams that a plain call is cut for, and blocks of at least a chunk (a shorter block
-// has more state than tokens to move), where the chain gets shorter by what the cut costs.
+// has more state than tokens to move), where the chain gets shorter by what the cut costs and its states do not take longer to move.
 int plan_pop_forward(const Shape& s, int block) {
   const long long streams = (long long)s.B * s.H * ((s.dk < s.dv ? s.dk : s.dv) / fpk::BV);
   if (block < fpk::CH || s.T <= block || 3 * streams > fpk_compute_units()) return 1;
   const int n = segment_count(s, block);
-  return cut_pays(s, n, block, false, block) ? n : 1;
+  return block_states_pay(s, n, block) && cut_pays(s, n, block, false, block) ? n : 1;
 }
 int plan_pop_backward(const Shape& s, int block) {
   const int n = plan_pop_forward(s, block);

@@ -125,6 +125,23 @@ def test_new_entry_points_check_their_arguments(lib):
     assert lib.fp_retention_bwd_split(p, p, p, null, dec, null, null, p, p, p, null, 1, 8, 2, 64, 64, null, 0, 0, None) == -1
 
 
+@pytest.mark.parametrize("cut,B,T,H,dk,dv,block", [
+    (True, 4, 1440, 4, 64, 128, 144),      # 5 MB of block states against a chain of 30 chunks
+    (True, 4, 4096, 4, 128, 128, 64),      # 67 MB, 64 chunks: just worth it
+    (False, 10, 4096, 4, 128, 128, 64),    # 168 MB against the same chain
+    (False, 4, 4096, 8, 128, 128, 64),
+    (False, 10, 4096, 8, 64, 64, 64),
+    (False, 5, 16384, 8, 128, 128, 64),    # 671 MB, 256 chunks
+    (True, 2, 16384, 4, 128, 128, 128),
+    (False, 4, 1440, 4, 64, 128, 1440),    # a single block
+    (False, 4, 1440, 16, 64, 128, 144),    # too many streams
+])
+def test_pop_calls_are_cut_where_their_states_are_worth_it(lib, cut, B, T, H, dk, dv, block):
+    """On a device of 256 compute units (what the library takes a machine without a GPU for)."""
+    segments = -(-T // block)
+    assert lib.fp_pop_retention_workspace_bytes(B, T, H, dk, dv, block) == (4 * B * segments * H * dk * dv if cut else 0)
+
+
 def test_new_python_wrappers_refuse_cpu_tensors():
     import torch
     from flash_pop_amd import flash_pop_retention_with_suffixes, retention_recurrent
