@@ -73,16 +73,19 @@ __global__ __launch_bounds__(fpk::DECODE_THREADS) void decode_step_kernel(const 
   fpk::decode_step(args, lds);
 }
 
+template <bool ONCE>
 __global__ __launch_bounds__(fpk::LAYER_THREADS) void rotary_qk_kernel(const fpk::RotaryArgs args) {
-  fpk::rotary_qk(args);
+  fpk::rotary_qk<ONCE>(args);
 }
 
+template <bool ONCE>
 __global__ __launch_bounds__(fpk::LAYER_THREADS) void gated_norm_fwd_kernel(const fpk::GatedNormArgs args) {
-  fpk::gated_norm_fwd(args);
+  fpk::gated_norm_fwd<ONCE>(args);
 }
 
+template <bool ONCE>
 __global__ __launch_bounds__(fpk::LAYER_THREADS) void gated_norm_bwd_kernel(const fpk::GatedNormArgs args) {
-  fpk::gated_norm_bwd(args);
+  fpk::gated_norm_bwd<ONCE>(args);
 }
 
 // LDS above 64 KB has to be opted into once per device and kernel.  One bit per kernel (`slot`)
@@ -476,8 +479,8 @@ int fpk_launch_rotary(const fpk::RotaryArgs& args, void* stream, const char** er
     *err = why;
     return 1;
   }
-  hipLaunchKernelGGL(rotary_qk_kernel, dim3((unsigned)blocks), dim3(fpk::LAYER_THREADS), 0,
-                     static_cast<hipStream_t>(stream), a);
+  hipLaunchKernelGGL(fpk::passes_caches(a) ? rotary_qk_kernel<true> : rotary_qk_kernel<false>, dim3((unsigned)blocks),
+                     dim3(fpk::LAYER_THREADS), 0, static_cast<hipStream_t>(stream), a);
   return launched(err);
 }
 
@@ -487,11 +490,9 @@ int fpk_launch_gated_norm(const fpk::GatedNormArgs& a, void* stream, const char*
     *err = why;
     return 1;
   }
-  if (a.out)
-    hipLaunchKernelGGL(gated_norm_fwd_kernel, dim3((unsigned)blocks), dim3(fpk::LAYER_THREADS), 0,
-                       static_cast<hipStream_t>(stream), a);
-  else
-    hipLaunchKernelGGL(gated_norm_bwd_kernel, dim3((unsigned)blocks), dim3(fpk::LAYER_THREADS), 0,
-                       static_cast<hipStream_t>(stream), a);
+  const bool once = fpk::passes_caches(a);
+  const auto kernel = a.out ? (once ? gated_norm_fwd_kernel<true> : gated_norm_fwd_kernel<false>)
+                            : (once ? gated_norm_bwd_kernel<true> : gated_norm_bwd_kernel<false>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(fpk::LAYER_THREADS), 0, static_cast<hipStream_t>(stream), a);
   return launched(err);
 }

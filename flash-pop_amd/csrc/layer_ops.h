@@ -12,16 +12,19 @@
 
 namespace fpk {
 
-// Every tensor here passes through once and is larger than the caches where time counts: loads and stores that do not claim
-// room in them.  B8 T4096 H16 128 x 128 (2.15 GB for both stages in both directions): 410 -> 377 us, 5.2 -> 5.7 TB/s; a
-// decode step of one or 256 sequences is as fast either way.
-FP_DEVICE u32x4 ld128_once(const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_m*>(p)); }
-FP_DEVICE void st128_once(uint16_t* p, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4_m*>(p)); }
+// Every tensor here passes through once.  Stores carry the hint not to claim room in the caches; with ONCE, for a launch whose
+// tensors are larger than those (passes_caches below), so do loads: those of a smaller one find their data there.
+template <bool ONCE>
+FP_DEVICE u32x4 load_once(const uint16_t* p) {
+  return ONCE ? __builtin_nontemporal_load(reinterpret_cast<const u32x4_m*>(p)) : ld128(p);
+}
+FP_DEVICE void store_once(uint16_t* p, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4_m*>(p)); }
 
 // ------------------------------------------------------------------------------------------
 // One thread: 8 adjacent features (4 rotation pairs) of one token, for p.heads_per_thread heads of
 // q and k (all of them when there are plenty of tokens: the sines and cosines are then computed
 // once per token; a single decode token is spread over more threads instead of more loop trips).
+template <bool ONCE>
 FP_DEVICE void rotary_qk(const RotaryArgs& p) {
   const int opr = p.d / 8;                                   // threads per token and head group
   const int hgroups = (p.H + p.heads_per_thread - 1) / p.heads_per_thread;
@@ -50,7 +53,7 @@ FP_DEVICE void rotary_qk(const RotaryArgs& p) {
       u32x4 v[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        if (h0 + u < h_end) v[u] = ld128_once(src + at0 + (size_t)(h0 + u) * p.d);
+        if (h0 + u < h_end) v[u] = load_once<ONCE>(src + at0 + (size_t)(h0 + u) * p.d);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
@@ -61,7 +64,7 @@ FP_DEVICE void rotary_qk(const RotaryArgs& p) {
           const float e = bf16_elem(v[u], 2 * j), d = bf16_elem(v[u], 2 * j + 1);
           o[j] = fprt::pack_bf16x2(e * cs[j] - d * sn[j], d * cs[j] + e * sn[j]);
         }
-        st128_once(dst + at0 + (size_t)(h0 + u) * p.d, o);
+        store_once(dst + at0 + (size_t)(h0 + u) * p.d, o);
       }
     }
   }
@@ -103,14 +106,15 @@ FP_DEVICE float round_bf16(float x) { return bf16_bits_to_float(float_to_bf16_bi
 
 // One thread: 8 adjacent values of one (row, head).  Threads past the last head take part in the
 // lane exchanges with zeros and touch no memory.
+template <bool ONCE>
 FP_DEVICE void gated_norm_fwd(const GatedNormArgs& p) {
   const int lanes = p.dv / 8;
   const long long unit = (long long)fprt::block_index() * LAYER_THREADS + fprt::thread_index();
   const bool live = unit / lanes < p.groups;
   const size_t at = (size_t)unit * 8;
   const u32x4 zero = {0, 0, 0, 0};
-  const u32x4 rv = live ? ld128_once(p.r + at) : zero;
-  const u32x4 gv = live ? ld128_once(p.g + at) : zero;
+  const u32x4 rv = live ? load_once<ONCE>(p.r + at) : zero;
+  const u32x4 gv = live ? load_once<ONCE>(p.g + at) : zero;
   const HeadStats st = head_stats(rv, lanes, p.dv, p.eps);
   float y[8];
 #pragma unroll
@@ -122,21 +126,22 @@ FP_DEVICE void gated_norm_fwd(const GatedNormArgs& p) {
   u32x4 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = fprt::pack_bf16x2(y[2 * e], y[2 * e + 1]);
-  if (live) st128_once(p.out + at, o);
+  if (live) store_once(p.out + at, o);
 }
 
 // With n^ = (r - mean) rstd, s = swish(g), dn = d_out * s:
 //   d_r = rstd (dn - mean(dn) - n^ mean(dn n^)),   d_g = d_out * n * swish'(g)
 // where n is n^ rounded to bf16 as the forward used it and swish'(g) = sig (1 + g (1 - sig)).
+template <bool ONCE>
 FP_DEVICE void gated_norm_bwd(const GatedNormArgs& p) {
   const int lanes = p.dv / 8;
   const long long unit = (long long)fprt::block_index() * LAYER_THREADS + fprt::thread_index();
   const bool live = unit / lanes < p.groups;
   const size_t at = (size_t)unit * 8;
   const u32x4 zero = {0, 0, 0, 0};
-  const u32x4 rv = live ? ld128_once(p.r + at) : zero;
-  const u32x4 gv = live ? ld128_once(p.g + at) : zero;
-  const u32x4 dv_ = live ? ld128_once(p.d_out + at) : zero;
+  const u32x4 rv = live ? load_once<ONCE>(p.r + at) : zero;
+  const u32x4 gv = live ? load_once<ONCE>(p.g + at) : zero;
+  const u32x4 dv_ = live ? load_once<ONCE>(p.d_out + at) : zero;
   const HeadStats st = head_stats(rv, lanes, p.dv, p.eps);
   float nh[8], dn[8], dg[8];
   float s1 = 0.f, s2 = 0.f;
@@ -160,12 +165,24 @@ FP_DEVICE void gated_norm_bwd(const GatedNormArgs& p) {
     o_g[e] = fprt::pack_bf16x2(dg[2 * e], dg[2 * e + 1]);
   }
   if (live) {
-    st128_once(p.d_r + at, o_r);
-    st128_once(p.d_g + at, o_g);
+    store_once(p.d_r + at, o_r);
+    store_once(p.d_g + at, o_g);
   }
 }
 
 // ------------------------------------------------------------------------------------------
+// Whether what a launch moves is more than the last-level cache (256 MB) holds of what the launch before left.  Measured, us, with
+// the hint on loads and stores | on stores | on neither (rotary + norm forward; rotary, op, norm forward; the same and backward):
+//   B4 T1024 H8 64 x 128    launches of 25 to 42 MB    12.4 | 11.1 | 12.4    35.8 | 34.8 | 36.0    106 | 103 | 102
+//   B8 T1024 H12 64 x 128   50 to 126 MB               26.8 | 24.8 | 24.7    52.6 | 50.2 | 47.5    140 | 134 | 136
+//   B2 T4096 H16 128 x 128  101 to 168 MB              51.5 | 50.2 | 48.8   111.1 | 108.2 | 108.8  273 | 272 | 272
+//   B8 T2048 H12 64 x 128   101 to 252 MB              45.2 | 41.5 | 40.9    90.1 | 87.1 | 87.9    248 | 258 | 262
+//   B4 T4096 H16 128 x 128  201 to 336 MB              85.7 | 80.8 | 93.9   186.3 | 192.4 | 189.6  490 | 494 | 495
+//   B8 T4096 H16 128 x 128  403 to 671 MB             163.3 | 170.8 | 178.0 276.6 | 290.9 | 292.8  736 | 771 | 785
+inline bool passes_caches(long long bytes) { return bytes >= 176000000LL; }
+inline bool passes_caches(const RotaryArgs& a) { return passes_caches((a.k_in ? 8LL : 4LL) * a.B * a.T * a.H * a.d); }
+inline bool passes_caches(const GatedNormArgs& a) { return passes_caches((a.out ? 6LL : 10LL) * a.groups * a.dv); }
+
 // Host side: argument checks and grid sizes, shared by the GPU launcher and the CPU test harness.
 // Return nullptr if the launch is valid (and the number of workgroups in `blocks`), else the reason.
 // (chooses a.heads_per_thread)

@@ -180,7 +180,7 @@ int fpk_launch_rotary(const fpk::RotaryArgs& args, void* /*stream*/, const char*
       fprt::g_lane.tid = t;
       fprt::g_lane.block = (int)blk;
       fprt::g_lane.grid = (int)blocks;
-      fpk::rotary_qk(a);
+      fpk::rotary_qk<false>(a);
     }
   }
   return 0;
@@ -193,7 +193,7 @@ int fpk_launch_gated_norm(const fpk::GatedNormArgs& a, void* /*stream*/, const c
     return 1;
   }
   return run_grid(fpk::LAYER_THREADS, (int)blocks, 0, [&](char*) {
-    if (a.out) fpk::gated_norm_fwd(a);
-    else fpk::gated_norm_bwd(a);
+    if (a.out) fpk::gated_norm_fwd<false>(a);
+    else fpk::gated_norm_bwd<false>(a);
   });
 }

@@ -164,3 +164,24 @@ def test_gated_group_norm_statistics_at_full_size(hip_lib):
     n = hp.raw_gated_norm_fwd(hip_lib, r, one).float().reshape(rows, H, dv)
     assert float(n.mean(-1).abs().max()) < 0.01
     assert float((n.square().mean(-1) - 1).abs().max()) < 0.01
+
+
+def test_large_launches_equal_small_ones():
+    """A launch that is larger than the caches loads with a hint (passes_caches in layer_ops.h); its results are those
+    of the same rows in two launches that are not."""
+    from flash_pop_amd import XPos, gated_group_norm
+    T, H, d = 6144, 16, 128                       # 201 MB for rotary, 151 and 252 MB for the norm, per launch of both halves
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, gate, dy = (torch.randn(2, T, H, d, generator=g, device=DEV).to(hp.BF16).requires_grad_(i < 3) for i in range(4))
+    xpos = XPos(d)
+
+    def step(rows):
+        rq, rk = xpos(q[rows], k[rows], 5)
+        y = gated_group_norm(q[rows], gate[rows].flatten(-2))
+        return (rq, rk, y, *torch.autograd.grad([rq, rk, y], [q, k, gate], [dy[rows], dy[rows], dy[rows].flatten(-2)]))
+
+    whole, parts = step(slice(0, 2)), [step(slice(i, i + 1)) for i in (0, 1)]
+    for i, got in enumerate(whole):
+        first, second = parts[0][i], parts[1][i]
+        ref = torch.cat((first, second)) if i < 3 else torch.cat((first[:1], second[1:]))
+        assert torch.equal(got, ref), i
