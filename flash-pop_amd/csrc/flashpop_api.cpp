@@ -770,8 +770,11 @@ int fp_retention_bwd_ckpt(const void* q, const void* k, const void* v, const voi
 size_t fp_retention_workspace_bytes(int B, int T, int H, int dk, int dv) {
   const Shape s{B, T, H, dk, dv};
   if (B < 1 || T < 1 || H < 1 || H > fpk::MAX_HEADS || !dim_ok(dk) || !dim_ok(dv)) return 0;
-  const int fwd = plan_forward(s), bwd = plan_backward(s);
-  return workspace_bytes(s, fwd > bwd ? fwd : bwd);
+  return workspace_bytes(s, plan_forward(s));   // (a backward is cut as its forward, or not at all)
+}
+
+size_t fp_retention_backward_workspace_bytes(int B, int T, int H, int dk, int dv) {
+  return fp_retention_workspace_bytes(B, T, H, dk, dv) ? workspace_bytes(Shape{B, T, H, dk, dv}, plan_backward(Shape{B, T, H, dk, dv})) : 0;
 }
 
 int fp_retention_fwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
@@ -843,6 +846,11 @@ size_t fp_pop_retention_workspace_bytes(int B, int T, int H, int dk, int dv, int
   const Shape s{B, T, H, dk, dv};
   if (B < 1 || T < 1 || H < 1 || H > fpk::MAX_HEADS || !dim_ok(dk) || !dim_ok(dv) || block_size < 1) return 0;
   return workspace_bytes(s, plan_pop_forward(s, block_size));
+}
+
+size_t fp_pop_retention_backward_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size) {
+  const Shape s{B, T, H, dk, dv};
+  return fp_pop_retention_workspace_bytes(B, T, H, dk, dv, block_size) ? workspace_bytes(s, plan_pop_backward(s, block_size)) : 0;
 }
 
 int fp_pop_retention_fwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
@@ -1000,6 +1008,6 @@ int fp_set_backward_choice(int choice, int checkpoint_every) {
 
 const char* fp_last_error(void) { return g_err; }
 
-int fp_version(void) { return 1008; }
+int fp_version(void) { return 1009; }
 
 }  // extern "C"

@@ -66,8 +66,8 @@ Tensor bytes_like(size_t n, const Tensor& t) { return at::empty({(int64_t)n}, t.
 Tensor state_like(const Tensor& t, const Shape& s) { return at::empty({s.B, s.H, s.dk, s.dv}, t.options()); }
 Tensor values_like(const Tensor& t, const Shape& s) { return at::empty({s.B, s.T, s.H, s.dv}, t.options()); }
 
-// What a forward leaves for its backward: states every `every` tokens, or (every = 0) the workspace of a forward that cut its
-// sequences into segments, which holds the state at the start of every segment.
+// What a forward leaves for its backward: states every `every` tokens, or (every = 0), where the backward is cut too, the workspace
+// of a forward that cut its sequences into segments, which holds the state at the start of every segment.
 struct Kept {
   Tensor t;
   int every = 0;
@@ -83,7 +83,7 @@ void retention_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
     Tensor ws = bytes_like(bytes, q);   // (from a stream-ordered allocator: handing it back right after the call is safe)
     check(fp_retention_fwd_split(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(o), ptr(s_out), n.B, n.T, n.H, n.dk, n.dv, ptr(ws),
                                  bytes, stream()));
-    if (for_backward) kept.t = ws;
+    if (for_backward && fp_retention_backward_workspace_bytes(n.B, n.T, n.H, n.dk, n.dv)) kept.t = ws;
     return;
   }
   int every = 0;
@@ -107,7 +107,7 @@ void pop_retention_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const 
     Tensor ws = bytes_like(bytes, q);
     check(fp_pop_retention_fwd_split(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(o), ptr(states), n.B, n.T, n.H, n.dk, n.dv, block,
                                      ptr(ws), bytes, stream()));
-    if (for_backward) kept.t = ws;
+    if (for_backward && fp_pop_retention_backward_workspace_bytes(n.B, n.T, n.H, n.dk, n.dv, block)) kept.t = ws;
     return;
   }
   check(fp_pop_retention_fwd(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(o), states.numel() ? ptr(states) : nullptr, n.B, n.T,
@@ -129,7 +129,7 @@ Grads retention_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Ten
     const void* const d_states = d_blocks.defined() && d_blocks.numel() ? ptr(d_blocks) : nullptr;
     Tensor ws = kept.t;
     if (!ws.defined()) {
-      if (const size_t bytes = fp_pop_retention_workspace_bytes(n.B, n.T, n.H, n.dk, n.dv, block)) ws = bytes_like(bytes, q);
+      if (const size_t bytes = fp_pop_retention_backward_workspace_bytes(n.B, n.T, n.H, n.dk, n.dv, block)) ws = bytes_like(bytes, q);
     }
     if (ws.defined())
       check(fp_pop_retention_bwd_split(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(d_o), d_states, ptr(r.dq), ptr(r.dk), ptr(r.dv),
@@ -147,7 +147,7 @@ Grads retention_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Ten
   }
   Tensor ws = kept.t;
   if (!ws.defined()) {
-    if (const size_t bytes = fp_retention_workspace_bytes(n.B, n.T, n.H, n.dk, n.dv)) ws = bytes_like(bytes, q);
+    if (const size_t bytes = fp_retention_backward_workspace_bytes(n.B, n.T, n.H, n.dk, n.dv)) ws = bytes_like(bytes, q);
   }
   if (ws.defined())
     check(fp_retention_bwd_split(ptr(q), ptr(k), ptr(v), ptr(s), g.data(), ptr(d_o), ptr(d_s_out), ptr(r.dq), ptr(r.dk), ptr(r.dv),

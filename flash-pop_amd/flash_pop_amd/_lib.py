@@ -28,6 +28,8 @@ SIGNATURES = {
     "fp_pop_retention_fwd": [_P, _P, _P, _P, _D, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "fp_pop_retention_bwd": [_P, _P, _P, _P, _D, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "fp_pop_retention_workspace_bytes": [_I, _I, _I, _I, _I, _I],
+    "fp_retention_backward_workspace_bytes": [_I, _I, _I, _I, _I],
+    "fp_pop_retention_backward_workspace_bytes": [_I, _I, _I, _I, _I, _I],
     "fp_pop_retention_fwd_split": [_P, _P, _P, _P, _D, _P, _P, _I, _I, _I, _I, _I, _I, _P, _Z, _P],
     "fp_pop_retention_bwd_split": [_P, _P, _P, _P, _D, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _Z, _I, _P],
     "fp_pop_fused_fwd": [_P] * 7 + [_D] + [_P] * 3 + [_I] * 7 + [_P],
@@ -51,8 +53,7 @@ def bind(path: str) -> ctypes.CDLL:
     for name, argtypes in SIGNATURES.items():
         fn = getattr(lib, name)          # AttributeError if the symbol is missing
         fn.argtypes = argtypes
-        fn.restype = {"fp_last_error": c_char_p, "fp_retention_workspace_bytes": c_size_t,
-                      "fp_pop_retention_workspace_bytes": c_size_t, "fp_retention_checkpoint_bytes": c_size_t}.get(name, c_int)
+        fn.restype = c_char_p if name == "fp_last_error" else c_size_t if name.endswith("_bytes") else c_int
     return lib
 
 

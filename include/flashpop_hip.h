@@ -96,8 +96,11 @@ int fp_retention_bwd_ckpt(const void* q, const void* k, const void* v, const voi
  *                                 for the same q, k, v, s0 and decays and nothing has written to it
  *                                 since; the backward then skips recomputing those states (one pass
  *                                 over k and v).  0: the workspace holds nothing of use.
- *                                 Either way its contents are undefined after the backward. */
+ *                                 Either way its contents are undefined after the backward.
+ *   fp_retention_backward_workspace_bytes  what the backward alone needs: 0 where only the forward is cut (the
+ *                                 workspace it leaves is of no use then), else the same bytes */
 size_t fp_retention_workspace_bytes(int B, int T, int H, int dk, int dv);
+size_t fp_retention_backward_workspace_bytes(int B, int T, int H, int dk, int dv);
 int fp_retention_fwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
                            void* o, void* s_out, int B, int T, int H, int dk, int dv, void* workspace,
                            size_t workspace_bytes, void* stream);
@@ -120,9 +123,10 @@ int fp_retention_fwd_split_static(const void* q, const void* k, const void* v, c
                                   void* stream);
 
 /* The POP entry points below for few streams and long sequences, cut at the blocks the way fp_retention_*_split cuts at
- * segments of its own choice; workspace and forward_states_kept as there.  0 bytes: the shape is not cut, and the calls are
+ * segments of its own choice; workspace, forward_states_kept and the two sizes as there.  0 bytes: the shape is not cut, and the calls are
  * fp_pop_retention_fwd / _bwd. */
 size_t fp_pop_retention_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size);
+size_t fp_pop_retention_backward_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size);
 int fp_pop_retention_fwd_split(const void* q, const void* k, const void* v, const void* s0, const double* head_decays,
                                void* o, void* block_states, int B, int T, int H, int dk, int dv, int block_size,
                                void* workspace, size_t workspace_bytes, void* stream);

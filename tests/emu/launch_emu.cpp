@@ -70,7 +70,10 @@ int fpk_stream_is_capturing(void* /*stream*/) { return g_emu_capturing; }
 
 // Pretends the chip has 8 compute units, so that small test shapes take the paths that large
 // ones take on a real device (several sequences per workgroup, split sequences).
-int fpk_launch_steps() { return 0; }   // the harness cuts whatever can be cut
+// By default launches cost nothing, so that the harness cuts whatever can be cut.
+static int g_emu_launch_steps = 0;
+extern "C" void emu_set_launch_steps(int steps) { g_emu_launch_steps = steps; }
+int fpk_launch_steps() { return g_emu_launch_steps; }
 int fpk_compute_units() { return 8; }
 
 // one translation unit per pair of head dimensions (fused_family.cpp)

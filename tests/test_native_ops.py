@@ -168,3 +168,38 @@ def test_in_place_steps_are_seen_by_the_graph(ops):
     with torch.inference_mode():
         state = s.clone()
     step(state, in_place=True)                                  # (has no version to advance)
+
+
+@pytest.fixture
+def launches_cost(emu):
+    """launches_cost(steps): what the harness's device takes a launch for, so that not everything that can be cut is"""
+    yield emu[0].emu_set_launch_steps
+    emu[0].emu_set_launch_steps(0)
+
+
+@pytest.mark.parametrize("T,block", [(650, 0), (326, 65)])
+def test_only_what_the_backward_uses_is_kept(emu, ops, launches_cost, T, block):
+    """The segment states of a cut forward go through the graph (and saved-tensor hooks) only if the backward is cut too; gradients
+    are the oracle's either way."""
+    lib, shape = emu[0], (1, T, 1, 64, 64) + ((block,) if block else ())
+    name = "fp_pop_retention" if block else "fp_retention"
+    forward, backward = getattr(lib, name + "_workspace_bytes"), getattr(lib, name + "_backward_workspace_bytes")
+    q, k, v, s = hp.make_inputs(1, T, 1, 64, 64, seed=T, state_std=0.3)
+    d_o, = hp.make_cotangents([(1, T, 1, 64)], seed=T)
+    q.requires_grad_()
+    call = (lambda: ops.flash_pop_retention(q, k, v, s, (0.97,), block)) if block else (lambda: ops.fused_chunk_retention(q, k, v, s, (0.97,)))
+    ref = (hp.oracle_pop(q, k, v, s, (0.97,), block, d_o, None) if block else hp.oracle_plain(q, k, v, s, (0.97,), d_o, None))[2][0]
+    seen = set()
+    for steps in range(40):
+        launches_cost(steps)
+        cut = (forward(*shape) > 0, backward(*shape) > 0)
+        if cut in seen or not cut[0]:
+            continue
+        seen.add(cut)
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t, lambda t: t):
+            out = call()[0]
+        assert len(packed) == (5 if cut[1] else 4)
+        hp.assert_close(torch.autograd.grad(out, q, d_o)[0], ref, f"dq, forward and backward cut: {cut}")
+    # (the cut of a POP call always pays for its backward too at a size that the harness can run)
+    assert seen == ({(True, True)} if block else {(True, True), (True, False)}), seen
