@@ -20,7 +20,7 @@ class FusedChunkRetention:
         if out is NotImplemented:
             if _ops.tracing():
                 return _ops.Traced.apply(FusedChunkRetention.apply, q, k, v, s, head_decays)
-            _ops.prepare(q, k, v, s, head_decays)
+            _ops.check_retention(q, k, v, s, head_decays)
             _ops.rejected("fused_chunk_retention")
         return out
 

@@ -15,6 +15,6 @@ def gated_group_norm(retention, gate, eps: float = 1e-6):
     if out is NotImplemented:
         if _ops.tracing():
             return _ops.Traced.apply(gated_group_norm, retention, gate, eps)
-        _ops.gated_norm_fwd(retention, gate, eps)   # raises
+        _ops.check_gated_norm(retention, gate)
         _ops.rejected("gated_group_norm")
     return out

@@ -24,7 +24,7 @@ def _refused(q, k, v, s, head_decays, block_size):
     """Raises for arguments that the native ops did not take; -> the shape if it is the suffixes' fault."""
     block_size = int(block_size)
     assert block_size >= 1, f"block_size must be positive, got {block_size}"
-    return _ops.prepare(q, k, v, s, head_decays)[4]
+    return _ops.check_retention(q, k, v, s, head_decays)
 
 
 class FlashPOPRetention:
@@ -53,7 +53,7 @@ class FlashPOPRetentionWithSuffixes:
             if _ops.tracing():
                 return _ops.Traced.apply(FlashPOPRetentionWithSuffixes.apply, q, k, v, s, head_decays, block_size, q_sfx, k_sfx, v_sfx)
             shape = _refused(q, k, v, s, head_decays, block_size)
-            _ops.prepare_suffixes(q_sfx, k_sfx, v_sfx, shape, int(block_size))
+            _ops.check_suffixes(q_sfx, k_sfx, v_sfx, shape, int(block_size))
             _ops.rejected("flash_pop_retention_with_suffixes")
         return out
 

@@ -40,6 +40,6 @@ class XPos:
         if out is NotImplemented:
             if _ops.tracing():
                 return _ops.Traced.apply(self, q, k, start_idx)
-            _ops.rotary_qk(q, k, theta, start_idx)   # raises
+            _ops.check_rotary(q, k, theta, start_idx)
             _ops.rejected("XPos")
         return out

@@ -203,3 +203,24 @@ def test_only_what_the_backward_uses_is_kept(emu, ops, launches_cost, T, block):
         hp.assert_close(torch.autograd.grad(out, q, d_o)[0], ref, f"dq, forward and backward cut: {cut}")
     # (the cut of a POP call always pays for its backward too at a size that the harness can run)
     assert seen == ({(True, True)} if block else {(True, True), (True, False)}), seen
+
+
+def test_pass_ops_refuse_graph_capture(emu, ops):
+    """Instantiating a HIP graph that holds the pass kernels has crashed the host process, so the retention ops raise, forward and
+    backward, while their stream records one (the harness's flag: nothing is recorded).  The small kernels can be recorded."""
+    calls = _calls(ops)
+    ins = {op: [t.requires_grad_() for t in inputs(1)] for op, (_, inputs) in calls.items()}
+    outs = {op: _tuple(call(*ins[op]))[0].sum() for op, (call, _) in calls.items()}
+    x = [t.detach()[:, 0] for t in ins["plain"][:3]]
+    emu[0].emu_set_capturing(1)
+    try:
+        for op, (call, _) in calls.items():
+            for run in (lambda: call(*ins[op]), lambda: torch.autograd.grad(outs[op], ins[op], allow_unused=True)):
+                if op in ("rotary", "norm"):
+                    run()
+                    continue
+                with pytest.raises(RuntimeError, match="cannot be captured into a HIP graph"):
+                    run()
+        ops.retention_recurrent(*x, DEC, None)
+    finally:
+        emu[0].emu_set_capturing(0)
