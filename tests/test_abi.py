@@ -125,6 +125,25 @@ def test_new_entry_points_check_their_arguments(lib):
     assert lib.fp_retention_bwd_split(p, p, p, null, dec, null, null, p, p, p, null, 1, 8, 2, 64, 64, null, 0, 0, None) == -1
 
 
+@pytest.mark.parametrize("segments,backward,B,T,H,dk,dv", [
+    (5, False, 1, 1152, 4, 64, 64),       # 18 chunks
+    (0, False, 1, 832, 4, 64, 64),        # 13
+    (20, True, 1, 5003, 12, 64, 128),
+    (0, False, 1, 1152, 12, 64, 128),
+    (5, False, 3, 1777, 8, 128, 128),     # the forward alone
+    (0, False, 3, 1152, 8, 128, 128),
+    (8, True, 2, 2560, 8, 128, 256),
+    (0, False, 2, 1792, 8, 128, 256),
+    (8, True, 2, 16384, 8, 128, 256),    # equal segments
+    (0, False, 8, 4096, 16, 128, 128),    # enough streams
+])
+def test_calls_are_cut_where_it_pays(lib, segments, backward, B, T, H, dk, dv):
+    """On a device of 256 compute units (what the library takes a machine without a GPU for)."""
+    bytes_ = 4 * B * segments * H * dk * dv
+    assert lib.fp_retention_workspace_bytes(B, T, H, dk, dv) == bytes_
+    assert lib.fp_retention_backward_workspace_bytes(B, T, H, dk, dv) == (bytes_ if backward else 0)
+
+
 @pytest.mark.parametrize("cut,B,T,H,dk,dv,block", [
     (True, 4, 1440, 4, 64, 128, 144),      # 5 MB of block states against a chain of 30 chunks
     (True, 4, 4096, 4, 128, 128, 64),      # 67 MB, 64 chunks: just worth it

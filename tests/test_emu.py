@@ -164,20 +164,22 @@ def test_split_sequences_fwd_bwd(emu_lib, B, T, H, dk, dv, state_std, segments):
     assert torch.equal(o2, o) and all(torch.equal(a, b) for a, b in zip(again, (dq, dk_, dv_, ds0)))
 
 
-@pytest.mark.parametrize("B,T,H,dk,dv,state_std,segments", [
-    (1, 257, 1, 64, 64, 0.5, 2),       # the last segment is one token
-    (1, 511, 1, 128, 128, 0.5, 2),     # one token short of two whole segments: the state-only kernel's chunk that begins before its segment
-    (1, 700, 1, 64, 128, None, 3),     # 11 chunks, the last one short, no initial state
-    (1, 704, 1, 64, 64, 0.5, 3),       # 11 whole chunks in segments of 4, 4 and 3
-    (2, 300, 1, 128, 128, 0.5, 1),     # too many streams for the harness's 8 units: not cut
-    (1, 300, 1, 128, 256, 0.3, 2),     # two workgroups per segment in the state-only kernel
-    (1, 330, 1, 256, 64, 0.3, 2),      # the state-only walk visits every chunk twice
-    (2, 330, 1, 64, 64, 0.5, 2),       # rows of the second sequence start inside a chunk
+@pytest.mark.parametrize("B,T,H,dk,dv,state_std,segments,gamma", [
+    (1, 257, 1, 64, 64, 0.5, 2, 0.9),       # the last segment is one token
+    (1, 511, 1, 128, 128, 0.5, 2, 0.9),     # one token short of two whole segments: a short last chunk in the state-only kernel
+    (1, 700, 1, 64, 128, None, 3, 0.9),     # 11 chunks, the last one short, no initial state
+    (1, 704, 1, 64, 64, 0.5, 3, 0.9),       # 11 whole chunks in segments of 4, 4 and 3
+    (2, 300, 1, 128, 128, 0.5, 1, 0.9),     # too many streams for the harness's 8 units: not cut
+    (1, 300, 1, 128, 256, 0.3, 2, 0.9),     # two workgroups per segment in the state-only kernel
+    (1, 330, 1, 256, 64, 0.3, 2, 0.9),      # the state-only walk visits every chunk twice
+    (2, 330, 1, 64, 64, 0.5, 2, 0.9),       # rows of the second sequence start inside a chunk
+    (1, 700, 1, 64, 64, 0.5, 3, 0.99),
+    (1, 620, 1, 128, 128, 0.5, 3, 0.99),
 ])
-def test_split_sequences_uneven(emu_lib, B, T, H, dk, dv, state_std, segments):
-    """Sequences that do not fall into equal segments of whole chunks, every segment with a decay strong enough that a
-    state one token off would show."""
-    decays = (0.9,) * H
+def test_split_sequences_uneven(emu_lib, B, T, H, dk, dv, state_std, segments, gamma):
+    """Sequences that do not fall into equal segments of whole chunks, with a decay strong enough that a state one token off
+    would show, and with one that leaves something of a state over a whole segment (0.99^256 = 0.08)."""
+    decays = (gamma,) * H
     q, k, v, s = hp.make_inputs(B, T, H, dk, dv, seed=T, state_std=state_std)
     d_o, d_s = hp.make_cotangents([(B, T, H, dv), (B, H, dk, dv)], seed=T + 1)
     o, S, nbytes, ws = hp.raw_split_fwd(emu_lib, q, k, v, s, decays, keep_workspace=True)

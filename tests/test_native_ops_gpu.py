@@ -13,7 +13,7 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("wanted", ["qkvs", "q", "s", "kv"])
-@pytest.mark.parametrize("T", [70, 1100])      # 1100: the sequences are cut into segments
+@pytest.mark.parametrize("T", [70, 1100, 2001])   # 1100: the forward is cut into segments; 2001: the backward too
 def test_gradients_of_some_inputs_from_some_outputs(wanted, T):
     from flash_pop_amd import fused_chunk_retention
     B, H, d = 1, 2, 64
@@ -59,9 +59,9 @@ def test_no_grad_in_place_changes_and_reuse():
 def test_saved_tensor_hooks_see_all_and_tangents_are_refused():
     from flash_pop_amd import XPos, flash_pop_retention, fused_chunk_retention, gated_group_norm
     decays = oracle.head_decays(2)
-    q, k, v, s = hp.make_inputs(1, 1600, 2, 64, 64, seed=8, state_std=0.3, device=DEV)
+    q, k, v, s = hp.make_inputs(1, 2001, 2, 64, 64, seed=8, state_std=0.3, device=DEV)
     q.requires_grad_()
-    for op, args in ((fused_chunk_retention, ()), (flash_pop_retention, (160,))):     # both cut into segments
+    for op, args in ((fused_chunk_retention, ()), (flash_pop_retention, (160,))):     # both cut into segments, both ways
         ref = torch.autograd.grad(op(q, k, v, s, decays, *args)[0].sum(), q)[0]
         packed = []
         with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.numel()) or t.cpu(), lambda t: t.to(DEV)):
@@ -84,8 +84,8 @@ def test_saved_tensor_hooks_see_all_and_tangents_are_refused():
 def test_threads_with_streams_of_their_own():
     from flash_pop_amd import fused_chunk_retention
     decays = oracle.head_decays(4)
-    q, k, v, s = hp.make_inputs(2, 1200, 4, 64, 64, seed=6, state_std=0.3, device=DEV)
-    d_o, = hp.make_cotangents([(2, 1200, 4, 64)], seed=7, device=DEV)
+    q, k, v, s = hp.make_inputs(2, 3001, 4, 64, 64, seed=6, state_std=0.3, device=DEV)   # cut into segments both ways
+    d_o, = hp.make_cotangents([(2, 3001, 4, 64)], seed=7, device=DEV)
 
     def step():
         leaves = [t.detach().clone().requires_grad_() for t in (q, k, v, s)]

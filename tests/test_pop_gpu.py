@@ -71,18 +71,59 @@ def test_pop_without_state_argument():
 
 
 def test_pop_outputs_equal_plain_outputs():
-    """The context outputs of the POP op are those of the plain entry point (same chunk partition
+    """The context outputs of a POP op that runs in one walk are those of the plain entry point (same chunk partition
     when block is a chunk multiple -> bit-identical), and its last block state is the plain final
     state.  The plain side is called through the C ABI: the Python op may cut such a shape into
-    segments, which rounds differently."""
+    segments, which rounds differently.  (So does a POP call that is cut at its blocks, by the order of fp32 sums.)"""
     from flash_pop_amd import flash_pop_retention, _lib
     B, T, H, d, block = 2, 1024, 4, 128, 128
+    assert _lib.load().fp_pop_retention_workspace_bytes(B, T, H, d, d, block) == 0
     decays = oracle.head_decays(H)
     q, k, v, s = hp.make_inputs(B, T, H, d, d, seed=21, state_std=0.1, device=DEV)
     o_pop, states = flash_pop_retention(q, k, v, s, decays, block)
     o, S = hp.raw_fwd(_lib.load(), q, k, v, s, decays)
     torch.cuda.synchronize()
     assert torch.equal(o_pop, o) and torch.equal(states[:, -1], S)
+
+
+@pytest.mark.parametrize("B,T,H,dk,dv,block", [
+    (1, 1500, 4, 128, 128, 144),   # the 128-wide state-only kernel, blocks and a tail that end inside a chunk
+    (2, 1000, 4, 128, 64, 100),    # the pass kernel's state-only walk, the sequence ends on a boundary
+    (1, 1500, 2, 256, 64, 144),
+    (1, 1537, 2, 128, 128, 128),   # whole chunks per block, a tail of one token
+    (1, 832, 2, 64, 64, 64),
+])
+def test_pop_split_entry_points(hip_lib, B, T, H, dk, dv, block):
+    """fp_pop_retention_*_split on shapes that are cut at their blocks, the backward from the states that the forward left and
+    from recomputed ones: against the oracle, and against the uncut entry points (order of fp32 sums; of the gradients, other
+    operands are weighed)."""
+    _say(f"[pop split] B{B} T{T} H{H} dk{dk} dv{dv} block={block}")
+    decays = oracle.head_decays(H, (5, 9))
+    q, k, v, s = hp.make_inputs(B, T, H, dk, dv, seed=T, state_std=0.3, device=DEV)
+    d_o, d_b = hp.make_cotangents([(B, T, H, dv), (B, T // block, H, dk, dv)], seed=T + 1, device=DEV)
+    nbytes = hip_lib.fp_pop_retention_workspace_bytes(B, T, H, dk, dv, block)
+    assert nbytes > 0 and hip_lib.fp_pop_retention_backward_workspace_bytes(B, T, H, dk, dv, block) == nbytes
+    ws, p, dec = torch.empty(nbytes, dtype=torch.uint8, device=DEV), hp._p, hp._dec(decays)
+    nan = lambda *shape: torch.full(shape, float("nan"), dtype=torch.bfloat16, device=DEV)
+    o, states = nan(*d_o.shape), nan(*d_b.shape)
+    assert hip_lib.fp_pop_retention_fwd_split(p(q), p(k), p(v), p(s), dec, p(o), p(states), B, T, H, dk, dv, block, p(ws), nbytes, None) == 0
+    kept = []
+    for forward_states in (1, 0):
+        kept.append([nan(*t.shape) for t in (q, k, v, s)])
+        assert hip_lib.fp_pop_retention_bwd_split(p(q), p(k), p(v), p(s), dec, p(d_o), p(d_b), *[p(g) for g in kept[-1]], B, T, H, dk, dv,
+                                                  block, p(ws), nbytes, forward_states, None) == 0
+    o1, states1 = hp.raw_pop_fwd(hip_lib, q, k, v, s, decays, block)
+    torch.cuda.synchronize()
+    o_ref, st_ref, refs = hp.oracle_pop(q, k, v, s, decays, block, d_o, d_b)
+    hp.assert_close(o, o_ref, "o", head_dim=2)
+    hp.assert_close(states, st_ref, "states", head_dim=2)
+    for name, grad, again, ref in zip(("dq", "dk", "dv", "ds0"), *kept, refs):
+        hp.assert_close(grad, ref, name, head_dim=1 if name == "ds0" else 2)
+        assert torch.equal(grad, again), name
+    # (a state element that moved by a few 2^-24 rounds to another bf16 operand in one case of 2^13, and dk of them make an output)
+    for name, cut, uncut in (("o", o, o1), ("states", states, states1)):
+        share = float((cut != uncut).float().mean())
+        assert share <= 2e-3, (name, share)
 
 
 def _suffix_case(B, N, block, Ls, H, dk, dv, seed, oracle_batches, oracle_device="cpu", literal=None):

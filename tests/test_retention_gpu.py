@@ -333,7 +333,12 @@ def test_decode_step_kernel_256_steps():
     hp.assert_close(s1, s1_ref, "state, no state")
 
 
-@pytest.mark.parametrize("B,T,H,dk,dv", [(1, 8192, 2, 128, 128), (1, 4096, 2, 256, 128), (2, 2240, 3, 128, 256)])
+@pytest.mark.parametrize("B,T,H,dk,dv", [
+    (1, 8192, 2, 128, 128), (1, 4096, 2, 256, 128), (2, 2240, 3, 128, 256),
+    # uneven segments, whose states are fp32: the last one ends inside a chunk
+    (1, 5003, 4, 128, 128), (1, 2501, 2, 128, 256), (2, 1500, 2, 64, 128), (1, 2000, 2, 192, 128), (1, 3001, 2, 256, 64),
+    (1, 2305, 4, 128, 128),   # ... is one token
+])
 def test_split_entry_points_long_sequence_few_streams(B, T, H, dk, dv):
     """fp_retention_*_split on shapes the library cuts into segments (a few streams on a 256-CU device; with
     256-wide keys the state-only walk visits every chunk twice; the last case has 7 segments of 5 chunks and two
@@ -347,6 +352,7 @@ def test_split_entry_points_long_sequence_few_streams(B, T, H, dk, dv):
     d_o, d_s = hp.make_cotangents([(B, T, H, dv), (B, H, dk, dv)], seed=78, device=DEV)
     o, S, nbytes = hp.raw_split_fwd(lib, q, k, v, s, decays)
     assert nbytes > 0 and nbytes % (2 * 2 * B * H * dk * dv) == 0, nbytes
+    assert lib.fp_retention_backward_workspace_bytes(B, T, H, dk, dv) == nbytes   # both directions are cut
     grads = hp.raw_split_bwd(lib, q, k, v, s, decays, d_o, d_s)
     o1, S1 = hp.raw_fwd(lib, q, k, v, s, decays)
     grads1 = hp.raw_bwd(lib, q, k, v, s, decays, d_o, d_s)
@@ -357,7 +363,7 @@ def test_split_entry_points_long_sequence_few_streams(B, T, H, dk, dv):
     hp.assert_close(S, S_ref, "S", head_dim=1)
     for n, g, r in zip(names, grads, g_ref):
         hp.assert_close(g, r, n, head_dim=1 if n == "ds0" else 2)
-    # the two routes differ only by the bf16 rounding of the segment states
+    # the two routes differ only by the rounding of the segment states (to bf16 between equal segments)
     hp.assert_close(o, o1.float(), "o vs unsplit", head_dim=2)
     for n, g, g1 in zip(names, grads, grads1):
         hp.assert_close(g, g1.float(), f"{n} vs unsplit", head_dim=1 if n == "ds0" else 2)
