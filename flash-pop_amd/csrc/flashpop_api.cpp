@@ -627,12 +627,12 @@ int backward_split(const Shape& s, const Shape& seg, const void* q, const void* 
   return run_dk_dv(a, b, stream, "dk / dv");
 }
 
-int check_workspace(const Shape& s, int segments, const void* workspace, size_t bytes) {
+int check_workspace(const Shape& s, int segments, const void* workspace, size_t bytes, const char* query = "fp_retention_workspace_bytes") {
   if (segments <= 1) return FP_OK;
-  if (!workspace) return fail(FP_ERR_NULL_POINTER, "workspace is NULL but fp_retention_workspace_bytes() is nonzero for this shape");
+  if (!workspace) return fail(FP_ERR_NULL_POINTER, "workspace is NULL but %s() is nonzero for this shape", query);
   if (bytes < workspace_bytes(s, segments))
-    return fail(FP_ERR_BAD_SHAPE, "workspace of %zu bytes is smaller than the %zu that fp_retention_workspace_bytes() asks for",
-                bytes, workspace_bytes(s, segments));
+    return fail(FP_ERR_BAD_SHAPE, "workspace of %zu bytes is smaller than the %zu that %s() asks for", bytes,
+                workspace_bytes(s, segments), query);
   if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return fail(FP_ERR_BAD_SHAPE, "workspace must be 16-byte aligned");
   return FP_OK;
 }
@@ -862,7 +862,7 @@ int fp_pop_retention_fwd_split(const void* q, const void* k, const void* v, cons
     return fp_pop_retention_fwd(q, k, v, s0, head_decays, o, block_states, B, T, H, dk, dv, block_size, stream);
   if (int rc = check_stream(stream, "fp_pop_retention_fwd_split")) return rc;
   if (!q || !k || !v || !o || !block_states) return fail(FP_ERR_NULL_POINTER, "q, k, v, o and block_states must not be NULL");
-  if (int rc = check_workspace(s, segments, workspace, workspace_bytes_given)) return rc;
+  if (int rc = check_workspace(s, segments, workspace, workspace_bytes_given, "fp_pop_retention_workspace_bytes")) return rc;
   return forward_split(s, block_segments(s, block_size), q, k, v, s0, head_decays, o, nullptr, workspace, stream,
                        BlockStates{out(block_states), nullptr, T / block_size});
 }
@@ -878,7 +878,7 @@ int fp_pop_retention_bwd_split(const void* q, const void* k, const void* v, cons
   if (int rc = check_stream(stream, "fp_pop_retention_bwd_split")) return rc;
   if (!q || !k || !v || !d_o || !dq || !dk_ || !dv_)
     return fail(FP_ERR_NULL_POINTER, "q, k, v, d_o, dq, dk and dv must not be NULL");
-  if (int rc = check_workspace(s, segments, workspace, workspace_bytes_given)) return rc;
+  if (int rc = check_workspace(s, segments, workspace, workspace_bytes_given, "fp_pop_retention_workspace_bytes")) return rc;
   return backward_split(s, block_segments(s, block_size), q, k, v, s0, head_decays, d_o, nullptr, dq, dk_, dv_, d_s0, workspace,
                         forward_states_kept != 0, stream, BlockStates{nullptr, in(d_block_states), T / block_size});
 }

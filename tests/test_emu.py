@@ -232,7 +232,8 @@ def test_pop_split_at_blocks(emu_lib, B, T, H, dk, dv, block, state_std, segment
             assert oracle.rms_error_ratio(g.float(), ref) <= 1.05 * oracle.rms_error_ratio(u.float(), ref), name
     if nbytes:   # argument checks come before any launch
         rc = lambda w, n: emu_lib.fp_pop_retention_fwd_split(p(q), p(k), p(v), p(s), dec, p(o), p(states), B, T, H, dk, dv, block, w, n, None)
-        assert rc(None, 0) == -1 and rc(p(ws), nbytes - 16) == -2
+        assert rc(None, 0) == -1 and b"fp_pop_retention_workspace_bytes" in emu_lib.fp_last_error()
+        assert rc(p(ws), nbytes - 16) == -2 and b"fp_pop_retention_workspace_bytes" in emu_lib.fp_last_error()
 
 
 @pytest.mark.parametrize("T,dk,dv,block", [
