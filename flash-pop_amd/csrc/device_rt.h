@@ -61,6 +61,8 @@ FP_DEVICE void wave_sync() { __builtin_amdgcn_wave_barrier(); }
 
 // Nothing may be moved across this point by the instruction scheduler.
 FP_DEVICE void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
+// A value that has to be there (a load: has to have arrived) at this point.
+FP_DEVICE void keep(u32x4 v) { asm volatile("" ::"v"(v)); }
 
 // Bounds-checked view of global memory (raw buffer resource): loads beyond `nbytes` return
 // zero and stores beyond it are dropped by the hardware, which is how ragged chunk tails

@@ -553,7 +553,8 @@ Shape block_segments(const Shape& s, int block) {
 int contributions(const Shape& seg, const double* decays, const void* w_rows, const void* z_rows, int reverse,
                   const Workspace& w, void* stream) {
   const float sc = 1.0f / std::sqrt((float)seg.dk);
-  if (seg.dk == fpk::FB_D && seg.dv % fpk::FB_D == 0) {   // the kernel that holds 128 x 128 of the state per workgroup
+  // the kernel that holds 128 x 128 of the state per workgroup
+  if (seg.dk == fpk::FB_D && seg.dv % fpk::FB_D == 0 && fpk::contrib_fits(seg.T, seg.H, seg.dv)) {
     fpk::ContribArgs c;
     std::memset(&c, 0, sizeof c);
     c.W = in(w_rows); c.Z = in(z_rows); c.U = w.contrib; c.U_lo = w.contrib_lo;

@@ -125,6 +125,9 @@ struct ContribArgs {
   float s_update;
   float log2g[MAX_HEADS];
 };
+// Whether the rows of whole chunks, those beyond a sequence's end included, have 32-bit byte offsets in that pass (one that wrapped
+// would come back into its view).
+inline bool contrib_fits(long long T, int H, int dB) { return (T + CH) * H * dB * 2 < (1LL << 32); }
 // One recurrent (decode) step for every (batch, head):  S' = gamma S + (scale k)^T v,  o = q S'.
 // q, k [B,H,dk]; v, o [B,H,dv]; S [B,H,dk,dv]; all bf16, fp32 arithmetic.  s_out may be s_in.
 struct DecodeArgs {

@@ -12,6 +12,8 @@
 // helpers are those of retention_bwd_fused.h); two more chunks are on their way in registers.  One
 // workgroup barrier per chunk.
 #pragma once
+#include <type_traits>
+
 #include "pass_args.h"
 #include "lds_access.h"
 #include "retention_bwd_fused.h"
@@ -86,8 +88,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     const fprt::BufView w = live ? wv : none, z = live ? zv : none;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int r = live ? t0 + ld_row + 32 * u : 0;
-      const uint32_t row = r < len ? r : len;   // beyond a short last chunk: row `len`, the first one beyond the views, reads as zero
+      const uint32_t row = live ? t0 + ld_row + 32 * u : 0u;   // rows of a short last chunk beyond `len` read as zeros (contrib_fits)
       pf[u] = fprt::buf_load128(w, row * roww + ld_piece * 16);
       pf[2 + u] = fprt::buf_load128(z, row * rowz + ld_piece * 16);
     }
@@ -115,14 +116,14 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   racc[0] = f32x16{0};
   racc[1] = f32x16{0};
 
-  // `L` tokens of the chunk are there.  Walking forward a short chunk is the last one and its weights count from its last token (in
-  // the order of the walk that carries a sequence through, so that a cut call gives the state of the uncut one); walking
-  // backward it is the first one, met with R = 0, and its weights are those of any other.
-  auto update = [&](int s, int L) {
+  // L: tokens of the chunk, where it is the short last one of a forward walk (CH otherwise): its weights count from its last token, as
+  // in the walk that carries a sequence through, so that a cut call gives the state of the uncut one.  (Walking backward a short
+  // chunk is the first one, met with R = 0, and its weights are those of any other.)
+  auto update = [&](int s, auto short_chunk, int L) {
+    constexpr bool SHORT = decltype(short_chunk)::value;
     const uint16_t* const Ws = TL + (2 * s) * FB_TILE;
     const uint16_t* const Zs = Ws + FB_TILE;
-    const bool whole = REV || L == CH;
-    const float decay = whole ? gL : fprt::exp2_approx((float)L * lg);
+    const float decay = SHORT ? fprt::exp2_approx((float)L * lg) : gL;
     u32x4 ua[4], ub0[4], ub1[4];
     auto request = [&](int tt) {
       const int t = REV ? tt : 3 - tt;
@@ -144,7 +145,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     fprt::sched_fence();
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
-      if (!whole) {
+      if (SHORT) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int left = L - 1 - 16 * (3 - tt) - nat_token(g, e);
@@ -166,22 +167,30 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   // Chunk it is multiplied from stage it & 1 while chunk it + 1 moves from registers into the
   // other stage and the loads of chunk it + 3 take its place; chunk it + 2 is on its way in the
   // second set of registers.
-  auto tokens = [&](int it) { return len - it * CH < CH ? len - it * CH : CH; };   // walking forward
+  const int nwhole = REV ? nch : len / CH;
   u32x4 pa[4], pb[4];
   load(0, pa);
   load(1, pb);
   stage(0, pa);
   load(2, pa);
   fprt::block_sync();
-  for (int it = 0; it < nch; it += 2) {
+  for (int it = 0; it < nwhole; it += 2) {
     stage(1, pb);
     load(it + 3, pb);
-    update(0, tokens(it));
+    update(0, std::false_type{}, CH);
     fprt::block_sync();
-    if (it + 1 >= nch) break;
+    if (it + 1 >= nwhole) break;
     stage(0, pa);
     load(it + 4, pa);
-    update(1, tokens(it + 1));
+    update(1, std::false_type{}, CH);
+    fprt::block_sync();
+  }
+  // (pb is wanted on both ways out of the loop, or the compiler moves its loads behind the break, a chunk later: 42 -> 46 us at
+  // B2 H8 T16384 dv 256)
+#pragma unroll
+  for (int u = 0; u < 4; ++u) fprt::keep(pb[u]);
+  if (nwhole < nch) {
+    update(nwhole & 1, std::true_type{}, len - nwhole * CH);
     fprt::block_sync();
   }
 
@@ -200,6 +209,7 @@ inline const char* check_contrib(const ContribArgs& a) {
     return "state-only pass: segments that do not cover their sequence";
   if (a.dB < FB_D || a.dB % FB_D != 0) return "state-only pass: Z must have a multiple of 128 columns";
   if (!a.W || !a.Z || !a.U) return "state-only pass: null pointer";
+  if (!contrib_fits(a.T, a.H, a.dB)) return "state-only pass: sequence too long";
   if ((long long)a.B * a.H * (a.dB / FB_D) > 0x7fffffffLL) return "state-only pass: too many sequences";
   return nullptr;
 }

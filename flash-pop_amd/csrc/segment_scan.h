@@ -33,19 +33,22 @@ FP_DEVICE void segment_scan_form(const ScanArgs& p) {
     for (int e = 0; e < SCAN_VEC; ++e) r[e] = 0.f;
   }
   auto segment = [&](int i) { return p.reverse ? p.S - 1 - i : i; };
-  auto block = [&](int m) { return (((size_t)b * p.nblk + m) * p.H + h) * p.M + in_mat; };
-  auto matrix = [&](int i) { return (((size_t)b * p.S + segment(i)) * p.H + h) * p.M + in_mat; };
+  const size_t step = (size_t)p.H * p.M;   // elements between the matrices of two segments, or blocks, of a sequence
+  const size_t block0 = (size_t)b * p.nblk * step + (size_t)h * p.M + in_mat, matrix0 = (size_t)b * p.S * step + (size_t)h * p.M + in_mat;
+  auto block = [&](int m) { return block0 + (size_t)m * step; };
+  auto joins = [&](int i) { return p.blocks_in && segment(i) < p.nblk; };
+  auto matrix = [&](int i) { return matrix0 + (size_t)segment(i) * step; };
   for (int i0 = 0; i0 < p.S; i0 += SCAN_AHEAD) {
     u32x4 u[SCAN_AHEAD], ulo[LO ? SCAN_AHEAD : 1], add[BLOCKS ? SCAN_AHEAD : 1];
-    // (init may be U: a batch is read before its first element is written)
+    // (init may be U: a batch is read before its first element is written.)  Every load is issued, those beyond the last segment or
+    // block on what another step reads as well: behind branches the compiler waits for each before the next (B1 H12 T5003 64 x 128,
+    // 20 segments: 13.2 us a launch so, 8.7 us without; B2 H8 T16384 128 x 256, 8 segments: 8.8, 7.2).
 #pragma unroll
     for (int j = 0; j < SCAN_AHEAD; ++j) {
-      if (BLOCKS) add[BLOCKS ? j : 0] = u32x4{0, 0, 0, 0};
-      if (i0 + j < p.S) {
-        u[j] = ld128(p.U + matrix(i0 + j));
-        if (LO) ulo[LO ? j : 0] = ld128(p.U_lo + matrix(i0 + j));
-        if (BLOCKS && p.blocks_in && segment(i0 + j) < p.nblk) add[BLOCKS ? j : 0] = ld128(p.blocks_in + block(segment(i0 + j)));
-      }
+      const int i = i0 + j < p.S ? i0 + j : p.S - 1;
+      u[j] = ld128(p.U + matrix(i));
+      if (LO) ulo[LO ? j : 0] = ld128(p.U_lo + matrix(i));
+      if (BLOCKS) add[BLOCKS ? j : 0] = ld128(joins(i) ? p.blocks_in + block(segment(i)) : p.U + matrix(i));
     }
 #pragma unroll
     for (int j = 0; j < SCAN_AHEAD; ++j) {
@@ -58,7 +61,7 @@ FP_DEVICE void segment_scan_form(const ScanArgs& p) {
       };
 #pragma unroll
       for (int e = 0; e < SCAN_VEC; ++e) {
-        if (BLOCKS) r[e] += bf16_elem(add[BLOCKS ? j : 0], e);
+        if (BLOCKS && joins(i0 + j)) r[e] += bf16_elem(add[BLOCKS ? j : 0], e);
       }
       if constexpr (LO) {
         store(p.init + matrix(i0 + j), UpperHalf{});
