@@ -1,8 +1,8 @@
 // The ops of flash_pop_amd as a CPython extension over the C ABI: argument checks, output and workspace allocation, launches and
 // autograd nodes in native code.  With these in Python, behind ctypes, a call of a few microseconds of kernels was bound by its host
 // work: 16 us a forward, 100 us and more a backward, which the autograd thread ran under the interpreter lock.  Before and
-// after, per pass: decode layer step B1 H12 64 x 128 (three calls) 53 -> 20 us, forward B1 H4 T512 64 x 64 28 -> 17 us (now its
-// three launches), forward + backward B3 H8 T1777 128 x 128 166 -> 89 us and B32 H4 T2048 64 x 64 148 -> 118 us (now their kernels).
+// after, per pass: decode layer step B1 H12 64 x 128 (three calls) 53 -> 21 us, forward B1 H4 T512 64 x 64 28 -> 17 us in three
+// launches (12.5 us in the one it is now), forward + backward B32 H4 T2048 64 x 64 148 -> 118 us (now its kernels).
 //
 // Functions return NotImplemented when an argument is not what they take, or the call is being traced; the Python wrappers then
 // raise the exception that says what is wrong, or make the call one that can be traced (flash_pop_amd/_ops.py).  Errors of the C ABI become RuntimeError.

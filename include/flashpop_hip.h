@@ -84,7 +84,8 @@ int fp_retention_bwd_ckpt(const void* q, const void* k, const void* v, const voi
  * The _split variants cut every sequence into segments that run as separate sequences (a
  * state-only pass and a scan give each segment its starting state first); they need scratch
  * memory from the caller.  Same arguments, results and error behaviour as fp_retention_fwd /
- * fp_retention_bwd otherwise; segment states pass through bf16.  No counterpart in the
+ * fp_retention_bwd otherwise; the states between segments of equal length pass through bf16, those between uneven ones
+ * are fp32 (in the workspace: the upper 16 bits of all elements, then the lower 16).  No counterpart in the
  * reference, whose kernels also walk a sequence serially (fused_chunk_fwd.py:95-187).
  *   fp_retention_workspace_bytes  scratch bytes the two calls need for this shape on the current
  *                                 device; 0 means they would not cut (and accept workspace = NULL)
@@ -123,7 +124,9 @@ int fp_retention_fwd_split_static(const void* q, const void* k, const void* v, c
                                   void* stream);
 
 /* The POP entry points below for few streams and long sequences, cut at the blocks the way fp_retention_*_split cuts at
- * segments of its own choice; workspace, forward_states_kept and the two sizes as there.  0 bytes: the shape is not cut, and the calls are
+ * segments of its own choice, where the states of all blocks are worth moving; the states between blocks are fp32.  Where blocks
+ * are whole 64-token chunks the o of a call that is not cut is that of fp_retention_fwd bit for bit; that of a cut one differs
+ * by the order of fp32 sums.  workspace, forward_states_kept and the two sizes as there.  0 bytes: the shape is not cut, and the calls are
  * fp_pop_retention_fwd / _bwd. */
 size_t fp_pop_retention_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size);
 size_t fp_pop_retention_backward_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size);
