@@ -622,6 +622,7 @@ PyObject* py_pop_with_suffixes(PyObject*, PyObject* const* a, Py_ssize_t nargs) 
 PyObject* py_decode_step(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (!count(nargs, 6)) return nullptr;
+  if (traced()) return not_implemented();
   Tensor q, k, v, s, o, s_out;
   Decays g;
   if (!as_tensor(a[0], q) || !as_tensor(a[1], k) || !as_tensor(a[2], v) || !as_tensor(a[3], s) || !q.defined() || !k.defined() || !v.defined())

@@ -17,6 +17,8 @@ def retention_recurrent(query, key, value, head_decays, prev_state, in_place=Fal
         head_decays = tuple(head_decays.flatten().tolist())
     out = _lib.native().decode_step(query, key, value, prev_state, head_decays, in_place)
     if out is NotImplemented:
+        if _ops.tracing():
+            return _ops.Traced.apply(retention_recurrent, query, key, value, head_decays, prev_state, in_place)
         _ops.check_decode_step(query, key, value, prev_state, head_decays, in_place)
         _ops.rejected("retention_recurrent")
     return out

@@ -83,6 +83,17 @@ def test_traced_programs_run_the_op_again(ops, op):
         torch.jit.trace(call, (ins[0][:, :1], *ins[1:]))
 
 
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.filterwarnings("ignore")
+def test_traced_programs_run_the_decode_step_again(ops, in_place):
+    step = lambda q, k, v, s: ops.retention_recurrent(q[:, 0], k[:, 0], v[:, 0], DEC, s, in_place=in_place)
+    traced = torch.jit.trace(step, tuple(t.clone() for t in _inputs(1)[:4]), check_trace=False)
+    ins, ins2 = _inputs(2)[:4], _inputs(2)[:4]
+    out, ref = traced(*ins), step(*ins2)
+    assert all(torch.equal(a, b) for a, b in zip((*out, ins[3]), (*ref, ins2[3])))
+    assert (out[1].data_ptr() == ins[3].data_ptr()) == in_place
+
+
 class _NoGradient(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x):
