@@ -80,6 +80,23 @@ int pop(int B, int T, int H, int dk, int dv, int block) {
   return done(rc, "pop", B, T, H, dk, dv, block);
 }
 
+// a POP call cut at its blocks
+int pop_split(int B, int T, int H, int dk, int dv, int block) {
+  std::vector<double> dec(H, 0.97);
+  const size_t nq = (size_t)B * T * H * dk, nv = (size_t)B * T * H * dv, ns = (size_t)B * H * dk * dv, nb = T / block;
+  uint16_t *q = buf(nq), *k = buf(nq), *v = buf(nv), *s = buf(ns), *o = buf(nv, false), *dO = buf(nv);
+  uint16_t *dq = buf(nq, false), *dk_ = buf(nq, false), *dv_ = buf(nv, false), *ds0 = buf(ns, false);
+  uint16_t *bs = buf(nb * ns, false), *dbs = buf(nb * ns);
+  const size_t wb = fp_pop_retention_workspace_bytes(B, T, H, dk, dv, block);
+  void* ws = wb ? aligned_alloc(16, wb) : nullptr;
+  int rc = wb ? 0 : -99;
+  if (!rc) rc = fp_pop_retention_fwd_split(q, k, v, s, dec.data(), o, bs, B, T, H, dk, dv, block, ws, wb, nullptr);
+  for (int kept = 1; kept >= 0; --kept)
+    if (!rc) rc = fp_pop_retention_bwd_split(q, k, v, s, dec.data(), dO, dbs, dq, dk_, dv_, ds0, B, T, H, dk, dv, block, ws, wb, kept, nullptr);
+  free(ws);
+  return done(rc, "pop split", B, T, H, dk, dv, block);
+}
+
 // forward with checkpoints every `every` tokens, then the backward that starts from them
 int checkpointed(int B, int T, int H, int every, int dk = 128, int dv = 128) {
   std::vector<double> dec(H, 0.97);
@@ -150,6 +167,9 @@ int main() {
   rc |= plain(1, 100, 1, 192, 192, false);    // three visits per chunk
   rc |= plain(1, 512, 1, 64, 128, true);      // cut into segments (state-only walk, scan)
   rc |= plain(1, 640, 1, 128, 256, true);     // ... with the state-only kernel for 128-wide keys, two workgroups per segment
+  rc |= plain(1, 511, 1, 128, 128, true);     // uneven segments, fp32 states: the last chunk of that kernel is short
+  rc |= plain(1, 257, 1, 64, 64, true);       // ... the last segment is one token
+  rc |= pop_split(1, 150, 1, 128, 128, 65);   // blocks and a tail that end inside chunks
   rc |= pop(1, 287, 1, 64, 128, 144);
   rc |= pop(2, 28, 1, 64, 64, 15);
   rc |= pop(1, 40, 1, 64, 64, 100);           // no full block
