@@ -463,7 +463,7 @@ int64_t as_block(PyObject* o) { return std::min<int64_t>(as_int(o), 1 << 30); }
 
 bool is_bf16(const Tensor& t) { return !t.defined() || (t.scalar_type() == at::kBFloat16 && fpt::on_device(t)); }
 
-// q, k [B,T,H,dk], v [B,T,H,dv], s [B,H,dk,dv] or none, H decays: what _ops.prepare asks for; makes them contiguous
+// q, k [B,T,H,dk], v [B,T,H,dv], s [B,H,dk,dv] or none, H decays: what _ops.check_retention asks for; makes them contiguous
 bool retention_args(PyObject* const* a, Tensor& q, Tensor& k, Tensor& v, Tensor& s, Decays& g, Shape& n) {
   if (!as_tensor(a[0], q) || !as_tensor(a[1], k) || !as_tensor(a[2], v) || !as_tensor(a[3], s) || !q.defined() || !k.defined() || !v.defined())
     return false;
