@@ -45,6 +45,8 @@
 //   the bf16 copy of dS, the next chunk's tiles and the staged outputs move
 //   -- barrier --
 #pragma once
+#include <type_traits>
+
 #include "pass_args.h"
 #include "lds_access.h"
 
@@ -242,20 +244,25 @@ FP_DEVICE void stage_tile(const Common& k, uint16_t* tile, const u32x4 (&pf)[FbT
 #pragma unroll
   for (int u = 0; u < G::NU; ++u) st128(tile + at<G::LD>(row0 + G::ROWS * u, 8 * piece), pf[u]);
 }
-// staging tile ([token][feature]) -> rows of an item in `dst` (chunks) or `dst_sfx` (suffixes)
+// Piece u < FbTile<D>::NU of this thread: from the staging tile ([token][feature]), and into the rows of an item
+template <int D>
+FP_DEVICE u32x4 staged_piece(const Common& k, const uint16_t* tile, int u) {
+  using G = FbTile<D>;
+  return ld128(tile + at<G::LD>(k.tid / G::PPR + G::ROWS * u, 8 * (k.tid % G::PPR)));
+}
+template <int D>
+FP_DEVICE void store_piece(const Common& k, const fprt::BufView& v, int u, u32x4 d) {
+  using G = FbTile<D>;
+  // non-temporal: the gradients are not read back here, and kept out of the caches they leave
+  // room for the rows that the other workgroup of the stream is about to read a second time
+  fprt::buf_store128_nt(v, (uint32_t)(k.tid / G::PPR + G::ROWS * u) * ((uint32_t)k.H * D * 2) + (k.tid % G::PPR) * 16, d);
+}
+// staging tile -> rows of an item in `dst` (chunks) or `dst_sfx` (suffixes)
 template <int D>
 FP_DEVICE void drain_tile(const Common& k, const uint16_t* tile, void* dst, void* dst_sfx, const Item& it) {
-  using G = FbTile<D>;
   const fprt::BufView v = item_view<D>(k, dst, dst_sfx, it);
-  const uint32_t rowp = (uint32_t)k.H * D * 2;
-  const int row0 = k.tid / G::PPR, piece = k.tid % G::PPR;
 #pragma unroll
-  for (int u = 0; u < G::NU; ++u) {
-    const int row = row0 + G::ROWS * u;
-    // non-temporal: the gradients are not read back here, and kept out of the caches they leave
-    // room for the rows that the other workgroup of the stream is about to read a second time
-    fprt::buf_store128_nt(v, (uint32_t)row * rowp + piece * 16, ld128(tile + at<G::LD>(row, 8 * piece)));
-  }
+  for (int u = 0; u < FbTile<D>::NU; ++u) store_piece<D>(k, v, u, staged_piece<D>(k, tile, u));
 }
 
 // 32 x 32 accumulator (rows n = nbase + acc_row(r, g), column token i) -> staging tile [i][n]
@@ -444,8 +451,8 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
   const float gL_full = fprt::exp2_approx((float)CH * lg);
 
   // FOLD: the chunks from the one past the end (empty; it carries the suffix at T) down to the first
-  auto item_of = [&](int it) { return FOLD ? chunk_item(k, k.nch - it) : item_backward(k, it); };
-  const int nitems = FOLD ? k.nch + 1 : item_count(k);
+  auto item_of = [&](int it) { return FOLD ? chunk_item(k, k.nch - it) : SFX ? item_backward(k, it) : chunk_item(k, k.nch - 1 - it); };
+  const int nitems = FOLD ? k.nch + 1 : SFX ? item_count(k) : k.nch;
   // FOLD: the suffix that hangs off the first token of the chunk visited it-th (L = 0: none), and this thread's
   // 16 bytes of its q_s (threads 0..255) or dO_s rows (threads 256..511)
   auto suffix_of = [&](int it) {
@@ -474,7 +481,7 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
     return p.d_blocks + (((size_t)k.b * nblocks + (t0 / p.blocks_every - 1)) * p.H + k.h) * DK * DV;
   };
   constexpr int BP = DK * (DV / 8) / FB_THREADS;   // 16-byte pieces of a state matrix per thread
-  Item cur = item_of(0), nxt = item_of(1), prev = cur;
+  Item cur = item_of(0), nxt = item_of(1), prev = Item{0u, 0, false};
   u32x4 pf_q[GK::NU], pf_g[GV::NU], pf_k[GK::NU], pf_v[GV::NU], pf_s = {0, 0, 0, 0};
   load_tile<DK, true>(k, p.q, p.q_sfx, cur, pf_q);   // q: read by this workgroup only
   load_tile<DV>(k, p.dO, p.dO_sfx, cur, pf_g);
@@ -488,10 +495,15 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
   stage_tile<DK>(k, Ks, pf_k);
   stage_tile<DV>(k, Vs, pf_v);
   if constexpr (FOLD) stage_suffix(pf_s);
-  load_tile<DK, true>(k, p.q, p.q_sfx, nxt, pf_q);
-  load_tile<DV>(k, p.dO, p.dO_sfx, nxt, pf_g);
+  // In the order of the loop's own loads: how many younger ones may still be on their way when a tile is wanted has to be the
+  // same on both ways into the loop, or the wait in it is for all of them, stores included (B32 H4 T2048 64 x 64: 76 -> 72 us).
+  fprt::sched_fence();
   load_tile<DK>(k, p.k, p.k_sfx, nxt, pf_k);
   load_tile<DV>(k, p.v, p.v_sfx, nxt, pf_v);
+  fprt::sched_fence();
+  load_tile<DK, true>(k, p.q, p.q_sfx, nxt, pf_q);
+  load_tile<DV>(k, p.dO, p.dO_sfx, nxt, pf_g);
+  fprt::sched_fence();
   fprt::block_sync();
   f32x16 racc[TPW];
 #pragma unroll
@@ -508,11 +520,20 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
     if constexpr (MODE == FB_PLAIN) {   // the loads of it + 2 chunks are on their way or done
       if (p.pace && k.tid == 0) fprt::pace_store(p.pace + stream, p.pace_base + (uint32_t)(it + 2));
     }
-    // ---- the previous item's outputs leave (nothing writes the staging tiles before the next barrier)
-    if (it > 0) {
-      drain_tile<DV>(k, OUTV, p.dv, p.dv_sfx, prev);
-      drain_tile<DK>(k, OUTK, p.dk, p.dk_sfx, prev);
-    }
+    // ---- the previous item's outputs leave during the first stretch (nothing writes the staging tiles before its barrier), a
+    // piece per k-step: leave(n), n = 0 .. OUTS.  Ahead of the stretch they held its products up for 1 000 to 1 400 of the 9 500
+    // cycles of a chunk step (128 x 128; B32 H4 T2048 64 x 64: 72 -> 62 us a launch).
+    const fprt::BufView dv_view = item_view<DV>(k, p.dv, p.dv_sfx, prev), dk_view = item_view<DK>(k, p.dk, p.dk_sfx, prev);
+    constexpr int OUTS = GV::NU + GK::NU;
+    u32x4 leaving;
+    auto leave = [&](int n) {
+      if (n >= 1 && n <= OUTS) {
+        if (n <= GV::NU) store_piece<DV>(k, dv_view, n - 1, leaving);
+        else store_piece<DK>(k, dk_view, n - 1 - GV::NU, leaving);
+      }
+      if (n < OUTS) leaving = n < GV::NU ? staged_piece<DV>(k, OUTV, n) : staged_piece<DK>(k, OUTK, n - GV::NU);
+    };
+    static_assert(OUTS < KS + 1, "a piece per k-step");
     // ---- stretch 1: scores D[j][i] = W[j] . X[i] and read-out wread(i) sum_a R^T[n][a] X[i][a], the
     // operands of a k-step requested a few k-steps ahead
     f32x16 acc[2], sc = {0};
@@ -528,6 +549,24 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
         ra[t] = pass == 0 ? frag_cols(rrow, t) : frag_rows<LDK>(Rt, tr_seq, t, 32 * rt);
       };
       constexpr int AHEAD = 2;   // k-steps of operands in flight (a third one costs the 128-wide instantiations their last registers)
+      // The products of the read-out (and, SCORES, of this wave's score tile: IB its rows of X), k-step by k-step.
+      auto products = [&](auto with_scores, auto ib) {
+        constexpr bool SCORES = decltype(with_scores)::value;
+        constexpr int IB = decltype(ib)::value;
+#pragma unroll
+        for (int t = 0; t < AHEAD; ++t) request(t);
+        leave(0);
+        fprt::sched_fence();
+#pragma unroll
+        for (int t = 0; t < KS; ++t) {
+          if (SCORES) sc = fprt::mfma_32x32x16_bf16(wf[t], IB ? x1[t] : x0[t], sc);
+          acc[0] = fprt::mfma_32x32x16_bf16(ra[t], x0[t], acc[0]);
+          acc[1] = fprt::mfma_32x32x16_bf16(ra[t], x1[t], acc[1]);
+          if (t + AHEAD < KS) request(t + AHEAD);
+          leave(t + 1);
+          fprt::sched_fence();
+        }
+      };
       if (sfx || !has_out) {   // no read-out: only the score tile
         if (scores) {
 #pragma unroll
@@ -540,30 +579,15 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
           for (int t = 0; t < KS; ++t) sc = fprt::mfma_32x32x16_bf16(wf[t], x0[t], sc);
           score_finish(sc, mw, s_jb == s_ib, true, c, g, xp_pass + rt * FB_XP, lane);
         }
+#pragma unroll
+        for (int n = 0; n <= OUTS; ++n) leave(n);
       } else if (scores) {
-#pragma unroll
-        for (int t = 0; t < AHEAD; ++t) request(t);
-        fprt::sched_fence();
-#pragma unroll
-        for (int t = 0; t < KS; ++t) {
-          sc = fprt::mfma_32x32x16_bf16(wf[t], s_ib ? x1[t] : x0[t], sc);
-          acc[0] = fprt::mfma_32x32x16_bf16(ra[t], x0[t], acc[0]);
-          acc[1] = fprt::mfma_32x32x16_bf16(ra[t], x1[t], acc[1]);
-          if (t + AHEAD < KS) request(t + AHEAD);
-          fprt::sched_fence();
-        }
+        // one copy per row block: a choice between operands in registers would cost four selects a k-step
+        if (s_ib) products(std::true_type{}, std::integral_constant<int, 1>{});
+        else products(std::true_type{}, std::integral_constant<int, 0>{});
         score_finish(sc, mw, s_jb == s_ib, true, c, g, xp_pass + rt * FB_XP, lane);
       } else {
-#pragma unroll
-        for (int t = 0; t < AHEAD; ++t) request(t);
-        fprt::sched_fence();
-#pragma unroll
-        for (int t = 0; t < KS; ++t) {
-          acc[0] = fprt::mfma_32x32x16_bf16(ra[t], x0[t], acc[0]);
-          acc[1] = fprt::mfma_32x32x16_bf16(ra[t], x1[t], acc[1]);
-          if (t + AHEAD < KS) request(t + AHEAD);
-          fprt::sched_fence();
-        }
+        products(std::false_type{}, std::integral_constant<int, 0>{});
       }
     }
     float wread0 = wread_full0, wread1 = wread_full1;
@@ -756,17 +780,17 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
   const TrLane tr_acc = tr_lane<LDK>(lane, TR_ACC), tr_nat_k = tr_lane<LDK>(lane, TR_NAT), tr_nat_v = tr_lane<LDV>(lane, TR_NAT);
 
   // The walk: without checkpoints the chunks in order; with them the segments from the last to the
-  // first, the chunks of a segment in order.  seg_chunks = chunks per segment.
+  // first, the chunks of a segment in order.  seg_chunks = chunks per segment; the last segment may be shorter.
   const int seg_chunks = p.ckpt ? p.ckpt_every / CH : k.nch;
   const int nseg = (k.nch + seg_chunks - 1) / seg_chunks;
-  auto chunk_of = [&](int it) {   // chunk visited in iteration `it`, -1 beyond the walk
-    if (it < 0 || it >= k.nch) return -1;
-    if (nseg == 1) return it;
-    // the last segment may be shorter than the others
-    const int tail = k.nch - (nseg - 1) * seg_chunks;
-    if (it < tail) return (nseg - 1) * seg_chunks + it;
-    const int j = it - tail;
-    return (nseg - 2 - j / seg_chunks) * seg_chunks + j % seg_chunks;
+  // a chunk of the walk and the first chunk of its segment; chunk -1 beyond the walk
+  struct Step {
+    int chunk, start;
+  };
+  auto step_after = [&](const Step& w) {
+    if (w.chunk < 0) return w;
+    if (w.chunk + 1 < k.nch && w.chunk + 1 < w.start + seg_chunks) return Step{w.chunk + 1, w.start};
+    return w.start > 0 ? Step{w.start - seg_chunks, w.start - seg_chunks} : Step{-1, 0};
   };
   // state matrix that a segment starts from: s0 for the first, else the checkpoint before it
   auto segment_state = [&](int seg) -> const uint16_t* {
@@ -776,7 +800,7 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
   };
   // item visited in iteration `it`
   // FOLD: the chunks in order and one more, empty, at T for the suffix there
-  auto item_of = [&](int it) { return SFX ? item_forward(k, it) : FOLD ? chunk_item(k, it) : chunk_item(k, chunk_of(it)); };
+  auto item_of = [&](int it, const Step& w) { return SFX ? item_forward(k, it) : FOLD ? chunk_item(k, it) : chunk_item(k, w.chunk); };
   const int nitems = SFX ? item_count(k) : FOLD ? k.nch + 1 : k.nch;
   // FOLD: the suffix that hangs off the first token of the chunk visited it-th (L = 0: none), this thread's 16 bytes
   // of its dO_s rows (32 rows, zero from row Ls on), and its rows of dq_s
@@ -801,7 +825,8 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
     fprt::buf_store128_nt(item_view<DK>(k, nullptr, p.dq_sfx, sx), (uint32_t)sq_row * ((uint32_t)k.H * DK * 2) + sq_piece * 16,
                           ld128(tile + at<LDK>(sq_row, 8 * sq_piece)));
   };
-  Item cur = item_of(0), nxt = item_of(1), prev = cur;
+  Step w0 = {(nseg - 1) * seg_chunks, (nseg - 1) * seg_chunks}, w1 = step_after(w0);
+  Item cur = item_of(0, w0), nxt = item_of(1, w1), prev = Item{0u, 0, false};
   u32x4 pf_x[GV::NU], pf_w[GV::NU], pf_z[GK::NU], pf_s = {0, 0, 0, 0};
   load_tile<DV>(k, p.dO, p.dO_sfx, cur, pf_x);
   load_tile<DV>(k, p.v, p.v_sfx, cur, pf_w);
@@ -839,17 +864,16 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
   //   3  the next chunk's W and Z tiles
   int patience = 256;   // polls of the pacing word that this workgroup affords in all
   for (int it = 0; it < nitems; ++it) {
-    const int next = SFX ? 0 : chunk_of(it + 1);
-    const bool fresh = !SFX && next >= 0 && next != chunk_of(it) + 1;   // the next chunk starts another segment
+    const bool fresh = MODE == FB_PLAIN && w1.chunk >= 0 && w1.start != w0.start;   // the next chunk starts another segment
+    const Step w2 = step_after(w1);
     const bool sfx = SFX && cur.sfx;
     const int L = cur.L;
-    const Item after = item_of(it + 2);
+    const Item after = item_of(it + 2, w2);
     if constexpr (MODE == FB_PLAIN) {
       // the loads that this iteration issues (behind its first barrier) open another segment: not before the reverse
       // workgroup has asked for that segment's last chunk
-      const int c2 = chunk_of(it + 2);
-      if (p.pace && nseg > 1 && c2 >= 0 && c2 % seg_chunks == 0 && k.tid == 0) {
-        const int last = (c2 + seg_chunks < k.nch ? c2 + seg_chunks : k.nch) - 1;
+      if (p.pace && nseg > 1 && w2.chunk >= 0 && w2.chunk == w2.start && k.tid == 0) {
+        const int last = (w2.start + seg_chunks < k.nch ? w2.start + seg_chunks : k.nch) - 1;
         const uint32_t want = p.pace_base + (uint32_t)(k.nch - last);
         while (patience > 0 && (int32_t)(fprt::pace_load(p.pace + stream) - want) < 0) {
           fprt::nap();
@@ -857,10 +881,9 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
         }
       }
     }
-    if (it > 0) {   // nothing writes the staging tile before the next barrier
-      drain_tile<DK>(k, OUT, p.dq, p.dq_sfx, prev);
-      if constexpr (FOLD) drain_suffix(it - 1);
-    }
+    // nothing writes the staging tile before the next barrier
+    drain_tile<DK>(k, OUT, p.dq, p.dq_sfx, prev);
+    if constexpr (FOLD) drain_suffix(it - 1);
     f32x16 acc[2];
     if constexpr (state_role) {
       if (rt < 3) {
@@ -1008,7 +1031,7 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
     // nobody reads this chunk's X tile or the old copy of R any more
     stage_tile<DV>(k, Xs, pf_x);
     load_tile<DV>(k, p.dO, p.dO_sfx, after, pf_x);
-    if (fresh) load_state<DK, DV, true>(k, Rt, segment_state(next / seg_chunks));   // the next segment's starting state
+    if (fresh) load_state<DK, DV, true>(k, Rt, segment_state(w1.start / seg_chunks));   // the next segment's starting state
     fprt::block_sync();
 
     stage_tile<DV>(k, Ws, pf_w);
@@ -1026,6 +1049,8 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
     prev = cur;
     cur = nxt;
     nxt = after;
+    w0 = w1;
+    w1 = w2;
   }
   drain_tile<DK>(k, OUT, p.dq, p.dq_sfx, prev);
   if constexpr (FOLD) drain_suffix(nitems - 1);

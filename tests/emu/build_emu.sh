@@ -9,7 +9,7 @@ cxx=${EMU_CXX:-/opt/rocm/llvm/bin/clang++}
 out=${EMU_OUT:-$here/libflashpop_emu.so}
 obj=$(mktemp -d)
 trap 'rm -rf "$obj"' EXIT
-flags="-std=c++17 ${EMU_OPT:--O2} -g -fPIC -pthread $EMU_FLAGS -I$here -I$csrc"
+flags="-std=c++17 -Wno-pass-failed ${EMU_OPT:--O2} -g -fPIC -pthread $EMU_FLAGS -I$here -I$csrc"
 pids=""
 for w in 64 128 192 256; do
   "$cxx" $flags -DEMU_FAMILY=$w -c "$here/pass_family.cpp" -o "$obj/pass_$w.o" & pids="$pids $!"
