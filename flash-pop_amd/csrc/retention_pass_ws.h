@@ -354,7 +354,8 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
 #pragma unroll
     for (int r = 0; r < 4; ++r) zg_off[r] = (4 * z_tg + r) * rowB + z_fq * 8;
     const int zt_off = (4 * z_fq) * T_LD + 4 * z_tg;
-    const int y_row = tid >> 2, y_col = (tid & 3) * 16;
+    // Y: rows y_row and y_row + 32, 16 bytes each, so that a store covers whole 128-byte pieces of rows
+    const int y_row = tid >> 3, y_col = (tid & 7) * 8;
     const uint32_t yg_off = y_row * rowB + y_col * 2;
 
     // Loads and stores are issued unconditionally (zero-length views when there is nothing to
@@ -401,13 +402,13 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     // Y tile of chunk c2 from LDS stage s to global; rows beyond its length are dropped
     auto drain_y = [&](const Chunk& c2, int s) {
       const uint16_t* src = YB + s * CH * YB_LD + y_row * YB_LD + y_col;
-      const u32x4 v0 = ld128(src), v1 = ld128(src + 8);
+      const u32x4 v0 = ld128(src), v1 = ld128(src + 32 * YB_LD);
       const bool live = c2.ok && !STATE;
       const fprt::BufView yv = fprt::make_buf(((SFX && c2.sfx) ? Ysg : Yg) + (live ? rowsB(c2) : 0),
                                               live ? (uint32_t)(c2.L - 1) * rowB + BV * 2 : 0u);
       // non-temporal: outputs are not read back by this launch and need not displace its inputs in the caches
       fprt::buf_store128_nt(yv, yg_off, v0);
-      fprt::buf_store128_nt(yv, yg_off + 16, v1);
+      fprt::buf_store128_nt(yv, yg_off + 32 * rowB, v1);
     };
 
     Chunk ck = first_chunk(slot), ck1 = chunk_after(ck), ckp = no_chunk;
