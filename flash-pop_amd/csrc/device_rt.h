@@ -79,6 +79,11 @@ FP_DEVICE void buf_store128(BufView b, uint32_t off, u32x4 v) { __builtin_amdgcn
 // the same with the non-temporal hint: data that nobody reads again soon need not stay in the caches
 FP_DEVICE u32x4 buf_load128_nt(BufView b, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(b.rsrc, off, 0, 2); }
 FP_DEVICE void buf_store128_nt(BufView b, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, b.rsrc, off, 0, 2); }
+// ... and written through (sc1): what the L2s still hold at a kernel's end has to go out before the next launch starts (fused
+// backward, B32 H4 T2048 64 x 64: 64 -> 60.5 us; no difference in launches that write little).  For stores that cover whole lines
+// only: a line that leaves in parts costs far more than this saves (the forward of B8 H16 T4096 128 x 128 storing half lines at
+// a time: 123 -> 185 us).
+FP_DEVICE void buf_store128_through(BufView b, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, b.rsrc, off, 0, 2 | 16); }
 FP_DEVICE void buf_store64(BufView b, uint32_t off, u32x2 v) { __builtin_amdgcn_raw_buffer_store_b64(v, b.rsrc, off, 0, 0); }
 
 // A word that another workgroup of the same launch polls (relaxed, device scope), and a short sleep between polls.

@@ -255,7 +255,7 @@ FP_DEVICE void store_piece(const Common& k, const fprt::BufView& v, int u, u32x4
   using G = FbTile<D>;
   // non-temporal: the gradients are not read back here, and kept out of the caches they leave
   // room for the rows that the other workgroup of the stream is about to read a second time
-  fprt::buf_store128_nt(v, (uint32_t)(k.tid / G::PPR + G::ROWS * u) * ((uint32_t)k.H * D * 2) + (k.tid % G::PPR) * 16, d);
+  fprt::buf_store128_through(v, (uint32_t)(k.tid / G::PPR + G::ROWS * u) * ((uint32_t)k.H * D * 2) + (k.tid % G::PPR) * 16, d);
 }
 // staging tile -> rows of an item in `dst` (chunks) or `dst_sfx` (suffixes)
 template <int D>
@@ -822,7 +822,7 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
     const Item sx = suffix_of(it);
     if (sx.L == 0 || sq_row >= 2 * FB_SFX_ROWS) return;
     const uint16_t* const tile = OUTS + ((it * CH / k.block) & 1) * SFX_OUT;
-    fprt::buf_store128_nt(item_view<DK>(k, nullptr, p.dq_sfx, sx), (uint32_t)sq_row * ((uint32_t)k.H * DK * 2) + sq_piece * 16,
+    fprt::buf_store128_through(item_view<DK>(k, nullptr, p.dq_sfx, sx), (uint32_t)sq_row * ((uint32_t)k.H * DK * 2) + sq_piece * 16,
                           ld128(tile + at<LDK>(sq_row, 8 * sq_piece)));
   };
   Step w0 = {(nseg - 1) * seg_chunks, (nseg - 1) * seg_chunks}, w1 = step_after(w0);
@@ -1194,11 +1194,11 @@ FP_DEVICE void suffix_intra_bwd(const FusedBwdArgs& p, char* lds) {
     }
     fprt::block_sync();
     // rows < Ls leave
-    if (live_v) fprt::buf_store128_nt(view(p.dv_sfx, m, p.Ls, DV), (uint32_t)rv * rowv + cv * 16, ld128(ODV + at<LDV>(rv, 8 * cv)));
+    if (live_v) fprt::buf_store128_through(view(p.dv_sfx, m, p.Ls, DV), (uint32_t)rv * rowv + cv * 16, ld128(ODV + at<LDV>(rv, 8 * cv)));
     if (live_k) {
       const uint32_t off = (uint32_t)rk * rowk + ck * 16;
-      fprt::buf_store128_nt(view(p.dk_sfx, m, p.Ls, DK), off, ld128(ODK + at<LDK>(rk, 8 * ck)));
-      fprt::buf_store128_nt(view(p.dq_sfx, m, p.Ls, DK), off, ld128(ODQ + at<LDK>(rk, 8 * ck)));
+      fprt::buf_store128_through(view(p.dk_sfx, m, p.Ls, DK), off, ld128(ODK + at<LDK>(rk, 8 * ck)));
+      fprt::buf_store128_through(view(p.dq_sfx, m, p.Ls, DK), off, ld128(ODQ + at<LDK>(rk, 8 * ck)));
     }
     // (the next pair's rows are staged by the thread that has just read this pair's results from the same places,
     // and every read of the input tiles is behind the barrier above)
