@@ -58,8 +58,9 @@ __global__ __launch_bounds__(fpk::FB_THREADS) void short_seq_fwd_kernel(const fp
   fpk::short_seq_fwd<DK, DV>(args, lds);
 }
 
+template <int VEC, int AHEAD>
 __global__ __launch_bounds__(fpk::SCAN_THREADS) void segment_scan_kernel(const fpk::ScanArgs args) {
-  fpk::segment_scan(args);
+  fpk::segment_scan<VEC, AHEAD>(args);
 }
 
 template <bool REV>
@@ -435,25 +436,15 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* stream, const char** err
 }
 
 int fpk_launch_scan(const fpk::ScanArgs& a, void* stream, const char** err) {
-  if (a.M % fpk::SCAN_VEC != 0 || a.B < 1 || a.S < 1 || a.H < 1 || !a.U || !a.init || !a.U_lo != !a.init_lo ||
-      (!a.U_lo && (a.blocks_in || a.blocks_out))) {
-    *err = "segment scan: bad arguments";
+  if (const char* why = fpk::check_scan(a)) {
+    *err = why;
     return 1;
   }
-  const long long items = (long long)a.B * a.H * (a.M / fpk::SCAN_VEC);
-  const long long blocks = (items + fpk::SCAN_THREADS - 1) / fpk::SCAN_THREADS;
-  if (blocks > 0x7fffffffLL) {
-    *err = "segment scan: too many state matrices";
-    return 1;
-  }
-  hipLaunchKernelGGL(segment_scan_kernel, dim3((unsigned)blocks), dim3(fpk::SCAN_THREADS), 0,
+  const bool narrow = fpk::scan_narrow(a, fpk_compute_units());
+  hipLaunchKernelGGL(narrow ? (segment_scan_kernel<fpk::SCAN_VEC_NARROW, fpk::SCAN_AHEAD_NARROW>) : (segment_scan_kernel<fpk::SCAN_VEC, fpk::SCAN_AHEAD>),
+                     dim3((unsigned)fpk::scan_blocks(a, narrow ? fpk::SCAN_VEC_NARROW : fpk::SCAN_VEC)), dim3(fpk::SCAN_THREADS), 0,
                      static_cast<hipStream_t>(stream), a);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    *err = hipGetErrorString(e);
-    return 1;
-  }
-  return 0;
+  return launched(err);
 }
 
 int fpk_launch_decode(const fpk::DecodeArgs& a, void* stream, const char** err) {

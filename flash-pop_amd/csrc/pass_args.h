@@ -203,8 +203,8 @@ constexpr int DECODE_THREADS = 256;
 constexpr int decode_lds_bytes(int dv) { return (DECODE_THREADS / (dv / 8)) * dv * 4; }
 
 constexpr int SCAN_THREADS = 256;
-constexpr int SCAN_VEC = 8;   // elements per thread
-constexpr int SCAN_AHEAD = 8;   // contributions requested together
+constexpr int SCAN_VEC = 8, SCAN_VEC_NARROW = 2;       // elements per thread
+constexpr int SCAN_AHEAD = 8, SCAN_AHEAD_NARROW = 12;   // contributions requested together
 
 // Rotary position embedding of q and k in one launch.  Pairs (x[2i], x[2i+1]) of every head are
 // rotated by the angle float(position) * theta[i], `sign` = -1 rotates back (the gradient).

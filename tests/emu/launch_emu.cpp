@@ -142,20 +142,20 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* /*stream*/, const char**
 }
 
 int fpk_launch_scan(const fpk::ScanArgs& a, void* /*stream*/, const char** err) {
-  if (a.M % fpk::SCAN_VEC != 0 || a.B < 1 || a.S < 1 || a.H < 1 || !a.U || !a.init || !a.U_lo != !a.init_lo ||
-      (!a.U_lo && (a.blocks_in || a.blocks_out))) {
-    *err = "segment scan: bad arguments";
+  if (const char* why = fpk::check_scan(a)) {
+    *err = why;
     return 1;
   }
-  const long long items = (long long)a.B * a.H * (a.M / fpk::SCAN_VEC);
-  const int blocks = (int)((items + fpk::SCAN_THREADS - 1) / fpk::SCAN_THREADS);
+  const bool narrow = fpk::scan_narrow(a, fpk_compute_units());
+  const int blocks = (int)fpk::scan_blocks(a, narrow ? fpk::SCAN_VEC_NARROW : fpk::SCAN_VEC);
   // no barriers inside: the lanes can run one after another on this thread
   for (int blk = 0; blk < blocks; ++blk) {
     for (int t = 0; t < fpk::SCAN_THREADS; ++t) {
       fprt::g_lane.tid = t;
       fprt::g_lane.block = blk;
       fprt::g_lane.grid = blocks;
-      fpk::segment_scan(a);
+      if (narrow) fpk::segment_scan<fpk::SCAN_VEC_NARROW, fpk::SCAN_AHEAD_NARROW>(a);
+      else fpk::segment_scan<fpk::SCAN_VEC, fpk::SCAN_AHEAD>(a);
     }
   }
   return 0;
