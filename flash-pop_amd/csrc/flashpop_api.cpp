@@ -553,12 +553,12 @@ Shape block_segments(const Shape& s, int block) {
 int contributions(const Shape& seg, const double* decays, const void* w_rows, const void* z_rows, int reverse,
                   const Workspace& w, void* stream) {
   const float sc = 1.0f / std::sqrt((float)seg.dk);
-  // the kernel that holds 128 x 128 of the state per workgroup
-  if (seg.dk == fpk::FB_D && seg.dv % fpk::FB_D == 0 && fpk::contrib_fits(seg.T, seg.H, seg.dv)) {
+  // the kernel that holds whole columns of the state per workgroup
+  if ((seg.dk == 64 || seg.dk == fpk::FB_D) && fpk::contrib_fits(seg.T, seg.H, seg.dk, seg.dv)) {
     fpk::ContribArgs c;
     std::memset(&c, 0, sizeof c);
     c.W = in(w_rows); c.Z = in(z_rows); c.U = w.contrib; c.U_lo = w.contrib_lo;
-    c.B = seg.B; c.T = seg.T; c.H = seg.H; c.dB = seg.dv; c.reverse = reverse;
+    c.B = seg.B; c.T = seg.T; c.H = seg.H; c.dk = seg.dk; c.dB = seg.dv; c.reverse = reverse;
     c.segs = seg.segs; c.total = seg.total;
     c.s_update = reverse ? 1.f : sc;
     for (int h = 0; h < seg.H; ++h) c.log2g[h] = (float)std::log2(decays[h]);

@@ -63,10 +63,10 @@ __global__ __launch_bounds__(fpk::SCAN_THREADS) void segment_scan_kernel(const f
   fpk::segment_scan<VEC, AHEAD>(args);
 }
 
-template <bool REV>
-__global__ __launch_bounds__(fpk::FB_THREADS) void segment_contrib_kernel(const fpk::ContribArgs args) {
+template <int DK, int NC, int NTH, bool REV>
+__global__ __launch_bounds__(NTH) void segment_contrib_kernel(const fpk::ContribArgs args) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  fpk::segment_contrib<REV>(args, lds);
+  fpk::segment_contrib<DK, NC, NTH, REV>(args, lds);
 }
 
 __global__ __launch_bounds__(fpk::DECODE_THREADS) void decode_step_kernel(const fpk::DecodeArgs args) {
@@ -94,8 +94,8 @@ __global__ __launch_bounds__(fpk::LAYER_THREADS) void gated_norm_bwd_kernel(cons
 // no thread calls hipFuncSetAttribute for it again (which matters to callers that capture
 // launches into a graph after a warm-up run).  Setting the attribute twice in a race is harmless.
 constexpr int kMaxDevices = 64;
-static_assert(2 * fpk::PASS_KERNELS <= 57, "one bit per kernel instantiation, single and paired; the top six for the others");
-std::atomic<uint64_t> g_armed[kMaxDevices][2];   // slots 0..63: pass kernels and the small ones; 64..127: the fused backward family
+static_assert(2 * fpk::PASS_KERNELS <= 64, "one bit per kernel instantiation, single and paired");
+std::atomic<uint64_t> g_armed[kMaxDevices][2];   // bits 0..63: pass kernels; 64..: the fused backward family, short sequences, state-only pass
 
 template <typename Kernel, typename... More>
 int launch(Kernel kernel, int threads, int lds, int slot, int passes, hipStream_t stream, const char** err,
@@ -400,39 +400,28 @@ int fpk_launch_short_bwd(const fpk::FusedBwdArgs& a, void* stream, const char** 
   return launch_short_bwd<64, 64>(a, 3, st, err);
 }
 
+namespace {
+
+template <int DK, int NC, int NTH, bool REV>
+int launch_contrib(const fpk::ContribArgs& a, int slot, hipStream_t st, const char** err) {
+  constexpr int lds = fpk::ContribTile<DK, NC, NTH>::lds_bytes;
+  if (arm(reinterpret_cast<const void*>(segment_contrib_kernel<DK, NC, NTH, REV>), lds, 64 + 28 + slot, err)) return 1;
+  hipLaunchKernelGGL((segment_contrib_kernel<DK, NC, NTH, REV>), dim3((unsigned)(a.B * a.H * (a.dB / NC))), dim3(NTH), lds, st, a);
+  return launched(err);
+}
+
+}  // namespace
+
 int fpk_launch_contrib(const fpk::ContribArgs& a, void* stream, const char** err) {
   if (const char* why = fpk::check_contrib(a)) {
     *err = why;
     return 1;
   }
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) {
-    *err = "hipGetDevice failed";
-    return 1;
-  }
-  const void* const kernel = a.reverse ? reinterpret_cast<const void*>(segment_contrib_kernel<true>)
-                                       : reinterpret_cast<const void*>(segment_contrib_kernel<false>);
-  const uint64_t bit = 1ull << (a.reverse ? 60 : 61);
-  const bool tracked = dev >= 0 && dev < kMaxDevices;
-  if (!tracked || !(g_armed[dev][0].load(std::memory_order_acquire) & bit)) {
-    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, fpk::sc_lds_bytes()) != hipSuccess) {
-      (void)hipGetLastError();
-      *err = "hipFuncSetAttribute(MaxDynamicSharedMemorySize) failed";
-      return 1;
-    }
-    if (tracked) g_armed[dev][0].fetch_or(bit, std::memory_order_release);
-  }
-  const dim3 grid((unsigned)(a.B * a.H * (a.dB / fpk::FB_D))), threads(fpk::FB_THREADS);
-  if (a.reverse)
-    hipLaunchKernelGGL(segment_contrib_kernel<true>, grid, threads, fpk::sc_lds_bytes(), static_cast<hipStream_t>(stream), a);
-  else
-    hipLaunchKernelGGL(segment_contrib_kernel<false>, grid, threads, fpk::sc_lds_bytes(), static_cast<hipStream_t>(stream), a);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    *err = hipGetErrorString(e);
-    return 1;
-  }
-  return 0;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (a.dk == 64) return a.reverse ? launch_contrib<64, 64, 256, true>(a, 0, st, err) : launch_contrib<64, 64, 256, false>(a, 1, st, err);
+  if (fpk::contrib_columns(a) == 64)
+    return a.reverse ? launch_contrib<128, 64, 256, true>(a, 2, st, err) : launch_contrib<128, 64, 256, false>(a, 3, st, err);
+  return a.reverse ? launch_contrib<128, 128, 512, true>(a, 4, st, err) : launch_contrib<128, 128, 512, false>(a, 5, st, err);
 }
 
 int fpk_launch_scan(const fpk::ScanArgs& a, void* stream, const char** err) {

@@ -111,23 +111,23 @@ struct ScanArgs {
   int Tlast;             // tokens of the last segment (1 .. Tseg)
   float log2g[MAX_HEADS];
 };
-// State-only pass for states of 128 rows (segment_contrib.h): U[b][h] = what sequence b adds to a
+// State-only pass for states of 64 or 128 rows (segment_contrib.h): U[b][h] = what sequence b adds to a
 // zero state, sum_j weight(j) W[j]^T Z[j] with weight(j) = s_update gamma^(T - 1 - j) walking forward
-// (`reverse` = 0) and s_update gamma^(j + 1) walking backward.  W [B,T,H,128], Z [B,T,H,dB],
-// U [B,H,128,dB], bf16; dB a multiple of 128.  `segs`, `total` as in PassArgs.
+// (`reverse` = 0) and s_update gamma^(j + 1) walking backward.  W [B,T,H,dk], Z [B,T,H,dB],
+// U [B,H,dk,dB], bf16; dB a multiple of 64.  `segs`, `total` as in PassArgs.
 struct ContribArgs {
   const uint16_t* W;
   const uint16_t* Z;
   uint16_t* U;
   uint16_t* U_lo;        // the lower halves if U is fp32 (see PassArgs::Rout_lo), nullable
-  int B, T, H, dB, reverse;
+  int B, T, H, dk, dB, reverse;
   int segs, total;
   float s_update;
   float log2g[MAX_HEADS];
 };
 // Whether the rows of whole chunks, those beyond a sequence's end included, have 32-bit byte offsets in that pass (one that wrapped
 // would come back into its view).
-inline bool contrib_fits(long long T, int H, int dB) { return (T + CH) * H * dB * 2 < (1LL << 32); }
+inline bool contrib_fits(long long T, int H, int dk, int dB) { return (T + CH) * H * (dk > dB ? dk : dB) * 2 < (1LL << 32); }
 // One recurrent (decode) step for every (batch, head):  S' = gamma S + (scale k)^T v,  o = q S'.
 // q, k [B,H,dk]; v, o [B,H,dv]; S [B,H,dk,dv]; all bf16, fp32 arithmetic.  s_out may be s_in.
 struct DecodeArgs {
@@ -264,7 +264,7 @@ int fpk_launch_short_fwd(const fpk::ShortFwdArgs& args, void* stream, const char
 // Launches the segment scan.  Same conventions as fpk_launch_pass.
 int fpk_launch_scan(const fpk::ScanArgs& args, void* stream, const char** err);
 
-// Launches the state-only pass for states of 128 rows (B H dB / 128 workgroups).  Same conventions.
+// Launches the state-only pass for states of 64 or 128 rows.  Same conventions.
 int fpk_launch_contrib(const fpk::ContribArgs& args, void* stream, const char** err);
 
 // Bytes of the library's own scratch array (one per device, see fpk_static_scratch).

@@ -130,15 +130,20 @@ int fpk_launch_short_fwd(const fpk::ShortFwdArgs& a, void* /*stream*/, const cha
   return emu_short_fwd_64_64(a);
 }
 
+template <int DK, int NC, int NTH>
+static int run_contrib(const fpk::ContribArgs& a) {
+  return run_grid(NTH, a.B * a.H * (a.dB / NC), fpk::ContribTile<DK, NC, NTH>::lds_bytes, [&](char* l) {
+    if (a.reverse) fpk::segment_contrib<DK, NC, NTH, true>(a, l);
+    else fpk::segment_contrib<DK, NC, NTH, false>(a, l);
+  });
+}
+
 int fpk_launch_contrib(const fpk::ContribArgs& a, void* /*stream*/, const char** err) {
   if (const char* why = fpk::check_contrib(a)) {
     *err = why;
     return 1;
   }
-  return run_grid(fpk::FB_THREADS, a.B * a.H * (a.dB / fpk::FB_D), fpk::sc_lds_bytes(), [&](char* l) {
-    if (a.reverse) fpk::segment_contrib<true>(a, l);
-    else fpk::segment_contrib<false>(a, l);
-  });
+  return a.dk == 64 ? run_contrib<64, 64, 256>(a) : fpk::contrib_columns(a) == 64 ? run_contrib<128, 64, 256>(a) : run_contrib<128, 128, 512>(a);
 }
 
 int fpk_launch_scan(const fpk::ScanArgs& a, void* /*stream*/, const char** err) {

@@ -287,6 +287,26 @@ def test_cut_final_state_follows_the_uncut_walk(emu_lib, T, dk, dv):
     assert n > 0 and share <= 1e-3, share
 
 
+@pytest.mark.parametrize("T,dk,dv", [
+    (257, 64, 64),      # 64-row states: a last segment of one token
+    (575, 64, 192),     # ... three workgroups per segment, a last chunk of 63 tokens
+    (513, 128, 64),     # 128-row states, 64 columns per workgroup
+    (577, 128, 192),    # ... a last segment of one token (uneven cuts all: equal segments hand bf16 states on, a step in 2^8)
+])
+def test_state_only_pass_in_64_columns(emu_lib, T, dk, dv):
+    """What the segments add to the carried state, 64 columns per workgroup: the final state is the uncut call's (up to the half
+    step in 2^13 of test_cut_final_state_follows_the_uncut_walk; gamma = 0.97 over the last 64 tokens: the short chunk counts),
+    and the gradient of the initial state, which the walk back gives, meets the oracle."""
+    q, k, v, s = hp.make_inputs(1, T, 1, dk, dv, seed=T, state_std=0.5)
+    d_o, d_s = hp.make_cotangents([(1, T, 1, dv), (1, 1, dk, dv)], seed=T + 1)
+    o, S, n = hp.raw_split_fwd(emu_lib, q, k, v, s, (0.97,))
+    _, S1 = hp.raw_fwd(emu_lib, q, k, v, s, (0.97,))
+    assert n > 0 and (S != S1).float().mean().item() <= 1e-3
+    o_ref, _, (_, _, _, gs) = hp.oracle_plain(q, k, v, s, (0.97,), d_o, d_s)
+    ds0 = hp.raw_split_bwd(emu_lib, q, k, v, s, (0.97,), d_o, d_s)[3]
+    _check_all([("o", o, o_ref), ("ds0", ds0, gs)])
+
+
 @pytest.mark.parametrize("B,nblk,block,Ls,H,state_std,dk,dv", [
     (1, 2, 128, 16, 1, 0.5, 128, 128),     # two chunks per block
     (1, 4, 64, 64, 1, None, 128, 128),     # block == chunk, suffixes as long as a chunk, no initial state
