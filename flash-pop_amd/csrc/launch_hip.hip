@@ -7,6 +7,7 @@
 #include "segment_contrib.h"
 #include "retention_bwd_fused.h"
 #include "short_seq.h"
+#include "pop_fold_fwd.h"
 #include "decode_step.h"
 #include "layer_ops.h"
 
@@ -44,6 +45,11 @@ template <int DK, int DV>
 __global__ __launch_bounds__(fpk::SI_THREADS) void suffix_intra_bwd_kernel(const fpk::FusedBwdArgs args) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   fpk::suffix_intra_bwd<DK, DV>(args, lds);
+}
+
+__global__ __launch_bounds__(fpk::PF_THREADS) void pop_fold_fwd_kernel(const fpk::PassArgs args) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  fpk::pop_fold_fwd(args, lds, fpk::place_workgroup(fprt::block_index(), fprt::grid_size(), 1).wg);
 }
 
 template <int DK, int DV>
@@ -242,15 +248,6 @@ struct DeviceMultiRun {
 
 }  // namespace
 
-int fpk_launch_pass(const fpk::PassArgs& args, void* stream, const char** err) {
-  fpk::PassArgs a = args;
-  if (const char* why = fpk::plan_pass(a, fpk_compute_units())) {
-    *err = why;
-    return 1;
-  }
-  return fpk::dispatch_pass(a, DeviceRun{a, static_cast<hipStream_t>(stream), err});
-}
-
 int fpk_launch_passes(const fpk::PassArgs* const* passes, int n, void* stream, const char** err) {
   if (n == 1) return fpk_launch_pass(*passes[0], stream, err);
   fpk::PassArgs planned[fpk::MAX_PASSES_PER_LAUNCH];
@@ -294,6 +291,21 @@ int launched(const char** err) {
 }
 
 }  // namespace
+
+int fpk_launch_pass(const fpk::PassArgs& args, void* stream, const char** err) {
+  fpk::PassArgs a = args;
+  if (const char* why = fpk::plan_pass(a, fpk_compute_units())) {
+    *err = why;
+    return 1;
+  }
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (fpk::pop_folds(a)) {
+    if (arm(reinterpret_cast<const void*>(pop_fold_fwd_kernel), fpk::pf_lds_bytes(), 64 + 34, err)) return 1;
+    hipLaunchKernelGGL(pop_fold_fwd_kernel, dim3((unsigned)(a.B * a.H * (a.dB / fpk::BV))), dim3(fpk::PF_THREADS), fpk::pf_lds_bytes(), st, a);
+    return launched(err);
+  }
+  return fpk::dispatch_pass(a, DeviceRun{a, st, err});
+}
 
 namespace {
 

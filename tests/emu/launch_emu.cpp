@@ -6,6 +6,7 @@
 #include "segment_contrib.h"
 #include "retention_bwd_fused.h"
 #include "short_seq.h"
+#include "pop_fold_fwd.h"
 #include "decode_step.h"
 #include "layer_ops.h"
 
@@ -42,6 +43,11 @@ int fpk_launch_pass(const fpk::PassArgs& args, void* /*stream*/, const char** er
   if (const char* why = fpk::plan_pass(a, fpk_compute_units())) {
     *err = why;
     return 1;
+  }
+  if (fpk::pop_folds(a)) {
+    const int nwg = a.B * a.H * (a.dB / fpk::BV);
+    return run_grid(fpk::PF_THREADS, nwg, fpk::pf_lds_bytes(),
+                    [&](char* l) { fpk::pop_fold_fwd(a, l, fpk::place_workgroup(fprt::block_index(), nwg, 1).wg); });
   }
   return run_family(&a, 1);
 }

@@ -140,6 +140,23 @@ def test_fused_pop_fwd_bwd(emu_lib, B, nblk, block, Ls, H, dk, dv, state_std, ta
     _check_all([(n, g, r) for n, g, r in zip(FUSED_NAMES, grads, g_ref)])
 
 
+@pytest.mark.parametrize("B,nblk,block,Ls,H,dv,state_std", [
+    (1, 3, 65, 16, 1, 64, 0.5),      # a chunk of one token per block
+    (1, 2, 128, 1, 1, 192, None),    # the longest blocks it takes, one-token suffixes, three column tiles, no initial state
+    (2, 4, 15, 15, 2, 64, 0.5),      # blocks shorter than a row block
+    (1, 1, 63, 16, 1, 128, 0.5),     # a single short block
+])
+def test_folded_forward(emu_lib, B, nblk, block, Ls, H, dv, state_std):
+    """The forward that takes suffixes as part of the chunks at their boundaries (64-wide keys)."""
+    decays = oracle.head_decays(H, (4, 9))
+    q, k, v, s = hp.make_inputs(B, nblk * block, H, 64, dv, seed=block + Ls, state_std=state_std)
+    sfx = hp.make_suffix_inputs(B, nblk, Ls, H, 64, dv, seed=block + Ls + 1)
+    o, o_sfx, S = hp.raw_fused_fwd(emu_lib, q, k, v, s, sfx, decays, block)
+    cot = hp.make_cotangents([tuple(v.shape), tuple(sfx[2].shape), (B, H, 64, dv)], seed=1)
+    o_ref, os_ref, S_ref, _ = hp.oracle_fused(q, k, v, s, sfx, decays, block, cot)
+    _check_all([("o", o, o_ref), ("o_sfx", o_sfx, os_ref), ("s_out", S, S_ref)])
+
+
 @pytest.mark.parametrize("B,T,H,dk,dv,state_std,segments", [
     (1, 512, 1, 64, 64, 0.5, 2),       # the harness pretends to have 8 compute units: 1 stream -> 2 segments of 4 chunks
     (1, 1024, 1, 64, 128, None, 4),    # dk != dv, no initial state, 4 segments
