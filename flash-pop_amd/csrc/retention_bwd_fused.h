@@ -195,6 +195,12 @@ FP_DEVICE Item item_forward(const Common& k, int it) {
 }
 FP_DEVICE int item_count(const Common& k) { return k.block == 0 ? k.nch : 1 + k.nblk * (k.spb + 1); }
 
+// FOLD: a chunk as chunk `chunk` of block `block`, stepped from chunk to chunk (a suffix hangs off chunk 0 of its block); asking
+// the chunk's number for it took several divisions a step (B8 H12 T2048 64 x 128, blocks of 64: 95.8 -> 93.1 us a launch).
+struct Boundary {
+  int chunk, block;
+};
+
 FP_DEVICE Common make_common(const FusedBwdArgs& p, int stream) {
   Common k;
   k.tid = fprt::thread_index();
@@ -453,17 +459,14 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
   // FOLD: the chunks from the one past the end (empty; it carries the suffix at T) down to the first
   auto item_of = [&](int it) { return FOLD ? chunk_item(k, k.nch - it) : SFX ? item_backward(k, it) : chunk_item(k, k.nch - 1 - it); };
   const int nitems = FOLD ? k.nch + 1 : SFX ? item_count(k) : k.nch;
-  // FOLD: the suffix that hangs off the first token of the chunk visited it-th (L = 0: none), and this thread's
+  // FOLD: the suffix that hangs off the first token of a chunk (L = 0: none), and this thread's
   // 16 bytes of its q_s (threads 0..255) or dO_s rows (threads 256..511)
-  auto suffix_of = [&](int it) {
-    const int t0 = (k.nch - it) * CH;
-    return it >= 0 && it < nitems && t0 % k.block == 0 ? suffix_item(k, t0 / k.block) : Item{0u, 0, false};
-  };
+  auto suffix_at = [&](const Boundary& w) { return FOLD && w.chunk == 0 && w.block >= 0 ? suffix_item(k, w.block) : Item{0u, 0, false}; };
   const bool sfx_q = k.tid < 256;
   const int sfx_i = k.tid & 255;
   const int sfx_row = sfx_q ? sfx_i / GK::PPR : sfx_i / GV::PPR, sfx_piece = sfx_q ? sfx_i % GK::PPR : sfx_i % GV::PPR;
-  auto load_suffix = [&](int it) {
-    Item sx = suffix_of(it);
+  auto load_suffix = [&](const Boundary& w) {
+    Item sx = suffix_at(w);
     if (sfx_row >= FB_SFX_ROWS) sx.L = 0;
     sx.sfx = true;
     if (sfx_q) return fprt::buf_load128(item_view<DK>(k, nullptr, p.q_sfx, sx), (uint32_t)sfx_row * ((uint32_t)k.H * DK * 2) + sfx_piece * 16);
@@ -487,7 +490,8 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
   load_tile<DV>(k, p.dO, p.dO_sfx, cur, pf_g);
   load_tile<DK>(k, p.k, p.k_sfx, cur, pf_k);
   load_tile<DV>(k, p.v, p.v_sfx, cur, pf_v);
-  if constexpr (FOLD) pf_s = load_suffix(0);
+  Boundary here = {0, k.nblk};   // FOLD: the chunk at T
+  if constexpr (FOLD) pf_s = load_suffix(here);
   // the gradient that the walk starts from: that of the final state, or (BLOCKS) of a block that ends with the sequence
   load_state<DK, DV, false>(k, Rt, BLOCKS ? block_grad(k.T) : p.ds_out ? p.ds_out + (size_t)stream * DK * DV : nullptr);
   stage_tile<DK>(k, Qs, pf_q);
@@ -604,7 +608,8 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
     fprt::block_sync();
 
     // FOLD: the next chunk's suffix rows travel during this stretch only (registers are scarce in the first one)
-    if constexpr (FOLD) pf_s = load_suffix(it + 1);
+    const Boundary below = here.chunk > 0 ? Boundary{here.chunk - 1, here.block} : Boundary{k.spb - 1, here.block - 1};
+    if constexpr (FOLD) pf_s = load_suffix(below);
     // BLOCKS: this chunk starts at a block boundary: the gradient of the state there travels during this stretch
     const uint16_t* const inject = BLOCKS && !cur.sfx && L > 0 ? block_grad((int)(cur.row - (uint32_t)k.b * k.T)) : nullptr;
     u32x4 pf_b[BP];
@@ -673,7 +678,7 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
     }
     if constexpr (FOLD) {
       // the suffix at this chunk's first token: what it adds to dS is not decayed (it reads the state as it is there)
-      if (owns && suffix_of(it).L > 0) {
+      if (owns && suffix_at(here).L > 0) {
         const u32x4 ua = frag_rows<LDK>(QS, tr_nat_k, 0, 32 * at_);
         u32x4 ub[TPW];
 #pragma unroll
@@ -731,6 +736,7 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
     prev = cur;
     cur = nxt;
     nxt = after;
+    here = below;
   }
   drain_tile<DV>(k, OUTV, p.dv, p.dv_sfx, prev);
   drain_tile<DK>(k, OUTK, p.dk, p.dk_sfx, prev);
@@ -802,15 +808,15 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
   // FOLD: the chunks in order and one more, empty, at T for the suffix there
   auto item_of = [&](int it, const Step& w) { return SFX ? item_forward(k, it) : FOLD ? chunk_item(k, it) : chunk_item(k, w.chunk); };
   const int nitems = SFX ? item_count(k) : FOLD ? k.nch + 1 : k.nch;
-  // FOLD: the suffix that hangs off the first token of the chunk visited it-th (L = 0: none), this thread's 16 bytes
+  // FOLD: the suffix that hangs off the first token of a chunk (L = 0: none), this thread's 16 bytes
   // of its dO_s rows (32 rows, zero from row Ls on), and its rows of dq_s
-  auto suffix_of = [&](int it) {
-    return it >= 0 && it < nitems && (it * CH) % k.block == 0 ? suffix_item(k, it * CH / k.block) : Item{0u, 0, false};
+  auto suffix_at = [&](const Boundary& w) {
+    return FOLD && w.chunk == 0 && w.block >= 0 && w.block <= k.nblk ? suffix_item(k, w.block) : Item{0u, 0, false};
   };
   const int sx_row = k.tid / GV::PPR, sx_piece = k.tid % GV::PPR;     // dO_s: 32 rows of DV / 8 pieces
   const int sq_row = k.tid / GK::PPR, sq_piece = k.tid % GK::PPR;     // dq_s: 32 rows of DK / 8 pieces
-  auto load_suffix = [&](int it) {
-    Item sx = suffix_of(it);
+  auto load_suffix = [&](const Boundary& w) {
+    Item sx = suffix_at(w);
     if (sx_row >= 2 * FB_SFX_ROWS) sx.L = 0;
     sx.sfx = true;
     return fprt::buf_load128(item_view<DV>(k, nullptr, p.dO_sfx, sx), (uint32_t)sx_row * ((uint32_t)k.H * DV * 2) + sx_piece * 16);
@@ -818,10 +824,10 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
   auto stage_suffix = [&](u32x4 v) {
     if (sx_row < 2 * FB_SFX_ROWS) st128(XS + at<LDV>(sx_row, 8 * sx_piece), v);
   };
-  auto drain_suffix = [&](int it) {
-    const Item sx = suffix_of(it);
+  auto drain_suffix = [&](const Boundary& w) {
+    const Item sx = suffix_at(w);
     if (sx.L == 0 || sq_row >= 2 * FB_SFX_ROWS) return;
-    const uint16_t* const tile = OUTS + ((it * CH / k.block) & 1) * SFX_OUT;
+    const uint16_t* const tile = OUTS + (w.block & 1) * SFX_OUT;
     fprt::buf_store128_through(item_view<DK>(k, nullptr, p.dq_sfx, sx), (uint32_t)sq_row * ((uint32_t)k.H * DK * 2) + sq_piece * 16,
                           ld128(tile + at<LDK>(sq_row, 8 * sq_piece)));
   };
@@ -831,7 +837,8 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
   load_tile<DV>(k, p.dO, p.dO_sfx, cur, pf_x);
   load_tile<DV>(k, p.v, p.v_sfx, cur, pf_w);
   load_tile<DK>(k, p.k, p.k_sfx, cur, pf_z);
-  if constexpr (FOLD) pf_s = load_suffix(0);
+  Boundary behind = {0, -1}, here = {0, 0};   // FOLD
+  if constexpr (FOLD) pf_s = load_suffix(here);
   // R[a][n] = S[n][a]: the copy is the state matrix as it is stored
   load_state<DK, DV, true>(k, Rt, segment_state(nseg - 1));
   stage_tile<DV>(k, Xs, pf_x);
@@ -883,7 +890,7 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
     }
     // nothing writes the staging tile before the next barrier
     drain_tile<DK>(k, OUT, p.dq, p.dq_sfx, prev);
-    if constexpr (FOLD) drain_suffix(it - 1);
+    if constexpr (FOLD) drain_suffix(behind);
     f32x16 acc[2];
     if constexpr (state_role) {
       if (rt < 3) {
@@ -937,7 +944,7 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
       }
       if constexpr (FOLD) {
         // the suffix at this chunk's first token reads the same R: its rows of dq_s, as far as they come from the state
-        const Item sx = suffix_of(it);
+        const Item sx = suffix_at(here);
         if (sx.L > 0) {
           const uint16_t* const xsrow = XS + at<LDV>(c, 8 * g);
           f32x16 as = {0};
@@ -952,14 +959,15 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
           for (int t = 0; t < KS; ++t) as = fprt::mfma_32x32x16_bf16(ra[t], xs[t], as);
 #pragma unroll
           for (int r = 0; r < 16; ++r) as[r] *= wread0;
-          put_output<LDK>(OUTS + ((it * CH / k.block) & 1) * SFX_OUT, c, 32 * rt, g, as);
+          put_output<LDK>(OUTS + (here.block & 1) * SFX_OUT, c, 32 * rt, g, as);
         }
       }
     }
     fprt::block_sync();
 
     // FOLD: the next chunk's suffix rows travel during the second stretch only (registers are scarce in the first)
-    if constexpr (FOLD) pf_s = load_suffix(it + 1);
+    const Boundary ahead = here.chunk + 1 < k.spb ? Boundary{here.chunk + 1, here.block} : Boundary{0, here.block + 1};
+    if constexpr (FOLD) pf_s = load_suffix(ahead);
     if constexpr (!state_role) {
       // Y^T[n][i] += sum_j Z^T[n][j] P^T[j][i]; tokens j < 32 reach both halves (tiles (0,0), (0,1)),
       // the others only the second
@@ -1051,9 +1059,11 @@ FP_DEVICE void fused_bwd_forward(const FusedBwdArgs& p, char* lds, int stream) {
     nxt = after;
     w0 = w1;
     w1 = w2;
+    behind = here;
+    here = ahead;
   }
   drain_tile<DK>(k, OUT, p.dq, p.dq_sfx, prev);
-  if constexpr (FOLD) drain_suffix(nitems - 1);
+  if constexpr (FOLD) drain_suffix(behind);
 }
 
 // launch index -> kind and stream: the reverse workgroups (the longer ones) come first
