@@ -33,6 +33,10 @@ FP_DEVICE uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
 }
 
+// The lower (upper) halves of two words as one, that of `a` in bits 0..15 (v_perm_b32).
+FP_DEVICE uint32_t lower_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+FP_DEVICE uint32_t upper_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
 // 2^x for x <= 0 (v_exp_f32, ~1 ulp; results below the normal range flush to zero).
 FP_DEVICE float exp2_approx(float x) { return __builtin_amdgcn_exp2f(x); }
 // full-precision elementary functions for the elementwise kernels

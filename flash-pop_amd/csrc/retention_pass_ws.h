@@ -388,14 +388,9 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int w = e >> 1;
-        u32x2 d;
-        if (e & 1) {
-          d[0] = (fr.z[0][w] >> 16) | (fr.z[1][w] & 0xffff0000u);
-          d[1] = (fr.z[2][w] >> 16) | (fr.z[3][w] & 0xffff0000u);
-        } else {
-          d[0] = (fr.z[0][w] & 0xffffu) | (fr.z[1][w] << 16);
-          d[1] = (fr.z[2][w] & 0xffffu) | (fr.z[3][w] << 16);
-        }
+        u32x2 d;   // (halves joined by shifts and masks are formed when the words arrive, an item early)
+        d[0] = (e & 1) ? fprt::upper_halves(fr.z[0][w], fr.z[1][w]) : fprt::lower_halves(fr.z[0][w], fr.z[1][w]);
+        d[1] = (e & 1) ? fprt::upper_halves(fr.z[2][w], fr.z[3][w]) : fprt::lower_halves(fr.z[2][w], fr.z[3][w]);
         st64(zt + zt_off + e * T_LD, d);
       }
     };
@@ -417,9 +412,13 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     feed_load_z(feed, ck);
     feed_store_x(feed, 0);
     feed_store_z(feed, 0);
-    feed_load_x(feed, ck1);
-    feed_load_z(feed, ck1);
-    fprt::block_sync();   // stage 0 is filled, item 1 is on its way
+    // Item 1 on its way, stage 0 filled.  Every copy of the loop below does this for itself: with one set of loads ahead of all of
+    // them their registers are not the ones that a copy keeps its loads in, and it waits for all of them in every other item.
+    auto enter = [&] {
+      feed_load_x(feed, ck1);
+      feed_load_z(feed, ck1);
+      fprt::block_sync();
+    };
 
     // One item.  `feed` holds item it + 1 on entry; once its parts have gone into LDS they are
     // reloaded with item it + 2.  Returns false after the last item.  `half` is the parity of `it`
@@ -564,10 +563,13 @@ FP_DEVICE void retention_pass_ws(const PassArgs& p, const PassTensors& io, char*
     // Three copies of the loop, chosen once per wave: two live tiles and this wave makes one of
     // them; one live tile made by this wave; one live tile made by the partner.
     if (other_live) {
+      enter();
       walk_visits<NH>([&](auto part, int it) { return iteration(part, Half<1>{}, Half<1>{}, it); });
     } else if (makes_diag) {
+      enter();
       walk_visits<NH>([&](auto part, int it) { return iteration(part, Half<1>{}, Half<0>{}, it); });
     } else {
+      enter();
       walk_visits<NH>([&](auto part, int it) { return iteration(part, Half<0>{}, Half<0>{}, it); });
     }
     return;

@@ -76,6 +76,8 @@ FP_DEVICE uint32_t pack_bf16x2(float lo, float hi) {
   return (uint32_t)f32_to_bf16_rne(lo) | ((uint32_t)f32_to_bf16_rne(hi) << 16);
 }
 
+FP_DEVICE uint32_t lower_halves(uint32_t a, uint32_t b) { return (a & 0xffffu) | (b << 16); }
+FP_DEVICE uint32_t upper_halves(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
 FP_DEVICE float exp2_approx(float x) { return std::exp2(x); }
 FP_DEVICE void sincos_f32(float x, float& s, float& c) { s = std::sin(x); c = std::cos(x); }
 FP_DEVICE float sigmoid_f32(float x) { return 1.0f / (1.0f + std::exp(-x)); }
