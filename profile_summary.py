@@ -16,7 +16,7 @@ import subprocess
 import sys
 from collections import defaultdict
 
-OURS = ("retention_", "suffix_intra", "short_seq", "segment_scan", "segment_contrib", "decode_step", "rotary_qk", "gated_norm")
+OURS = ("retention_", "pop_fold", "suffix_intra", "short_seq", "segment_scan", "segment_contrib", "decode_step", "rotary_qk", "gated_norm")
 COPY_KIB = 1 << 20   # the calibration copies 1 GiB
 
 
