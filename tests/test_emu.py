@@ -292,7 +292,7 @@ def test_cut_calls_carry_fp32_states(emu_lib, choose_backward, T, dk, dv, block)
 @pytest.mark.parametrize("T,dk,dv", [
     (511, 128, 128),    # the 128-wide state-only kernel, a last chunk of 63 tokens
     (257, 128, 256),    # of one token, two workgroups per segment
-    (330, 64, 128),     # the pass kernel's state-only walk
+    (330, 64, 128),     # 64-row states, a last chunk of 10 tokens
 ])
 def test_cut_final_state_follows_the_uncut_walk(emu_lib, T, dk, dv):
     """The state-only walk of a cut call takes the chunks of the uncut one, the short one last, and weighs the same keys the

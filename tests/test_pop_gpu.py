@@ -88,7 +88,7 @@ def test_pop_outputs_equal_plain_outputs():
 
 @pytest.mark.parametrize("B,T,H,dk,dv,block", [
     (1, 1500, 4, 128, 128, 144),   # the 128-wide state-only kernel, blocks and a tail that end inside a chunk
-    (2, 1000, 4, 128, 64, 100),    # the pass kernel's state-only walk, the sequence ends on a boundary
+    (2, 1000, 4, 128, 64, 100),    # 64 columns of a state per workgroup, the sequence ends on a boundary
     (1, 1500, 2, 256, 64, 144),
     (1, 1537, 2, 128, 128, 128),   # whole chunks per block, a tail of one token
     (1, 832, 2, 64, 64, 64),
