@@ -328,7 +328,7 @@ int launch_bwd_fused(const fpk::FusedBwdArgs& a, int slot, hipStream_t st, const
     if (launched(err)) return 1;
     // what stays inside the suffixes, after the part of dq_s that comes from the carried state is written
     const long long pairs = (long long)a.B * (a.T / a.block + 1) * a.H;
-    const long long wgs = 8LL * fpk_compute_units();
+    const long long wgs = (long long)fpk::SI_PER_CU * fpk_compute_units();
     hipLaunchKernelGGL((suffix_intra_bwd_kernel<DK, DV>), dim3((unsigned)(pairs < wgs ? pairs : wgs)), dim3(fpk::SI_THREADS),
                        lds_si, st, a);
     return launched(err);

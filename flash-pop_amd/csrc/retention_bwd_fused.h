@@ -1088,16 +1088,25 @@ FP_DEVICE void fused_bwd(const FusedBwdArgs& p, char* lds, int block) {
 // wrote, so that the sum is rounded once); the next pair's rows are on their way in registers meanwhile.  The three
 // products are the dv pass, the dk pass and the dq pass of the chunk kernels above on one 16-token tile, and are written
 // with their pieces.
+//
+// Bound by latency (B8 H12 T2048 64 x 128) or by the bytes' way (B8 H16 T4096 128 x 128: 273 MB at 5.2 TB/s).  Tiles of 16
+// rows, lanes of tokens 16 .. 31 reading those of 0 .. 15 again (their columns of a product are dropped, their rows are the
+// second k-step, which nobody reads): half the LDS of 32-row tiles with zeros, so that registers (3 waves per SIMD) and not
+// LDS (2 workgroups per unit at 128 x 128) say how many workgroups run at once.  The grid is that many, each walking several
+// pairs with the next one's rows on their way: 18.9 -> 15.5 us at the first shape against 8 per unit, of which most had one pair
+// or two, 53.0 -> 52.0 at the second (20.5 and 55.4 us before the tiles); 2 / 4 / 6 per unit 18.1 / 19.4 / 17.5 and 49.9 / 56.9
+// / 51.9; registers cut to 4 waves per SIMD 18.0 and 52.8.
 constexpr int SI_THREADS = 256;
-// q, k, dk, dq (dk wide) and v, dO, dv (dv wide), 32 rows each; score tiles
-constexpr int si_lds_bytes(int dk, int dv) { return 2 * (2 * FB_SFX_ROWS * (4 * (dk + 8) + 3 * (dv + 8)) + 3 * FB_XP); }
+constexpr int SI_PER_CU = 3;
+// q, k, dk, dq (dk wide) and v, dO, dv (dv wide), 16 rows each; score tiles
+constexpr int si_lds_bytes(int dk, int dv) { return 2 * (FB_SFX_ROWS * (4 * (dk + 8) + 3 * (dv + 8)) + 3 * FB_XP); }
 
 template <int DK, int DV>
 FP_DEVICE void suffix_intra_bwd(const FusedBwdArgs& p, char* lds) {
   using namespace fb;
   constexpr int LDK = DK + 8, LDV = DV + 8;
-  constexpr int TK = 2 * FB_SFX_ROWS * LDK, TV = 2 * FB_SFX_ROWS * LDV;   // tiles of 32 rows (a score tile wants 32)
-  const int tid = fprt::thread_index(), wave = tid >> 6, lane = tid & 63, g = lane >> 5, c = lane & 31;
+  constexpr int TK = FB_SFX_ROWS * LDK, TV = FB_SFX_ROWS * LDV;
+  const int tid = fprt::thread_index(), wave = tid >> 6, lane = tid & 63, g = lane >> 5, c = lane & 31, i16 = c & 15;
   uint16_t* const Qs = reinterpret_cast<uint16_t*>(lds);   // inputs: rows >= Ls are zero
   uint16_t* const Ks = Qs + TK;
   uint16_t* const Vs = Ks + TK;
@@ -1114,10 +1123,10 @@ FP_DEVICE void suffix_intra_bwd(const FusedBwdArgs& p, char* lds) {
   const TrLane tr_acc_k = tr_lane<LDK>(lane, TR_ACC), tr_acc_v = tr_lane<LDV>(lane, TR_ACC);
   // pass of the score tile this wave makes (waves 0..2): X, W and whether it is the backward-walking kind
   //   0 dv: X = k, W = q, reverse     1 dk: X = v, W = dO, reverse     2 dq: X = dO, W = v, forward
-  const uint16_t* const s_xrow = wave == 0 ? Ks + at<LDK>(c, 8 * g) : wave == 1 ? Vs + at<LDV>(c, 8 * g) : Gs + at<LDV>(c, 8 * g);
-  const uint16_t* const s_wrow = wave == 0   ? Qs + at<LDK>(score_row(c), 8 * g)
-                                 : wave == 1 ? Gs + at<LDV>(score_row(c), 8 * g)
-                                             : Vs + at<LDV>(score_row(c), 8 * g);
+  const uint16_t* const s_xrow = wave == 0 ? Ks + at<LDK>(i16, 8 * g) : wave == 1 ? Vs + at<LDV>(i16, 8 * g) : Gs + at<LDV>(i16, 8 * g);
+  const uint16_t* const s_wrow = wave == 0   ? Qs + at<LDK>(score_row(i16), 8 * g)
+                                 : wave == 1 ? Gs + at<LDV>(score_row(i16), 8 * g)
+                                             : Vs + at<LDV>(score_row(i16), 8 * g);
 
   auto view = [&](const void* base, int m, int rows, int D) {
     const char* ptr = static_cast<const char*>(base) + ((size_t)(m / p.H) * p.Ls * p.H + (size_t)(m % p.H)) * D * 2;
@@ -1138,11 +1147,8 @@ FP_DEVICE void suffix_intra_bwd(const FusedBwdArgs& p, char* lds) {
     r.d = fprt::buf_load128(view(p.dO_sfx, mm, nv, DV), offv);
   };
 
-  // rows 16 .. 31 of every tile are never written below: they start, and stay, zero
-  for (int i = tid * 8; i < 4 * TK + 3 * TV; i += SI_THREADS * 8) st128(Qs + i, u32x4{0, 0, 0, 0});
   Rows cur;
   load(fprt::block_index(), cur);
-  fprt::block_sync();
   for (int m = fprt::block_index(); m < pairs; m += fprt::grid_size()) {
     const float lg = p.log2g[m % p.H];
     if (live_k) {
@@ -1190,17 +1196,17 @@ FP_DEVICE void suffix_intra_bwd(const FusedBwdArgs& p, char* lds) {
       const u32x4 za = frag_rows<LDV>(Gs, tr_acc_v, 0, 32 * wave), pq = ld128(XP + lane * 8);
       f32x16 acc = {0};
       acc = fprt::mfma_32x32x16_bf16(za, pq, acc);
-      put_output<LDV>(ODV, c, 32 * wave, g, acc);
+      if (c < FB_SFX_ROWS) put_output<LDV>(ODV, c, 32 * wave, g, acc);
     }
     if (32 * wave < DK) {
       const u32x4 zq = frag_rows<LDK>(Qs, tr_acc_k, 0, 32 * wave), pk = ld128(XP + FB_XP + lane * 8);
       f32x16 acc = {0};
       acc = fprt::mfma_32x32x16_bf16(zq, pk, acc);
-      put_output<LDK>(ODK, c, 32 * wave, g, acc);
+      if (c < FB_SFX_ROWS) put_output<LDK>(ODK, c, 32 * wave, g, acc);
       const u32x4 zk = frag_rows<LDK>(Ks, tr_acc_k, 0, 32 * wave), pd = ld128(XP + 2 * FB_XP + lane * 8);
-      acc = get_state<LDK>(ODQ, c, 32 * wave, g);   // the layout put_output writes: [token][feature]
+      acc = get_state<LDK>(ODQ, i16, 32 * wave, g);   // the layout put_output writes: [token][feature]
       acc = fprt::mfma_32x32x16_bf16(zk, pd, acc);
-      put_output<LDK>(ODQ, c, 32 * wave, g, acc);
+      if (c < FB_SFX_ROWS) put_output<LDK>(ODQ, c, 32 * wave, g, acc);
     }
     fprt::block_sync();
     // rows < Ls leave
