@@ -9,7 +9,14 @@
 // of its waves, so W is read once per NC columns, Z once, and nothing else moves.  The W and Z tiles
 // of a chunk sit row-major in LDS (two stages) and both MFMA operands come from them through the
 // transposing LDS read (the tile layout and the operand helpers are those of retention_bwd_fused.h);
-// two more chunks are on their way in registers.  One workgroup barrier per chunk.  The sum leaves
+// two more chunks are on their way in registers.  One workgroup barrier per chunk.
+//
+// 64 columns: bit for bit what the pass kernel's state-only walk gives (which takes keys of 192 and 256): chunks are cut from
+// where the walk starts, so that walking backward the short one is the first of the sequence, every weight is a power of gamma of
+// its own, and the tokens are summed in order (ContribTile::AS_WALK).  128 columns: chunks from the first token on in both
+// directions, weights of a k-step from those of the one before.
+//
+// The sum leaves
 // through the transposing read as well (16 bits at a time it took as long as four chunks: 128 x 128,
 // B12 T448 H8 17.1 -> 11.5 us a launch, B16 T2048 H8 dv 256 44.6 -> 40.5).
 //
@@ -33,6 +40,7 @@ struct ContribTile {
   static constexpr int W = CH * LDW, STAGE = W + CH * LDZ;              // elements
   static constexpr int NRT = DK / 32, TPW = NRT * (NC / 32) / (NTH / 64);   // 32-row blocks of R; 32 x 32 tiles of it per wave
   static constexpr int NW = CH * (DK / 8) / NTH, NZ = CH * (NC / 8) / NTH;  // 16-byte pieces per thread
+  static constexpr bool AS_WALK = NC == BV;
   // two stages of a W and a Z tile; the copy of R that the final store reads takes their place
   static constexpr int lds_bytes = 2 * 2 * STAGE;
   static_assert(2 * STAGE >= NC * LDW, "the state copy fits where the tiles were");
@@ -67,11 +75,17 @@ FP_DEVICE void put_contribution(const ContribArgs& p, uint16_t* Rt, uint16_t* ds
   }
 }
 
+// AS_WALK: token j of a k-step lies in tile row `walk_row(j)` of it, so that element e of a TR_NAT operand is token
+// walk_token(g, e), as in the pass kernel's operands
+FP_DEVICE int walk_row(int j) { return (j & ~15) | ((j & 3) << 2) | ((j & 4) >> 1) | ((j & 8) >> 3); }
+FP_DEVICE int walk_token(int g, int e) { return 4 * g + (e & 3) + 8 * (e >> 2); }
+
 template <int DK, int NC, int NTH, bool REV>
 FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   using namespace fb;
   using G = ContribTile<DK, NC, NTH>;
   constexpr int LDW = G::LDW, LDZ = G::LDZ, TPW = G::TPW;
+  constexpr bool AS_WALK = G::AS_WALK;
   const int tid = fprt::thread_index(), wave = tid >> 6, lane = tid & 63, g = lane >> 5, c = lane & 31;
   // the workgroups of one (sequence, head) differ by a multiple of the stream count: with a multiple
   // of 8 streams they sit on the same XCD and share the W rows in its L2
@@ -87,14 +101,13 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   const uint32_t roww = (uint32_t)p.H * DK * 2, rowz = (uint32_t)p.H * p.dB * 2;   // bytes between tokens
   const char* const wbase = reinterpret_cast<const char*>(p.W) + (row0 * p.H + h) * DK * 2;
   const char* const zbase = reinterpret_cast<const char*>(p.Z) + (row0 * p.H + h) * p.dB * 2 + (size_t)ct * NC * 2;
-  const fprt::BufView wv = fprt::make_buf(wbase, (uint32_t)(len - 1) * roww + DK * 2);
-  const fprt::BufView zv = fprt::make_buf(zbase, (uint32_t)(len - 1) * rowz + NC * 2);
-  const fprt::BufView none = fprt::make_buf(wbase, 0u);   // visits beyond the walk read zeros and move nothing
 
   uint16_t* const TL = reinterpret_cast<uint16_t*>(lds);   // stage s: W tile at s G::STAGE, Z tile behind it
   // this thread's 16-byte pieces: rows w_row + RW u of W, z_row + RZ u of Z
   constexpr int RW = NTH / (DK / 8), RZ = NTH / (NC / 8);
   const int w_row = tid / (DK / 8), w_piece = tid % (DK / 8), z_row = tid / (NC / 8), z_piece = tid % (NC / 8);
+  const int w_off = at<LDW>(AS_WALK ? walk_row(w_row) : w_row, 8 * w_piece), z_off = at<LDZ>(AS_WALK ? walk_row(z_row) : z_row, 8 * z_piece);
+  static_assert(RW % 16 == 0 && RZ % 16 == 0, "a thread's rows have the same place in their k-steps");
   struct Rows {
     u32x4 w[G::NW], z[G::NZ];
   };
@@ -102,9 +115,11 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   // registers <- the chunk visited it-th
   auto load = [&](int it, Rows& pf) {
     const bool live = it < nch;
-    const int t0 = (REV ? nch - 1 - it : it) * CH;
-    const fprt::BufView w = live ? wv : none, z = live ? zv : none;
-    // rows of a short last chunk beyond `len` read as zeros (contrib_fits)
+    const int end = AS_WALK && REV ? len - it * CH : len;
+    const int t0 = !(AS_WALK && REV) ? (REV ? nch - 1 - it : it) * CH : end > CH ? end - CH : 0;
+    // rows of a short chunk from `end` on read as zeros (contrib_fits); visits beyond the walk read zeros and move nothing
+    const fprt::BufView w = fprt::make_buf(wbase, live ? (uint32_t)(end - 1) * roww + DK * 2 : 0u);
+    const fprt::BufView z = fprt::make_buf(zbase, live ? (uint32_t)(end - 1) * rowz + NC * 2 : 0u);
 #pragma unroll
     for (int u = 0; u < G::NW; ++u) pf.w[u] = fprt::buf_load128(w, (live ? t0 + w_row + RW * u : 0u) * roww + w_piece * 16);
 #pragma unroll
@@ -113,29 +128,36 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   auto stage = [&](int s, const Rows& pf) {
     uint16_t* const st = TL + s * G::STAGE;
 #pragma unroll
-    for (int u = 0; u < G::NW; ++u) st128(st + at<LDW>(w_row + RW * u, 8 * w_piece), pf.w[u]);
+    for (int u = 0; u < G::NW; ++u) st128(st + w_off + RW * u * LDW, pf.w[u]);
 #pragma unroll
-    for (int u = 0; u < G::NZ; ++u) st128(st + G::W + at<LDZ>(z_row + RZ * u, 8 * z_piece), pf.z[u]);
+    for (int u = 0; u < G::NZ; ++u) st128(st + G::W + z_off + RZ * u * LDZ, pf.z[u]);
   };
 
   // this wave's tiles of R: rows a = 32 at_ .., columns n = 32 (nt0 + u) .., u < TPW
   const int at_ = wave % G::NRT, nt0 = (wave / G::NRT) * TPW;
   const TrLane tr_w = tr_lane<LDW>(lane, TR_NAT), tr_z = tr_lane<LDZ>(lane, TR_NAT);
-  // weights of the k-step taken first (the last 16 tokens walking forward, the first 16 walking
-  // backward); each further k-step is 16 tokens further from where the state is read
-  float wk_first[8];
+  auto weight = [&](int e) { return p.s_update * fprt::exp2_approx((float)(e > 0 ? e : 0) * lg); };
+  // Weights of a whole chunk.  AS_WALK: of every k-step.  Else of the k-step taken first (the last 16 tokens walking forward, the
+  // first 16 walking backward); each further k-step is 16 tokens further from where the state is read.
+  constexpr int NWK = AS_WALK ? 4 : 1;
+  float wk_whole[NWK][8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
-    wk_first[e] = p.s_update * fprt::exp2_approx((float)(REV ? nat_token(g, e) + 1 : 15 - nat_token(g, e)) * lg);
+  for (int t = 0; t < NWK; ++t) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int j = AS_WALK ? 16 * t + walk_token(g, e) : REV ? nat_token(g, e) : 48 + nat_token(g, e);
+      wk_whole[t][e] = weight(REV ? j + 1 : CH - 1 - j);
+    }
+  }
   const float g16 = fprt::exp2_approx(16.f * lg), gL = fprt::exp2_approx((float)CH * lg);
 
   f32x16 racc[TPW];
 #pragma unroll
   for (int u = 0; u < TPW; ++u) racc[u] = f32x16{0};
 
-  // L: tokens of the chunk, where it is the short last one of a forward walk (CH otherwise): its weights count from its last token, as
-  // in the walk that carries a sequence through, so that a cut call gives the state of the uncut one.  (Walking backward a short
-  // chunk is the first one, met with R = 0, and its weights are those of any other.)
+  // L: tokens of the chunk, where it is the short one that ends the walk (CH otherwise).  Walking forward its weights count from its
+  // last token, as in the walk that carries a sequence through, so that a cut call gives the state of the uncut one.  (Walking
+  // backward they are those of any other chunk; with 128 columns the short chunk is met first, with R = 0.)
   auto update = [&](int s, auto short_chunk, int L) {
     constexpr bool SHORT = decltype(short_chunk)::value;
     const uint16_t* const Ws = TL + s * G::STAGE;
@@ -143,7 +165,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     const float decay = SHORT ? fprt::exp2_approx((float)L * lg) : gL;
     u32x4 ua[4], ub[4][TPW];
     auto request = [&](int tt) {
-      const int t = REV ? tt : 3 - tt;
+      const int t = AS_WALK || REV ? tt : 3 - tt;
       ua[tt] = frag_rows<LDW>(Ws, tr_w, t, 32 * at_);
 #pragma unroll
       for (int u = 0; u < TPW; ++u) ub[tt][u] = frag_rows<LDZ>(Zs, tr_z, t, 32 * (nt0 + u));
@@ -158,22 +180,22 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     }
     float wk[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) wk[e] = wk_first[e];
+    for (int e = 0; e < 8; ++e) wk[e] = wk_whole[0][e];
     fprt::sched_fence();
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
-      if (SHORT) {
+      if (SHORT && !REV) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int left = L - 1 - 16 * (3 - tt) - nat_token(g, e);
-          wk[e] = p.s_update * fprt::exp2_approx((float)(left > 0 ? left : 0) * lg);
-        }
+        for (int e = 0; e < 8; ++e) wk[e] = weight(L - 1 - (AS_WALK ? 16 * tt + walk_token(g, e) : 16 * (3 - tt) + nat_token(g, e)));
+      } else if (AS_WALK) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) wk[e] = wk_whole[AS_WALK ? tt : 0][e];
       }
       const u32x4 wa = weigh(ua[tt], wk);
 #pragma unroll
       for (int u = 0; u < TPW; ++u) racc[u] = fprt::mfma_32x32x16_bf16(wa, ub[tt][u], racc[u]);
       if (tt + 2 < 4) request(tt + 2);
-      if (tt < 3) {
+      if (!AS_WALK && tt < 3) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) wk[e] *= g16;
       }
@@ -184,7 +206,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   // Chunk it is multiplied from stage it & 1 while chunk it + 1 moves from registers into the
   // other stage and the loads of chunk it + 3 take its place; chunk it + 2 is on its way in the
   // second set of registers.
-  const int nwhole = REV ? nch : len / CH;
+  const int nwhole = REV && !AS_WALK ? nch : len / CH;
   Rows pa, pb;
   load(0, pa);
   load(1, pb);

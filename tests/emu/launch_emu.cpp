@@ -152,6 +152,28 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* /*stream*/, const char**
   return a.dk == 64 ? run_contrib<64, 64, 256>(a) : fpk::contrib_columns(a) == 64 ? run_contrib<128, 64, 256>(a) : run_contrib<128, 128, 512>(a);
 }
 
+// What every sequence (segment) adds to a zero state, U in fp32 halves, by the state-only kernel or (`walk`) by the pass kernel's
+// state-only walk: the two have to agree bit for bit where the former takes 64 columns.
+extern "C" int emu_state_only(int walk, const uint16_t* W, const uint16_t* Z, uint16_t* U, uint16_t* U_lo, int B, int T, int H, int dk,
+                              int dv, int segs, int total, int reverse, float log2g) {
+  const char* msg = "";
+  if (!walk) {
+    fpk::ContribArgs c = {};
+    c.W = W; c.Z = Z; c.U = U; c.U_lo = U_lo;
+    c.B = B; c.T = T; c.H = H; c.dk = dk; c.dB = dv; c.segs = segs; c.total = total; c.reverse = reverse;
+    c.s_update = reverse ? 1.f : 0.125f;
+    for (int h = 0; h < H; ++h) c.log2g[h] = log2g / (float)(h + 1);
+    return fpk_launch_contrib(c, nullptr, &msg);
+  }
+  fpk::PassArgs a = {};
+  a.X = W; a.W = W; a.Z = Z; a.Rout = U; a.Rout_lo = U_lo;
+  a.B = B; a.T = T; a.H = H; a.dA = dk; a.dB = dv; a.segs = segs; a.total = total; a.reverse = reverse; a.state_only = 1;
+  a.rs_a = dv; a.rs_n = 1;
+  a.s_intra = a.s_read = 1.f; a.s_update = reverse ? 1.f : 0.125f;
+  for (int h = 0; h < H; ++h) a.log2g[h] = log2g / (float)(h + 1);
+  return fpk_launch_pass(a, nullptr, &msg);
+}
+
 int fpk_launch_scan(const fpk::ScanArgs& a, void* /*stream*/, const char** err) {
   if (const char* why = fpk::check_scan(a)) {
     *err = why;

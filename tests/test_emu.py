@@ -2,6 +2,7 @@
 tests/emu/) and compares with the oracle.  This checks indexing, chunk scheduling, the pass
 mapping and ragged/unaligned handling without a GPU; it assumes the documented MFMA lane
 layout, which only the GPU parity tests can confirm."""
+import ctypes
 import os
 import subprocess
 
@@ -302,6 +303,29 @@ def test_cut_final_state_follows_the_uncut_walk(emu_lib, T, dk, dv):
     _, S1 = hp.raw_fwd(emu_lib, q, k, v, s, (0.97,))
     share = (S != S1).float().mean().item()
     assert n > 0 and share <= 1e-3, share
+
+
+@pytest.mark.parametrize("reverse", (0, 1))
+@pytest.mark.parametrize("T,total,dk,dv", [
+    (144, 360, 64, 64),     # a short chunk in every segment, the last one shorter still
+    (128, 257, 64, 192),    # whole chunks, a last segment of one token; three workgroups per segment
+    (63, 63, 64, 64),       # less than a chunk
+    (215, 215, 128, 64),    # 128 rows, 64 columns
+    (64, 191, 128, 192),
+])
+def test_state_only_kernel_matches_the_walk(emu_lib, T, total, dk, dv, reverse):
+    """Where the state-only kernel takes 64 columns it cuts the chunks, weighs the operands and sums as the pass kernel's
+    state-only walk does, in either direction: same bits."""
+    segs, H = -(-total // T), 2
+    w, _, z, _ = hp.make_inputs(1, total, H, dk, dv, seed=T + dv)
+    out = []
+    for walk in (0, 1):
+        u = torch.zeros(2, segs, H, dk, dv, dtype=torch.int16)
+        rc = emu_lib.emu_state_only(walk, hp._p(w), hp._p(z), hp._p(u[0]), hp._p(u[1]), segs, T, H, dk, dv,
+                                    segs, total, reverse, ctypes.c_float(-0.03))
+        assert rc == 0
+        out.append(u)
+    assert out[0].any() and torch.equal(out[0], out[1])
 
 
 @pytest.mark.parametrize("T,dk,dv", [
