@@ -299,7 +299,7 @@ int fpk_launch_pass(const fpk::PassArgs& args, void* stream, const char** err) {
     return 1;
   }
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (fpk::pop_folds(a)) {
+  if (fpk::pop_folds(a, fpk_compute_units())) {
     if (arm(reinterpret_cast<const void*>(pop_fold_fwd_kernel), fpk::pf_lds_bytes(), 64 + 34, err)) return 1;
     hipLaunchKernelGGL(pop_fold_fwd_kernel, dim3((unsigned)(a.B * a.H * (a.dB / fpk::BV))), dim3(fpk::PF_THREADS), fpk::pf_lds_bytes(), st, a);
     return launched(err);

@@ -350,12 +350,26 @@ FP_DEVICE void pop_fold_fwd(const PassArgs& p, char* lds, int wg) {
   }
 }
 
-// Whether the kernel above takes a planned pass: a forward with suffixes that fit beside a chunk, keys of 64, whole blocks of at
-// most two chunks.  Its step is longer than a plain chunk's in the suffix walk, so it needs suffixes to save: us a call, walk ->
-// here, B8 T2048 H8 64 x 128 (suffixes of 16 but where said) blocks of 32 (B4 T1024) 76 -> 54, 64 (H12) 77 -> 61, 128 (one token) 60 -> 55,
-// 192 51 -> 52, 200 63 -> 65, 1024 (B2 T4096 H4) 85 -> 95.
-inline bool pop_folds(const PassArgs& a) {
-  return a.Ls > 0 && a.Ls <= PF_SFX && !a.reverse && a.dA == PF_DK && a.T == a.nblk * a.block && a.rs_n == 1 && a.block <= 2 * CH;
+// Whether the kernel above takes a planned pass on a device of `compute_units`: a forward with suffixes that fit beside a chunk,
+// keys of 64, whole blocks of at most a chunk and a half or so, where it is the faster one.  Its step takes about 1.7 us against 1.1 for
+// an item of the walk, and a workgroup half a microsecond longer to start, so it needs enough suffixes to save, and of 64 x 64
+// states on a full device, where the bytes count too, more of them (512 a token and tile; 384 at 64 x 128, 320 at 64 x 256).
+// Speed here over that of the walk, inputs not in a cache, 128 to 1 024 workgroups, blocks of 16 to 64 tokens:
+//                1 block        2 blocks       3 blocks       4 blocks       6 blocks       12 blocks      32 blocks
+//   64 x 64      .79 to .94     .84 to 1.02    .89 to 1.07    .93 to 1.11    .94 to 1.18    1.01 to 1.29   1.08 to 1.41
+//   64 x 128     .85 to .92     .90 to 1.00    .97 to 1.06    1.01 to 1.11   1.02 to 1.20   1.09 to 1.30   1.13 to 1.41
+//   64 x 256     .85 to .95     .93 to 1.00    .97 to 1.08    1.03 to 1.13   1.06 to 1.19   1.09 to 1.30   1.10 to 1.40
+// (the longer the block the lower; 32 workgroups of 64 x 64: 4 blocks of 64 1.08, 6 blocks 1.13), blocks of 72 to 96, 104 and 128:
+//                4 blocks                          8 blocks                           12 blocks
+//   64 x 64      .95 to 1.00, .92 to .99, .90      .99 to 1.06, .95 to 1.03, .89      1.01 to 1.08, .97 to 1.04, .93 to 1.00
+//   64 x 128     .97 to 1.00, .97 to 1.00, .92     1.02 to 1.07, 1.01 to 1.06, .89    1.03 to 1.09, 1.02 to 1.08, .94 to 1.03
+//   64 x 256     .98 to 1.02, .99 to 1.00, .93     1.02 to 1.06, 1.01 to 1.06, .94    1.03 to 1.09, 1.03 to 1.08, .94 to 1.05
+inline bool pop_folds(const PassArgs& a, int compute_units) {
+  if (a.Ls <= 0 || a.Ls > PF_SFX || a.reverse || a.dA != PF_DK || a.T != a.nblk * a.block || a.rs_n != 1) return false;
+  const bool by_bytes = a.dB == BV && 2LL * a.B * a.H > compute_units;
+  if (a.block > CH) return a.block <= (a.dB == BV ? 96 : 104) && a.nblk >= (by_bytes ? 12 : 8);
+  if (by_bytes) return a.nblk >= 3 && 4 * a.nblk >= a.block - 16;
+  return a.nblk >= (2 * a.block <= CH ? 3 : 4);
 }
 
 }  // namespace fpk

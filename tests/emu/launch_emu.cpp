@@ -44,7 +44,7 @@ int fpk_launch_pass(const fpk::PassArgs& args, void* /*stream*/, const char** er
     *err = why;
     return 1;
   }
-  if (fpk::pop_folds(a)) {
+  if (fpk::pop_folds(a, fpk_compute_units())) {
     const int nwg = a.B * a.H * (a.dB / fpk::BV);
     return run_grid(fpk::PF_THREADS, nwg, fpk::pf_lds_bytes(),
                     [&](char* l) { fpk::pop_fold_fwd(a, l, fpk::place_workgroup(fprt::block_index(), nwg, 1).wg); });
@@ -150,6 +150,14 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* /*stream*/, const char**
     return 1;
   }
   return a.dk == 64 ? run_contrib<64, 64, 256>(a) : fpk::contrib_columns(a) == 64 ? run_contrib<128, 64, 256>(a) : run_contrib<128, 128, 512>(a);
+}
+
+// The rule that chooses the forward of a POP call with suffixes, on a device of `compute_units`
+extern "C" int emu_pop_folds(int B, int T, int H, int dk, int dv, int block, int Ls, int compute_units) {
+  fpk::PassArgs a = {};
+  a.B = B; a.T = T; a.H = H; a.dA = dk; a.dB = dv; a.block = block; a.nblk = T / block; a.Ls = Ls;
+  a.rs_a = dv; a.rs_n = 1;
+  return fpk::pop_folds(a, compute_units);
 }
 
 // What every sequence (segment) adds to a zero state, U in fp32 halves, by the state-only kernel or (`walk`) by the pass kernel's

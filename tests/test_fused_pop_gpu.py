@@ -77,6 +77,27 @@ def test_fused_parity_sweep(B, N, block, Ls, H, dk, dv):
     run_fused(B, N, block, Ls, H, dk, dv, 0.3, seed=N * block + Ls, decay_range=(5, 12))
 
 
+@pytest.mark.parametrize("B,N,block,Ls,H,dv,state_std", [
+    (2, 8, 65, 16, 4, 64, 0.3),      # a chunk of one token per block
+    (1, 9, 96, 1, 2, 192, None),     # the longest blocks, one-token suffixes, three column tiles, no initial state
+    (2, 5, 64, 7, 4, 256, 0.3),      # four column tiles
+    (17, 8, 90, 16, 8, 128, 0.3),    # more workgroups than compute units
+    (37, 4, 64, 16, 7, 192, 0.3),    # ... several rounds of them, no multiple of the XCDs
+    (9, 12, 63, 15, 31, 64, None),   # ... one tile of columns
+])
+def test_folded_forward_sizes(hip_lib, B, N, block, Ls, H, dv, state_std):
+    """64-wide keys, whole blocks and short suffixes: the forward that takes a suffix as part of the chunk at its boundary."""
+    _say(f"[folded fwd] B{B} N{N} block{block} Ls{Ls} H{H} dv{dv} s0={state_std}")
+    decays = oracle.head_decays(H, (5, 12))
+    q, k, v, s = hp.make_inputs(B, N * block, H, 64, dv, seed=block + dv, state_std=state_std, device=DEV)
+    sfx = hp.make_suffix_inputs(B, N, Ls, H, 64, dv, seed=block + 1, device=DEV)
+    o, o_sfx, S = hp.raw_fused_fwd(hip_lib, q, k, v, s, sfx, decays, block)
+    torch.cuda.synchronize()
+    o_ref, os_ref, S_ref = hp.oracle_fused(q, k, v, s, sfx, decays, block, device=DEV)
+    for name, got, ref, head_dim in (("o", o, o_ref, 2), ("o_sfx", o_sfx, os_ref, 2), ("last S", S, S_ref, 1)):
+        hp.assert_close(got, ref, name, head_dim=head_dim)
+
+
 @pytest.mark.parametrize("B,N,block,Ls,H,dk,dv,tail", [
     (2, 3, 64, 16, 4, 128, 128, 40),     # tokens after the last block boundary, fewer than a chunk
     (2, 2, 144, 16, 2, 64, 128, 100),    # ... more than a chunk (the reference's generation block size)
