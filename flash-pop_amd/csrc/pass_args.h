@@ -128,6 +128,15 @@ struct ContribArgs {
 // Whether the rows of whole chunks, those beyond a sequence's end included, have 32-bit byte offsets in that pass (one that wrapped
 // would come back into its view).
 inline bool contrib_fits(long long T, int H, int dk, int dB) { return (T + CH) * H * (dk > dB ? dk : dB) * 2 < (1LL << 32); }
+// Whether that pass is the faster form of a state-only pass over `seqs` sequences, else it is the pass kernel's state-only walk, 64
+// columns of a state per workgroup of 512 threads, one per unit.  128 columns: always (B16 T2048 H8 128 x 256: 40.5 us against 66).
+// 64 columns: workgroups of 256 threads, several to a unit, and the same bits, so it takes more of them than there are units to
+// win.  Walk -> that pass, us a launch, workgroups on 256 units:
+//   128 rows   96 wg 7.8 -> 9.4   160 wg 10.1 -> 11.2   256 wg 12.7 -> 15.6   288 wg 12.5 -> 11.0   384 wg 33.2 -> 27.6
+//   64 rows    96 wg 7.1 -> 7.1   160 wg 7.0 -> 7.7     256 wg 9.6 -> 10.4    320 wg 11.6 -> 10.0   512 wg 17.1 -> 13.4   768 wg 28.8 -> 17.4
+inline bool contrib_pays(long long seqs, int H, int dk, int dB, int compute_units) {
+  return (dk == 128 && dB % 128 == 0) || seqs * H * (dB / BV) > compute_units;
+}
 // One recurrent (decode) step for every (batch, head):  S' = gamma S + (scale k)^T v,  o = q S'.
 // q, k [B,H,dk]; v, o [B,H,dv]; S [B,H,dk,dv]; all bf16, fp32 arithmetic.  s_out may be s_in.
 struct DecodeArgs {

@@ -152,6 +152,9 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* /*stream*/, const char**
   return a.dk == 64 ? run_contrib<64, 64, 256>(a) : fpk::contrib_columns(a) == 64 ? run_contrib<128, 64, 256>(a) : run_contrib<128, 128, 512>(a);
 }
 
+// The rule that chooses the state-only pass
+extern "C" int emu_contrib_pays(int seqs, int H, int dk, int dv, int compute_units) { return fpk::contrib_pays(seqs, H, dk, dv, compute_units); }
+
 // The rule that chooses the forward of a POP call with suffixes, on a device of `compute_units`
 extern "C" int emu_pop_folds(int B, int T, int H, int dk, int dv, int block, int Ls, int compute_units) {
   fpk::PassArgs a = {};
