@@ -62,8 +62,6 @@ struct FbTile {
   static constexpr int ROWS = FB_THREADS / PPR;    // rows that one sweep of the 512 threads covers
   static constexpr int NU = CH / ROWS;             // sweeps per tile = pieces per thread
 };
-constexpr int FB_LD = FbTile<FB_D>::LD;     // the 128-wide tile (what the state-only kernel of segment_contrib.h uses too)
-constexpr int FB_TILE = FbTile<FB_D>::ELEMS;
 constexpr int FB_XP = 32 * 32;              // elements of one score tile in operand layout
 // How POP suffixes take part in the walks:
 //   FB_PLAIN  none
@@ -95,7 +93,6 @@ namespace fb {
 // element offset of (row, col) in a tile of pitch LD
 template <int LD>
 FP_DEVICE int at(int row, int col) { return row * LD + col; }
-FP_DEVICE int at(int row, int col) { return at<FB_LD>(row, col); }
 
 // Operand that runs along the columns of a tile: columns 16 t + 8 g .. + 7 of the lane's row.
 // `rowp` points at column 8 g of that row.
@@ -124,7 +121,6 @@ FP_DEVICE TrLane tr_lane(int lane, TrOrder order) {
   const int r_hi = order == TR_NAT ? r_lo + 1 : order == TR_ACC ? r_lo + 2 : r_lo + 4;
   return TrLane{r_lo * LD + col, r_hi * LD + col};
 }
-FP_DEVICE TrLane tr_lane(int lane, TrOrder order) { return tr_lane<FB_LD>(lane, order); }
 // token (within its k-step) of element e of a TR_NAT operand
 FP_DEVICE int nat_token(int g, int e) { return 2 * g + 4 * (e & 3) + (e >> 2); }
 // row of the score tile that accumulator row m stands for: within each group of 16, m = 8 h + 4 g + e
@@ -138,7 +134,6 @@ FP_DEVICE u32x4 frag_rows(const uint16_t* tile, const TrLane& tl, int t, int cba
   const u32x2 hi = fprt::lds_read_tr16_b64(p + tl.hi);
   return u32x4{lo[0], lo[1], hi[0], hi[1]};
 }
-FP_DEVICE u32x4 frag_rows(const uint16_t* tile, const TrLane& tl, int t, int cbase) { return frag_rows<FB_LD>(tile, tl, t, cbase); }
 
 // eight packed bf16 times eight weights
 FP_DEVICE u32x4 weigh(u32x4 v, const float (&w)[8]) {
@@ -180,7 +175,6 @@ FP_DEVICE Item suffix_item(const Common& k, int n) { return Item{((uint32_t)k.b 
 // Walking backward with suffixes: the suffix at T, then per block (from the last) its chunks
 // from the last to the first and the suffix at its lower boundary.
 FP_DEVICE Item item_backward(const Common& k, int it) {
-  if (k.block == 0) return chunk_item(k, k.nch - 1 - it);
   if (it <= 0) return it == 0 ? suffix_item(k, k.nblk) : Item{0u, 0, false};
   const int j = it - 1, blk = k.nblk - 1 - j / (k.spb + 1), r = j % (k.spb + 1);
   if (blk < 0) return Item{0u, 0, false};
@@ -188,12 +182,11 @@ FP_DEVICE Item item_backward(const Common& k, int it) {
 }
 // Walking forward with suffixes: per block the suffix at its lower boundary and its chunks, then the suffix at T.
 FP_DEVICE Item item_forward(const Common& k, int it) {
-  if (k.block == 0) return chunk_item(k, it);
   const int blk = it / (k.spb + 1), r = it % (k.spb + 1);
   if (it < 0 || blk > k.nblk || (blk == k.nblk && r > 0)) return Item{0u, 0, false};
   return r == 0 ? suffix_item(k, blk) : chunk_item(k, blk * k.spb + r - 1);
 }
-FP_DEVICE int item_count(const Common& k) { return k.block == 0 ? k.nch : 1 + k.nblk * (k.spb + 1); }
+FP_DEVICE int item_count(const Common& k) { return 1 + k.nblk * (k.spb + 1); }
 
 // FOLD: a chunk as chunk `chunk` of block `block`, stepped from chunk to chunk (a suffix hangs off chunk 0 of its block); asking
 // the chunk's number for it took several divisions a step (B8 H12 T2048 64 x 128, blocks of 64: 95.8 -> 93.1 us a launch).
@@ -259,7 +252,7 @@ FP_DEVICE u32x4 staged_piece(const Common& k, const uint16_t* tile, int u) {
 template <int D>
 FP_DEVICE void store_piece(const Common& k, const fprt::BufView& v, int u, u32x4 d) {
   using G = FbTile<D>;
-  // non-temporal: the gradients are not read back here, and kept out of the caches they leave
+  // written through, non-temporal: the gradients are not read back here, and kept out of the caches they leave
   // room for the rows that the other workgroup of the stream is about to read a second time
   fprt::buf_store128_through(v, (uint32_t)(k.tid / G::PPR + G::ROWS * u) * ((uint32_t)k.H * D * 2) + (k.tid % G::PPR) * 16, d);
 }
@@ -287,7 +280,6 @@ FP_DEVICE void put_output(uint16_t* tile, int i, int nbase, int g, const f32x16&
 // accumulator tile (rows a = abase + acc_row, column n) -> Rt
 template <int LD>
 FP_DEVICE void put_state(uint16_t* Rt, int n, int abase, int g, const f32x16& acc) { put_output<LD>(Rt, n, abase, g, acc); }
-FP_DEVICE void put_state(uint16_t* Rt, int n, int abase, int g, const f32x16& acc) { put_output<FB_LD>(Rt, n, abase, g, acc); }
 template <int LD>
 FP_DEVICE f32x16 get_state(const uint16_t* Rt, int n, int abase, int g) {
   f32x16 acc;
