@@ -1083,11 +1083,16 @@ FP_DEVICE void fused_bwd(const FusedBwdArgs& p, char* lds, int block) {
 //
 // Bound by latency (B8 H12 T2048 64 x 128) or by the bytes' way (B8 H16 T4096 128 x 128: 273 MB at 5.2 TB/s).  Tiles of 16
 // rows, lanes of tokens 16 .. 31 reading those of 0 .. 15 again (their columns of a product are dropped, their rows are the
-// second k-step, which nobody reads): half the LDS of 32-row tiles with zeros, so that registers (3 waves per SIMD) and not
-// LDS (2 workgroups per unit at 128 x 128) say how many workgroups run at once.  The grid is that many, each walking several
-// pairs with the next one's rows on their way: 18.9 -> 15.5 us at the first shape against 8 per unit, of which most had one pair
-// or two, 53.0 -> 52.0 at the second (20.5 and 55.4 us before the tiles); 2 / 4 / 6 per unit 18.1 / 19.4 / 17.5 and 49.9 / 56.9
-// / 51.9; registers cut to 4 waves per SIMD 18.0 and 52.8.
+// second k-step, which nobody reads): half the LDS of 32-row tiles with zeros (20.5 -> 18.9 and 55.4 -> 53.0 us a launch at these
+// two), so that registers and not LDS say how many workgroups run at once: three per unit, four at 64 x 64.
+//
+// The grid is SI_PER_CU workgroups per unit, each walking several pairs with the next one's rows on their way.  Three are the best
+// or within 2 % of it for every pair of dimensions; what the number changes beside the workgroups in flight is how evenly the
+// pairs divide.  2 / 3 / 4 / 8 per unit, the whole backward in us, 12 and 33 pairs per unit (B8 H12 T2048, B8 H16 T4096):
+//   64 x 64     85.3 /  83.5 /  81.9 /  84.0   176.2 / 169.4 / 166.5 / 168.5
+//   64 x 128   114.8 / 111.9 / 116.2 / 115.2   247.9 / 240.8 / 249.7 / 244.6
+//   128 x 64   117.0 / 115.5 / 117.9 / 117.3   248.7 / 245.3 / 254.8 / 248.1
+//   128 x 128  152.7 / 153.6 / 155.3 / 153.7   341.8 / 346.1 / 350.2 / 345.7
 constexpr int SI_THREADS = 256;
 constexpr int SI_PER_CU = 3;
 // q, k, dk, dq (dk wide) and v, dO, dv (dv wide), 16 rows each; score tiles
