@@ -425,16 +425,19 @@ int plan_segments(const Shape& s) {
 }
 // Whether n segments shorten the chain of chunk steps by what the cut costs: its extra launches, and the segment states
 // that it moves.  Forward, measured at 1.1 us (64-wide keys) to 1.4 us (128) a step on the 256-unit device, uncut -> cut:
-//   64 x 64    H4 B1        18 chunks 23.5 -> 20.3 us, 13 chunks 18.2 -> 19.9
-//   64 x 128   H12 B1       79 chunks 90.7 -> 39.6,    18 chunks 23.9 -> 22.2,  13 chunks 18.5 -> 20.9
-//   128 x 128  H8 B3        28 chunks 44.1 -> 38.5,    18 chunks 30.0 -> 35.3
-//   128 x 256  H8 B2        40 chunks 61.1 -> 51.5,    28 chunks 44.2 -> 46.4
-// Backward (the uncut passes share launches, or are the fused kernel with its longer step; the cut has four launches):
-//   64 x 64    H4 B1        28 chunks 35.4 -> 30.6,    18 chunks 24.3 -> 29.6
-//   64 x 64    H12 B6       40 chunks 84.9 -> 81.8,    28 chunks 61.6 -> 64.9 (fused)
-//   64 x 128   H12 B1       18 chunks 53.7 -> 43.4,    13 chunks 41.3 -> 42.3
-//   128 x 128  H16 B1       79 chunks 119 -> 91,       40 chunks 62.4 -> 63.4,  28 chunks 45.6 -> 56.9
-//   128 x 256  H8 B2        28 chunks 121 -> 84,       18 chunks 81.0 -> 78.9
+//   64 x 64    H4 B1        18 chunks 23.8 -> 19.9 us, 16 chunks 21.8 -> 18.5,  13 chunks 18.4 -> 19.7
+//   64 x 128   H12 B1       79 chunks 89.6 -> 32.8,    18 chunks 24.4 -> 20.9,  13 chunks 18.9 -> 20.6
+//   128 x 128  H8 B3        28 chunks 44.0 -> 30.7,    18 chunks 30.0 -> 29.3,  13 chunks 23.5 -> 28.7
+//   128 x 256  H8 B2        40 chunks 60.0 -> 38.6,    28 chunks 43.9 -> 33.8,  18 chunks 30.0 -> 38.3
+// Backward (the uncut passes share launches, or are the fused kernel with its longer step; the cut has four launches and the
+// forward's states):
+//   64 x 64    H4 B1        28 chunks 35.3 -> 27.8,    18 chunks 24.8 -> 28.7
+//   64 x 64    H12 B6       79 chunks 132 -> 133,      40 chunks 69.8 -> 79.5,  28 chunks 50.5 -> 63.6 (fused)
+//   64 x 128   H12 B1       18 chunks 54.3 -> 41.9,    13 chunks 41.4 -> 40.9
+//   128 x 128  H16 B1       79 chunks 116 -> 82,       40 chunks 61.8 -> 50.8,  28 chunks 45.1 -> 44.6
+//   128 x 256  H8 B2        28 chunks 119 -> 68,       18 chunks 80.0 -> 70.9,  13 chunks 60.8 -> 61.8
+// The line dates from slower state-only passes, scans and fused backwards: it leaves calls of 16 to 18 chunks uncut that a cut
+// would shorten (128 x 256 up to 28), and cuts the backward of 64 x 64 on 72 streams from 40 chunks on.
 // `block`: a POP call, whose chunks end at its blocks and whose gradient passes share fewer launches (64 x 128, B4 H4 T1440
 // in blocks of 144, 30 chunks, with the suffix call and the launches between the two: 200 -> 166 us).
 bool cut_pays(const Shape& s, int n, int tokens, bool backward, int block = 0) {
@@ -466,10 +469,10 @@ int plan_backward(const Shape& s) {
 // moves 2.  There are as many states as blocks, however many fill the chip, and the cut call streams them at 3.5 to 4.5 TB/s
 // while the uncut one walks, 1.4 to 2 us a chunk: 6.8 MB a step tell the two apart (three steps: the launches).  Uncut -> cut,
 // forward / backward, us:
-//   128 x 128  blocks of 64    B10 H4 T4096   132 -> 259 / 226 -> 399      B4 H4 T4096   131 -> 110 / 225 -> 161
-//   128 x 128  blocks of 144   B10 H4 T16384  593 -> 678 / 934 -> 1091     B4 H8 T4096   145 -> 137 / 237 -> 231
-//   64 x 128   blocks of 64    B6 H8 T4096     99 -> 131 / 216 -> 231      B6 H4 T2048    52 -> 47 / 162 -> 80
-//   64 x 64    blocks of 64    B10 H8 T4096    98 -> 120 / 174 -> 217      B6 H8 T16384  452 -> 377 / 672 -> 594
+//   128 x 128  blocks of 64    B10 H4 T4096   131 -> 227 / 226 -> 355      B4 H4 T4096   130 -> 97 / 226 -> 148
+//   128 x 128  blocks of 144   B10 H4 T16384  589 -> 595 / 926 -> 1014     B4 H8 T4096   145 -> 119 / 237 -> 217
+//   64 x 128   blocks of 64    B6 H8 T4096     98 -> 144 / 193 -> 258      B6 H4 T2048    52 -> 52 / 163 -> 81
+//   64 x 64    blocks of 64    B10 H8 T4096    98 -> 123 / 160 -> 236      B6 H8 T16384  444 -> 432 / 665 -> 667
 bool block_states_pay(const Shape& s, int segments, int block) {
   if (fpk_launch_steps() <= 0) return true;   // (a device whose launches cost nothing)
   const double chunks = (double)segments * ((block + fpk::CH - 1) / fpk::CH);
