@@ -168,8 +168,14 @@ int main() {
   rc |= plain(1, 512, 1, 64, 128, true);      // cut into segments (state-only walk, scan)
   rc |= plain(1, 640, 1, 128, 256, true);     // ... with the state-only kernel for 128-wide keys, two workgroups per segment
   rc |= plain(1, 511, 1, 128, 128, true);     // uneven segments, fp32 states: the last chunk of that kernel is short
-  rc |= plain(1, 257, 1, 64, 64, true);       // ... the last segment is one token
+  rc |= plain(1, 257, 1, 64, 64, true);       // ... in the state-only walk, the last segment is one token
+  rc |= plain(1, 512, 1, 256, 64, true);      // the state-only walk with two visits per chunk
+  rc |= plain(1, 511, 1, 192, 64, true);      // ... with three, fp32 states
+  rc |= plain(1, 768, 1, 64, 256, true);      // the state-only kernel for 64-wide keys (more workgroups than units)
+  rc |= plain(1, 700, 1, 64, 256, true);      // ... short chunks at either end of a walk, fp32 states
   rc |= pop_split(1, 150, 1, 128, 128, 65);   // blocks and a tail that end inside chunks
+  rc |= pop_split(1, 600, 1, 128, 64, 65);    // ... the state-only kernel for 128 rows and 64 columns
+  rc |= pop_split(1, 600, 1, 64, 64, 65);     // ... for 64 rows
   rc |= pop(1, 287, 1, 64, 128, 144);
   rc |= pop(2, 28, 1, 64, 64, 15);
   rc |= pop(1, 40, 1, 64, 64, 100);           // no full block
@@ -180,6 +186,7 @@ int main() {
   rc |= fused(1, 1, 80, 5, 1, 64, 128, 30);   // tokens after the last block boundary
   rc |= fused(1, 0, 90, 12, 1, 64, 64, 70);   // no full block
   rc |= fused(1, 2, 64, 100, 1, 128, 64);     // suffixes in two parts
+  rc |= fused(1, 8, 90, 16, 1, 64, 64);       // the forward that folds suffixes into chunks: two chunks a block, the longest suffixes
   fp_set_backward_choice(2, -1);        // one short stream would not take this path by itself
   rc |= fused(1, 4, 64, 16, 1, 128, 128);     // backward in the kernel that carries dS once, suffixes as extra stops
   rc |= plain(1, 210, 1, 128, 128, false);    // the same kernel without suffixes, ragged last chunk
