@@ -412,7 +412,7 @@ def gpu_leg(args):
             "tokens": i["tokens"],
             "ms_per_step": round(l5_ms, 4),
             "roofline": step_roofline("layer5", i, l5_ms, l5_fwd, l5_bwd,
-                                      "suffix walk of the pass kernel (forward); the backward kernels of this shape"),
+                                      "forward with the suffixes folded into the chunks; fused backward with folded suffixes + suffix_intra_bwd_kernel"),
         }
         del step
     if not args.no_layer:
