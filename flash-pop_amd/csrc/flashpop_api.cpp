@@ -557,8 +557,7 @@ int contributions(const Shape& seg, const double* decays, const void* w_rows, co
                   const Workspace& w, void* stream) {
   const float sc = 1.0f / std::sqrt((float)seg.dk);
   // the kernel that holds whole columns of the state per workgroup
-  if ((seg.dk == 64 || seg.dk == fpk::FB_D) && fpk::contrib_fits(seg.T, seg.H, seg.dk, seg.dv) &&
-      fpk::contrib_pays(seg.B, seg.H, seg.dk, seg.dv, fpk_compute_units())) {
+  if (fpk::contrib_pays(seg.B, seg.T, seg.H, seg.dk, seg.dv, fpk_compute_units()) && fpk::contrib_fits(seg.T, seg.H, seg.dk, seg.dv)) {
     fpk::ContribArgs c;
     std::memset(&c, 0, sizeof c);
     c.W = in(w_rows); c.Z = in(z_rows); c.U = w.contrib; c.U_lo = w.contrib_lo;

@@ -431,9 +431,7 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* stream, const char** err
   }
   const hipStream_t st = static_cast<hipStream_t>(stream);
   if (a.dk == 64) return a.reverse ? launch_contrib<64, 64, 256, true>(a, 0, st, err) : launch_contrib<64, 64, 256, false>(a, 1, st, err);
-  if (fpk::contrib_columns(a) == 64)
-    return a.reverse ? launch_contrib<128, 64, 256, true>(a, 2, st, err) : launch_contrib<128, 64, 256, false>(a, 3, st, err);
-  return a.reverse ? launch_contrib<128, 128, 512, true>(a, 4, st, err) : launch_contrib<128, 128, 512, false>(a, 5, st, err);
+  return a.reverse ? launch_contrib<128, 128, 512, true>(a, 2, st, err) : launch_contrib<128, 128, 512, false>(a, 3, st, err);
 }
 
 int fpk_launch_scan(const fpk::ScanArgs& a, void* stream, const char** err) {

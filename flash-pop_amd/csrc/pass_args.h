@@ -114,7 +114,7 @@ struct ScanArgs {
 // State-only pass for states of 64 or 128 rows (segment_contrib.h): U[b][h] = what sequence b adds to a
 // zero state, sum_j weight(j) W[j]^T Z[j] with weight(j) = s_update gamma^(T - 1 - j) walking forward
 // (`reverse` = 0) and s_update gamma^(j + 1) walking backward.  W [B,T,H,dk], Z [B,T,H,dB],
-// U [B,H,dk,dB], bf16; dB a multiple of 64.  `segs`, `total` as in PassArgs.
+// U [B,H,dk,dB], bf16; dB a multiple of dk.  `segs`, `total` as in PassArgs.
 struct ContribArgs {
   const uint16_t* W;
   const uint16_t* Z;
@@ -129,13 +129,21 @@ struct ContribArgs {
 // would come back into its view).
 inline bool contrib_fits(long long T, int H, int dk, int dB) { return (T + CH) * H * (dk > dB ? dk : dB) * 2 < (1LL << 32); }
 // Whether that pass is the faster form of a state-only pass over `seqs` sequences, else it is the pass kernel's state-only walk, 64
-// columns of a state per workgroup of 512 threads, one per unit.  128 columns: always (B16 T2048 H8 128 x 256: 40.5 us against 66).
-// 64 columns: workgroups of 256 threads, several to a unit, and the same bits, so it takes more of them than there are units to
-// win.  Walk -> that pass, us a launch, workgroups on 256 units:
-//   128 rows   96 wg 7.8 -> 9.4   160 wg 10.1 -> 11.2   256 wg 12.7 -> 15.6   288 wg 12.5 -> 11.0   384 wg 33.2 -> 27.6
-//   64 rows    96 wg 7.1 -> 7.1   160 wg 7.0 -> 7.7     256 wg 9.6 -> 10.4    320 wg 11.6 -> 10.0   512 wg 17.1 -> 13.4   768 wg 28.8 -> 17.4
-inline bool contrib_pays(long long seqs, int H, int dk, int dB, int compute_units) {
-  return (dk == 128 && dB % 128 == 0) || seqs * H * (dB / BV) > compute_units;
+// columns of a state per workgroup of 512 threads, which go from sequence to sequence with the next one's rows on their way.
+// 128 x 128 of a state per workgroup: always (B16 T2048 H8 128 x 256: 40.5 us against 66).  64 x 64: workgroups of 256 threads,
+// several to a unit, and the same bits, so it takes more of them than there are units to win, and of short sequences not too
+// many.  Speed over the walk's at 256 units, 64 x 64 / 64 x 128 (96 workgroups 1.00, 160 .91, 256 .92):
+//                   288 wg         384            512            768            1024           1296           2048           4096
+//   1 chunk         1.07 / 1.08    1.06 / 1.05    1.01 / 1.02    1.01 / 1.04    .90 / .91      .89 / .92      .81 / .84      .79 / .77
+//   2               1.07 / 1.10    1.05 / 1.07    .98 / 1.01     .94 / 1.00     .87 / .96      .97 / 1.04     .88 / .89      .89 / .90
+//   4               1.22 / 1.25    1.15 / 1.20    1.03 / 1.09    .97 / 1.09     .91 / .94      1.05 / 1.09    .93 / .99      .95 / .97
+//   6               1.25 / 1.33    1.19 / 1.25    1.05 / 1.15    1.05 / 1.11    .97 / 1.00     1.10 / 1.15    1.01 / 1.04    .99 / 1.03
+//   12              1.35 / 1.45    1.26 / 1.34    1.15 / 1.21    1.09 / 1.27    1.06 / 1.08    1.21 / 1.28    1.07 / 1.14    1.04 / 1.00
+// 128 x 64 has no form of its own: 1.0 to 1.15 at 288 and 320 workgroups, .85 to 1.0 at 512, .75 to .9 from 640 on.
+inline bool contrib_pays(long long seqs, int T, int H, int dk, int dB, int compute_units) {
+  if (dk != 64) return dk == 128 && dB % 128 == 0;
+  const long long wgs = seqs * H * (dB / BV);
+  return wgs > compute_units && (wgs <= 3LL * compute_units || T > 4 * CH);
 }
 // One recurrent (decode) step for every (batch, head):  S' = gamma S + (scale k)^T v,  o = q S'.
 // q, k [B,H,dk]; v, o [B,H,dv]; S [B,H,dk,dv]; all bf16, fp32 arithmetic.  s_out may be s_in.

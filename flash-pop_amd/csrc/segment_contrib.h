@@ -11,19 +11,17 @@
 // transposing LDS read (the tile layout and the operand helpers are those of retention_bwd_fused.h);
 // two more chunks are on their way in registers.  One workgroup barrier per chunk.
 //
-// 64 columns: bit for bit what the pass kernel's state-only walk gives (which takes keys of 192 and 256): chunks are cut from
-// where the walk starts, so that walking backward the short one is the first of the sequence, every weight is a power of gamma of
-// its own, and the tokens are summed in order (ContribTile::AS_WALK).  128 columns: chunks from the first token on in both
-// directions, weights of a k-step from those of the one before.
+// 64 rows: 64 columns per workgroup of 256 threads (37 KB of LDS: several share a compute unit), bit for bit what the pass
+// kernel's state-only walk gives, which takes all other states and those calls that it is the faster one at (contrib_pays):
+// chunks are cut from where the walk starts, so that walking backward the short one is the first of the sequence, every weight is
+// a power of gamma of its own, and the tokens are summed in order (ContribTile::AS_WALK).  64 x 128, B20 T256 H12 11.1 us in the
+// walk, 8.4 here; B40 T144 H4 9.2, 6.9.  128 columns of a 64-row state per workgroup: 9.1 and 7.1.
 //
-// The sum leaves
-// through the transposing read as well (16 bits at a time it took as long as four chunks: 128 x 128,
+// 128 rows: 128 columns per workgroup of 512 threads; chunks from the first token on in both directions, weights of a k-step
+// from those of the one before.
+//
+// The sum leaves through the transposing read as well (16 bits at a time it took as long as four chunks: 128 x 128,
 // B12 T448 H8 17.1 -> 11.5 us a launch, B16 T2048 H8 dv 256 44.6 -> 40.5).
-//
-// 128 x 128 with 512 threads where Z has a multiple of 128 columns; 64 rows, or 64 columns, with 256
-// threads (37 to 53 KB of LDS: several workgroups share a compute unit): 64 x 128, B20 T256 H12
-// 11.1 us in the pass kernel's state-only walk, 8.4 here; B40 T144 H4 9.2, 6.9.  128 columns of a
-// 64-row state per workgroup: 9.1 and 7.1.
 #pragma once
 #include <type_traits>
 
@@ -243,16 +241,15 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   put_contribution<DK, NC, NTH>(p, TL, p.U_lo, stream, ct, tid, c, g, at_, nt0, racc, LowerHalf{});
 }
 
-// Host side, shared by the GPU launcher and the CPU test harness: argument check, and the columns of Z per workgroup.
-inline int contrib_columns(const ContribArgs& a) { return a.dk == FB_D && a.dB % FB_D == 0 ? FB_D : BV; }
+// Host side, shared by the GPU launcher and the CPU test harness: argument check.
 inline const char* check_contrib(const ContribArgs& a) {
   if (a.B < 1 || a.T < 1 || a.H < 1 || a.H > MAX_HEADS) return "state-only pass: B, T, H >= 1 expected";
   if (a.segs < 0 || (a.segs > 0 && (a.B % a.segs != 0 || a.total > (long long)a.segs * a.T || a.total <= (a.segs - 1LL) * a.T)))
     return "state-only pass: segments that do not cover their sequence";
-  if ((a.dk != 64 && a.dk != FB_D) || a.dB < BV || a.dB % BV != 0) return "state-only pass: W of 64 or 128 columns, Z of a multiple of 64";
+  if ((a.dk != 64 && a.dk != FB_D) || a.dB < a.dk || a.dB % a.dk != 0) return "state-only pass: W of 64 or 128 columns, Z of a multiple of them";
   if (!a.W || !a.Z || !a.U) return "state-only pass: null pointer";
   if (!contrib_fits(a.T, a.H, a.dk, a.dB)) return "state-only pass: sequence too long";
-  if ((long long)a.B * a.H * (a.dB / contrib_columns(a)) > 0x7fffffffLL) return "state-only pass: too many sequences";
+  if ((long long)a.B * a.H * (a.dB / a.dk) > 0x7fffffffLL) return "state-only pass: too many sequences";
   return nullptr;
 }
 

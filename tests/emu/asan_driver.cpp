@@ -174,8 +174,8 @@ int main() {
   rc |= plain(1, 768, 1, 64, 256, true);      // the state-only kernel for 64-wide keys (more workgroups than units)
   rc |= plain(1, 700, 1, 64, 256, true);      // ... short chunks at either end of a walk, fp32 states
   rc |= pop_split(1, 150, 1, 128, 128, 65);   // blocks and a tail that end inside chunks
-  rc |= pop_split(1, 600, 1, 128, 64, 65);    // ... the state-only kernel for 128 rows and 64 columns
-  rc |= pop_split(1, 600, 1, 64, 64, 65);     // ... for 64 rows
+  rc |= pop_split(1, 600, 1, 128, 64, 65);    // ... 128 rows and 64 columns: the state-only walk
+  rc |= pop_split(1, 600, 1, 64, 64, 65);     // ... 64 rows: the state-only kernel
   rc |= pop(1, 287, 1, 64, 128, 144);
   rc |= pop(2, 28, 1, 64, 64, 15);
   rc |= pop(1, 40, 1, 64, 64, 100);           // no full block

@@ -149,11 +149,13 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* /*stream*/, const char**
     *err = why;
     return 1;
   }
-  return a.dk == 64 ? run_contrib<64, 64, 256>(a) : fpk::contrib_columns(a) == 64 ? run_contrib<128, 64, 256>(a) : run_contrib<128, 128, 512>(a);
+  return a.dk == 64 ? run_contrib<64, 64, 256>(a) : run_contrib<128, 128, 512>(a);
 }
 
 // The rule that chooses the state-only pass
-extern "C" int emu_contrib_pays(int seqs, int H, int dk, int dv, int compute_units) { return fpk::contrib_pays(seqs, H, dk, dv, compute_units); }
+extern "C" int emu_contrib_pays(int seqs, int T, int H, int dk, int dv, int compute_units) {
+  return fpk::contrib_pays(seqs, T, H, dk, dv, compute_units);
+}
 
 // The rule that chooses the forward of a POP call with suffixes, on a device of `compute_units`
 extern "C" int emu_pop_folds(int B, int T, int H, int dk, int dv, int block, int Ls, int compute_units) {
@@ -164,7 +166,7 @@ extern "C" int emu_pop_folds(int B, int T, int H, int dk, int dv, int block, int
 }
 
 // What every sequence (segment) adds to a zero state, U in fp32 halves, by the state-only kernel or (`walk`) by the pass kernel's
-// state-only walk: the two have to agree bit for bit where the former takes 64 columns.
+// state-only walk: the two have to agree bit for bit where the former takes 64-row states.
 extern "C" int emu_state_only(int walk, const uint16_t* W, const uint16_t* Z, uint16_t* U, uint16_t* U_lo, int B, int T, int H, int dk,
                               int dv, int segs, int total, int reverse, float log2g) {
   const char* msg = "";

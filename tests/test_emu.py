@@ -346,11 +346,9 @@ def test_cut_final_state_follows_the_uncut_walk(emu_lib, T, dk, dv):
     (144, 360, 64, 64),     # a short chunk in every segment, the last one shorter still
     (128, 257, 64, 192),    # whole chunks, a last segment of one token; three workgroups per segment
     (63, 63, 64, 64),       # less than a chunk
-    (215, 215, 128, 64),    # 128 rows, 64 columns
-    (64, 191, 128, 192),
 ])
 def test_state_only_kernel_matches_the_walk(emu_lib, T, total, dk, dv, reverse):
-    """Where the state-only kernel takes 64 columns it cuts the chunks, weighs the operands and sums as the pass kernel's
+    """Where the state-only kernel takes 64-row states it cuts the chunks, weighs the operands and sums as the pass kernel's
     state-only walk does, in either direction: same bits."""
     segs, H = -(-total // T), 2
     w, _, z, _ = hp.make_inputs(1, total, H, dk, dv, seed=T + dv)
@@ -365,18 +363,20 @@ def test_state_only_kernel_matches_the_walk(emu_lib, T, total, dk, dv, reverse):
 
 
 def test_rule_of_the_state_only_pass(emu_lib):
-    """64 columns of a state per workgroup: the pass kernel's walk while its workgroups fit the units, as it is the faster one there
-    (128 x 64, 96 sequences and heads: 7.8 against 9.4 us)."""
+    """Which kernel sums the segments of a cut call, at 256 units: of 64-row states the state-only kernel where its workgroups are
+    more than the units, but not many of short segments (128 x 64, 1 296 of two chunks: 25 us in the walk, 32 in a kernel of 64
+    columns); the walk for all other states but those of 128 x 128."""
     pays = emu_lib.emu_contrib_pays
-    assert not pays(24, 4, 128, 64, 256) and not pays(64, 4, 128, 64, 256) and pays(65, 4, 128, 64, 256)
-    assert not pays(32, 4, 64, 128, 256) and pays(33, 4, 64, 128, 256)
-    assert pays(1, 1, 128, 128, 256) and pays(1, 1, 128, 256, 256) and not pays(1, 1, 128, 192, 256)
+    assert not pays(32, 1000, 4, 64, 128, 256) and pays(33, 64, 4, 64, 128, 256) and pays(96, 64, 4, 64, 128, 256)
+    assert not pays(97, 256, 4, 64, 128, 256) and pays(97, 257, 4, 64, 128, 256) and pays(4096, 257, 4, 64, 64, 256)
+    assert not pays(97, 1000, 8, 128, 64, 256) and not pays(108, 128, 12, 128, 64, 256) and not pays(97, 1000, 4, 128, 192, 256)
+    assert pays(1, 64, 1, 128, 128, 256) and pays(1000, 64, 8, 128, 256, 256)
 
 
 @pytest.mark.parametrize("T,dk,dv", [
     (257, 64, 64),      # 64-row states: a last segment of one token
     (575, 64, 192),     # ... three workgroups per segment, a last chunk of 63 tokens
-    (513, 128, 64),     # 128-row states, 64 columns per workgroup
+    (513, 128, 64),     # 128-row states, 64 columns per workgroup (the walk)
     (577, 128, 192),    # ... a last segment of one token (uneven cuts all: equal segments hand bf16 states on, a step in 2^8)
 ])
 def test_state_only_pass_in_64_columns(emu_lib, T, dk, dv):
