@@ -16,9 +16,9 @@
 //                       tiles of the next chunk and of its suffix, the way out of the staged outputs.
 //
 // Two workgroup barriers per step.  What bounds it: the feed waves' chain, 1 100 cycles for the scores, 1 400 for the tiles, 600
-// for the loads.  B8 H12 T2048 64 x 128, blocks of 64, suffixes of 16: 75.5 us a launch in the suffix walk (64 chunk items and 65
-// suffix items), 58 here.  128-wide keys were slower in it (B8 H16 T4096: 230 against 190 us; both roles need more than 256
-// registers) and stay with the walk.
+// for the loads.  B8 H12 T2048 64 x 128, blocks of 64, suffixes of 16: forwards in a row 79.8 us each in the suffix walk (64 chunk
+// items and 65 suffix items), 61.0 here; the launch in a traced training step 77.7 and 67.  128-wide keys were slower in it (B8 H16
+// T4096: 230 against 190 us; both roles need more than 256 registers) and stay with the walk.
 #pragma once
 #include <type_traits>
 
