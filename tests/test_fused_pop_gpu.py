@@ -70,8 +70,11 @@ def run_fused(B, N, block, Ls, H, dk, dv, state_std, seed, decay_range=None, ora
     (3, 8, 64, 16, 16, 128, 128),    # 48 streams: the fewest that take the backward with the suffixes folded into the chunks
     (8, 8, 64, 16, 12, 64, 128),     # ... the same backward for 64-wide keys (96 streams)
     (4, 4, 128, 40, 12, 128, 64),    # ... 64-wide values, suffixes as extra stops of the walks
-    (8, 8, 64, 9, 8, 64, 64),        # ... 64 x 64 states, folded suffixes of 9 tokens
-    (3, 4, 128, 33, 16, 128, 128),   # ... with suffixes too long to fold: stops of its walks
+    (8, 8, 64, 9, 8, 64, 64),        # 64 x 64 states on 64 streams: the passes
+    (8, 8, 64, 9, 12, 64, 64),       # ... on 96: the backward of the 48 streams above, folded suffixes of 9 tokens
+    (4, 8, 64, 16, 12, 128, 64),     # ... 128 x 64 states
+    (2, 5, 128, 1, 16, 128, 64),     # ... one-token suffixes, two chunks a block
+    (3, 4, 128, 33, 16, 128, 128),   # ... suffixes too long to fold: stops of its walks
 ])
 def test_fused_parity_sweep(B, N, block, Ls, H, dk, dv):
     run_fused(B, N, block, Ls, H, dk, dv, 0.3, seed=N * block + Ls, decay_range=(5, 12))
