@@ -73,9 +73,10 @@ FP_DEVICE void put_contribution(const ContribArgs& p, uint16_t* Rt, uint16_t* ds
   }
 }
 
-// AS_WALK: token j of a k-step lies in tile row `walk_row(j)` of it, so that element e of a TR_NAT operand is token
-// walk_token(g, e), as in the pass kernel's operands
-FP_DEVICE int walk_row(int j) { return (j & ~15) | ((j & 3) << 2) | ((j & 4) >> 1) | ((j & 8) >> 3); }
+// AS_WALK: row r of a tile holds token `walk_in_row(r)`, so that element e of a TR_NAT operand is token walk_token(g, e) of its
+// k-step, as in the pass kernel's operands.  (The threads fetch by that order and store row by row: with the rows' places permuted
+// at the stores instead, the rows of a wave meet in the same banks.)
+FP_DEVICE int walk_in_row(int r) { return (r & ~15) | ((r >> 2) & 3) | ((r & 2) << 1) | ((r & 1) << 3); }
 FP_DEVICE int walk_token(int g, int e) { return 4 * g + (e & 3) + 8 * (e >> 2); }
 
 template <int DK, int NC, int NTH, bool REV>
@@ -103,8 +104,9 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   uint16_t* const TL = reinterpret_cast<uint16_t*>(lds);   // stage s: W tile at s G::STAGE, Z tile behind it
   // this thread's 16-byte pieces: rows w_row + RW u of W, z_row + RZ u of Z
   constexpr int RW = NTH / (DK / 8), RZ = NTH / (NC / 8);
-  const int w_row = tid / (DK / 8), w_piece = tid % (DK / 8), z_row = tid / (NC / 8), z_piece = tid % (NC / 8);
-  const int w_off = at<LDW>(AS_WALK ? walk_row(w_row) : w_row, 8 * w_piece), z_off = at<LDZ>(AS_WALK ? walk_row(z_row) : z_row, 8 * z_piece);
+  const int w_place = tid / (DK / 8), w_piece = tid % (DK / 8), z_place = tid / (NC / 8), z_piece = tid % (NC / 8);
+  const int w_off = at<LDW>(w_place, 8 * w_piece), z_off = at<LDZ>(z_place, 8 * z_piece);
+  const int w_row = AS_WALK ? walk_in_row(w_place) : w_place, z_row = AS_WALK ? walk_in_row(z_place) : z_place;
   static_assert(RW % 16 == 0 && RZ % 16 == 0, "a thread's rows have the same place in their k-steps");
   struct Rows {
     u32x4 w[G::NW], z[G::NZ];
@@ -153,14 +155,14 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
 #pragma unroll
   for (int u = 0; u < TPW; ++u) racc[u] = f32x16{0};
 
-  // L: tokens of the chunk, where it is the short one that ends the walk (CH otherwise).  Walking forward its weights count from its
-  // last token, as in the walk that carries a sequence through, so that a cut call gives the state of the uncut one.  (Walking
-  // backward they are those of any other chunk; with 128 columns the short chunk is met first, with R = 0.)
+  // L: tokens of the chunk.  The short one that ends a walk forward (SHORT) has weights of its own, which count from its last
+  // token, as in the walk that carries a sequence through, so that a cut call gives the state of the uncut one.  Walking backward
+  // the weights are those of any other chunk, and with 128 columns the short chunk is met first, with R = 0.
   auto update = [&](int s, auto short_chunk, int L) {
     constexpr bool SHORT = decltype(short_chunk)::value;
     const uint16_t* const Ws = TL + s * G::STAGE;
     const uint16_t* const Zs = Ws + G::W;
-    const float decay = SHORT ? fprt::exp2_approx((float)L * lg) : gL;
+    const float decay = SHORT || (AS_WALK && REV) ? fprt::exp2_approx((float)L * lg) : gL;
     u32x4 ua[4], ub[4][TPW];
     auto request = [&](int tt) {
       const int t = AS_WALK || REV ? tt : 3 - tt;
@@ -182,7 +184,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     fprt::sched_fence();
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
-      if (SHORT && !REV) {
+      if (SHORT) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) wk[e] = weight(L - 1 - (AS_WALK ? 16 * tt + walk_token(g, e) : 16 * (3 - tt) + nat_token(g, e)));
       } else if (AS_WALK) {
@@ -204,7 +206,8 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   // Chunk it is multiplied from stage it & 1 while chunk it + 1 moves from registers into the
   // other stage and the loads of chunk it + 3 take its place; chunk it + 2 is on its way in the
   // second set of registers.
-  const int nwhole = REV && !AS_WALK ? nch : len / CH;
+  const int nwhole = REV ? nch : len / CH;
+  auto tokens = [&](int it) { return AS_WALK && REV && len - it * CH < CH ? len - it * CH : CH; };
   Rows pa, pb;
   load(0, pa);
   load(1, pb);
@@ -214,12 +217,12 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   for (int it = 0; it < nwhole; it += 2) {
     stage(1, pb);
     load(it + 3, pb);
-    update(0, std::false_type{}, CH);
+    update(0, std::false_type{}, tokens(it));
     fprt::block_sync();
     if (it + 1 >= nwhole) break;
     stage(0, pa);
     load(it + 4, pa);
-    update(1, std::false_type{}, CH);
+    update(1, std::false_type{}, tokens(it + 1));
     fprt::block_sync();
   }
   // (pb is wanted on both ways out of the loop, or the compiler moves its loads behind the break, a chunk later: 42 -> 46 us at
