@@ -116,14 +116,17 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   auto load = [&](int it, Rows& pf) {
     const bool live = it < nch;
     const int end = AS_WALK && REV ? len - it * CH : len;
-    const int t0 = !(AS_WALK && REV) ? (REV ? nch - 1 - it : it) * CH : end > CH ? end - CH : 0;
-    // rows of a short chunk from `end` on read as zeros (contrib_fits); visits beyond the walk read zeros and move nothing
+    const int first = !(AS_WALK && REV) ? (REV ? nch - 1 - it : it) * CH : end > CH ? end - CH : 0;
+    // rows of a short chunk from `end` on read as zeros (contrib_fits); visits beyond the walk read zeros and move nothing.  (One row
+    // offset for all of a thread's loads: chosen per load, the choice became branches around them, behind which every wait is for all.)
     const fprt::BufView w = fprt::make_buf(wbase, live ? (uint32_t)(end - 1) * roww + DK * 2 : 0u);
     const fprt::BufView z = fprt::make_buf(zbase, live ? (uint32_t)(end - 1) * rowz + NC * 2 : 0u);
+    const uint32_t t0 = live ? first : 0;
+    const uint32_t wo = (t0 + w_row) * roww + w_piece * 16, zo = (t0 + z_row) * rowz + z_piece * 16;
 #pragma unroll
-    for (int u = 0; u < G::NW; ++u) pf.w[u] = fprt::buf_load128(w, (live ? t0 + w_row + RW * u : 0u) * roww + w_piece * 16);
+    for (int u = 0; u < G::NW; ++u) pf.w[u] = fprt::buf_load128(w, wo + (uint32_t)(RW * u) * roww);
 #pragma unroll
-    for (int u = 0; u < G::NZ; ++u) pf.z[u] = fprt::buf_load128(z, (live ? t0 + z_row + RZ * u : 0u) * rowz + z_piece * 16);
+    for (int u = 0; u < G::NZ; ++u) pf.z[u] = fprt::buf_load128(z, zo + (uint32_t)(RZ * u) * rowz);
   };
   auto stage = [&](int s, const Rows& pf) {
     uint16_t* const st = TL + s * G::STAGE;
@@ -132,6 +135,11 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
 #pragma unroll
     for (int u = 0; u < G::NZ; ++u) st128(st + G::W + z_off + RZ * u * LDZ, pf.z[u]);
   };
+
+  Rows pa, pb;   // the first two chunks travel while the weights are made
+  load(0, pa);
+  load(1, pb);
+  fprt::sched_fence();
 
   // this wave's tiles of R: rows a = 32 at_ .., columns n = 32 (nt0 + u) .., u < TPW
   const int at_ = wave % G::NRT, nt0 = (wave / G::NRT) * TPW;
@@ -146,7 +154,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int j = AS_WALK ? 16 * t + walk_token(g, e) : REV ? nat_token(g, e) : 48 + nat_token(g, e);
-      wk_whole[t][e] = weight(REV ? j + 1 : CH - 1 - j);
+      wk_whole[t][e] = p.s_update * fprt::exp2_approx((float)(REV ? j + 1 : CH - 1 - j) * lg);
     }
   }
   const float g16 = fprt::exp2_approx(16.f * lg), gL = fprt::exp2_approx((float)CH * lg);
@@ -208,9 +216,6 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
   // second set of registers.
   const int nwhole = REV ? nch : len / CH;
   auto tokens = [&](int it) { return AS_WALK && REV && len - it * CH < CH ? len - it * CH : CH; };
-  Rows pa, pb;
-  load(0, pa);
-  load(1, pb);
   stage(0, pa);
   load(2, pa);
   fprt::block_sync();
