@@ -437,7 +437,8 @@ int plan_segments(const Shape& s) {
 //   128 x 128  H16 B1       79 chunks 116 -> 82,       40 chunks 61.8 -> 50.8,  28 chunks 45.1 -> 44.6
 //   128 x 256  H8 B2        28 chunks 119 -> 68,       18 chunks 80.0 -> 70.9,  13 chunks 60.8 -> 61.8
 // The line dates from slower state-only passes, scans and fused backwards: it leaves calls of 16 to 18 chunks uncut that a cut
-// would shorten (128 x 256 up to 28), and cuts the backward of 64 x 64 on 72 streams from 40 chunks on.
+// would shorten (128 x 256 up to 28), and cuts the backward of 64 x 64 on 72 streams from 40 chunks on.  (Measured before the
+// state-only passes got another 0.3 to 0.8 us shorter.)
 // `block`: a POP call, whose chunks end at its blocks and whose gradient passes share fewer launches (64 x 128, B4 H4 T1440
 // in blocks of 144, 30 chunks, with the suffix call and the launches between the two: 200 -> 166 us).
 bool cut_pays(const Shape& s, int n, int tokens, bool backward, int block = 0) {

@@ -130,20 +130,19 @@ struct ContribArgs {
 inline bool contrib_fits(long long T, int H, int dk, int dB) { return (T + CH) * H * (dk > dB ? dk : dB) * 2 < (1LL << 32); }
 // Whether that pass is the faster form of a state-only pass over `seqs` sequences, else it is the pass kernel's state-only walk, 64
 // columns of a state per workgroup of 512 threads, which go from sequence to sequence with the next one's rows on their way.
-// 128 x 128 of a state per workgroup: always (B16 T2048 H8 128 x 256: 40.5 us against 66).  64 x 64: workgroups of 256 threads,
-// several to a unit, and the same bits, so it takes more of them than there are units to win, and of short sequences not too
-// many.  Speed over the walk's at 256 units, 64 x 64 / 64 x 128 (96 workgroups 1.00, 160 .91, 256 .92):
-//                   288 wg         384            512            768            1024           1296           2048           4096
-//   1 chunk         1.07 / 1.08    1.06 / 1.05    1.01 / 1.02    1.01 / 1.04    .90 / .91      .89 / .92      .81 / .84      .79 / .77
-//   2               1.07 / 1.10    1.05 / 1.07    .98 / 1.01     .94 / 1.00     .87 / .96      .97 / 1.04     .88 / .89      .89 / .90
-//   4               1.22 / 1.25    1.15 / 1.20    1.03 / 1.09    .97 / 1.09     .91 / .94      1.05 / 1.09    .93 / .99      .95 / .97
-//   6               1.25 / 1.33    1.19 / 1.25    1.05 / 1.15    1.05 / 1.11    .97 / 1.00     1.10 / 1.15    1.01 / 1.04    .99 / 1.03
-//   12              1.35 / 1.45    1.26 / 1.34    1.15 / 1.21    1.09 / 1.27    1.06 / 1.08    1.21 / 1.28    1.07 / 1.14    1.04 / 1.00
-// 128 x 64 has no form of its own: 1.0 to 1.15 at 288 and 320 workgroups, .85 to 1.0 at 512, .75 to .9 from 640 on.
+// 128 x 128 of a state per workgroup: always (B16 T2048 H8 128 x 256: 44 us against 67; the least, B12 T448 H8, 12.0 against 11.0).
+// 64 x 64, with the same bits as the walk: but for many workgroups of short sequences.  Speed over the walk's at 256 units, inputs
+// not in a cache up to 768 workgroups, 64 x 64 / 64 x 128:
+//                   64 wg          160            256            320            768            1024           1296           2048           4096
+//   1 chunk         1.04 / 1.03    1.00 / 1.01    .98 / 1.00     1.10 / 1.09    .97 / .99      .90 / .96      .92 / .92      .85 / .85      .85 / .81
+//   2               1.08 / 1.07    1.05 / 1.04    1.01 / 1.03    1.13 / 1.16    .98 / 1.01     .92 / .99      1.01 / 1.07    .91 / .94      .91 / .95
+//   4               1.11 / 1.11    1.10 / 1.10    1.06 / 1.07    1.27 / 1.31    1.03 / 1.12    .96 / 1.00     1.11 / 1.15    .98 / 1.05     .95 / 1.05
+//   6               1.16 / 1.17    1.13 / 1.15    1.09 / 1.12    1.29 / 1.41    1.04 / 1.16    1.03 / 1.07    1.12 / 1.18    1.04 / 1.11    1.00 / 1.10
+//   12              1.25 / 1.25    1.17 / 1.21    1.16 / 1.18    1.42 / 1.57    1.11 / 1.23    1.07 / 1.14    1.18 / 1.29    1.08 / 1.18    1.05 / 1.00
+// 128 x 64 has no form of its own: one lost to the walk from 512 workgroups on (.75 to .93 times its speed).
 inline bool contrib_pays(long long seqs, int T, int H, int dk, int dB, int compute_units) {
   if (dk != 64) return dk == 128 && dB % 128 == 0;
-  const long long wgs = seqs * H * (dB / BV);
-  return wgs > compute_units && (wgs <= 3LL * compute_units || T > 4 * CH);
+  return seqs * H * (dB / BV) <= 3LL * compute_units || T > 4 * CH;
 }
 // One recurrent (decode) step for every (batch, head):  S' = gamma S + (scale k)^T v,  o = q S'.
 // q, k [B,H,dk]; v, o [B,H,dv]; S [B,H,dk,dv]; all bf16, fp32 arithmetic.  s_out may be s_in.

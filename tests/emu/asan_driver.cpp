@@ -165,13 +165,13 @@ int main() {
   rc |= plain(1, 65, 1, 64, 256, false);      // two visits per chunk, state read transposed
   rc |= plain(1, 130, 1, 256, 64, false);     // two visits per chunk, state as stored
   rc |= plain(1, 100, 1, 192, 192, false);    // three visits per chunk
-  rc |= plain(1, 512, 1, 64, 128, true);      // cut into segments (state-only walk, scan)
+  rc |= plain(1, 512, 1, 64, 128, true);      // cut into segments (state-only kernel for 64-row states, scan)
   rc |= plain(1, 640, 1, 128, 256, true);     // ... with the state-only kernel for 128-wide keys, two workgroups per segment
   rc |= plain(1, 511, 1, 128, 128, true);     // uneven segments, fp32 states: the last chunk of that kernel is short
-  rc |= plain(1, 257, 1, 64, 64, true);       // ... in the state-only walk, the last segment is one token
+  rc |= plain(1, 257, 1, 64, 64, true);       // ... 64-row states, the last segment is one token
   rc |= plain(1, 512, 1, 256, 64, true);      // the state-only walk with two visits per chunk
   rc |= plain(1, 511, 1, 192, 64, true);      // ... with three, fp32 states
-  rc |= plain(1, 768, 1, 64, 256, true);      // the state-only kernel for 64-wide keys (more workgroups than units)
+  rc |= plain(1, 768, 1, 64, 256, true);      // the state-only kernel for 64-wide keys, more workgroups than units
   rc |= plain(1, 700, 1, 64, 256, true);      // ... short chunks at either end of a walk, fp32 states
   rc |= pop_split(1, 150, 1, 128, 128, 65);   // blocks and a tail that end inside chunks
   rc |= pop_split(1, 600, 1, 128, 64, 65);    // ... 128 rows and 64 columns: the state-only walk

@@ -292,7 +292,7 @@ def test_pop_split_at_blocks(emu_lib, B, T, H, dk, dv, block, state_std, segment
 
 @pytest.mark.parametrize("T,dk,dv,block", [
     (256, 128, 128, 64),   # POP cut at its blocks, 128-wide keys
-    (150, 256, 64, 64),    # the same through the pass kernel's state-only walk, a tail after the last block
+    (150, 256, 64, 64),    # the same through the state-only kernel for 64-row states, a tail after the last block
     (330, 256, 64, 0),     # the plain op in uneven segments
 ])
 def test_cut_calls_carry_fp32_states(emu_lib, choose_backward, T, dk, dv, block):
@@ -363,11 +363,10 @@ def test_state_only_kernel_matches_the_walk(emu_lib, T, total, dk, dv, reverse):
 
 
 def test_rule_of_the_state_only_pass(emu_lib):
-    """Which kernel sums the segments of a cut call, at 256 units: of 64-row states the state-only kernel where its workgroups are
-    more than the units, but not many of short segments (128 x 64, 1 296 of two chunks: 25 us in the walk, 32 in a kernel of 64
-    columns); the walk for all other states but those of 128 x 128."""
+    """Which kernel sums the segments of a cut call, at 256 units: of 64-row states the state-only kernel but for many workgroups
+    of short segments (4 096 of a chunk: 28 us in the walk, 34 in the kernel); the walk for all other states but those of 128 x 128."""
     pays = emu_lib.emu_contrib_pays
-    assert not pays(32, 1000, 4, 64, 128, 256) and pays(33, 64, 4, 64, 128, 256) and pays(96, 64, 4, 64, 128, 256)
+    assert pays(1, 64, 1, 64, 64, 256) and pays(32, 1000, 4, 64, 128, 256) and pays(96, 64, 4, 64, 128, 256)
     assert not pays(97, 256, 4, 64, 128, 256) and pays(97, 257, 4, 64, 128, 256) and pays(4096, 257, 4, 64, 64, 256)
     assert not pays(97, 1000, 8, 128, 64, 256) and not pays(108, 128, 12, 128, 64, 256) and not pays(97, 1000, 4, 128, 192, 256)
     assert pays(1, 64, 1, 128, 128, 256) and pays(1000, 64, 8, 128, 256, 256)

@@ -92,8 +92,9 @@ def test_pop_outputs_equal_plain_outputs():
     (1, 1500, 2, 256, 64, 144),
     (1, 1537, 2, 128, 128, 128),   # whole chunks per block, a tail of one token
     (1, 832, 2, 64, 64, 64),
-    (4, 1440, 4, 64, 128, 144),    # more state-only workgroups than units: the state-only kernel for 64-row states
+    (4, 1440, 4, 64, 128, 144),    # the state-only kernel for 64-row states, more workgroups than units
     (2, 1500, 16, 64, 64, 144),    # ... a short chunk in every segment, a tail of less than a chunk
+    (4, 2048, 16, 64, 64, 128),    # many short segments of such states: the state-only walk
 ])
 def test_pop_split_entry_points(hip_lib, B, T, H, dk, dv, block):
     """fp_pop_retention_*_split on shapes that are cut at their blocks, the backward from the states that the forward left and

@@ -338,7 +338,7 @@ def test_decode_step_kernel_256_steps():
     # uneven segments, whose states are fp32: the last one ends inside a chunk
     (1, 5003, 4, 128, 128), (1, 2501, 2, 128, 256), (2, 1500, 2, 64, 128), (1, 2000, 2, 192, 128), (1, 3001, 2, 256, 64),
     (1, 2305, 4, 128, 128),   # ... is one token
-    (1, 5003, 12, 64, 128),   # more state-only workgroups than units: the state-only kernel for 64-row states
+    (1, 5003, 12, 64, 128),   # the state-only kernel for 64-row states, more workgroups than units
     (1, 3000, 8, 64, 192),    # ... three column tiles
 ])
 def test_split_entry_points_long_sequence_few_streams(B, T, H, dk, dv):
