@@ -68,6 +68,12 @@ FP_DEVICE void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
 // A value that has to be there (a load: has to have arrived) at this point.
 FP_DEVICE void keep(u32x4 v) { asm volatile("" ::"v"(v)); }
 
+// The same value, of which the compiler knows nothing: what follows from it is computed where it is used, not kept in registers
+FP_DEVICE int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 // Bounds-checked view of global memory (raw buffer resource): loads beyond `nbytes` return
 // zero and stores beyond it are dropped by the hardware, which is how ragged chunk tails
 // are handled without branches.  Offsets are bytes from `base`, below 4 GiB.
@@ -89,6 +95,33 @@ FP_DEVICE void buf_store128_nt(BufView b, uint32_t off, u32x4 v) { __builtin_amd
 // a time: 123 -> 185 us).
 FP_DEVICE void buf_store128_through(BufView b, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, b.rsrc, off, 0, 2 | 16); }
 FP_DEVICE void buf_store64(BufView b, uint32_t off, u32x2 v) { __builtin_amdgcn_raw_buffer_store_b64(v, b.rsrc, off, 0, 0); }
+
+// Global memory -> LDS without a way through registers: lane l's 16 bytes at byte `off` of the view land at byte 16 l from `lds`, which
+// is the same in every lane (zeros, where they are beyond the view).  Asynchronous: what it wrote may be read after fill_wait
+// and a barrier.  Inline assembly, because the compiler would put a wait for every copy in flight before every LDS read
+// that follows; nothing but LDS is written, so there is no register for it to lose track of.
+struct FillView {
+  u32x4 words;   // the buffer resource, uniform
+};
+FP_DEVICE uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+FP_DEVICE FillView make_fill(const void* base, uint32_t nbytes) {
+  const uint64_t p = reinterpret_cast<uint64_t>(base);
+  return FillView{u32x4{uniform((uint32_t)p), uniform((uint32_t)(p >> 32) & 0xffffu), uniform(nbytes), 0x00020000u}};
+}
+typedef uint32_t LdsAddress;
+FP_DEVICE LdsAddress lds_address(const char* p) { return uniform((uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p)); }
+// ONCE: with the non-temporal hint
+template <bool ONCE>
+FP_DEVICE void fill_lds(const FillView& v, uint32_t off, LdsAddress lds) {
+  if (ONCE) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(lds), "v"(off), "s"(v.words) : "memory", "m0");
+  else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(v.words) : "memory", "m0");
+}
+// Until at most N of this wave's loads, copies and stores are still under way (they end in order).
+template <int N>
+FP_DEVICE void fill_wait() {
+  static_assert(N >= 0 && N < 64, "six bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 
 // A word that another workgroup of the same launch polls (relaxed, device scope), and a short sleep between polls.
 FP_DEVICE void pace_store(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }

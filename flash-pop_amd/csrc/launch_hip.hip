@@ -34,6 +34,21 @@ __global__ __launch_bounds__(fpk::NTHREADS_WS) void retention_pass_multi_kernel(
   fpk::retention_pass_ws<DA, MODE, NH>(first, io, lds, id.wg, nwg);
 }
 
+// The same for dA = 64 without suffixes (MODE: fpk::FillMode); one pass: a direction each, so that a launch fetches the code of one
+template <int MODE, bool REV>
+__global__ __launch_bounds__(fpk::FP_THREADS) void retention_pass_fill_kernel(const fpk::PassArgs args) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  fpk::retention_pass_fill_dir<MODE, REV>(args, fpk::tensors_of(args), lds, fpk::place_workgroup(fprt::block_index(), fprt::grid_size(), 1).wg);
+}
+template <int MODE>
+__global__ __launch_bounds__(fpk::FP_THREADS) void retention_pass_fill_multi_kernel(const fpk::PassArgs first, const fpk::PassTensors second,
+                                                                                   const fpk::PassTensors third, const int passes) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const fpk::WorkgroupId id = fpk::place_workgroup(fprt::block_index(), fprt::grid_size() / passes, passes);
+  const fpk::PassTensors io = id.pass == 0 ? fpk::tensors_of(first) : id.pass == 1 ? second : third;
+  fpk::retention_pass_fill<MODE>(first, io, lds, id.wg);
+}
+
 // MODE: how POP suffixes take part (fpk::FbMode): none, as extra stops of the walks, or (at most 16 tokens) folded into
 // the chunks at their boundaries, with suffix_intra_bwd_kernel for what stays inside such a suffix
 template <int DK, int DV, int MODE>
@@ -100,7 +115,9 @@ __global__ __launch_bounds__(fpk::LAYER_THREADS) void gated_norm_bwd_kernel(cons
 // no thread calls hipFuncSetAttribute for it again (which matters to callers that capture
 // launches into a graph after a warm-up run).  Setting the attribute twice in a race is harmless.
 constexpr int kMaxDevices = 64;
-static_assert(2 * fpk::PASS_KERNELS <= 64, "one bit per kernel instantiation, single and paired");
+// retention_pass_fill_kernel walking backward: its bit is that many behind that of the same walk forward, behind all of those
+constexpr int kFillReverse = 2 * fpk::PASS_KERNELS;
+static_assert(kFillReverse + fpk::FILL_SLOTS <= 64, "one bit per kernel instantiation, single and paired");
 std::atomic<uint64_t> g_armed[kMaxDevices][2];   // bits 0..63: pass kernels; 64..: the fused backward family, short sequences, state-only pass
 
 template <typename Kernel, typename... More>
@@ -231,6 +248,11 @@ struct DeviceRun {
   int go(int slot) const {
     return launch(retention_pass_ws_kernel<DA, MODE, NH>, fpk::NTHREADS_WS, fpk::lds_bytes_ws(DA), slot, 1, stream, err, a);
   }
+  template <int MODE>
+  int fill(int slot) const {
+    return a.reverse ? launch(retention_pass_fill_kernel<MODE, true>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot + kFillReverse, 1, stream, err, a)
+                     : launch(retention_pass_fill_kernel<MODE, false>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot, 1, stream, err, a);
+  }
 };
 
 struct DeviceMultiRun {
@@ -243,6 +265,11 @@ struct DeviceMultiRun {
     return launch(retention_pass_multi_kernel<DA, MODE, NH>, fpk::NTHREADS_WS, fpk::lds_bytes_ws(DA),
                   fpk::PASS_KERNELS + slot, n, stream, err, planned[0], fpk::tensors_of(planned[1]),
                   fpk::tensors_of(planned[n - 1]), n);
+  }
+  template <int MODE>
+  int fill(int slot) const {
+    return launch(retention_pass_fill_multi_kernel<MODE>, fpk::FP_THREADS, fpk::fp_lds_bytes(), fpk::PASS_KERNELS + slot, n, stream,
+                  err, planned[0], fpk::tensors_of(planned[1]), fpk::tensors_of(planned[n - 1]), n);
   }
 };
 

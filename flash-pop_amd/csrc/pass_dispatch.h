@@ -5,11 +5,13 @@
 
 #include "pass_args.h"
 #include "retention_pass_ws.h"
+#include "retention_pass_fill.h"
 
 namespace fpk {
 
 // Number of kernel instantiations `dispatch_pass` can pick from (its `slot` argument is below this).
 constexpr int PASS_KERNELS = 22;
+constexpr int FILL_SLOTS = 5;   // those of retention_pass_fill.h are below this
 
 // Checks what the walks assume about `a` and chooses a.slots (workgroups per (head, column tile))
 // for a device with `compute_units` units.  Returns nullptr, or a message for the caller.
@@ -89,8 +91,8 @@ inline const char* plan_passes(PassArgs* planned, const PassArgs* const* passes,
   return nullptr;
 }
 
-// Calls run.template go<DA, MODE, NH>(slot) for the instantiation a planned `a` needs; `slot`
-// numbers the instantiations 0 .. PASS_KERNELS - 1.
+// Calls run.template go<DA, MODE, NH>(slot), or run.template fill<MODE>(slot) for the kernel of retention_pass_fill.h,
+// for the instantiation a planned `a` needs; `slot` numbers the instantiations 0 .. PASS_KERNELS - 1.
 template <typename Run>
 int dispatch_pass(const PassArgs& a, Run&& run) {
   const bool blocks = a.block > 0 && (a.Bout || a.Bin);
@@ -100,10 +102,10 @@ int dispatch_pass(const PassArgs& a, Run&& run) {
   if (a.dA == 64) {
     if (suffix_any) return run.template go<64, WALK_SUFFIX_ANY, 1>(14);
     if (suffix) return run.template go<64, WALK_SUFFIX, 1>(0);
-    if (blocks) return run.template go<64, WALK_BLOCKS, 1>(1);
+    if (blocks) return run.template fill<FILL_BLOCKS>(1);
     if (a.state_only) return run.template go<64, WALK_STATE, 1>(2);
-    if (multi) return run.template go<64, WALK_MULTI, 1>(3);
-    return run.template go<64, WALK_PLAIN, 1>(4);
+    if (multi) return run.template fill<FILL_MULTI>(3);
+    return run.template fill<FILL_PLAIN>(4);
   }
   if (a.dA == 128) {
     if (suffix_any) return run.template go<128, WALK_SUFFIX_ANY, 1>(15);

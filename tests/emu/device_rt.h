@@ -85,6 +85,7 @@ FP_DEVICE float rsqrt_f32(float x) { return 1.0f / std::sqrt(x); }
 
 FP_DEVICE void sched_fence() {}
 FP_DEVICE void keep(u32x4) {}
+FP_DEVICE int opaque(int x) { return x; }
 FP_DEVICE void pace_store(uint32_t* p, uint32_t v) { __atomic_store_n(p, v, __ATOMIC_RELAXED); }
 FP_DEVICE uint32_t pace_load(const uint32_t* p) { return __atomic_load_n(p, __ATOMIC_RELAXED); }
 FP_DEVICE void nap() {}
@@ -141,5 +142,18 @@ FP_DEVICE void buf_store64(BufView b, uint32_t off, u32x2 v) {
 FP_DEVICE u32x4 buf_load128_nt(BufView b, uint32_t off) { return buf_load128(b, off); }
 FP_DEVICE void buf_store128_nt(BufView b, uint32_t off, u32x4 v) { buf_store128(b, off, v); }
 FP_DEVICE void buf_store128_through(BufView b, uint32_t off, u32x4 v) { buf_store128(b, off, v); }
+
+typedef BufView FillView;
+FP_DEVICE FillView make_fill(const void* base, uint32_t nbytes) { return make_buf(base, nbytes); }
+FP_DEVICE uint32_t uniform(uint32_t x) { return x; }
+typedef char* LdsAddress;
+FP_DEVICE LdsAddress lds_address(char* p) { return p; }
+template <bool ONCE>
+FP_DEVICE void fill_lds(const FillView& v, uint32_t off, LdsAddress lds) {
+  const u32x4 d = buf_load128(v, off);
+  std::memcpy(lds + 16 * (g_lane.tid & 63), &d, 16);
+}
+template <int N>
+FP_DEVICE void fill_wait() {}
 
 }  // namespace fprt

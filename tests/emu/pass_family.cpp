@@ -30,6 +30,21 @@ struct FamilyRun {
       return 1;   // another width's translation unit
     }
   }
+  template <int MODE>
+  int fill(int /*slot*/) const {
+    if constexpr (fpk::FP_DA == EMU_FAMILY) {
+      const fpk::PassArgs& a = planned[0];
+      const int nwg = a.slots * a.H * (a.dB / fpk::BV);
+      const fpk::PassArgs* const p = planned;
+      const int passes = n;
+      return run_grid(fpk::FP_THREADS, passes * nwg, fpk::fp_lds_bytes(), [&](char* l) {
+        const fpk::WorkgroupId id = fpk::place_workgroup(fprt::block_index(), nwg, passes);
+        fpk::retention_pass_fill<MODE>(a, fpk::tensors_of(p[id.pass]), l, id.wg);
+      });
+    } else {
+      return 1;
+    }
+  }
 };
 
 }  // namespace

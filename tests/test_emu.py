@@ -643,3 +643,25 @@ def test_gated_group_norm(emu_lib, rows, H, dv):
     d_r_ref, d_g_ref = hp.oracle_gated_norm_grads(r, gate, d_out)
     hp.assert_close(d_r, d_r_ref, "d_r")
     hp.assert_close(d_g, d_g_ref, "d_g")
+
+
+@pytest.mark.parametrize("B,T,state_std", [
+    (1, 33, 0.5), (1, 64, None), (1, 65, 0.5), (2, 128, 0.5), (1, 193, 0.5), (1, 257, None),   # one chunk to five: fewer than are under way, and more
+    (17, 64, 0.5), (18, 65, 0.5), (17, 129, 0.5),   # several sequences per workgroup (8 units), of one chunk to three
+])
+def test_pass_of_64_wide_rows(emu_lib, choose_backward, B, T, state_std):
+    """The pass whose rows are copied straight into LDS, in all four roles: forward and the three gradient passes."""
+    choose_backward(PASSES)
+    test_plain_fwd_bwd(emu_lib, B, T, 1, 64, 64, state_std)
+
+
+def test_pass_of_64_wide_rows_fp32_states_every_chunk(emu_lib):
+    """Segments of one chunk with fp32 states, several per workgroup: a state's two tiles are taken in turn by three chunks in a row."""
+    test_pop_split_at_blocks(emu_lib, 1, 1300, 1, 64, 64, 64, 0.5, 21)
+
+
+@pytest.mark.parametrize("T,block", [(192, 64), (300, 64), (200, 40), (260, 130)])
+def test_pass_of_64_wide_rows_blocks(emu_lib, choose_backward, T, block):
+    """Block states leave, and their gradients join, at every chunk and at some of them."""
+    choose_backward(PASSES)
+    test_pop_fwd_bwd(emu_lib, 1, T, 1, 64, 64, block)

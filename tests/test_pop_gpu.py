@@ -176,3 +176,8 @@ def test_config4_pop_with_suffixes():
     (N + 1 = 65 per sequence, the first from S0).  Every sequence against the oracle, which runs on the GPU."""
     _suffix_case(B=8, N=64, block=64, Ls=16, H=16, dk=128, dv=128, seed=40, oracle_batches=range(8), oracle_device=DEV,
                  literal={})
+
+
+def test_pop_split_single_chunk_segments(hip_lib):
+    """64-token blocks of 64 x 64 states, more segments than units: every chunk of the passes brings fp32 states of its own."""
+    test_pop_split_entry_points(hip_lib, 1, 8192, 4, 64, 64, 64)

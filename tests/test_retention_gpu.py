@@ -477,3 +477,19 @@ def test_non_finite_future_keys_do_not_reach_earlier_outputs():
     torch.cuda.synchronize()
     assert torch.isfinite(o_bad[:, :t0].float()).all()
     assert torch.equal(o_bad[:, :t0], o_clean)
+
+
+@pytest.mark.parametrize("B,T,H,dv,state_std", [
+    (2, 64, 3, 64, 0.1), (1, 65, 3, 128, None), (2, 128, 2, 64, 0.1), (1, 191, 4, 64, 0.1), (1, 193, 4, 192, 0.1), (2, 257, 2, 256, 0.1),
+    (70, 64, 4, 64, 0.1), (75, 65, 4, 64, 0.1), (40, 150, 12, 128, None),   # more workgroups than units: several sequences each
+    (24, 700, 12, 64, 0.1),                                                 # ... with checkpoints (uncut: a workgroup per sequence)
+])
+def test_pass_of_64_wide_rows(hip_lib, B, T, H, dv, state_std):
+    """The pass whose rows are copied straight into LDS, in the forward and (by choice) in the three gradient passes, around the
+    number of chunks that are under way at a time."""
+    for choice in (0, 1):
+        assert hip_lib.fp_set_backward_choice(choice, -1) == 0
+        try:
+            run_plain(B, T, H, 64, dv, state_std, seed=T + choice, oracle_batches=sorted({0, B // 2, B - 1}), oracle_device=DEV)
+        finally:
+            assert hip_lib.fp_set_backward_choice(0, -1) == 0
