@@ -7,7 +7,6 @@
 #include "segment_contrib.h"
 #include "retention_bwd_fused.h"
 #include "short_seq.h"
-#include "pop_fold_fwd.h"
 #include "decode_step.h"
 #include "layer_ops.h"
 
@@ -60,11 +59,6 @@ template <int DK, int DV>
 __global__ __launch_bounds__(fpk::SI_THREADS) void suffix_intra_bwd_kernel(const fpk::FusedBwdArgs args) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   fpk::suffix_intra_bwd<DK, DV>(args, lds);
-}
-
-__global__ __launch_bounds__(fpk::PF_THREADS) void pop_fold_fwd_kernel(const fpk::PassArgs args) {
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  fpk::pop_fold_fwd(args, lds, fpk::place_workgroup(fprt::block_index(), fprt::grid_size(), 1).wg);
 }
 
 template <int DK, int DV>
@@ -250,8 +244,11 @@ struct DeviceRun {
   }
   template <int MODE>
   int fill(int slot) const {
-    return a.reverse ? launch(retention_pass_fill_kernel<MODE, true>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot + kFillReverse, 1, stream, err, a)
-                     : launch(retention_pass_fill_kernel<MODE, false>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot, 1, stream, err, a);
+    if constexpr (MODE == fpk::FILL_FOLD)
+      return launch(retention_pass_fill_kernel<MODE, false>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot, 1, stream, err, a);
+    else
+      return a.reverse ? launch(retention_pass_fill_kernel<MODE, true>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot + kFillReverse, 1, stream, err, a)
+                       : launch(retention_pass_fill_kernel<MODE, false>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot, 1, stream, err, a);
   }
 };
 
@@ -268,8 +265,13 @@ struct DeviceMultiRun {
   }
   template <int MODE>
   int fill(int slot) const {
-    return launch(retention_pass_fill_multi_kernel<MODE>, fpk::FP_THREADS, fpk::fp_lds_bytes(), fpk::PASS_KERNELS + slot, n, stream,
-                  err, planned[0], fpk::tensors_of(planned[1]), fpk::tensors_of(planned[n - 1]), n);
+    if constexpr (MODE == fpk::FILL_FOLD) {   // (the pass of a forward: it has a launch of its own)
+      *err = "walk with folded suffixes: one pass per launch";
+      return 1;
+    } else {
+      return launch(retention_pass_fill_multi_kernel<MODE>, fpk::FP_THREADS, fpk::fp_lds_bytes(), fpk::PASS_KERNELS + slot, n, stream, err,
+                    planned[0], fpk::tensors_of(planned[1]), fpk::tensors_of(planned[n - 1]), n);
+    }
   }
 };
 
@@ -326,11 +328,6 @@ int fpk_launch_pass(const fpk::PassArgs& args, void* stream, const char** err) {
     return 1;
   }
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (fpk::pop_folds(a, fpk_compute_units())) {
-    if (arm(reinterpret_cast<const void*>(pop_fold_fwd_kernel), fpk::pf_lds_bytes(), 64 + 34, err)) return 1;
-    hipLaunchKernelGGL(pop_fold_fwd_kernel, dim3((unsigned)(a.B * a.H * (a.dB / fpk::BV))), dim3(fpk::PF_THREADS), fpk::pf_lds_bytes(), st, a);
-    return launched(err);
-  }
   return fpk::dispatch_pass(a, DeviceRun{a, st, err});
 }
 

@@ -10,8 +10,8 @@
 namespace fpk {
 
 // Number of kernel instantiations `dispatch_pass` can pick from (its `slot` argument is below this).
-constexpr int PASS_KERNELS = 22;
-constexpr int FILL_SLOTS = 5;   // those of retention_pass_fill.h are below this
+constexpr int PASS_KERNELS = 23;
+constexpr int FILL_SLOTS = 5;   // those of retention_pass_fill.h that walk either way are below this
 
 // Checks what the walks assume about `a` and chooses a.slots (workgroups per (head, column tile))
 // for a device with `compute_units` units.  Returns nullptr, or a message for the caller.
@@ -100,6 +100,7 @@ int dispatch_pass(const PassArgs& a, Run&& run) {
   // trailing tokens after the last block boundary, or suffixes in several parts: the general suffix walk
   const bool suffix_any = suffix && (a.T != a.nblk * a.block || a.Ls > CH);
   if (a.dA == 64) {
+    if (pop_folds(a)) return run.template fill<FILL_FOLD>(22);
     if (suffix_any) return run.template go<64, WALK_SUFFIX_ANY, 1>(14);
     if (suffix) return run.template go<64, WALK_SUFFIX, 1>(0);
     if (blocks) return run.template fill<FILL_BLOCKS>(1);

@@ -1,5 +1,5 @@
 // Retention pass (see pass_args.h for the recurrence) whose tiles go from global memory into LDS without passing through
-// registers: dA = 64, without suffixes.
+// registers: dA = 64; of the walks with suffixes the forward one whose suffixes fit beside a chunk.
 //
 // One workgroup owns one (batch, head) stream and 64 columns of Z, Y and R.  Its waves have one of three roles:
 //
@@ -42,8 +42,11 @@ constexpr int FP_Q_LD = 2 * (32 + 8);     // row pitch of a carry wave's quarter
 constexpr int FP_Q = 32 * FP_Q_LD;
 
 // FILL_MULTI: a workgroup may walk several sequences (p.slots < p.B); FILL_BLOCKS: chunks end at block boundaries, where block
-// states leave (Bout, walking forward) or their gradients join (Bin, walking backward)
-enum FillMode { FILL_PLAIN = 0, FILL_MULTI = 1, FILL_BLOCKS = 2 };
+// states leave (Bout, walking forward) or their gradients join (Bin, walking backward).  FILL_FOLD: chunks end at block boundaries
+// of a POP call, and a suffix of at most FP_SFX tokens is part of the chunk that starts at its boundary, whose state it reads: a
+// fourth score tile, a second read-out, 16 more rows of every tensor.  The suffix at T hangs off one more, empty, chunk.
+enum FillMode { FILL_PLAIN = 0, FILL_MULTI = 1, FILL_BLOCKS = 2, FILL_FOLD = 3 };
+constexpr int FP_SFX = 16;
 
 // A tile of 64 tokens x 64 features
 struct FillTile {
@@ -63,7 +66,7 @@ constexpr int fp_lds_bytes() {
          + 2 * FillTile::BYTES                // W weighted
          + 2 * 3 * FP_P                       // scores
          + 2 * 4 * FP_Q                       // staged output
-         + 4 * FillTile::BYTES;               // states that enter
+         + 4 * FillTile::BYTES;               // states that enter; FILL_FOLD: the suffixes' tiles
 }
 
 namespace pp {
@@ -86,17 +89,19 @@ struct Chunk {
   uint32_t row;        // its first row among all rows of a tensor
   int b;               // its sequence
   bool first;          // starts its sequence
-  int bound, blk;      // FILL_BLOCKS: tokens up to the next boundary, block that the chunk belongs to
+  int bound, blk;      // FILL_BLOCKS, FILL_FOLD: tokens up to the next boundary, block that the chunk belongs to
+  int sfx;             // FILL_FOLD: the suffix at its first token, -1: none
   uint32_t base;       // the sequence's first row
   int len;             // ... and tokens
 };
+FP_DEVICE bool live(const Chunk& k) { return k.L > 0 || k.sfx >= 0; }
 // The chunks of sequence `slot`, then (FILL_MULTI) of slot + slots, ...  Without divisions and, but for a change of the sequence, branches.
 template <int MODE, bool REV>
 struct ChunkWalk {
   const PassArgs& p;
   FP_DEVICE void place(Chunk& k) const {
     k.L = k.left < CH ? k.left : CH;
-    if (MODE == FILL_BLOCKS) k.L = k.bound < k.L ? k.bound : k.L;
+    if (MODE == FILL_BLOCKS || MODE == FILL_FOLD) k.L = k.bound < k.L ? k.bound : k.L;
     k.row = REV ? k.base + (uint32_t)(k.left - k.L) : k.base + (uint32_t)(k.len - k.left);
   }
   FP_DEVICE Chunk first(int b) const {
@@ -105,14 +110,15 @@ struct ChunkWalk {
     k.first = true;
     k.len = p.T;
     k.base = (uint32_t)b * p.T;
-    if (MODE != FILL_BLOCKS && p.segs > 0) {   // (the last segment may be shorter)
+    if ((MODE == FILL_PLAIN || MODE == FILL_MULTI) && p.segs > 0) {   // (the last segment may be shorter)
       const int seg = b % p.segs, left = p.total - seg * p.T;
       k.len = left < p.T ? left : p.T;
       k.base = (uint32_t)(b / p.segs) * p.total + (uint32_t)seg * p.T;
     }
     k.left = b < p.B ? k.len : 0;
     k.blk = k.bound = 0;
-    if (MODE == FILL_BLOCKS) {
+    k.sfx = MODE == FILL_FOLD ? 0 : -1;
+    if (MODE == FILL_BLOCKS || MODE == FILL_FOLD) {
       k.blk = REV ? (p.T - 1) / p.block : 0;
       k.bound = REV ? p.T - k.blk * p.block : p.block;
     }
@@ -124,10 +130,11 @@ struct ChunkWalk {
     n.left = k.left - k.L;
     n.first = false;
     if (MODE == FILL_MULTI && k.L > 0 && n.left == 0) return first(k.b + p.slots);
-    if (MODE == FILL_BLOCKS) {
+    if (MODE == FILL_BLOCKS || MODE == FILL_FOLD) {
       const bool crosses = k.bound == k.L;
       n.bound = crosses ? p.block : k.bound - k.L;
       n.blk = k.blk + (crosses ? (REV ? -1 : 1) : 0);
+      if (MODE == FILL_FOLD) n.sfx = crosses && k.L > 0 ? n.blk : -1;
     }
     place(n);
     return n;
@@ -152,14 +159,20 @@ template <int MODE, bool REV>
 FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io, char* lds, int wg) {
   using namespace pp;
   using TT = FillTile;
-  constexpr bool MULTI = MODE == FILL_MULTI, BLOCKS = MODE == FILL_BLOCKS;
+  constexpr bool MULTI = MODE == FILL_MULTI, BLOCKS = MODE == FILL_BLOCKS, FOLD = MODE == FILL_FOLD;
+  static_assert(!FOLD || !REV, "suffixes: forward only");
   constexpr int DA = FP_DA, AHEAD = FP_AHEAD, KS = DA / 16, NAB = DA / 32;
-  constexpr int COPIES = 3 * TT::PER_WAVE;   // of a move wave, per chunk
+  constexpr int COPIES = 3 * TT::PER_WAVE + (FOLD ? 2 : 0);   // of a move wave, per chunk
   static_assert(AHEAD == 3, "the waits below");
 
   // X and W of a chunk are done with when it is carried, Z a step later
   constexpr int X0 = 0, W0 = X0 + AHEAD * TT::BYTES, Z0 = W0 + AHEAD * TT::BYTES, WW0 = Z0 + (AHEAD + 1) * TT::BYTES,
-                P0 = WW0 + 2 * TT::BYTES, Q0 = P0 + 2 * 3 * FP_P, S0 = Q0 + 2 * 4 * FP_Q;
+                P0 = WW0 + 2 * TT::BYTES, Q0 = P0 + 2 * 3 * FP_P,
+                END = Q0 + 2 * 4 * FP_Q, S0 = FOLD ? Q0 : END;
+  // FOLD: tiles of 16 rows (X and Z are both read when the chunk is carried); the state that enters takes the output stages' place
+  constexpr int SB = FP_SFX * TT::PITCH, XS0 = END, WS0 = XS0 + (AHEAD + 1) * SB, ZS0 = WS0 + AHEAD * SB, PS0 = ZS0 + (AHEAD + 1) * SB,
+                QS0 = PS0 + 2 * FP_P / 2, QS_HALF = FP_SFX * FP_Q_LD, QS_STAGE = 2 * QS_HALF;
+  static_assert(QS0 + 2 * QS_STAGE <= fp_lds_bytes() && S0 + 4 * TT::BYTES * (FOLD ? 0 : 1) <= fp_lds_bytes() && TT::BYTES <= 2 * 4 * FP_Q, "the tiles fit");
   auto at = [&](int byte) { return reinterpret_cast<uint16_t*>(lds + byte); };
   // the stage after one that starts `off` bytes into the rings of X and W, into that of Z
   auto next_x = [](int off) { return off == (AHEAD - 1) * TT::BYTES ? 0 : off + TT::BYTES; };
@@ -175,6 +188,7 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
   // backward).  These and the first are copied into LDS like the rows, this workgroup's 64 columns of R, [a][n] or, where R = S^T
   // (`tposed`), [n][a].  Four tiles taken in turn, or two pairs where the states are fp32, upper and lower halves.
   const bool tposed = io.rs_a == 1, halves = io.R0lo != nullptr;
+  auto sfx_row = [&](const Chunk& k) { return ((uint32_t)k.b * (p.nblk + 1) + (k.sfx > 0 ? k.sfx : 0)) * p.Ls; };
   auto brings_state = [&](const Chunk& k) { return MULTI ? io.R0 && k.first && k.L > 0 : BLOCKS && REV && io.Bin && walk.at_block_end(k); };
   auto state_tile = [&](int n) { return S0 + (halves ? (n & 1) * 2 : n & 3) * TT::BYTES; };
   auto matrix = [&](auto* base, int b) { return base + ((size_t)b * p.H + h) * p.dA * p.dB; };
@@ -213,9 +227,26 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
       fill(fprt::make_fill(Xg + (size_t)k.row * rowA, k.L > 0 ? (uint32_t)(k.L - 1) * rowA + DA * 2 : 0u), offA, rowA, X0 + sx);
       fill(fprt::make_fill(Zg + (size_t)k.row * rowB, k.L > 0 ? (uint32_t)(k.L - 1) * rowB + BV * 2 : 0u), offB, rowB, Z0 + sz);
     };
+    // FOLD: the 16 rows of a tensor are two copies, of X by wave 0, of W by wave 1 and of Z by the other two (as many each)
+    auto copy_suffix = [&](const Chunk& k, int sx, int sz) {
+      if constexpr (FOLD) {
+        const uint32_t pitch = fw < 2 ? rowA : rowB;
+        const char* const from = (fw == 0 ? reinterpret_cast<const char*>(io.Xs) + headA : fw == 1 ? reinterpret_cast<const char*>(io.Ws) + headA
+                                                                                               : reinterpret_cast<const char*>(io.Zs) + headB);
+        const int to = fw == 0 ? XS0 + sz / (TT::BYTES / SB) : fw == 1 ? WS0 + sx / (TT::BYTES / SB) : ZS0 + sz / (TT::BYTES / SB);
+        const fprt::FillView v = fprt::make_fill(from + (size_t)sfx_row(k) * pitch, k.sfx >= 0 ? (uint32_t)(p.Ls - 1) * pitch + 128 : 0u);
+        const int l = lane / TT::PPR;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int row = TT::ROWS * u + l;
+          fprt::fill_lds<false>(v, (uint32_t)row * pitch + (uint32_t)((lane % TT::PPR) ^ TT::key(row)) * 16, lds0 + (to + 1024 * u));
+        }
+      }
+    };
     auto copy = [&](const Chunk& k, int sx, int sz) {
       copy_w(k, sx);
       copy_xz(k, sx, sz);
+      copy_suffix(k, sx, sz);
     };
     const uint32_t rowR = 2u * (uint32_t)(tposed ? io.rs_n : io.rs_a);
     auto copy_tile = [&](const uint16_t* m, int to) {
@@ -275,7 +306,7 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
     int sx = 0, sz = 0, sp = 0;   // stages of chunk i
     bool late = false;            // the state of chunk i + 1 has not been asked for
 #pragma nounroll
-    while (c1.L > 0) {
+    while (live(c1)) {
       // The rows of W and those of X and Z not at once: where T * H * dA is a power of two all of them are on the same channels of
       // the memory (B16 T4096 H16, 64 values: 112 -> 101 us a launch).
       const int sx1 = next_x(sx);
@@ -287,7 +318,9 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
       if (state) copy_state(c2);
       copy_w(c3, sx);
       weigh(c1, sx1, sp ^ 1);
-      copy_xz(c3, sx, sz == 0 ? AHEAD * TT::BYTES : sz - TT::BYTES);
+      const int sz3 = sz == 0 ? AHEAD * TT::BYTES : sz - TT::BYTES;
+      copy_xz(c3, sx, sz3);
+      copy_suffix(c3, sx, sz3);
       // chunk i + 2 has arrived, its state and what is behind it may still be on its way
       if (!state) fprt::fill_wait<COPIES>();
       else if (!halves) fprt::fill_wait<COPIES + TT::PER_WAVE>();
@@ -318,9 +351,13 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
       // non-temporal: outputs are not read back by this launch and need not displace its inputs in the caches
       fprt::buf_store128_nt(yv, y_off, v0);
       fprt::buf_store128_nt(yv, y_off + 32 * rowB, v1);
+      if (FOLD && k.sfx >= 0 && t < 8 * FP_SFX) {
+        const fprt::BufView sv = fprt::make_buf(reinterpret_cast<char*>(io.Ys) + headB + (size_t)sfx_row(k) * rowB, (uint32_t)(p.Ls - 1) * rowB + BV * 2);
+        fprt::buf_store128_nt(sv, y_off, ld128(at(QS0 + sp * QS_STAGE + (y_piece >> 2) * QS_HALF + y_row * FP_Q_LD + 16 * (y_piece & 3))));
+      }
     };
-    // The diagonal score tiles by waves 0 and 1 of the role, the other live one by wave 2
-    const bool diagonal = fw < 2;
+    // The diagonal score tiles by waves 0 and 1 of the role, the other live one by wave 2, a suffix's by wave 3 (which has none otherwise)
+    const bool of_suffix = FOLD && fw == 3, scores = FOLD || fw < 3, diagonal = fw < 2 || of_suffix;
     const int s_ib = fw == 0 ? 0 : fw == 1 ? 1 : REV ? 0 : 1, s_jb = diagonal ? s_ib : 1 - s_ib;   // rows of X, rows of W
     float mw[16];
     uint32_t keep[8];      // bits to keep after conversion: a masked score is cleared, so that inf or nan cannot leak through 0 * x
@@ -334,14 +371,17 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
       const int d0 = REV ? acc_row(2 * e, g) - c : c - acc_row(2 * e, g), d1 = REV ? acc_row(2 * e + 1, g) - c : c - acc_row(2 * e + 1, g);
       keep[e] = diagonal ? ((d0 >= 0 ? 0x0000ffffu : 0u) | (d1 >= 0 ? 0xffff0000u : 0u)) : 0xffffffffu;
     }
-    const int x_at = X0 + TT::at(32 * s_ib + c, g), w_at = W0 + TT::at(32 * s_jb + c, g);
-    const int p_out = P0 + (diagonal ? s_ib : 2) * FP_P + lane * 16;
+    const int x_at = of_suffix ? XS0 + TT::at(c & (FP_SFX - 1), g) : X0 + TT::at(32 * s_ib + c, g);
+    const int w_at = of_suffix ? WS0 + TT::at(c & (FP_SFX - 1), g) : W0 + TT::at(32 * s_jb + c, g);
+    const int p_out = (of_suffix ? PS0 : P0 + (diagonal ? s_ib : 2) * FP_P) + lane * 16, p_stage = of_suffix ? FP_P / 2 : 3 * FP_P;
     u32x4 xf[KS], wf[KS];
-    auto score_load = [&](int sx) {
+    // sz: FOLD, the stage in the ring of suffixes' X
+    auto score_load = [&](int sx, int sz) {
+      const int ow = of_suffix ? sx / (TT::BYTES / SB) : sx, ox = of_suffix ? sz / (TT::BYTES / SB) : sx;
 #pragma unroll
       for (int k = 0; k < KS; ++k) {
-        wf[k] = ld128(at((w_at + sx) ^ (32 * k)));
-        xf[k] = ld128(at((x_at + sx) ^ (32 * k)));
+        wf[k] = ld128(at((w_at + ow) ^ (32 * k)));
+        xf[k] = ld128(at((x_at + ox) ^ (32 * k)));
       }
     };
     auto score = [&](int sp) {
@@ -357,25 +397,28 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
           const int r = 8 * k + 2 * e;
           d[e] = fprt::pack_bf16x2(sc[r] * mw[r], sc[r + 1] * mw[r + 1]) & keep[4 * k + e];
         }
-        st128(at(p_out + sp * 3 * FP_P + 1024 * k), d);
+        if (k == 0 || !of_suffix) st128(at(p_out + sp * p_stage + 1024 * k), d);
       }
     };
 
     Chunk c0 = walk.first(slot), cp = c0, c1 = walk.after(c0);
     cp.L = 0;
+    cp.sfx = -1;
     fprt::block_sync();
-    if (fw < 3) {
-      score_load(0);
+    if (scores) {
+      score_load(0, 0);
       score(0);
     }
     fprt::block_sync();
-    int sx = 0, sp = 0;   // stages of chunk i
+    int sx = 0, sz = 0, sp = 0;   // stages of chunk i
 #pragma nounroll
-    while (c1.L > 0) {
+    while (live(c1)) {
       sx = next_x(sx);
-      if (fw < 3) score_load(sx);
+      if (FOLD) sz = next_z(sz);
+      const bool now = of_suffix ? c1.sfx >= 0 : scores;
+      if (now) score_load(sx, sz);
       drain(cp, sp ^ 1);
-      if (fw < 3) score(sp ^ 1);
+      if (now) score(sp ^ 1);
       fprt::block_sync();
       cp = c0; c0 = c1;
       c1 = walk.after(c1);
@@ -473,6 +516,7 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
   const float gL_full = fprt::exp2_approx((float)CH * lg);
   const int p_at = P0 + lane * 16;
   const int y_at = quarter + c * FP_Q_LD + 16 * g;
+  const int xs_at = XS0 + TT::at(c & (FP_SFX - 1), g), ys_at = QS0 + ns * QS_HALF + (c & (FP_SFX - 1)) * FP_Q_LD + 16 * g;
 
   fprt::block_sync();
   if (io.R0) enter();
@@ -512,8 +556,30 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
     for (int k = 0; k < 4; ++k) z[k] = z_frag(Z0 + sz, k);
     // ---- read-out of the carried state, Y^T[n][i] = sum_a R[a][n] X[i][a]
     f32x16 acc = {0};
+    if (FOLD && ih == 0 && cur.sfx >= 0) {   // and the suffix's, whose rows are 0 .. 15 of a block
+      const int os = sz / (TT::BYTES / SB);
+      f32x16 accs = {0};
+      u32x4 xs[KS];
 #pragma unroll
-    for (int k = 0; k < KS; ++k) acc = fprt::mfma_32x32x16_bf16(packed(racc[k >> 1], k & 1), xf[k], acc);
+      for (int k = 0; k < KS; ++k) xs[k] = ld128(at((xs_at + os) ^ (32 * k)));
+      const u32x4 zs = z_frag(ZS0 + os, 0), ps = ld128(at(PS0 + lane * 16 + sp * (FP_P / 2)));
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        const u32x4 ra = packed(racc[k >> 1], k & 1);
+        acc = fprt::mfma_32x32x16_bf16(ra, xf[k], acc);
+        accs = fprt::mfma_32x32x16_bf16(ra, xs[k], accs);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) accs[r] *= wread_fwd;
+      accs = fprt::mfma_32x32x16_bf16(zs, ps, accs);
+      if (c < FP_SFX) {
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) st128(at(ys_at + sp * QS_STAGE + 32 * hf), packed(accs, hf));
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < KS; ++k) acc = fprt::mfma_32x32x16_bf16(packed(racc[k >> 1], k & 1), xf[k], acc);
+    }
     fprt::sched_fence();
     // ---- what the update needs is requested, R decays, the read-out is scaled
     u32x4 wa[4][NAB];
@@ -567,7 +633,7 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) st128(at(y_at + sp * 4 * FP_Q + 32 * hf), packed(acc, hf));
     fprt::block_sync();
-    if (nxt.L == 0) {
+    if (!live(nxt)) {
       if (BLOCKS && !REV && io.Bout && walk.at_block_end(cur)) leave(block_matrix(io.Bout, cur), sp ^ 1);
       if (io.Rout) leave(matrix(io.Rout, cur.b), sp ^ 1);
       return;
@@ -583,8 +649,26 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
 
 template <int MODE>
 FP_DEVICE void retention_pass_fill(const PassArgs& p, const PassTensors& io, char* lds, int wg) {
-  if (io.reverse) retention_pass_fill_dir<MODE, true>(p, io, lds, wg);
-  else retention_pass_fill_dir<MODE, false>(p, io, lds, wg);
+  if constexpr (MODE != FILL_FOLD) {
+    if (io.reverse) return retention_pass_fill_dir<MODE, true>(p, io, lds, wg);
+  }
+  retention_pass_fill_dir<MODE, false>(p, io, lds, wg);
+}
+
+// Whether a planned pass is a walk with folded suffixes: a forward whose suffixes fit beside a chunk, whole blocks.  The suffix walk of
+// retention_pass_ws.h, a suffix one more item of it, takes the others.  Speed here over that of the walk, 16-token suffixes, inputs not in
+// a cache, blocks of 16 to 64 tokens:
+//                workgroups    1 block         2 blocks        4 blocks        12 blocks       32 blocks
+//   64 x 64      32            1.11 to 1.12    1.27            1.46 to 1.47    1.78 to 1.81    1.94 to 2.01
+//                256           1.03 to 1.13    1.06 to 1.25    1.20 to 1.41    1.12 to 1.67    1.29 to 1.85
+//                1024          .99 to 1.13     1.08 to 1.27    1.21 to 1.40    1.41 to 1.69    1.23 to 1.96
+//   64 x 128     128           1.11 to 1.12    1.26 to 1.28    1.43 to 1.46    1.67 to 1.76    1.87 to 1.91
+//                1024          1.04 to 1.13    1.16 to 1.29    1.32 to 1.44    1.54 to 1.77    1.56 to 1.95
+//   64 x 256     1024          1.07 to 1.13    1.21 to 1.30    1.37 to 1.48    1.61 to 1.73    1.72 to 1.96
+// blocks of 72 to 128 tokens, 128 to 512 workgroups: 2 blocks 1.10 to 1.31, 12 blocks 1.16 to 1.61.
+// B8 H12 T2048 64 x 128, blocks of 64: 76.1 us in the walk, 44.4 here (61.0 in a kernel of two roles whose rows went through registers).
+inline bool pop_folds(const PassArgs& a) {
+  return a.Ls > 0 && a.Ls <= FP_SFX && !a.reverse && a.dA == FP_DA && a.T == a.nblk * a.block && a.rs_n == 1;
 }
 
 }  // namespace fpk

@@ -6,7 +6,6 @@
 #include "segment_contrib.h"
 #include "retention_bwd_fused.h"
 #include "short_seq.h"
-#include "pop_fold_fwd.h"
 #include "decode_step.h"
 #include "layer_ops.h"
 
@@ -43,11 +42,6 @@ int fpk_launch_pass(const fpk::PassArgs& args, void* /*stream*/, const char** er
   if (const char* why = fpk::plan_pass(a, fpk_compute_units())) {
     *err = why;
     return 1;
-  }
-  if (fpk::pop_folds(a, fpk_compute_units())) {
-    const int nwg = a.B * a.H * (a.dB / fpk::BV);
-    return run_grid(fpk::PF_THREADS, nwg, fpk::pf_lds_bytes(),
-                    [&](char* l) { fpk::pop_fold_fwd(a, l, fpk::place_workgroup(fprt::block_index(), nwg, 1).wg); });
   }
   return run_family(&a, 1);
 }
@@ -157,12 +151,12 @@ extern "C" int emu_contrib_pays(int seqs, int T, int H, int dk, int dv, int comp
   return fpk::contrib_pays(seqs, T, H, dk, dv, compute_units);
 }
 
-// The rule that chooses the forward of a POP call with suffixes, on a device of `compute_units`
-extern "C" int emu_pop_folds(int B, int T, int H, int dk, int dv, int block, int Ls, int compute_units) {
+// The rule that chooses the forward of a POP call with suffixes (the same on any device)
+extern "C" int emu_pop_folds(int B, int T, int H, int dk, int dv, int block, int Ls, int /*compute_units*/) {
   fpk::PassArgs a = {};
   a.B = B; a.T = T; a.H = H; a.dA = dk; a.dB = dv; a.block = block; a.nblk = T / block; a.Ls = Ls;
   a.rs_a = dv; a.rs_n = 1;
-  return fpk::pop_folds(a, compute_units);
+  return fpk::pop_folds(a);
 }
 
 // What every sequence (segment) adds to a zero state, U in fp32 halves, by the state-only kernel or (`walk`) by the pass kernel's

@@ -143,18 +143,17 @@ def test_fused_pop_fwd_bwd(emu_lib, B, nblk, block, Ls, H, dk, dv, state_std, ta
 
 @pytest.mark.parametrize("B,nblk,block,Ls,H,dv,state_std", [
     (1, 3, 65, 16, 1, 64, 0.5),      # a chunk of one token per block
-    (1, 2, 128, 1, 1, 192, None),    # the longest blocks it takes, one-token suffixes, three column tiles, no initial state
+    (1, 2, 128, 1, 1, 192, None),    # two chunks per block, one-token suffixes, three column tiles, no initial state
     (2, 4, 15, 15, 2, 64, 0.5),      # blocks shorter than a row block
     (1, 1, 63, 16, 1, 128, 0.5),     # a single short block
-    (1, 8, 65, 16, 1, 64, 0.5),      # what the rule gives to the folding kernel: a chunk of one token per block
-    (1, 8, 96, 1, 2, 64, None),      # ... the longest blocks, one-token suffixes, two heads, no initial state
+    (1, 8, 65, 16, 1, 64, 0.5),      # more chunks than are under way: of one token per block
+    (1, 8, 96, 1, 2, 64, None),      # ... of half a chunk, one-token suffixes, two heads, no initial state
     (1, 4, 63, 16, 1, 192, 0.5),     # ... blocks of less than a chunk, three column tiles
     (3, 3, 15, 15, 1, 256, 0.5),     # ... twelve workgroups on eight units
 ])
 def test_folded_forward(emu_lib, B, nblk, block, Ls, H, dv, state_std):
-    """64-wide keys and short suffixes: taken as part of the chunks at their boundaries, or (few blocks) as items of the walk."""
-    folds = nblk >= (3 if block <= 32 else 4 if block <= 64 else 8) and block <= 96
-    assert emu_lib.emu_pop_folds(B, nblk * block, H, 64, dv, block, Ls, 8) == folds
+    """64-wide keys and short suffixes: taken as part of the chunks at their boundaries."""
+    assert emu_lib.emu_pop_folds(B, nblk * block, H, 64, dv, block, Ls, 8) == 1
     decays = oracle.head_decays(H, (4, 9))
     q, k, v, s = hp.make_inputs(B, nblk * block, H, 64, dv, seed=block + Ls, state_std=state_std)
     sfx = hp.make_suffix_inputs(B, nblk, Ls, H, 64, dv, seed=block + Ls + 1)
@@ -166,23 +165,23 @@ def test_folded_forward(emu_lib, B, nblk, block, Ls, H, dv, state_std):
 
 @pytest.mark.parametrize("folds,B,nblk,H,dk,dv,block,Ls", [
     (1, 8, 32, 12, 64, 128, 64, 16),
-    (0, 8, 1, 12, 64, 128, 64, 16),       # too few blocks: the walk is faster
-    (0, 8, 3, 12, 64, 128, 33, 16),
+    (1, 8, 1, 12, 64, 128, 64, 16),       # a single block
+    (1, 8, 3, 12, 64, 128, 33, 16),
     (1, 8, 4, 12, 64, 128, 64, 16),
     (1, 8, 3, 12, 64, 256, 32, 16),
-    (0, 8, 2, 12, 64, 256, 1, 1),
-    (0, 8, 7, 8, 64, 128, 72, 3),         # two chunks a block
+    (1, 8, 2, 12, 64, 256, 1, 1),
+    (1, 8, 7, 8, 64, 128, 72, 3),         # two chunks a block
     (1, 8, 8, 8, 64, 128, 96, 3),
     (1, 8, 8, 8, 64, 256, 104, 3),
-    (0, 8, 64, 8, 64, 256, 105, 3),
-    (0, 4, 64, 8, 64, 64, 97, 3),
-    (1, 4, 4, 32, 64, 64, 64, 16),        # 64 x 64 states on half of the device
-    (0, 129, 11, 1, 64, 64, 64, 16),      # ... on more of it: the bytes count
+    (1, 8, 64, 8, 64, 256, 105, 3),
+    (1, 4, 64, 8, 64, 64, 97, 3),
+    (1, 4, 4, 32, 64, 64, 64, 16),        # 64 x 64 states
+    (1, 129, 11, 1, 64, 64, 64, 16),      # ... where the bytes count
     (1, 129, 12, 1, 64, 64, 64, 16),
-    (0, 17, 3, 8, 64, 64, 32, 16),
+    (1, 17, 3, 8, 64, 64, 32, 16),
     (1, 17, 4, 8, 64, 64, 32, 16),
     (1, 17, 3, 8, 64, 64, 16, 16),
-    (0, 17, 11, 8, 64, 64, 80, 16),
+    (1, 17, 11, 8, 64, 64, 80, 16),
     (1, 17, 12, 8, 64, 64, 80, 16),
     (0, 8, 32, 12, 128, 128, 64, 16),     # never: 128-wide keys, longer suffixes
     (0, 8, 32, 12, 64, 128, 64, 17),
