@@ -48,6 +48,20 @@ __global__ __launch_bounds__(fpk::FP_THREADS) void retention_pass_fill_multi_ker
   fpk::retention_pass_fill<MODE>(first, io, lds, id.wg);
 }
 
+// The same for dA = 128 with 128 columns per workgroup
+template <bool REV>
+__global__ __launch_bounds__(fpk::PW_THREADS) void retention_pass_wide_kernel(const fpk::PassArgs args) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  fpk::retention_pass_wide_dir<REV>(args, fpk::tensors_of(args), lds, fpk::place_workgroup(fprt::block_index(), fprt::grid_size(), 1).wg);
+}
+__global__ __launch_bounds__(fpk::PW_THREADS) void retention_pass_wide_multi_kernel(const fpk::PassArgs first, const fpk::PassTensors second,
+                                                                                   const fpk::PassTensors third, const int passes) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const fpk::WorkgroupId id = fpk::place_workgroup(fprt::block_index(), fprt::grid_size() / passes, passes);
+  const fpk::PassTensors io = id.pass == 0 ? fpk::tensors_of(first) : id.pass == 1 ? second : third;
+  fpk::retention_pass_wide(first, io, lds, id.wg);
+}
+
 // MODE: how POP suffixes take part (fpk::FbMode): none, as extra stops of the walks, or (at most 16 tokens) folded into
 // the chunks at their boundaries, with suffix_intra_bwd_kernel for what stays inside such a suffix
 template <int DK, int DV, int MODE>
@@ -109,13 +123,13 @@ __global__ __launch_bounds__(fpk::LAYER_THREADS) void gated_norm_bwd_kernel(cons
 // no thread calls hipFuncSetAttribute for it again (which matters to callers that capture
 // launches into a graph after a warm-up run).  Setting the attribute twice in a race is harmless.
 constexpr int kMaxDevices = 64;
-// retention_pass_fill_kernel walking backward: its bit is that many behind that of the same walk forward, behind all of those
-constexpr int kFillReverse = 2 * fpk::PASS_KERNELS;
-static_assert(kFillReverse + fpk::FILL_SLOTS <= 64, "one bit per kernel instantiation, single and paired");
+// retention_pass_fill_kernel and retention_pass_wide_kernel walking backward: of the former a bit is that many behind that of the same walk forward, behind all of those
+constexpr int kFillReverse = 2 * fpk::PASS_KERNELS, kWideReverse = kFillReverse + fpk::FILL_SLOTS;
+static_assert(kWideReverse < 64, "one bit per kernel instantiation, single and paired");
 std::atomic<uint64_t> g_armed[kMaxDevices][2];   // bits 0..63: pass kernels; 64..: the fused backward family, short sequences, state-only pass
 
 template <typename Kernel, typename... More>
-int launch(Kernel kernel, int threads, int lds, int slot, int passes, hipStream_t stream, const char** err,
+int launch(Kernel kernel, int threads, int lds, int slot, int nwg, hipStream_t stream, const char** err,
            const fpk::PassArgs& a, const More&... more) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
@@ -132,7 +146,6 @@ int launch(Kernel kernel, int threads, int lds, int slot, int passes, hipStream_
     }
     if (tracked) g_armed[dev][0].fetch_or(1ull << slot, std::memory_order_release);
   }
-  const int nwg = a.slots * a.H * (a.dB / fpk::BV) * passes;
   hipLaunchKernelGGL(kernel, dim3(nwg), dim3(threads), lds, stream, a, more...);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -240,15 +253,20 @@ struct DeviceRun {
   const char** err;
   template <int DA, int MODE, int NH>
   int go(int slot) const {
-    return launch(retention_pass_ws_kernel<DA, MODE, NH>, fpk::NTHREADS_WS, fpk::lds_bytes_ws(DA), slot, 1, stream, err, a);
+    return launch(retention_pass_ws_kernel<DA, MODE, NH>, fpk::NTHREADS_WS, fpk::lds_bytes_ws(DA), slot, fpk::pass_workgroups(a), stream, err, a);
   }
   template <int MODE>
   int fill(int slot) const {
     if constexpr (MODE == fpk::FILL_FOLD)
-      return launch(retention_pass_fill_kernel<MODE, false>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot, 1, stream, err, a);
+      return launch(retention_pass_fill_kernel<MODE, false>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot, fpk::pass_workgroups(a), stream, err, a);
     else
-      return a.reverse ? launch(retention_pass_fill_kernel<MODE, true>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot + kFillReverse, 1, stream, err, a)
-                       : launch(retention_pass_fill_kernel<MODE, false>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot, 1, stream, err, a);
+      return a.reverse ? launch(retention_pass_fill_kernel<MODE, true>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot + kFillReverse, fpk::pass_workgroups(a),
+                                stream, err, a)
+                       : launch(retention_pass_fill_kernel<MODE, false>, fpk::FP_THREADS, fpk::fp_lds_bytes(), slot, fpk::pass_workgroups(a), stream, err, a);
+  }
+  int wide(int slot) const {
+    return a.reverse ? launch(retention_pass_wide_kernel<true>, fpk::PW_THREADS, fpk::pw_lds_bytes(), kWideReverse, fpk::wide_workgroups(a), stream, err, a)
+                     : launch(retention_pass_wide_kernel<false>, fpk::PW_THREADS, fpk::pw_lds_bytes(), slot, fpk::wide_workgroups(a), stream, err, a);
   }
 };
 
@@ -260,7 +278,7 @@ struct DeviceMultiRun {
   template <int DA, int MODE, int NH>
   int go(int slot) const {
     return launch(retention_pass_multi_kernel<DA, MODE, NH>, fpk::NTHREADS_WS, fpk::lds_bytes_ws(DA),
-                  fpk::PASS_KERNELS + slot, n, stream, err, planned[0], fpk::tensors_of(planned[1]),
+                  fpk::PASS_KERNELS + slot, n * fpk::pass_workgroups(planned[0]), stream, err, planned[0], fpk::tensors_of(planned[1]),
                   fpk::tensors_of(planned[n - 1]), n);
   }
   template <int MODE>
@@ -269,9 +287,13 @@ struct DeviceMultiRun {
       *err = "walk with folded suffixes: one pass per launch";
       return 1;
     } else {
-      return launch(retention_pass_fill_multi_kernel<MODE>, fpk::FP_THREADS, fpk::fp_lds_bytes(), fpk::PASS_KERNELS + slot, n, stream, err,
-                    planned[0], fpk::tensors_of(planned[1]), fpk::tensors_of(planned[n - 1]), n);
+      return launch(retention_pass_fill_multi_kernel<MODE>, fpk::FP_THREADS, fpk::fp_lds_bytes(), fpk::PASS_KERNELS + slot,
+                    n * fpk::pass_workgroups(planned[0]), stream, err, planned[0], fpk::tensors_of(planned[1]), fpk::tensors_of(planned[n - 1]), n);
     }
+  }
+  int wide(int slot) const {
+    return launch(retention_pass_wide_multi_kernel, fpk::PW_THREADS, fpk::pw_lds_bytes(), fpk::PASS_KERNELS + slot, n * fpk::wide_workgroups(planned[0]),
+                  stream, err, planned[0], fpk::tensors_of(planned[1]), fpk::tensors_of(planned[n - 1]), n);
   }
 };
 
@@ -284,7 +306,7 @@ int fpk_launch_passes(const fpk::PassArgs* const* passes, int n, void* stream, c
     *err = why;
     return 1;
   }
-  return fpk::dispatch_pass(planned[0], DeviceMultiRun{planned, n, static_cast<hipStream_t>(stream), err});
+  return fpk::dispatch_pass(planned[0], n, fpk_compute_units(), DeviceMultiRun{planned, n, static_cast<hipStream_t>(stream), err});
 }
 
 namespace {
@@ -328,7 +350,7 @@ int fpk_launch_pass(const fpk::PassArgs& args, void* stream, const char** err) {
     return 1;
   }
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  return fpk::dispatch_pass(a, DeviceRun{a, st, err});
+  return fpk::dispatch_pass(a, 1, fpk_compute_units(), DeviceRun{a, st, err});
 }
 
 namespace {

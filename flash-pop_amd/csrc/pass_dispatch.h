@@ -6,11 +6,12 @@
 #include "pass_args.h"
 #include "retention_pass_ws.h"
 #include "retention_pass_fill.h"
+#include "retention_pass_wide.h"
 
 namespace fpk {
 
 // Number of kernel instantiations `dispatch_pass` can pick from (its `slot` argument is below this).
-constexpr int PASS_KERNELS = 23;
+constexpr int PASS_KERNELS = 24;
 constexpr int FILL_SLOTS = 5;   // those of retention_pass_fill.h that walk either way are below this
 
 // Checks what the walks assume about `a` and chooses a.slots (workgroups per (head, column tile))
@@ -91,10 +92,16 @@ inline const char* plan_passes(PassArgs* planned, const PassArgs* const* passes,
   return nullptr;
 }
 
-// Calls run.template go<DA, MODE, NH>(slot), or run.template fill<MODE>(slot) for the kernel of retention_pass_fill.h,
-// for the instantiation a planned `a` needs; `slot` numbers the instantiations 0 .. PASS_KERNELS - 1.
+// Workgroups of a planned pass: a column tile of `slots` sequences each, or in the kernel of retention_pass_wide.h twice the columns of
+// one sequence.
+inline int pass_workgroups(const PassArgs& a) { return a.slots * a.H * (a.dB / BV); }
+inline int wide_workgroups(const PassArgs& a) { return a.B * a.H * (a.dB / PW_D); }
+
+// Calls run.template go<DA, MODE, NH>(slot), run.template fill<MODE>(slot) for the kernel of retention_pass_fill.h or run.wide(slot) for
+// that of retention_pass_wide.h, for the instantiation that a launch of `passes` like the planned `a` needs; `slot` numbers the
+// instantiations 0 .. PASS_KERNELS - 1.
 template <typename Run>
-int dispatch_pass(const PassArgs& a, Run&& run) {
+int dispatch_pass(const PassArgs& a, int passes, int compute_units, Run&& run) {
   const bool blocks = a.block > 0 && (a.Bout || a.Bin);
   const bool suffix = a.Ls > 0, multi = a.slots < a.B;
   // trailing tokens after the last block boundary, or suffixes in several parts: the general suffix walk
@@ -113,6 +120,7 @@ int dispatch_pass(const PassArgs& a, Run&& run) {
     if (suffix) return run.template go<128, WALK_SUFFIX, 1>(5);
     if (blocks) return run.template go<128, WALK_BLOCKS, 1>(6);
     if (a.state_only) return run.template go<128, WALK_STATE, 1>(7);
+    if (pass_is_wide(a, passes, compute_units)) return run.wide(23);
     if (multi) return run.template go<128, WALK_MULTI, 1>(8);
     return run.template go<128, WALK_PLAIN, 1>(9);
   }

@@ -30,6 +30,19 @@ struct FamilyRun {
       return 1;   // another width's translation unit
     }
   }
+  int wide(int /*slot*/) const {
+    if constexpr (fpk::PW_D == EMU_FAMILY) {
+      const fpk::PassArgs& a = planned[0];
+      const int nwg = fpk::wide_workgroups(a), passes = n;
+      const fpk::PassArgs* const p = planned;
+      return run_grid(fpk::PW_THREADS, passes * nwg, fpk::pw_lds_bytes(), [&](char* l) {
+        const fpk::WorkgroupId id = fpk::place_workgroup(fprt::block_index(), nwg, passes);
+        fpk::retention_pass_wide(a, fpk::tensors_of(p[id.pass]), l, id.wg);
+      });
+    } else {
+      return 1;
+    }
+  }
   template <int MODE>
   int fill(int /*slot*/) const {
     if constexpr (fpk::FP_DA == EMU_FAMILY) {
@@ -52,5 +65,5 @@ struct FamilyRun {
 #define EMU_CAT2(a, b) a##b
 #define EMU_CAT(a, b) EMU_CAT2(a, b)
 int EMU_CAT(emu_pass_, EMU_FAMILY)(const fpk::PassArgs* planned, int n) {
-  return fpk::dispatch_pass(planned[0], FamilyRun{planned, n});
+  return fpk::dispatch_pass(planned[0], n, fpk_compute_units(), FamilyRun{planned, n});
 }

@@ -664,3 +664,15 @@ def test_pass_of_64_wide_rows_blocks(emu_lib, choose_backward, T, block):
     """Block states leave, and their gradients join, at every chunk and at some of them."""
     choose_backward(PASSES)
     test_pop_fwd_bwd(emu_lib, 1, T, 1, 64, 64, block)
+
+
+@pytest.mark.parametrize("B,T,H,dv,state_std", [
+    (5, 33, 1, 128, 0.5), (5, 64, 1, 128, None), (3, 65, 1, 256, 0.5), (5, 96, 1, 128, 0.5),   # fewer halves of chunks than are under way
+    (5, 161, 1, 128, 0.5), (2, 200, 2, 256, None), (5, 257, 1, 128, 0.5),                        # more
+    (9, 400, 1, 128, 0.5),                                                                       # more workgroups than units (8)
+])
+def test_pass_of_128_columns_per_workgroup(emu_lib, choose_backward, B, T, H, dv, state_std):
+    """The pass with 128 columns per workgroup and half a chunk per step, in the roles that it has: forward and dv pass, with values of
+    128 the dq and dk passes (which share a launch with it)."""
+    choose_backward(PASSES)
+    test_plain_fwd_bwd(emu_lib, B, T, H, 128, dv, state_std)

@@ -493,3 +493,19 @@ def test_pass_of_64_wide_rows(hip_lib, B, T, H, dv, state_std):
             run_plain(B, T, H, 64, dv, state_std, seed=T + choice, oracle_batches=sorted({0, B // 2, B - 1}), oracle_device=DEV)
         finally:
             assert hip_lib.fp_set_backward_choice(0, -1) == 0
+
+
+@pytest.mark.parametrize("B,T,H,dv,state_std", [
+    (10, 40, 16, 128, 0.1), (10, 64, 16, 128, None), (9, 65, 8, 256, 0.1), (10, 97, 16, 128, 0.1), (9, 128, 8, 256, None),
+    (10, 161, 16, 128, 0.1), (6, 200, 16, 256, 0.1), (10, 450, 16, 128, None), (33, 400, 8, 256, 0.1),
+    (2, 5000, 8, 256, 0.1),   # cut unevenly: segments from fp32 states
+])
+def test_pass_of_128_columns_per_workgroup(hip_lib, B, T, H, dv, state_std):
+    """The pass with 128 columns per workgroup and half a chunk per step, in the forward and (by choice) in the gradient passes,
+    around the number of halves that are under way at a time."""
+    for choice in (0, 1):
+        assert hip_lib.fp_set_backward_choice(choice, -1) == 0
+        try:
+            run_plain(B, T, H, 128, dv, state_std, seed=T + choice, oracle_batches=sorted({0, B // 2, B - 1}), oracle_device=DEV)
+        finally:
+            assert hip_lib.fp_set_backward_choice(0, -1) == 0
