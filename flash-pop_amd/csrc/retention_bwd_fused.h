@@ -476,6 +476,11 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
     return p.d_blocks + (((size_t)k.b * nblocks + (t0 / p.blocks_every - 1)) * p.H + k.h) * DK * DV;
   };
   constexpr int BP = DK * (DV / 8) / FB_THREADS;   // 16-byte pieces of a state matrix per thread
+  // 128 x 128: q of the chunk after next is asked for behind the third stretch's barrier, not in the stretch, which is the shortest and
+  // held up by four pieces' loads, and not together with dO, whose rows are on the same channels of the memory where T * H * 128 is a power
+  // of two (launches in a row, B8 H16 T4096 252 -> 243 us, B4 H24 230 -> 221; dO behind it 249 and 224, both 254 and 237, k and v behind the second
+  // stretch's 264 and 244; 64 x 128: neutral to 1 % slower).
+  constexpr bool Q_LATE = DK == FB_D && DV == FB_D && (MODE == FB_PLAIN || FOLD);   // (the modes it was measured in)
   Item cur = item_of(0), nxt = item_of(1), prev = Item{0u, 0, false};
   u32x4 pf_q[GK::NU], pf_g[GV::NU], pf_k[GK::NU], pf_v[GV::NU], pf_s = {0, 0, 0, 0};
   load_tile<DK, true>(k, p.q, p.q_sfx, cur, pf_q);   // q: read by this workgroup only
@@ -497,8 +502,10 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
   load_tile<DK>(k, p.k, p.k_sfx, nxt, pf_k);
   load_tile<DV>(k, p.v, p.v_sfx, nxt, pf_v);
   fprt::sched_fence();
-  load_tile<DK, true>(k, p.q, p.q_sfx, nxt, pf_q);
+  if (!Q_LATE) load_tile<DK, true>(k, p.q, p.q_sfx, nxt, pf_q);
   load_tile<DV>(k, p.dO, p.dO_sfx, nxt, pf_g);
+  fprt::sched_fence();
+  if (Q_LATE) load_tile<DK, true>(k, p.q, p.q_sfx, nxt, pf_q);
   fprt::sched_fence();
   fprt::block_sync();
   f32x16 racc[TPW];
@@ -721,10 +728,11 @@ FP_DEVICE void fused_bwd_reverse(const FusedBwdArgs& p, char* lds, int stream) {
     }
     stage_tile<DK>(k, Qs, pf_q);
     stage_tile<DV>(k, Gs, pf_g);
-    load_tile<DK, true>(k, p.q, p.q_sfx, after, pf_q);
+    if (!Q_LATE) load_tile<DK, true>(k, p.q, p.q_sfx, after, pf_q);
     load_tile<DV>(k, p.dO, p.dO_sfx, after, pf_g);
     if constexpr (FOLD) stage_suffix(pf_s);
     fprt::block_sync();
+    if (Q_LATE) load_tile<DK, true>(k, p.q, p.q_sfx, after, pf_q);
     prev = cur;
     cur = nxt;
     nxt = after;
