@@ -60,7 +60,8 @@ FP_DEVICE void retention_pass_wide_dir(const PassArgs& p, const PassTensors& io,
   auto half_row = [](int half) { return REV ? PW_ROWS * (1 - half) : PW_ROWS * half; };
   auto half_rows = [&](const Chunk& k, int half) {
     const int n = k.L - half_row(half);
-    return n < 0 ? 0 : n < PW_ROWS ? n : PW_ROWS;
+    // (walking backward it became one vector instruction, and every store a loop over lanes that might differ: 1.68 us a chunk, 1.54 without)
+    return (int)fprt::uniform((uint32_t)(n < 0 ? 0 : n < PW_ROWS ? n : PW_ROWS));
   };
 
   if (wave >= 4) {
