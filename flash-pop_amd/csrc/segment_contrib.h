@@ -20,8 +20,10 @@
 // 128 rows: 128 columns per workgroup of 512 threads; chunks from the first token on in both directions, weights of a k-step
 // from those of the one before.
 //
-// The sum leaves through the transposing read as well (16 bits at a time it took as long as four chunks: 128 x 128,
-// B12 T448 H8 17.1 -> 11.5 us a launch, B16 T2048 H8 dv 256 44.6 -> 40.5).
+// The sum leaves in whole lines: a lane holds eight consecutive columns of a row, which go through a row-major LDS tile (16 bits at a time
+// it took as long as four chunks: 128 x 128, B12 T448 H8 17.1 -> 11.5 us a launch; in pieces of 32 bytes, through the transposing read, which
+// took a second round for the lower halves, the launch of B1 H16 T1152 128 x 128 in segments of 4, 4, 4, 4 and 2 chunks took 11.5 us, so
+// 10.0, written through 9.4; of equal segments, T1280, 8.1 -> 7.4; the forward of B2 H8 T1152 128 x 256 29.4 -> 27.4).
 #pragma once
 #include <type_traits>
 
@@ -39,37 +41,32 @@ struct ContribTile {
   static constexpr int NRT = DK / 32, TPW = NRT * (NC / 32) / (NTH / 64);   // 32-row blocks of R; 32 x 32 tiles of it per wave
   static constexpr int NW = CH * (DK / 8) / NTH, NZ = CH * (NC / 8) / NTH;  // 16-byte pieces per thread
   static constexpr bool AS_WALK = NC == BV;
-  // two stages of a W and a Z tile; the copy of R that the final store reads takes their place
+  // two stages of a W and a Z tile; R on its way out (both halves of it) takes their place
   static constexpr int lds_bytes = 2 * 2 * STAGE;
-  static_assert(2 * STAGE >= NC * LDW, "the state copy fits where the tiles were");
+  static_assert(2 * STAGE >= 2 * DK * LDZ, "both halves of R fit where the tiles were");
   static_assert(NRT * (NC / 32) % (NTH / 64) == 0 && (NTH / 64) % NRT == 0, "whole tiles per wave");
 };
 
-// R (accumulator tiles of all waves), 16 bits of each element, through the LDS tile Rt -> its NC columns of matrix `stream` of dst
-template <int DK, int NC, int NTH, typename Part>
-FP_DEVICE void put_contribution(const ContribArgs& p, uint16_t* Rt, uint16_t* dst, int stream, int ct, int tid, int c, int g,
-                                int at_, int nt0, const f32x16 (&racc)[ContribTile<DK, NC, NTH>::TPW], Part part) {
-  using namespace fb;
-  constexpr int LDW = DK + 8, PPR = NC / 8;
+// Row m of a group of 16 of an accumulator tile stands for column 8 (bit 2) + 4 (bit 3) + (bits 0, 1) of R: a lane then holds eight
+// consecutive columns of a row.  The Z operand is read in that order: the pieces of four columns change places.
+template <int LD>
+FP_DEVICE fb::TrLane swapped_columns(int lane) {
+  const fb::TrLane tr = fb::tr_lane<LD>(lane, fb::TR_NAT);
+  const int piece = lane & 3, moved = 4 * ((((piece & 1) << 1) | (piece >> 1)) - piece);
+  return fb::TrLane{tr.lo + moved, tr.hi + moved};
+}
+// 16 bits of each element of R (the tiles of this wave) -> the row-major LDS tile Rt, `column`: this lane's first
+template <int TPW, int LD, typename Part>
+FP_DEVICE void lay_contribution(uint16_t* Rt, int row, int column, const f32x16 (&racc)[TPW], Part part) {
 #pragma unroll
-  for (int u = 0; u < ContribTile<DK, NC, NTH>::TPW; ++u) {
+  for (int u = 0; u < TPW; ++u) {
 #pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-      u32x2 d;
-      d[0] = pack16(racc[u][4 * qd], racc[u][4 * qd + 1], part);
-      d[1] = pack16(racc[u][4 * qd + 2], racc[u][4 * qd + 3], part);
-      st64(Rt + at<LDW>(32 * (nt0 + u) + c, 32 * at_ + 8 * qd + 4 * g), d);
+    for (int hf = 0; hf < 2; ++hf) {
+      u32x4 d;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d[e] = pack16(racc[u][8 * hf + 2 * e], racc[u][8 * hf + 2 * e + 1], part);
+      st128(Rt + fb::at<LD>(row, column + 32 * u + 16 * hf), d);
     }
-  }
-  fprt::block_sync();
-  char* const ubase = reinterpret_cast<char*>(dst) + ((size_t)stream * DK * p.dB + (size_t)ct * NC) * 2;
-  const fprt::BufView uv = fprt::make_buf(ubase, (uint32_t)(DK - 1) * p.dB * 2 + NC * 2);
-  // back through the transposing read: eight columns n of a row a per lane
-  const TrLane tr = tr_lane<LDW>(tid & 63, TR_SEQ);
-#pragma unroll
-  for (int i = 0; i < DK * PPR / NTH; ++i) {
-    const int pc = (tid >> 6) + (NTH / 64) * i, t = pc % (NC / 16), a32 = pc / (NC / 16);   // k-step of n, 32 rows of R
-    fprt::buf_store128(uv, (uint32_t)(32 * a32 + c) * p.dB * 2 + (16 * t + 8 * g) * 2, frag_rows<LDW>(Rt, tr, t, 32 * a32));
   }
 }
 
@@ -143,7 +140,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
 
   // this wave's tiles of R: rows a = 32 at_ .., columns n = 32 (nt0 + u) .., u < TPW
   const int at_ = wave % G::NRT, nt0 = (wave / G::NRT) * TPW;
-  const TrLane tr_w = tr_lane<LDW>(lane, TR_NAT), tr_z = tr_lane<LDZ>(lane, TR_NAT);
+  const TrLane tr_w = tr_lane<LDW>(lane, TR_NAT), tr_z = swapped_columns<LDZ>(lane);
   auto weight = [&](int e) { return p.s_update * fprt::exp2_approx((float)(e > 0 ? e : 0) * lg); };
   // Weights of a whole chunk.  AS_WALK: of every k-step.  Else of the k-step taken first (the last 16 tokens walking forward, the
   // first 16 walking backward); each further k-step is 16 tokens further from where the state is read.
@@ -201,7 +198,7 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
       }
       const u32x4 wa = weigh(ua[tt], wk);
 #pragma unroll
-      for (int u = 0; u < TPW; ++u) racc[u] = fprt::mfma_32x32x16_bf16(wa, ub[tt][u], racc[u]);
+      for (int u = 0; u < TPW; ++u) racc[u] = fprt::mfma_32x32x16_bf16(ub[tt][u], wa, racc[u]);
       if (tt + 2 < 4) request(tt + 2);
       if (!AS_WALK && tt < 3) {
 #pragma unroll
@@ -241,12 +238,33 @@ FP_DEVICE void segment_contrib(const ContribArgs& p, char* lds) {
     fprt::block_sync();
   }
 
-  // R -> its columns of the rows of U[b][h] (element (a, n) at a * dB + n), as bf16 or in fp32 halves; every read of the
-  // tiles is behind the last barrier
-  if (!p.U_lo) return put_contribution<DK, NC, NTH>(p, TL, p.U, stream, ct, tid, c, g, at_, nt0, racc, AsBf16{});
-  put_contribution<DK, NC, NTH>(p, TL, p.U, stream, ct, tid, c, g, at_, nt0, racc, UpperHalf{});
+  // R -> its columns of the rows of U[b][h] (element (a, n) at a * dB + n), as bf16 or in fp32 halves, in whole lines through LDS; every
+  // read of the tiles is behind the last barrier
+  uint16_t* const lower = TL + DK * LDZ;
+  const int row = 32 * at_ + c, column = 32 * nt0 + 8 * g;
+  if (p.U_lo) {
+    lay_contribution<TPW, LDZ>(TL, row, column, racc, UpperHalf{});
+    lay_contribution<TPW, LDZ>(lower, row, column, racc, LowerHalf{});
+  } else {
+    lay_contribution<TPW, LDZ>(TL, row, column, racc, AsBf16{});
+  }
   fprt::block_sync();
-  put_contribution<DK, NC, NTH>(p, TL, p.U_lo, stream, ct, tid, c, g, at_, nt0, racc, LowerHalf{});
+  const size_t matrix = (size_t)stream * DK * p.dB + (size_t)ct * NC;
+  // Written through from 2 MB a plane on (then and written back at the kernel's end, whole calls, us): B1 H16 T2001 128 x 128, 2.6 MB,
+  // 27.1 and 27.4; B1 H12 T5003 64 x 128, 3.9 MB, 28.2 and 28.8; below, B1 H4 T2048 64 x 64, .25 MB, 15.5 and 15.3, T4129 18.7 and 18.3.
+  const bool through = (size_t)p.B * p.H * DK * p.dB * 2 >= (2u << 20);
+  auto put = [&](uint16_t* dst, const uint16_t* Rt) {
+    const fprt::BufView uv = fprt::make_buf(dst + matrix, (uint32_t)(DK - 1) * p.dB * 2 + NC * 2);
+#pragma unroll
+    for (int i = 0; i < DK * (NC / 8) / NTH; ++i) {
+      const uint32_t to = (uint32_t)(z_place + RZ * i) * p.dB * 2 + z_piece * 16;
+      const u32x4 d = ld128(Rt + z_off + RZ * i * LDZ);
+      if (through) fprt::buf_store128_through(uv, to, d);
+      else fprt::buf_store128(uv, to, d);
+    }
+  };
+  put(p.U, TL);
+  if (p.U_lo) put(p.U_lo, lower);
 }
 
 // Host side, shared by the GPU launcher and the CPU test harness: argument check.
