@@ -426,7 +426,8 @@ int plan_segments(const Shape& s) {
 // Whether n segments shorten the chain of chunk steps by what the cut costs: its extra launches, and the segment states that it moves.
 // Counted in steps of 64-wide keys, 0.72 us on the 256-unit device (chunk_step); a launch is four of them with what its kernel takes to
 // begin and end.  States in fp32 halves (segments of unequal lengths, and blocks) take another three.  Measured uncut -> cut, us, inputs
-// in the caches, the same tensors again and again; forward:
+// in the caches, the same tensors again and again (before the state-only pass stored whole lines: 18 chunks of 128 x 256 cut 28.8 there, 27.4
+// with them; the line was not moved for it); forward:
 //   64 x 64    H4 B1        20 chunks 18.5 -> 15.2,  18 chunks 17.1 -> 16.5,  16 chunks 15.7 -> 15.1,  13 chunks 13.3 -> 16.4
 //   64 x 128   H12 B1       20 chunks 18.8 -> 16.1,  18 chunks 17.4 -> 18.1,  16 chunks 16.0 -> 16.0,  13 chunks 13.7 -> 17.6
 //   128 x 128  H8 B3        20 chunks 32.3 -> 23.2,  18 chunks 29.6 -> 28.3,  16 chunks 26.8 -> 22.5,  12 chunks 21.2 -> 21.9
