@@ -423,63 +423,35 @@ int plan_segments(const Shape& s) {
   }
   return even > 1 && 4 * (chunks / even) * fpk::CH <= 5 * tokens ? even : segment_count(s, tokens);
 }
-// Whether n segments shorten the chain of chunk steps by what the cut costs: its extra launches, and the segment states that it moves.
-// Counted in steps of 64-wide keys, 0.72 us on the 256-unit device (chunk_step); a launch is four of them with what its kernel takes to
-// begin and end.  States in fp32 halves (segments of unequal lengths, and blocks) take another three.  Measured uncut -> cut, us, inputs
-// in the caches, the same tensors again and again (before the state-only pass stored whole lines: 18 chunks of 128 x 256 cut 28.8 there, 27.4
-// with them; the line was not moved for it); forward:
-//   64 x 64    H4 B1        20 chunks 18.5 -> 15.2,  18 chunks 17.1 -> 16.5,  16 chunks 15.7 -> 15.1,  13 chunks 13.3 -> 16.4
-//   64 x 128   H12 B1       20 chunks 18.8 -> 16.1,  18 chunks 17.4 -> 18.1,  16 chunks 16.0 -> 16.0,  13 chunks 13.7 -> 17.6
-//   128 x 128  H8 B3        20 chunks 32.3 -> 23.2,  18 chunks 29.6 -> 28.3,  16 chunks 26.8 -> 22.5,  12 chunks 21.2 -> 21.9
-//   128 x 256  H8 B2        28 chunks 43.5 -> 26.7,  20 chunks 32.4 -> 24.1,  16 chunks 26.8 -> 23.5,  12 chunks 21.2 -> 22.9
-//   256 x 256  H8 B1        16 chunks 45.3 -> 31.9,  13 chunks 37.9 -> 37.9,  12 chunks 35.4 -> 31.1,   9 chunks 27.7 -> 35.6
+// Whether n segments shorten the chain of chunk steps by what the cut costs: its extra launches, and the segment states
+// that it moves.  Forward, measured at 1.1 us (64-wide keys) to 1.4 us (128) a step on the 256-unit device, uncut -> cut:
+//   64 x 64    H4 B1        18 chunks 23.8 -> 19.9 us, 16 chunks 21.8 -> 18.5,  13 chunks 18.4 -> 19.7
+//   64 x 128   H12 B1       79 chunks 89.6 -> 32.8,    18 chunks 24.4 -> 20.9,  13 chunks 18.9 -> 20.6
+//   128 x 128  H8 B3        28 chunks 44.0 -> 30.7,    18 chunks 30.0 -> 29.3,  13 chunks 23.5 -> 28.7
+//   128 x 256  H8 B2        40 chunks 60.0 -> 38.6,    28 chunks 43.9 -> 33.8,  18 chunks 30.0 -> 38.3
 // Backward (the uncut passes share launches, or are the fused kernel with its longer step; the cut has four launches and the
 // forward's states):
-//   64 x 64    H4 B1        32 chunks 27.4 -> 22.8,  28 chunks 24.6 -> 22.7,  24 chunks 21.8 -> 22.6
-//   64 x 64    H12 B6       60 chunks 102 -> 81,     40 chunks 69.3 -> 64.6,  28 chunks 50.3 -> 52.1 (fused)
-//   64 x 128   H12 B1       20 chunks 51.4 -> 35.3,  16 chunks 42.7 -> 35.0,  13 chunks 36.2 -> 37.7
-//   128 x 128  H16 B1       28 chunks 44.1 -> 34.5,  24 chunks 38.3 -> 33.8,  20 chunks 33.0 -> 33.4,  16 chunks 27.4 -> 32.4
-//   128 x 256  H8 B2        28 chunks 118 -> 58,     20 chunks 87.1 -> 54.1,  16 chunks 71.3 -> 53.3,  13 chunks 60.0 -> 60.1
-//   256 x 256  H8 B1        20 chunks 56.3 -> 62.0,  16 chunks 46.3 -> 49.1
-// POP calls (pop_cut_pays) keep an older line, further out for wide keys: cut, their o is no longer that of the plain call bit for bit,
-// which callers rely on for 12 to 16 chunks (128 x 128, H4 B2).  It leaves forward / backward, uncut -> cut:
-//   64 x 64    H4 B1        6 blocks of 144 19.5 -> 17.4 / 35.9 -> 24.6 (cut),   4 blocks of 256 17.2 -> 17.7 / 35.0 -> 25.9
-//   64 x 128   H4 B4        8 blocks of 144 25.3 -> 22.3 / 98.7 -> 40.3 (cut),   6 blocks of 144 20.0 -> 20.4 / 77.8 -> 37.8 (cut)
-//   128 x 128  H8 B1        6 blocks of 256 43.0 -> 26.5 / 80.0 -> 37.3 (cut),   4 blocks of 256 29.9 -> 24.9 / 56.2 -> 35.1
-//   256 x 256  H8 B1        6 blocks of 256 75.8 -> 42.8 / 140 -> 72,            4 blocks of 256 52.1 -> 38.8 / 96.6 -> 56.8
-double chunk_step(int dk) { return dk == 64 ? 1. : dk == 128 ? 1.9 : 3.; }   // of a pass whose keys are dk wide
-// Waves of the state-only pass over `streams` sequences
-long long contrib_waves(const Shape& s, long long streams) {
-  return waves(streams * (s.dk == fpk::FB_D && s.dv % fpk::FB_D == 0 ? s.dv / fpk::FB_D : s.dv / fpk::BV));
-}
-bool cut_pays(const Shape& s, int n, int tokens, bool backward) {
+//   64 x 64    H4 B1        28 chunks 35.3 -> 27.8,    18 chunks 24.8 -> 28.7
+//   64 x 64    H12 B6       79 chunks 132 -> 133,      40 chunks 69.8 -> 79.5,  28 chunks 50.5 -> 63.6 (fused)
+//   64 x 128   H12 B1       18 chunks 54.3 -> 41.9,    13 chunks 41.4 -> 40.9
+//   128 x 128  H16 B1       79 chunks 116 -> 82,       40 chunks 61.8 -> 50.8,  28 chunks 45.1 -> 44.6
+//   128 x 256  H8 B2        28 chunks 119 -> 68,       18 chunks 80.0 -> 70.9,  13 chunks 60.8 -> 61.8
+// The line dates from slower state-only passes, scans and fused backwards: it leaves calls of 16 to 18 chunks uncut that a cut
+// would shorten (128 x 256 up to 28), and cuts the backward of 64 x 64 on 72 streams from 40 chunks on.  (Measured before the
+// state-only passes got another 0.3 to 0.8 us shorter.)
+// `block`: a POP call, whose chunks end at its blocks and whose gradient passes share fewer launches (64 x 128, B4 H4 T1440
+// in blocks of 144, 30 chunks, with the suffix call and the launches between the two: 200 -> 166 us).
+bool cut_pays(const Shape& s, int n, int tokens, bool backward, int block = 0) {
   const int launch = fpk_launch_steps();   // what a launch costs, in chunk steps
   if (launch <= 0) return true;
-  const long long each = (tokens + fpk::CH - 1) / fpk::CH, chunks = (s.T + fpk::CH - 1LL) / fpk::CH;
+  const long long each = (tokens + fpk::CH - 1) / fpk::CH, chunks = block > 0 ? n * each : (s.T + fpk::CH - 1LL) / fpk::CH;
   const long long streams = (long long)s.B * s.H * n, tk = s.dk / fpk::BV, tv = s.dv / fpk::BV;
-  const double k_step = chunk_step(s.dk), v_step = chunk_step(s.dv), contrib = k_step * contrib_waves(s, streams);
-  if (!backward) {
-    const bool even = (long long)tokens * n == s.T;
-    return k_step * chunks - each * (contrib + k_step * waves(streams * tv)) >= launch * (even ? 2. : 2.75);
-  }
-  // dq and dk walk rows as wide as the values, dv rows as wide as the keys; uncut, dq shares the launch of dk, and all three share one
-  // where the widths are equal
-  const bool equal = s.dk == s.dv;
-  const double uncut = use_fused_backward(s, nullptr) ? 1.1 * (k_step + v_step) : equal ? k_step : k_step + v_step;
-  const double dk_dv = equal ? k_step * waves(2 * streams * tk) : v_step * waves(streams * tk) + k_step * waves(streams * tv);
-  return uncut * chunks - each * (contrib + v_step * waves(streams * tk) + dk_dv) >= launch * 4;
-}
-// The same for a POP call cut at its n blocks, in chunk steps of its own width (the chunks end at the blocks).
-bool pop_cut_pays(const Shape& s, int n, int block, bool backward) {
-  const int launch = fpk_launch_steps();
-  if (launch <= 0) return true;
-  const long long each = (block + fpk::CH - 1) / fpk::CH, chunks = n * each;
-  const long long streams = (long long)s.B * s.H * n, tk = s.dk / fpk::BV, tv = s.dv / fpk::BV, contrib = contrib_waves(s, streams);
   const double matrix = s.dk * s.dv / 16384.;
+  const long long contrib = waves(streams * (s.dk == fpk::FB_D && s.dv % fpk::FB_D == 0 ? s.dv / fpk::FB_D : tv));
   if (!backward) return chunks - each * (contrib + waves(streams * tv)) >= launch * (2 + 1.25 * matrix);
-  const bool equal = s.dk == s.dv, fused = use_fused_backward(s, nullptr) && block % fpk::CH == 0;
-  const long long uncut = fused ? 7 * chunks / 4 : (equal ? 2 : 3) * chunks;
-  const long long dk_dv = equal ? waves(2 * streams * tk) : waves(streams * tk) + waves(streams * tv);
+  const long long dk_dv = s.dk == s.dv ? waves(2 * streams * tk) : waves(streams * tk) + waves(streams * tv);
+  const bool fused = use_fused_backward(s, nullptr) && block % fpk::CH == 0;
+  const long long uncut = fused ? 7 * chunks / 4 : ((s.dk == s.dv ? 1 : 2) + (block > 0 ? 1 : 0)) * chunks;
   return uncut - each * (contrib + waves(streams * tk) + dk_dv) >= launch * (2.5 + 1.75 * matrix);
 }
 // Forward and backward cut a sequence the same way, so that the states the forward leaves at the start of every segment
@@ -517,11 +489,11 @@ int plan_pop_forward(const Shape& s, int block) {
   const long long streams = (long long)s.B * s.H * ((s.dk < s.dv ? s.dk : s.dv) / fpk::BV);
   if (block < fpk::CH || s.T <= block || 3 * streams > fpk_compute_units()) return 1;
   const int n = segment_count(s, block);
-  return block_states_pay(s, n, block) && pop_cut_pays(s, n, block, false) ? n : 1;
+  return block_states_pay(s, n, block) && cut_pays(s, n, block, false, block) ? n : 1;
 }
 int plan_pop_backward(const Shape& s, int block) {
   const int n = plan_pop_forward(s, block);
-  return n > 1 && pop_cut_pays(s, n, block, true) ? n : 1;
+  return n > 1 && cut_pays(s, n, block, true, block) ? n : 1;
 }
 
 size_t workspace_bytes(const Shape& s, int segments) {
