@@ -96,10 +96,13 @@ FP_DEVICE void buf_store128_nt(BufView b, uint32_t off, u32x4 v) { __builtin_amd
 FP_DEVICE void buf_store128_through(BufView b, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, b.rsrc, off, 0, 2 | 16); }
 FP_DEVICE void buf_store64(BufView b, uint32_t off, u32x2 v) { __builtin_amdgcn_raw_buffer_store_b64(v, b.rsrc, off, 0, 0); }
 
-// Global memory -> LDS without a way through registers: lane l's 16 bytes at byte `off` of the view land at byte 16 l from `lds`, which
-// is the same in every lane (zeros, where they are beyond the view).  Asynchronous: what it wrote may be read after fill_wait
-// and a barrier.  Inline assembly, because the compiler would put a wait for every copy in flight before every LDS read
-// that follows; nothing but LDS is written, so there is no register for it to lose track of.
+// Global memory -> LDS without a way through registers: lane l's 16 bytes at byte `off[u]` of the view land at byte 16 l from
+// `lds` + STEP u, which is the same in every lane (zeros, where they are beyond the view).  Asynchronous: what it wrote may be read after
+// fill_wait and a barrier.  Inline assembly, because the compiler would put a wait for every copy in flight before every LDS read
+// that follows; nothing but LDS is written, so there is no register for it to lose track of.  The compiler does not see the buffer
+// instructions either, so the wait states that these need are here: five behind a vector instruction (v_readfirstlane) that wrote a
+// word of the view, which may be the one right before this, and one behind m0.  All copies of a view at once, so that the five are
+// paid once.
 struct FillView {
   u32x4 words;   // the buffer resource, uniform
 };
@@ -111,11 +114,27 @@ FP_DEVICE FillView make_fill(const void* base, uint32_t nbytes) {
 typedef uint32_t LdsAddress;
 FP_DEVICE LdsAddress lds_address(const char* p) { return uniform((uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p)); }
 // ONCE: with the non-temporal hint
-template <bool ONCE>
-FP_DEVICE void fill_lds(const FillView& v, uint32_t off, LdsAddress lds) {
-  if (ONCE) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(lds), "v"(off), "s"(v.words) : "memory", "m0");
-  else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(v.words) : "memory", "m0");
+#define FP_COPY_FIRST(HINT) "s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %3, %1, 0 offen" HINT " lds"
+#define FP_COPY_NEXT(OFF, HINT) "\n\ts_add_u32 m0, m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %" #OFF ", %1, 0 offen" HINT " lds"
+template <bool ONCE, int STEP>
+FP_DEVICE void fill_lds(const FillView& v, const uint32_t (&off)[2], LdsAddress lds) {
+  if (ONCE)
+    asm volatile(FP_COPY_FIRST(" nt") FP_COPY_NEXT(4, " nt")
+                 ::"s"(lds), "s"(v.words), "n"(STEP), "v"(off[0]), "v"(off[1]) : "memory", "m0", "scc");
+  else
+    asm volatile(FP_COPY_FIRST("") FP_COPY_NEXT(4, "")
+                 ::"s"(lds), "s"(v.words), "n"(STEP), "v"(off[0]), "v"(off[1]) : "memory", "m0", "scc");
 }
+template <bool ONCE, int STEP>
+FP_DEVICE void fill_lds(const FillView& v, const uint32_t (&off)[8], LdsAddress lds) {
+  static_assert(!ONCE, "not with the hint");
+  asm volatile(FP_COPY_FIRST("") FP_COPY_NEXT(4, "") FP_COPY_NEXT(5, "") FP_COPY_NEXT(6, "") FP_COPY_NEXT(7, "") FP_COPY_NEXT(8, "")
+               FP_COPY_NEXT(9, "") FP_COPY_NEXT(10, "")
+               ::"s"(lds), "s"(v.words), "n"(STEP), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]), "v"(off[5]),
+               "v"(off[6]), "v"(off[7]) : "memory", "m0", "scc");
+}
+#undef FP_COPY_FIRST
+#undef FP_COPY_NEXT
 // Until at most N of this wave's loads, copies and stores are still under way (they end in order).
 template <int N>
 FP_DEVICE void fill_wait() {

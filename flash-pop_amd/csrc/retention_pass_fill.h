@@ -212,13 +212,9 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
     // this wave's part of 64 rows into a tile at `to`
     auto fill = [&](const fprt::FillView& v, uint32_t off, uint32_t pitch, int to) {
       const fprt::LdsAddress dst = lds0 + (to + 1024 * fw);
-      if (once) {
-#pragma unroll
-        for (int u = 0; u < TT::PER_WAVE; ++u) fprt::fill_lds<true>(v, off + 4 * TT::ROWS * u * pitch, dst + 4096 * u);
-      } else {
-#pragma unroll
-        for (int u = 0; u < TT::PER_WAVE; ++u) fprt::fill_lds<false>(v, off + 4 * TT::ROWS * u * pitch, dst + 4096 * u);
-      }
+      const uint32_t offs[TT::PER_WAVE] = {off, off + 4 * TT::ROWS * pitch};
+      if (once) fprt::fill_lds<true, 4096>(v, offs, dst);
+      else fprt::fill_lds<false, 4096>(v, offs, dst);
     };
     auto copy_w = [&](const Chunk& k, int sx) {
       fill(fprt::make_fill(Wg + (size_t)k.row * rowA, k.L > 0 ? (uint32_t)(k.L - 1) * rowA + DA * 2 : 0u), offA, rowA, W0 + sx);
@@ -235,12 +231,13 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
                                                                                                : reinterpret_cast<const char*>(io.Zs) + headB);
         const int to = fw == 0 ? XS0 + sz / (TT::BYTES / SB) : fw == 1 ? WS0 + sx / (TT::BYTES / SB) : ZS0 + sz / (TT::BYTES / SB);
         const fprt::FillView v = fprt::make_fill(from + (size_t)sfx_row(k) * pitch, k.sfx >= 0 ? (uint32_t)(p.Ls - 1) * pitch + 128 : 0u);
-        const int l = lane / TT::PPR;
+        uint32_t off[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const int row = TT::ROWS * u + l;
-          fprt::fill_lds<false>(v, (uint32_t)row * pitch + (uint32_t)((lane % TT::PPR) ^ TT::key(row)) * 16, lds0 + (to + 1024 * u));
+          const int row = TT::ROWS * u + lane / TT::PPR;
+          off[u] = (uint32_t)row * pitch + (uint32_t)((lane % TT::PPR) ^ TT::key(row)) * 16;
         }
+        fprt::fill_lds<false, 1024>(v, off, lds0 + to);
       }
     };
     auto copy = [&](const Chunk& k, int sx, int sz) {

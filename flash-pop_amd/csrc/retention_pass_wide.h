@@ -170,8 +170,10 @@ FP_DEVICE void retention_pass_wide_dir(const PassArgs& p, const PassTensors& io,
     auto copy = [&](const Chunk& k, int half, int stage) {
       const int rows = half_rows(k, half);
       const fprt::FillView v = fprt::make_fill(from + (size_t)(k.row + half_row(half)) * pitch, rows > 0 ? (uint32_t)(rows - 1) * pitch + PW_PITCH : 0u);
+      uint32_t offs[COPIES];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) fprt::fill_lds<false>(v, off[u & 3] + (u >> 2) * 16 * pitch, lds0 + (ring + stage + 1024 * u));
+      for (int u = 0; u < COPIES; ++u) offs[u] = off[u & 3] + (u >> 2) * 16 * pitch;
+      fprt::fill_lds<false, 1024>(v, offs, lds0 + (ring + stage));
     };
     // W weighted for the state update, by waves 2 and 3: rows 4 u + lane / 16, u = 4 (fw - 2) .. + 3
     auto weight = [&](int half, int u, int L) {

@@ -148,10 +148,12 @@ FP_DEVICE FillView make_fill(const void* base, uint32_t nbytes) { return make_bu
 FP_DEVICE uint32_t uniform(uint32_t x) { return x; }
 typedef char* LdsAddress;
 FP_DEVICE LdsAddress lds_address(char* p) { return p; }
-template <bool ONCE>
-FP_DEVICE void fill_lds(const FillView& v, uint32_t off, LdsAddress lds) {
-  const u32x4 d = buf_load128(v, off);
-  std::memcpy(lds + 16 * (g_lane.tid & 63), &d, 16);
+template <bool ONCE, int STEP, int N>
+FP_DEVICE void fill_lds(const FillView& v, const uint32_t (&off)[N], LdsAddress lds) {
+  for (int u = 0; u < N; ++u) {
+    const u32x4 d = buf_load128(v, off[u]);
+    std::memcpy(lds + STEP * u + 16 * (g_lane.tid & 63), &d, 16);
+  }
 }
 template <int N>
 FP_DEVICE void fill_wait() {}
