@@ -371,11 +371,24 @@ FP_DEVICE void retention_pass_wide_dir(const PassArgs& p, const PassTensors& io,
         for (int r = 0; r < 16; ++r) racc[a][r] *= gL;
       }
     }
+    // The two tiles of half 1 are summed in the order of retention_pass_ws.h, whose waves begin with the tile that they made themselves,
+    // those of the odd column blocks the other one: a call's o has the same bits whether it leaves block states (there) or not (here)
+    auto own_tile = [&]() {
 #pragma unroll
-    for (int k = 0; k < 2; ++k) acc = fprt::mfma_32x32x16_bf16(z[k], pd[k], acc);
-    if (half == 1) {
+      for (int k = 0; k < 2; ++k) acc = fprt::mfma_32x32x16_bf16(z[k], pd[k], acc);
+    };
+    auto other_tile = [&]() {
 #pragma unroll
       for (int k = 0; k < 2; ++k) acc = fprt::mfma_32x32x16_bf16(zp[k], po[k], acc);
+    };
+    if (half == 0) {
+      own_tile();
+    } else if (ns & 1) {
+      other_tile();
+      own_tile();
+    } else {
+      own_tile();
+      other_tile();
     }
     fprt::sched_fence();
     request_w(1);

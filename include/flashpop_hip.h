@@ -125,8 +125,8 @@ int fp_retention_fwd_split_static(const void* q, const void* k, const void* v, c
 
 /* The POP entry points below for few streams and long sequences, cut at the blocks the way fp_retention_*_split cuts at
  * segments of its own choice, where the states of all blocks are worth moving; the states between blocks are fp32.  Where blocks
- * are whole 64-token chunks the o of a call that is not cut is that of fp_retention_fwd bit for bit; that of a cut one differs
- * by the order of fp32 sums.  workspace, forward_states_kept and the two sizes as there.  0 bytes: the shape is not cut, and the calls are
+ * are whole 64-token chunks and sequences longer than 32 tokens (which have a kernel of their own) the o of a call that is not cut is
+ * that of fp_retention_fwd bit for bit, and so is that of fp_retention_fwd_ckpt; that of a cut one differs by the order of fp32 sums.  workspace, forward_states_kept and the two sizes as there.  0 bytes: the shape is not cut, and the calls are
  * fp_pop_retention_fwd / _bwd. */
 size_t fp_pop_retention_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size);
 size_t fp_pop_retention_backward_workspace_bytes(int B, int T, int H, int dk, int dv, int block_size);

@@ -676,3 +676,22 @@ def test_pass_of_128_columns_per_workgroup(emu_lib, choose_backward, B, T, H, dv
     128 the dq and dk passes (which share a launch with it)."""
     choose_backward(PASSES)
     test_plain_fwd_bwd(emu_lib, B, T, H, 128, dv, state_std)
+
+
+@pytest.mark.parametrize("B,T,dv,block", [
+    (6, 256, 128, 64),     # a block state behind every chunk
+    (3, 320, 256, 128),    # two column blocks per workgroup, tokens after the last boundary
+])
+def test_outputs_do_not_depend_on_block_states(emu_lib, B, T, dv, block):
+    """128-wide keys on more than half of the units: the plain forward runs in the kernel with 128 columns per workgroup, one that leaves
+    block states (POP, checkpoints) in the one with 64.  o is the same bit for bit, and so is the state after the last token."""
+    decays = oracle.head_decays(1, (4, 9))
+    q, k, v, s = hp.make_inputs(B, T, 1, 128, dv, seed=T + dv, state_std=0.5)
+    o, S = hp.raw_fwd(emu_lib, q, k, v, s, decays)
+    o_pop, states = hp.raw_pop_fwd(emu_lib, q, k, v, s, decays, block)
+    assert torch.equal(o, o_pop)
+    assert T % block != 0 or torch.equal(S, states[:, -1])
+    if dv == 128:
+        d_o, d_s = hp.make_cotangents([(B, T, 1, dv), (B, 1, 128, dv)], seed=T)
+        o_ckpt, S_ckpt = hp.raw_ckpt_fwd_bwd(emu_lib, q, k, v, s, decays, d_o, d_s, 128)[:2]
+        assert torch.equal(o, o_ckpt) and torch.equal(S, S_ckpt)

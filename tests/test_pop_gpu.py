@@ -87,6 +87,27 @@ def test_pop_outputs_equal_plain_outputs():
 
 
 @pytest.mark.parametrize("B,T,H,dk,dv,block", [
+    (10, 576, 16, 128, 128, 64),    # 160 workgroups of 128 columns in the plain call
+    (9, 576, 8, 128, 256, 192),     # 144
+    (24, 704, 16, 128, 128, 128),   # 384, more than there are units
+    (24, 640, 12, 64, 128, 64),     # 64-wide keys
+])
+def test_outputs_do_not_depend_on_block_states(hip_lib, B, T, H, dk, dv, block):
+    """Calls of many workgroups, where a plain forward may run in another kernel than one that leaves block states or checkpoints: o and
+    the last state are the same bit for bit."""
+    decays = oracle.head_decays(H)
+    q, k, v, s = hp.make_inputs(B, T, H, dk, dv, seed=T, state_std=0.1, device=DEV)
+    assert hip_lib.fp_retention_workspace_bytes(B, T, H, dk, dv) == hip_lib.fp_pop_retention_workspace_bytes(B, T, H, dk, dv, block) == 0
+    o, S = hp.raw_fwd(hip_lib, q, k, v, s, decays)
+    o_pop, states = hp.raw_pop_fwd(hip_lib, q, k, v, s, decays, block)
+    assert torch.equal(o_pop, o) and (T % block != 0 or torch.equal(states[:, -1], S))
+    if dv == 128:
+        d_o, d_s = hp.make_cotangents([(B, T, H, dv), (B, H, dk, dv)], seed=T, device=DEV)
+        o_ckpt, S_ckpt = hp.raw_ckpt_fwd_bwd(hip_lib, q, k, v, s, decays, d_o, d_s, 512)[:2]
+        assert torch.equal(o_ckpt, o) and torch.equal(S_ckpt, S)
+
+
+@pytest.mark.parametrize("B,T,H,dk,dv,block", [
     (1, 1500, 4, 128, 128, 144),   # the 128-wide state-only kernel, blocks and a tail that end inside a chunk
     (2, 1000, 4, 128, 64, 100),    # 64 columns of a state per workgroup, the sequence ends on a boundary
     (1, 1500, 2, 256, 64, 144),
