@@ -306,7 +306,7 @@ int fpk_launch_passes(const fpk::PassArgs* const* passes, int n, void* stream, c
     *err = why;
     return 1;
   }
-  return fpk::dispatch_pass(planned[0], n, fpk_compute_units(), DeviceMultiRun{planned, n, static_cast<hipStream_t>(stream), err});
+  return fpk::dispatch_pass(planned, n, fpk_compute_units(), DeviceMultiRun{planned, n, static_cast<hipStream_t>(stream), err});
 }
 
 namespace {
@@ -350,7 +350,7 @@ int fpk_launch_pass(const fpk::PassArgs& args, void* stream, const char** err) {
     return 1;
   }
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  return fpk::dispatch_pass(a, 1, fpk_compute_units(), DeviceRun{a, st, err});
+  return fpk::dispatch_pass(&a, 1, fpk_compute_units(), DeviceRun{a, st, err});
 }
 
 namespace {

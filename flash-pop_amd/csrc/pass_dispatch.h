@@ -2,6 +2,7 @@
 // launcher and the CPU thread harness so that both take the same decisions.
 #pragma once
 #include <cstring>
+#include <initializer_list>
 
 #include "pass_args.h"
 #include "retention_pass_ws.h"
@@ -11,7 +12,7 @@
 namespace fpk {
 
 // Number of kernel instantiations `dispatch_pass` can pick from (its `slot` argument is below this).
-constexpr int PASS_KERNELS = 24;
+constexpr int PASS_KERNELS = 27;
 constexpr int FILL_SLOTS = 5;   // those of retention_pass_fill.h that walk either way are below this
 
 // Checks what the walks assume about `a` and chooses a.slots (workgroups per (head, column tile))
@@ -97,21 +98,37 @@ inline const char* plan_passes(PassArgs* planned, const PassArgs* const* passes,
 inline int pass_workgroups(const PassArgs& a) { return a.slots * a.H * (a.dB / BV); }
 inline int wide_workgroups(const PassArgs& a) { return a.B * a.H * (a.dB / PW_D); }
 
+// Whether everything that the kernels of retention_pass_fill.h and retention_pass_wide.h copy straight into LDS, 16 bytes at a time,
+// starts at a multiple of them (rows and matrices are).  The pass kernel's loads into registers take any address.
+inline bool copies_aligned(const PassArgs& a) {
+  uintptr_t at = 0;
+  for (const uint16_t* t : {a.X, a.W, a.Z, a.R0, a.R0lo, a.Bin, a.Xs, a.Ws, a.Zs}) at |= reinterpret_cast<uintptr_t>(t);
+  return at % 16 == 0;
+}
+
 // Calls run.template go<DA, MODE, NH>(slot), run.template fill<MODE>(slot) for the kernel of retention_pass_fill.h or run.wide(slot) for
-// that of retention_pass_wide.h, for the instantiation that a launch of `passes` like the planned `a` needs; `slot` numbers the
+// that of retention_pass_wide.h, for the instantiation that a launch of the `n` planned passes needs; `slot` numbers the
 // instantiations 0 .. PASS_KERNELS - 1.
 template <typename Run>
-int dispatch_pass(const PassArgs& a, int passes, int compute_units, Run&& run) {
+int dispatch_pass(const PassArgs* planned, int n, int compute_units, Run&& run) {
+  const PassArgs& a = planned[0];
+  bool copies = true;
+  for (int i = 0; i < n; ++i) copies = copies && copies_aligned(planned[i]);
   const bool blocks = a.block > 0 && (a.Bout || a.Bin);
   const bool suffix = a.Ls > 0, multi = a.slots < a.B;
   // trailing tokens after the last block boundary, or suffixes in several parts: the general suffix walk
   const bool suffix_any = suffix && (a.T != a.nblk * a.block || a.Ls > CH);
   if (a.dA == 64) {
-    if (pop_folds(a)) return run.template fill<FILL_FOLD>(22);
+    if (copies && pop_folds(a)) return run.template fill<FILL_FOLD>(22);
     if (suffix_any) return run.template go<64, WALK_SUFFIX_ANY, 1>(14);
     if (suffix) return run.template go<64, WALK_SUFFIX, 1>(0);
-    if (blocks) return run.template fill<FILL_BLOCKS>(1);
     if (a.state_only) return run.template go<64, WALK_STATE, 1>(2);
+    if (!copies) {
+      if (blocks) return run.template go<64, WALK_BLOCKS, 1>(24);
+      if (multi) return run.template go<64, WALK_MULTI, 1>(25);
+      return run.template go<64, WALK_PLAIN, 1>(26);
+    }
+    if (blocks) return run.template fill<FILL_BLOCKS>(1);
     if (multi) return run.template fill<FILL_MULTI>(3);
     return run.template fill<FILL_PLAIN>(4);
   }
@@ -120,7 +137,7 @@ int dispatch_pass(const PassArgs& a, int passes, int compute_units, Run&& run) {
     if (suffix) return run.template go<128, WALK_SUFFIX, 1>(5);
     if (blocks) return run.template go<128, WALK_BLOCKS, 1>(6);
     if (a.state_only) return run.template go<128, WALK_STATE, 1>(7);
-    if (pass_is_wide(a, passes, compute_units)) return run.wide(23);
+    if (copies && pass_is_wide(a, n, compute_units)) return run.wide(23);
     if (multi) return run.template go<128, WALK_MULTI, 1>(8);
     return run.template go<128, WALK_PLAIN, 1>(9);
   }

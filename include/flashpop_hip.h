@@ -6,7 +6,8 @@
  * launches inside one of those four methods; the citation names that method.
  *
  * Conventions common to all entry points
- *   - every tensor pointer is DEVICE memory, bf16 (2 bytes/element), contiguous, in the
+ *   - every tensor pointer is DEVICE memory, bf16 (2 bytes/element), contiguous, at any multiple of 2 bytes
+ *     (at a multiple of 16 where an entry point says so; the fastest kernels run where all are), in the
  *     reference's layouts: q, k, dq, dk [B,T,H,dk]; v, o, d_o, dv [B,T,H,dv]; states
  *     [B,H,dk,dv]; block states [B, T/block_size, H, dk, dv]
  *   - head_decays is HOST memory: H doubles, gamma_h in (0, 1]

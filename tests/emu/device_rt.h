@@ -6,6 +6,7 @@
 #include <pthread.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstring>
 
@@ -148,9 +149,11 @@ FP_DEVICE FillView make_fill(const void* base, uint32_t nbytes) { return make_bu
 FP_DEVICE uint32_t uniform(uint32_t x) { return x; }
 typedef char* LdsAddress;
 FP_DEVICE LdsAddress lds_address(char* p) { return p; }
+inline std::atomic<int> g_misaligned_fills{0};   // copies from addresses that are not multiples of their 16 bytes
 template <bool ONCE, int STEP, int N>
 FP_DEVICE void fill_lds(const FillView& v, const uint32_t (&off)[N], LdsAddress lds) {
   for (int u = 0; u < N; ++u) {
+    if ((uint64_t)off[u] + 16 <= v.nbytes && (reinterpret_cast<uintptr_t>(v.base) + off[u]) % 16 != 0) ++g_misaligned_fills;
     const u32x4 d = buf_load128(v, off[u]);
     std::memcpy(lds + STEP * u + 16 * (g_lane.tid & 63), &d, 16);
   }

@@ -65,5 +65,5 @@ struct FamilyRun {
 #define EMU_CAT2(a, b) a##b
 #define EMU_CAT(a, b) EMU_CAT2(a, b)
 int EMU_CAT(emu_pass_, EMU_FAMILY)(const fpk::PassArgs* planned, int n) {
-  return fpk::dispatch_pass(planned[0], n, fpk_compute_units(), FamilyRun{planned, n});
+  return fpk::dispatch_pass(planned, n, fpk_compute_units(), FamilyRun{planned, n});
 }

@@ -695,3 +695,48 @@ def test_outputs_do_not_depend_on_block_states(emu_lib, B, T, dv, block):
         d_o, d_s = hp.make_cotangents([(B, T, 1, dv), (B, 1, 128, dv)], seed=T)
         o_ckpt, S_ckpt = hp.raw_ckpt_fwd_bwd(emu_lib, q, k, v, s, decays, d_o, d_s, 128)[:2]
         assert torch.equal(o, o_ckpt) and torch.equal(S, S_ckpt)
+
+
+def _shifted(t):
+    """The same values two bytes behind where they would be aligned."""
+    if t is None:
+        return None
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype)
+    flat[1:] = t.flatten()
+    assert flat[1:].data_ptr() % 4 == 2
+    return flat[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("which,B,T,dk,dv,block,Ls", [
+    *[(which, 1, 100, 64, 64, 0, 0) for which in ("q", "k", "v", "s", "all")],   # one sequence per workgroup
+    *[(which, 9, 40, 64, 128, 0, 0) for which in ("k", "all")],                  # several
+    *[(which, 1, 150, 64, 64, 64, 0) for which in ("v", "s", "all")],            # block states
+    *[(which, 1, 128, 64, 64, 64, 16) for which in ("q", "s", "sfx", "all")],    # folded suffixes
+    *[(which, 6, 100, 128, 128, 0, 0) for which in ("q", "all")],                # 128 columns per workgroup
+])
+def test_tensors_that_are_not_aligned(emu_lib, choose_backward, which, B, T, dk, dv, block, Ls):
+    """Tensors at any address are taken, as by loads into registers, and none is copied straight into LDS from one that is no multiple of
+    16 bytes, for which such copies are not made."""
+    choose_backward(PASSES)
+    decays = oracle.head_decays(1, (4, 9))
+    q, k, v, s = hp.make_inputs(B, T, 1, dk, dv, seed=T, state_std=0.5)
+    move = lambda name, t: _shifted(t) if which in (name, "all") else t
+    ins = [move(name, t) for name, t in zip("qkvs", (q, k, v, s))]
+    emu_lib.emu_misaligned_fills()
+    if Ls:
+        sfx = hp.make_suffix_inputs(B, T // block, Ls, 1, dk, dv, seed=T + 1)
+        got = hp.raw_fused_fwd(emu_lib, *ins, [move("sfx", t) for t in sfx], decays, block)
+        ref = hp.oracle_fused(q, k, v, s, sfx, decays, block)
+    elif block:
+        d_o, d_b = hp.make_cotangents([(B, T, 1, dv), (B, T // block, 1, dk, dv)], seed=T)
+        got = hp.raw_pop_fwd(emu_lib, *ins, decays, block) + hp.raw_pop_bwd(emu_lib, *ins, decays, block, move("v", d_o), move("s", d_b))
+        o_ref, st_ref, grads = hp.oracle_pop(q, k, v, s, decays, block, d_o, d_b)
+        ref = (o_ref, st_ref, *grads)
+    else:
+        d_o, d_s = hp.make_cotangents([(B, T, 1, dv), (B, 1, dk, dv)], seed=T)
+        got = hp.raw_fwd(emu_lib, *ins, decays) + hp.raw_bwd(emu_lib, *ins, decays, move("v", d_o), move("s", d_s))
+        o_ref, S_ref, grads = hp.oracle_plain(q, k, v, s, decays, d_o, d_s)
+        ref = (o_ref, S_ref, *grads)
+    assert emu_lib.emu_misaligned_fills() == 0
+    for i, (g, r) in enumerate(zip(got, ref)):
+        hp.assert_close(g, r, f"output {i}")

@@ -509,3 +509,37 @@ def test_pass_of_128_columns_per_workgroup(hip_lib, B, T, H, dv, state_std):
             run_plain(B, T, H, 128, dv, state_std, seed=T + choice, oracle_batches=sorted({0, B // 2, B - 1}), oracle_device=DEV)
         finally:
             assert hip_lib.fp_set_backward_choice(0, -1) == 0
+
+
+@pytest.mark.parametrize("B,T,H,dk,dv,block,Ls", [
+    (2, 193, 4, 64, 64, 0, 0), (75, 65, 4, 64, 64, 0, 0), (2, 300, 4, 64, 128, 64, 0), (2, 192, 4, 64, 128, 64, 16), (10, 97, 16, 128, 128, 0, 0),
+])
+def test_tensors_that_are_not_aligned(hip_lib, B, T, H, dk, dv, block, Ls):
+    """Tensors two bytes behind a multiple of 16, which the kernels that copy rows straight into LDS do not take, against the oracle."""
+    def shifted(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        flat[1:] = t.flatten()
+        return flat[1:].view(t.shape)
+
+    decays = oracle.head_decays(H)
+    q, k, v, s = hp.make_inputs(B, T, H, dk, dv, seed=T, state_std=0.1, device=DEV)
+    ins = [shifted(t) for t in (q, k, v, s)]
+    assert all(t.data_ptr() % 16 == 2 for t in ins)
+    d_o, d_s = hp.make_cotangents([(B, T, H, dv), (B, H, dk, dv)], seed=T + 1, device=DEV)
+    assert hip_lib.fp_set_backward_choice(1, -1) == 0
+    try:
+        if Ls:
+            sfx = hp.make_suffix_inputs(B, T // block, Ls, H, dk, dv, seed=T, device=DEV)
+            got = hp.raw_fused_fwd(hip_lib, *ins, [shifted(t) for t in sfx], decays, block)
+            ref = hp.oracle_fused(q, k, v, s, sfx, decays, block, device=DEV)
+        elif block:
+            got, ref = hp.raw_pop_fwd(hip_lib, *ins, decays, block), hp.oracle_pop(q, k, v, s, decays, block, device=DEV)
+        else:
+            got = hp.raw_fwd(hip_lib, *ins, decays) + hp.raw_bwd(hip_lib, *ins, decays, shifted(d_o), shifted(d_s))
+            o_ref, S_ref, grads = hp.oracle_plain(q, k, v, s, decays, d_o, d_s, device=DEV)
+            ref = (o_ref, S_ref, *grads)
+        torch.cuda.synchronize()
+    finally:
+        assert hip_lib.fp_set_backward_choice(0, -1) == 0
+    for i, (g, r) in enumerate(zip(got, ref)):
+        hp.assert_close(g, r, f"output {i}", head_dim=2 if g.dim() == 4 and g.shape[2] == H and g.shape[1] != H else None)
