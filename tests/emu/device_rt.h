@@ -5,10 +5,12 @@
 #pragma once
 #include <pthread.h>
 #include <stdint.h>
+#include <unistd.h>
 
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <deque>
 
 #define FP_DEVICE inline __attribute__((always_inline))
 
@@ -37,7 +39,16 @@ extern thread_local LaneCtx g_lane;
 FP_DEVICE int thread_index() { return g_lane.tid; }
 FP_DEVICE int block_index() { return g_lane.block; }
 FP_DEVICE int grid_size() { return g_lane.grid; }
-FP_DEVICE void block_sync() { pthread_barrier_wait(g_lane.wg_bar); }
+// A test can have the lanes below `threads` (above, if negative) come late out of every workgroup barrier: what the others do at once then
+// comes before everything that these do.
+struct Lag {
+  int threads, microseconds;
+};
+inline Lag g_lag{0, 0};
+FP_DEVICE void block_sync() {
+  pthread_barrier_wait(g_lane.wg_bar);
+  if (g_lag.threads != 0 && (g_lag.threads > 0 ? g_lane.tid < g_lag.threads : g_lane.tid >= -g_lag.threads)) usleep(g_lag.microseconds);
+}
 
 FP_DEVICE float bf16_to_f32(uint16_t b) {
   uint32_t u = (uint32_t)b << 16;
@@ -123,20 +134,43 @@ struct BufView {
   uint32_t nbytes;
 };
 FP_DEVICE BufView make_buf(const void* base, uint32_t nbytes) { return BufView{static_cast<const char*>(base), nbytes}; }
-FP_DEVICE u32x4 buf_load128(BufView b, uint32_t off) {
+// What a lane has under way: copies into LDS and, counted with them, its other loads and stores.  They end in order.  A copy lands as late
+// as it may, when a wait (fill_wait) is for it, and until then its place in LDS holds a pattern (nan): what reads it too early, or
+// what it overwrites too early, shows.
+struct UnderWay {
+  char* to;   // nullptr: no copy
+  u32x4 data;
+};
+inline thread_local std::deque<UnderWay> g_under_way;
+FP_DEVICE void counted() {
+  if (!g_under_way.empty()) g_under_way.push_back(UnderWay{nullptr, u32x4{0u, 0u, 0u, 0u}});   // (ahead of the first copy it makes no difference)
+}
+inline void land(size_t left) {
+  for (; g_under_way.size() > left; g_under_way.pop_front()) {
+    if (g_under_way.front().to) std::memcpy(g_under_way.front().to, &g_under_way.front().data, 16);
+  }
+}
+FP_DEVICE u32x4 bytes_at(BufView b, uint32_t off) {
   u32x4 v = {0u, 0u, 0u, 0u};
   if ((uint64_t)off + 16 <= b.nbytes) std::memcpy(&v, b.base + off, 16);
   return v;
 }
+FP_DEVICE u32x4 buf_load128(BufView b, uint32_t off) {
+  counted();
+  return bytes_at(b, off);
+}
 FP_DEVICE u32x2 buf_load64(BufView b, uint32_t off) {
+  counted();
   u32x2 v = {0u, 0u};
   if ((uint64_t)off + 8 <= b.nbytes) std::memcpy(&v, b.base + off, 8);
   return v;
 }
 FP_DEVICE void buf_store128(BufView b, uint32_t off, u32x4 v) {
+  counted();
   if ((uint64_t)off + 16 <= b.nbytes) std::memcpy(const_cast<char*>(b.base) + off, &v, 16);
 }
 FP_DEVICE void buf_store64(BufView b, uint32_t off, u32x2 v) {
+  counted();
   if ((uint64_t)off + 8 <= b.nbytes) std::memcpy(const_cast<char*>(b.base) + off, &v, 8);
 }
 // the non-temporal forms differ only in how the device's caches treat the data
@@ -154,11 +188,12 @@ template <bool ONCE, int STEP, int N>
 FP_DEVICE void fill_lds(const FillView& v, const uint32_t (&off)[N], LdsAddress lds) {
   for (int u = 0; u < N; ++u) {
     if ((uint64_t)off[u] + 16 <= v.nbytes && (reinterpret_cast<uintptr_t>(v.base) + off[u]) % 16 != 0) ++g_misaligned_fills;
-    const u32x4 d = buf_load128(v, off[u]);
-    std::memcpy(lds + STEP * u + 16 * (g_lane.tid & 63), &d, 16);
+    char* const to = lds + STEP * u + 16 * (g_lane.tid & 63);
+    std::memset(to, 0xff, 16);
+    g_under_way.push_back(UnderWay{to, bytes_at(v, off[u])});
   }
 }
 template <int N>
-FP_DEVICE void fill_wait() {}
+FP_DEVICE void fill_wait() { land(N); }
 
 }  // namespace fprt

@@ -149,6 +149,8 @@ int fpk_launch_contrib(const fpk::ContribArgs& a, void* /*stream*/, const char**
 // Copies into LDS since the last call that were not from a multiple of 16 bytes
 extern "C" int emu_misaligned_fills() { return fprt::g_misaligned_fills.exchange(0); }
 
+extern "C" void emu_set_lag(int threads, int microseconds) { fprt::g_lag = fprt::Lag{threads, microseconds}; }
+
 // The rule that chooses the state-only pass
 extern "C" int emu_contrib_pays(int seqs, int T, int H, int dk, int dv, int compute_units) {
   return fpk::contrib_pays(seqs, T, H, dk, dv, compute_units);

@@ -16,6 +16,7 @@ int run_grid(int nthreads, int nwg, int lds_bytes, Body body) {
   pthread_barrier_init(&wg_bar, nullptr, nthreads);
   std::vector<fprt::WaveShared> waves(nthreads / 64);
   for (auto& w : waves) pthread_barrier_init(&w.bar, nullptr, 64);
+  std::atomic<int> unfinished{0};   // workgroups' lanes that ended with copies into LDS under way
   std::vector<std::thread> lanes;
   for (int t = 0; t < nthreads; ++t) {
     lanes.emplace_back([&, t] {
@@ -26,6 +27,13 @@ int run_grid(int nthreads, int nwg, int lds_bytes, Body body) {
       for (int wg = 0; wg < nwg; ++wg) {
         fprt::g_lane.block = wg;
         body(lds->data());
+        for (const auto& u : fprt::g_under_way) {
+          if (u.to) {
+            ++unfinished;
+            break;
+          }
+        }
+        fprt::g_under_way.clear();
         pthread_barrier_wait(&wg_bar);
       }
     });
@@ -34,7 +42,7 @@ int run_grid(int nthreads, int nwg, int lds_bytes, Body body) {
   for (auto& w : waves) pthread_barrier_destroy(&w.bar);
   pthread_barrier_destroy(&wg_bar);
   delete lds;
-  return 0;
+  return unfinished != 0;
 }
 
 }  // namespace

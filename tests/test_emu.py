@@ -659,6 +659,25 @@ def test_pass_of_64_wide_rows_fp32_states_every_chunk(emu_lib):
     test_pop_split_at_blocks(emu_lib, 1, 1300, 1, 64, 64, 64, 0.5, 21)
 
 
+def test_pass_of_64_wide_rows_fp32_states_every_second_chunk(emu_lib):
+    """... of two chunks: the state of a chunk is asked for in the step that carries the last one that brought its own."""
+    test_pop_split_at_blocks(emu_lib, 1, 1300, 1, 64, 64, 128, 0.5, 11)
+
+
+@pytest.mark.parametrize("late", [256, -256], ids=["carry", "others"])
+def test_copies_do_not_overtake_what_reads_them(emu_lib, choose_backward, late):
+    """The waves that carry the state (the first four) come late out of every barrier, or all others do: nothing is copied, scored, weighed
+    or stored over what a wave of the same step still reads."""
+    emu_lib.emu_set_lag(late, 3000)
+    try:
+        test_pop_split_at_blocks(emu_lib, 1, 2304, 1, 64, 64, 64, 0.5, 36)   # five fp32 states in a row for half of the workgroups
+        test_folded_forward(emu_lib, 1, 6, 65, 16, 1, 64, 0.5)
+        choose_backward(PASSES)
+        test_pass_of_128_columns_per_workgroup(emu_lib, choose_backward, 5, 300, 1, 128, 0.5)
+    finally:
+        emu_lib.emu_set_lag(0, 0)
+
+
 @pytest.mark.parametrize("T,block", [(192, 64), (300, 64), (200, 40), (260, 130)])
 def test_pass_of_64_wide_rows_blocks(emu_lib, choose_backward, T, block):
     """Block states leave, and their gradients join, at every chunk and at some of them."""
