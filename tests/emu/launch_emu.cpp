@@ -156,12 +156,35 @@ extern "C" int emu_contrib_pays(int seqs, int T, int H, int dk, int dv, int comp
   return fpk::contrib_pays(seqs, T, H, dk, dv, compute_units);
 }
 
-// The rule that chooses the forward of a POP call with suffixes (the same on any device)
-extern "C" int emu_pop_folds(int B, int T, int H, int dk, int dv, int block, int Ls, int /*compute_units*/) {
-  fpk::PassArgs a = {};
-  a.B = B; a.T = T; a.H = H; a.dA = dk; a.dB = dv; a.block = block; a.nblk = T / block; a.Ls = Ls;
-  a.rs_a = dv; a.rs_n = 1;
-  return fpk::pop_folds(a);
+// The kernel (its number in dispatch_pass) that a launch of `passes` alike takes on a device of `compute_units`; block: with block
+// states, or with suffixes of Ls tokens
+namespace {
+struct Slot {
+  template <int DA, int MODE, int NH>
+  int go(int slot) const { return slot; }
+  template <int MODE>
+  int fill(int slot) const { return slot; }
+  int wide(int slot) const { return slot; }
+};
+}  // namespace
+extern "C" int emu_pass_kernel(int passes, int B, int T, int H, int dA, int dB, int block, int Ls, int reverse, int compute_units) {
+  alignas(16) static uint16_t some[8];
+  fpk::PassArgs a[fpk::MAX_PASSES_PER_LAUNCH] = {};
+  for (int i = 0; i < passes; ++i) {
+    a[i].X = a[i].W = a[i].Z = some;
+    a[i].Y = some;
+    a[i].B = B; a[i].T = T; a[i].H = H; a[i].dA = dA; a[i].dB = dB;
+    a[i].block = block; a[i].nblk = block > 0 ? T / block : 0; a[i].Ls = Ls; a[i].reverse = reverse;
+    a[i].rs_a = dB; a[i].rs_n = 1;
+    if (Ls > 0) {
+      a[i].Xs = a[i].Ws = a[i].Zs = some;
+      a[i].Ys = some;
+    } else if (block > 0) {
+      a[i].Bout = some;
+    }
+    if (fpk::plan_pass(a[i], compute_units)) return -1;
+  }
+  return fpk::dispatch_pass(a, passes, compute_units, Slot{});
 }
 
 // What every sequence (segment) adds to a zero state, U in fp32 halves, by the state-only kernel or (`walk`) by the pass kernel's

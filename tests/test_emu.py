@@ -32,6 +32,7 @@ def choose_backward(emu_lib):
 
 
 PASSES, FUSED, PACED = 1, 2, 3
+FOLD, WIDE = 22, 23   # two of the kernels' numbers in dispatch_pass
 
 
 def _check_all(pairs):
@@ -153,7 +154,7 @@ def test_fused_pop_fwd_bwd(emu_lib, B, nblk, block, Ls, H, dk, dv, state_std, ta
 ])
 def test_folded_forward(emu_lib, B, nblk, block, Ls, H, dv, state_std):
     """64-wide keys and short suffixes: taken as part of the chunks at their boundaries."""
-    assert emu_lib.emu_pop_folds(B, nblk * block, H, 64, dv, block, Ls, 8) == 1
+    assert emu_lib.emu_pass_kernel(1, B, nblk * block, H, 64, dv, block, Ls, 0, 8) == FOLD
     decays = oracle.head_decays(H, (4, 9))
     q, k, v, s = hp.make_inputs(B, nblk * block, H, 64, dv, seed=block + Ls, state_std=state_std)
     sfx = hp.make_suffix_inputs(B, nblk, Ls, H, 64, dv, seed=block + Ls + 1)
@@ -163,34 +164,45 @@ def test_folded_forward(emu_lib, B, nblk, block, Ls, H, dv, state_std):
     _check_all([("o", o, o_ref), ("o_sfx", o_sfx, os_ref), ("s_out", S, S_ref)])
 
 
-@pytest.mark.parametrize("folds,B,nblk,H,dk,dv,block,Ls", [
-    (1, 8, 32, 12, 64, 128, 64, 16),
-    (1, 8, 1, 12, 64, 128, 64, 16),       # a single block
-    (1, 8, 3, 12, 64, 128, 33, 16),
-    (1, 8, 4, 12, 64, 128, 64, 16),
-    (1, 8, 3, 12, 64, 256, 32, 16),
-    (1, 8, 2, 12, 64, 256, 1, 1),
-    (1, 8, 7, 8, 64, 128, 72, 3),         # two chunks a block
-    (1, 8, 8, 8, 64, 128, 96, 3),
-    (1, 8, 8, 8, 64, 256, 104, 3),
-    (1, 8, 64, 8, 64, 256, 105, 3),
-    (1, 4, 64, 8, 64, 64, 97, 3),
-    (1, 4, 4, 32, 64, 64, 64, 16),        # 64 x 64 states
-    (1, 129, 11, 1, 64, 64, 64, 16),      # ... where the bytes count
-    (1, 129, 12, 1, 64, 64, 64, 16),
-    (1, 17, 3, 8, 64, 64, 32, 16),
-    (1, 17, 4, 8, 64, 64, 32, 16),
-    (1, 17, 3, 8, 64, 64, 16, 16),
-    (1, 17, 11, 8, 64, 64, 80, 16),
-    (1, 17, 12, 8, 64, 64, 80, 16),
-    (0, 8, 32, 12, 128, 128, 64, 16),     # never: 128-wide keys, longer suffixes
-    (0, 8, 32, 12, 64, 128, 64, 17),
+@pytest.mark.parametrize("kernel,T,dk,dv,block,Ls", [
+    *[(FOLD, nblk * block, 64, dv, block, Ls) for dv in (64, 128, 256) for nblk, block, Ls in ((1, 1, 1), (1, 64, 16), (2, 105, 3), (64, 64, 16))],
+    (0, 2048, 64, 128, 64, 17),      # longer suffixes
+    (14, 2049, 64, 128, 64, 16),     # tokens after the last boundary
+    (5, 2048, 128, 128, 64, 16),     # 128-wide keys
 ])
-def test_rule_of_the_folded_forward(emu_lib, folds, B, nblk, H, dk, dv, block, Ls):
-    """Which POP calls with suffixes go to the folding kernel, at 256 units: those that it is faster at."""
-    assert emu_lib.emu_pop_folds(B, nblk * block, H, dk, dv, block, Ls, 256) == folds
-    if block > 1:
-        assert emu_lib.emu_pop_folds(B, nblk * block + 1, H, dk, dv, block, Ls, 256) == 0   # tokens after the last boundary
+def test_rule_of_the_folded_forward(emu_lib, kernel, T, dk, dv, block, Ls):
+    """Which POP calls with suffixes have them folded: those whose suffixes fit, whatever the number of blocks, streams and units.  Never
+    walking backward."""
+    for B, H, units in ((1, 1, 256), (8, 12, 256), (129, 1, 256), (1, 1, 8)):
+        assert emu_lib.emu_pass_kernel(1, B, T, H, dk, dv, block, Ls, 0, units) == kernel
+    assert emu_lib.emu_pass_kernel(1, 8, T, 12, dk, dv, block, Ls, 1, 256) == (0 if kernel == FOLD else kernel)
+
+
+@pytest.mark.parametrize("kernel,passes,B,T,H,dk,dv,block", [
+    (9, 1, 128, 2048, 1, 128, 128, 0),      # 128 columns per workgroup on half of the units: 64 columns each fit at once
+    (WIDE, 1, 129, 2048, 1, 128, 128, 0),
+    (9, 1, 4, 2048, 16, 128, 256, 0),
+    (WIDE, 1, 5, 1, 16, 128, 256, 0),       # any length while those of 128 columns fit
+    (9, 2, 64, 2048, 1, 128, 128, 0),       # two passes share a launch
+    (WIDE, 2, 65, 2048, 1, 128, 128, 0),
+    (WIDE, 3, 43, 2048, 1, 128, 128, 0),
+    (WIDE, 1, 256, 1, 1, 128, 128, 0),
+    (8, 1, 257, 383, 1, 128, 128, 0),       # more: sequences that are worth a workgroup
+    (WIDE, 1, 257, 384, 1, 128, 128, 0),
+    (8, 1, 129, 191, 1, 128, 256, 0),
+    (WIDE, 1, 129, 192, 1, 128, 256, 0),
+    (8, 1, 257, 4096, 1, 128, 192, 0),      # no whole number of 128 columns
+    (8, 1, 257, 4096, 1, 128, 64, 0),
+    (6, 1, 257, 4096, 1, 128, 128, 64),     # block states
+    (11, 1, 257, 4096, 1, 256, 128, 0),     # other keys
+    (1, 1, 257, 4096, 1, 64, 128, 64),
+    (3, 1, 129, 4096, 1, 64, 128, 0),
+    (4, 1, 128, 4096, 1, 64, 128, 0),
+])
+def test_rule_of_128_columns_per_workgroup(emu_lib, kernel, passes, B, T, H, dk, dv, block):
+    """Which passes run with 128 columns per workgroup, at 256 units, in either direction."""
+    for reverse in (0, 1):
+        assert emu_lib.emu_pass_kernel(passes, B, T, H, dk, dv, block, 0, reverse, 256) == kernel
 
 
 @pytest.mark.parametrize("B,T,H,dk,dv,state_std,segments", [
@@ -693,6 +705,7 @@ def test_pass_of_64_wide_rows_blocks(emu_lib, choose_backward, T, block):
 def test_pass_of_128_columns_per_workgroup(emu_lib, choose_backward, B, T, H, dv, state_std):
     """The pass with 128 columns per workgroup and half a chunk per step, in the roles that it has: forward and dv pass, with values of
     128 the dq and dk passes (which share a launch with it)."""
+    assert emu_lib.emu_pass_kernel(1, B, T, H, 128, dv, 0, 0, 0, 8) == WIDE
     choose_backward(PASSES)
     test_plain_fwd_bwd(emu_lib, B, T, H, 128, dv, state_std)
 

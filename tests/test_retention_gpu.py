@@ -503,6 +503,10 @@ def test_pass_of_64_wide_rows(hip_lib, B, T, H, dv, state_std):
 def test_pass_of_128_columns_per_workgroup(hip_lib, B, T, H, dv, state_std):
     """The pass with 128 columns per workgroup and half a chunk per step, in the forward and (by choice) in the gradient passes,
     around the number of halves that are under way at a time."""
+    # the lines of the rule that chooses it, which a CPU test holds the library to
+    segments = max(1, hip_lib.fp_retention_workspace_bytes(B, T, H, 128, dv) // (4 * B * H * 128 * dv))
+    workgroups, units = B * segments * H * dv // 128, torch.cuda.get_device_properties(0).multi_processor_count
+    assert 2 * workgroups > units and (workgroups <= units or T // segments * dv >= 384 * 128)
     for choice in (0, 1):
         assert hip_lib.fp_set_backward_choice(choice, -1) == 0
         try:
