@@ -37,7 +37,7 @@ __global__ __launch_bounds__(fpk::NTHREADS_WS) void retention_pass_multi_kernel(
 template <int MODE, bool REV>
 __global__ __launch_bounds__(fpk::FP_THREADS) void retention_pass_fill_kernel(const fpk::PassArgs args) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  fpk::retention_pass_fill_dir<MODE, REV>(args, fpk::tensors_of(args), lds, fpk::place_workgroup(fprt::block_index(), fprt::grid_size(), 1).wg);
+  fpk::retention_pass_fill_dir<MODE, REV, true>(args, fpk::tensors_of(args), lds, fpk::place_workgroup(fprt::block_index(), fprt::grid_size(), 1).wg);
 }
 template <int MODE>
 __global__ __launch_bounds__(fpk::FP_THREADS) void retention_pass_fill_multi_kernel(const fpk::PassArgs first, const fpk::PassTensors second,
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(fpk::FP_THREADS) void retention_pass_fill_multi_ker
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const fpk::WorkgroupId id = fpk::place_workgroup(fprt::block_index(), fprt::grid_size() / passes, passes);
   const fpk::PassTensors io = id.pass == 0 ? fpk::tensors_of(first) : id.pass == 1 ? second : third;
-  fpk::retention_pass_fill<MODE>(first, io, lds, id.wg);
+  fpk::retention_pass_fill<MODE, false>(first, io, lds, id.wg);
 }
 
 // The same for dA = 128 with 128 columns per workgroup

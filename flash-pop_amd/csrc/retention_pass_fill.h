@@ -148,14 +148,20 @@ struct ChunkWalk {
 
 }  // namespace pp
 
-// Whether the rows are copied with the cache hint: what a launch moves does not fit the caches, so that it serves nobody there.
-// B64 T2048 H4 64 x 64 (268 MB): 57.0 -> 53.6 us; below, the next launch finds some of it (the backward behind the forward of
-// B32 T2048 H4 64 x 64: 60 us, 65 with the hint in the forward).
+// Whether a pass moves more than the caches hold; rows of such a one that nobody reads again are copied with the cache hint (below, the
+// next launch finds some of them: the backward behind the forward of B32 T2048 H4 64 x 64, 134 MB, 60 us, 65 with the hint in the
+// forward).  Forward alone, and forward and backward of a training step, cold inputs, us: this rule; no hint at all; the hint on every row
+// of every launch:
+//   64 x 64    B64 T2048 H4     53.4, 170.7     56.2, 174.4     53.3, 181.1
+//              B64 T4096 H4     101.8, 344.7    108.3, 352.5    102.2, 365.5
+//   64 x 128   B16 T2048 H12    67.4, 223.2     70.7, 227.3     77.7, 235.2
+//              B32 T2048 H12    123.9, 419.4    141.1, 425.2    161.2, 429.2
+//   64 x 256   B16 T2048 H8     71.3, 259.0     77.3, 263.1     74.7, 266.6
 FP_DEVICE bool passes_caches(const PassArgs& p) { return (size_t)p.B * p.T * p.H * (p.dA + p.dB) * 4 > (200u << 20); }
 
 // Workgroup number `wg` of a pass; `io`: the tensors, walking direction and scales of this pass (a launch may hold several,
-// everything else in `p` is common to them).
-template <int MODE, bool REV>
+// everything else in `p` is common to them).  ALONE: the launch holds this pass only.
+template <int MODE, bool REV, bool ALONE>
 FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io, char* lds, int wg) {
   using namespace pp;
   using TT = FillTile;
@@ -201,27 +207,29 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
     // ================================= move waves =================================
     const int fw = wave & 3;
     // Copy u of this wave: rows ROWS (fw + 4 u) .. of a tile, whose keys do not depend on u
-    const int ra = TT::ROWS * fw + lane / TT::PPR, rb = TT::ROWS * fw + lane / TT::PPR;
-    const uint32_t offA = (uint32_t)ra * rowA + (uint32_t)((lane % TT::PPR) ^ TT::key(ra)) * 16;
-    const uint32_t offB = (uint32_t)rb * rowB + (uint32_t)((lane % TT::PPR) ^ TT::key(rb)) * 16;
+    const int row0 = TT::ROWS * fw + lane / TT::PPR, piece = (lane % TT::PPR) ^ TT::key(row0);
+    const uint32_t offA = (uint32_t)row0 * rowA + (uint32_t)piece * 16, offB = (uint32_t)row0 * rowB + (uint32_t)piece * 16;
     const fprt::LdsAddress lds0 = fprt::lds_address(lds);
     const char* const Xg = reinterpret_cast<const char*>(io.X) + headA;
     const char* const Wg = reinterpret_cast<const char*>(io.W) + headA;
     const char* const Zg = reinterpret_cast<const char*>(io.Z) + headB;
-    const bool once = passes_caches(p);
+    // X and W with the hint only where no other column tile reads them, nothing where several passes of a launch read the same rows.  A
+    // forward that leaves block states (checkpoints) has a backward behind it, which starts where it ended and reads q once but k and v twice:
+    // there X alone.
+    const bool once = ALONE && passes_caches(p), x_once = once && ntile == 1, w_once = x_once && !BLOCKS, z_once = once && !BLOCKS;
     // this wave's part of 64 rows into a tile at `to`
-    auto fill = [&](const fprt::FillView& v, uint32_t off, uint32_t pitch, int to) {
+    auto fill = [&](const fprt::FillView& v, uint32_t off, uint32_t pitch, int to, bool hint) {
       const fprt::LdsAddress dst = lds0 + (to + 1024 * fw);
       const uint32_t offs[TT::PER_WAVE] = {off, off + 4 * TT::ROWS * pitch};
-      if (once) fprt::fill_lds<true, 4096>(v, offs, dst);
+      if (hint) fprt::fill_lds<true, 4096>(v, offs, dst);
       else fprt::fill_lds<false, 4096>(v, offs, dst);
     };
     auto copy_w = [&](const Chunk& k, int sx) {
-      fill(fprt::make_fill(Wg + (size_t)k.row * rowA, k.L > 0 ? (uint32_t)(k.L - 1) * rowA + DA * 2 : 0u), offA, rowA, W0 + sx);
+      fill(fprt::make_fill(Wg + (size_t)k.row * rowA, k.L > 0 ? (uint32_t)(k.L - 1) * rowA + DA * 2 : 0u), offA, rowA, W0 + sx, w_once);
     };
     auto copy_xz = [&](const Chunk& k, int sx, int sz) {
-      fill(fprt::make_fill(Xg + (size_t)k.row * rowA, k.L > 0 ? (uint32_t)(k.L - 1) * rowA + DA * 2 : 0u), offA, rowA, X0 + sx);
-      fill(fprt::make_fill(Zg + (size_t)k.row * rowB, k.L > 0 ? (uint32_t)(k.L - 1) * rowB + BV * 2 : 0u), offB, rowB, Z0 + sz);
+      fill(fprt::make_fill(Xg + (size_t)k.row * rowA, k.L > 0 ? (uint32_t)(k.L - 1) * rowA + DA * 2 : 0u), offA, rowA, X0 + sx, x_once);
+      fill(fprt::make_fill(Zg + (size_t)k.row * rowB, k.L > 0 ? (uint32_t)(k.L - 1) * rowB + BV * 2 : 0u), offB, rowB, Z0 + sz, z_once);
     };
     // FOLD: the 16 rows of a tensor are two copies, of X by wave 0, of W by wave 1 and of Z by the other two (as many each)
     auto copy_suffix = [&](const Chunk& k, int sx, int sz) {
@@ -249,8 +257,8 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
     auto copy_tile = [&](const uint16_t* m, int to) {
       const fprt::FillView v = fprt::make_fill(reinterpret_cast<const char*>(m) + (tposed ? (size_t)tile * BV * rowR : (size_t)tile * BV * 2), 63 * rowR + 128);
       const int l = fprt::opaque(lane);
-      const uint32_t off = (uint32_t)(TT::ROWS * fw + l / TT::PPR) * rowR + (uint32_t)((l % TT::PPR) ^ TT::key(rb)) * 16;
-      fill(v, off, rowR, to);
+      const uint32_t off = (uint32_t)(TT::ROWS * fw + l / TT::PPR) * rowR + (uint32_t)((l % TT::PPR) ^ TT::key(row0)) * 16;
+      fill(v, off, rowR, to, false);
     };
     int states = 0;   // asked for so far
     auto copy_initial = [&](int b) {
@@ -644,12 +652,12 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
   }
 }
 
-template <int MODE>
+template <int MODE, bool ALONE>
 FP_DEVICE void retention_pass_fill(const PassArgs& p, const PassTensors& io, char* lds, int wg) {
   if constexpr (MODE != FILL_FOLD) {
-    if (io.reverse) return retention_pass_fill_dir<MODE, true>(p, io, lds, wg);
+    if (io.reverse) return retention_pass_fill_dir<MODE, true, ALONE>(p, io, lds, wg);
   }
-  retention_pass_fill_dir<MODE, false>(p, io, lds, wg);
+  retention_pass_fill_dir<MODE, false, ALONE>(p, io, lds, wg);
 }
 
 // Whether a planned pass is a walk with folded suffixes: a forward whose suffixes fit beside a chunk, whole blocks.  The suffix walk of

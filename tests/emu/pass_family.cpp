@@ -52,7 +52,8 @@ struct FamilyRun {
       const int passes = n;
       return run_grid(fpk::FP_THREADS, passes * nwg, fpk::fp_lds_bytes(), [&](char* l) {
         const fpk::WorkgroupId id = fpk::place_workgroup(fprt::block_index(), nwg, passes);
-        fpk::retention_pass_fill<MODE>(a, fpk::tensors_of(p[id.pass]), l, id.wg);
+        if (passes == 1) fpk::retention_pass_fill<MODE, true>(a, fpk::tensors_of(p[id.pass]), l, id.wg);
+        else fpk::retention_pass_fill<MODE, false>(a, fpk::tensors_of(p[id.pass]), l, id.wg);
       });
     } else {
       return 1;
