@@ -156,6 +156,14 @@ extern "C" int emu_contrib_pays(int seqs, int T, int H, int dk, int dv, int comp
   return fpk::contrib_pays(seqs, T, H, dk, dv, compute_units);
 }
 
+// The rule that chooses the forward of a POP call with suffixes (the same on any device)
+extern "C" int emu_pop_folds(int B, int T, int H, int dk, int dv, int block, int Ls, int /*compute_units*/) {
+  fpk::PassArgs a = {};
+  a.B = B; a.T = T; a.H = H; a.dA = dk; a.dB = dv; a.block = block; a.nblk = T / block; a.Ls = Ls;
+  a.rs_a = dv; a.rs_n = 1;
+  return fpk::pop_folds(a);
+}
+
 // The kernel (its number in dispatch_pass) that a launch of `passes` alike takes on a device of `compute_units`; block: with block
 // states, or with suffixes of Ls tokens
 namespace {

@@ -154,6 +154,7 @@ def test_fused_pop_fwd_bwd(emu_lib, B, nblk, block, Ls, H, dk, dv, state_std, ta
 ])
 def test_folded_forward(emu_lib, B, nblk, block, Ls, H, dv, state_std):
     """64-wide keys and short suffixes: taken as part of the chunks at their boundaries."""
+    assert emu_lib.emu_pop_folds(B, nblk * block, H, 64, dv, block, Ls, 8) == 1
     assert emu_lib.emu_pass_kernel(1, B, nblk * block, H, 64, dv, block, Ls, 0, 8) == FOLD
     decays = oracle.head_decays(H, (4, 9))
     q, k, v, s = hp.make_inputs(B, nblk * block, H, 64, dv, seed=block + Ls, state_std=state_std)
@@ -164,13 +165,43 @@ def test_folded_forward(emu_lib, B, nblk, block, Ls, H, dv, state_std):
     _check_all([("o", o, o_ref), ("o_sfx", o_sfx, os_ref), ("s_out", S, S_ref)])
 
 
+@pytest.mark.parametrize("folds,B,nblk,H,dk,dv,block,Ls", [
+    (1, 8, 32, 12, 64, 128, 64, 16),
+    (1, 8, 1, 12, 64, 128, 64, 16),       # a single block
+    (1, 8, 3, 12, 64, 128, 33, 16),
+    (1, 8, 4, 12, 64, 128, 64, 16),
+    (1, 8, 3, 12, 64, 256, 32, 16),
+    (1, 8, 2, 12, 64, 256, 1, 1),
+    (1, 8, 7, 8, 64, 128, 72, 3),         # two chunks a block
+    (1, 8, 8, 8, 64, 128, 96, 3),
+    (1, 8, 8, 8, 64, 256, 104, 3),
+    (1, 8, 64, 8, 64, 256, 105, 3),
+    (1, 4, 64, 8, 64, 64, 97, 3),
+    (1, 4, 4, 32, 64, 64, 64, 16),        # 64 x 64 states
+    (1, 129, 11, 1, 64, 64, 64, 16),      # ... where the bytes count
+    (1, 129, 12, 1, 64, 64, 64, 16),
+    (1, 17, 3, 8, 64, 64, 32, 16),
+    (1, 17, 4, 8, 64, 64, 32, 16),
+    (1, 17, 3, 8, 64, 64, 16, 16),
+    (1, 17, 11, 8, 64, 64, 80, 16),
+    (1, 17, 12, 8, 64, 64, 80, 16),
+    (0, 8, 32, 12, 128, 128, 64, 16),     # never: 128-wide keys, longer suffixes
+    (0, 8, 32, 12, 64, 128, 64, 17),
+])
+def test_rule_of_the_folded_forward(emu_lib, folds, B, nblk, H, dk, dv, block, Ls):
+    """Which POP calls with suffixes go to the folding kernel, at 256 units: those that it is faster at."""
+    assert emu_lib.emu_pop_folds(B, nblk * block, H, dk, dv, block, Ls, 256) == folds
+    if block > 1:
+        assert emu_lib.emu_pop_folds(B, nblk * block + 1, H, dk, dv, block, Ls, 256) == 0   # tokens after the last boundary
+
+
 @pytest.mark.parametrize("kernel,T,dk,dv,block,Ls", [
     *[(FOLD, nblk * block, 64, dv, block, Ls) for dv in (64, 128, 256) for nblk, block, Ls in ((1, 1, 1), (1, 64, 16), (2, 105, 3), (64, 64, 16))],
     (0, 2048, 64, 128, 64, 17),      # longer suffixes
     (14, 2049, 64, 128, 64, 16),     # tokens after the last boundary
     (5, 2048, 128, 128, 64, 16),     # 128-wide keys
 ])
-def test_rule_of_the_folded_forward(emu_lib, kernel, T, dk, dv, block, Ls):
+def test_kernel_of_a_forward_with_suffixes(emu_lib, kernel, T, dk, dv, block, Ls):
     """Which POP calls with suffixes have them folded: those whose suffixes fit, whatever the number of blocks, streams and units.  Never
     walking backward."""
     for B, H, units in ((1, 1, 256), (8, 12, 256), (129, 1, 256), (1, 1, 8)):

@@ -17,4 +17,16 @@ def test_all_entry_points_under_asan_and_ubsan(tmp_path):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=0", UBSAN_OPTIONS="print_stacktrace=1")
     res = subprocess.run([exe], capture_output=True, text=True, env=env, timeout=1500)
     assert res.returncode == 0, res.stdout[-3000:] + res.stderr[-6000:]
-    assert res.stdout.count("ok ") == 55 and "FAILED" not in res.stdout, res.stdout
+    assert res.stdout.count("ok ") == 50 and "FAILED" not in res.stdout, res.stdout
+
+
+def test_128_columns_per_workgroup_under_asan_and_ubsan(tmp_path):
+    """Ragged halves, both directions and a cut call in the kernel with 128 columns per workgroup."""
+    exe = str(tmp_path / "asan_driver")
+    build_env = dict(os.environ, EMU_OUT=exe, EMU_MAIN=os.path.join(EMU, "asan_driver.cpp"), EMU_OPT="-O1",
+                     EMU_FLAGS="-fsanitize=address,undefined -fno-sanitize-recover=all -fno-omit-frame-pointer")
+    subprocess.run([os.path.join(EMU, "build_emu.sh")], check=True, env=build_env)
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=0", UBSAN_OPTIONS="print_stacktrace=1")
+    res = subprocess.run([exe, "wide"], capture_output=True, text=True, env=env, timeout=1500)
+    assert res.returncode == 0, res.stdout[-3000:] + res.stderr[-6000:]
+    assert res.stdout.count("ok ") == 5 and "FAILED" not in res.stdout, res.stdout
