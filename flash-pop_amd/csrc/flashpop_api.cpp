@@ -424,21 +424,23 @@ int plan_segments(const Shape& s) {
   return even > 1 && 4 * (chunks / even) * fpk::CH <= 5 * tokens ? even : segment_count(s, tokens);
 }
 // Whether n segments shorten the chain of chunk steps by what the cut costs: its extra launches, and the segment states
-// that it moves.  Forward, measured at 1.1 us (64-wide keys) to 1.4 us (128) a step on the 256-unit device, uncut -> cut:
-//   64 x 64    H4 B1        18 chunks 23.8 -> 19.9 us, 16 chunks 21.8 -> 18.5,  13 chunks 18.4 -> 19.7
-//   64 x 128   H12 B1       79 chunks 89.6 -> 32.8,    18 chunks 24.4 -> 20.9,  13 chunks 18.9 -> 20.6
-//   128 x 128  H8 B3        28 chunks 44.0 -> 30.7,    18 chunks 30.0 -> 29.3,  13 chunks 23.5 -> 28.7
-//   128 x 256  H8 B2        40 chunks 60.0 -> 38.6,    28 chunks 43.9 -> 33.8,  18 chunks 30.0 -> 38.3
+// that it moves.  Forward on the 256-unit device, launches in a row, a step there 0.72 us (64-wide keys) or 1.4 (128), uncut -> cut, *: the
+// line cuts it:
+//   64 x 64    H4 B1     13 chunks 12.9 -> 16.2 us   16 chunks 15.3 -> 15.2   18 chunks 16.6 -> 16.5*  28 chunks 23.8 -> 15.4*
+//   64 x 64    H12 B6    28 chunks 24.6 -> 27.6      40 chunks 33.3 -> 33.6*  79 chunks 61.9 -> 53.6*
+//   64 x 128   H12 B1    13 chunks 13.2 -> 17.7      18 chunks 17.0 -> 18.1   28 chunks 24.2 -> 17.3*  79 chunks 61.8 -> 29.2*
+//   128 x 128  H8 B3     13 chunks 22.3 -> 25.5      18 chunks 29.1 -> 26.5   28 chunks 43.0 -> 29.1*
+//   128 x 256  H8 B2     13 chunks 22.3 -> 27.4      18 chunks 29.2 -> 27.9   28 chunks 43.0 -> 26.9   40 chunks 59.8 -> 31.4*
 // Backward (the uncut passes share launches, or are the fused kernel with its longer step; the cut has four launches and the
 // forward's states):
-//   64 x 64    H4 B1        28 chunks 35.3 -> 27.8,    18 chunks 24.8 -> 28.7
-//   64 x 64    H12 B6       79 chunks 132 -> 133,      40 chunks 69.8 -> 79.5,  28 chunks 50.5 -> 63.6 (fused)
-//   64 x 128   H12 B1       18 chunks 54.3 -> 41.9,    13 chunks 41.4 -> 40.9
-//   128 x 128  H16 B1       79 chunks 116 -> 82,       40 chunks 61.8 -> 50.8,  28 chunks 45.1 -> 44.6
-//   128 x 256  H8 B2        28 chunks 119 -> 68,       18 chunks 80.0 -> 70.9,  13 chunks 60.8 -> 61.8
-// The line dates from slower state-only passes, scans and fused backwards: it leaves calls of 16 to 18 chunks uncut that a cut
-// would shorten (128 x 256 up to 28), and cuts the backward of 64 x 64 on 72 streams from 40 chunks on.  (Measured before the
-// state-only passes got another 0.3 to 0.8 us shorter.)
+//   64 x 64    H4 B1     18 chunks 16.6 -> 24.2      28 chunks 23.8 -> 22.5*  40 chunks 32.5 -> 22.8*
+//   64 x 64    H12 B6    28 chunks 50.2 -> 51.2      40 chunks 69.7 -> 64.5*  79 chunks 133 -> 106* (uncut: fused)
+//   64 x 128   H12 B1    13 chunks 35.0 -> 37.8      18 chunks 45.8 -> 38.4   28 chunks 67.6 -> 36.2*  79 chunks 178 -> 54.2*
+//   128 x 128  H16 B1    18 chunks 29.3 -> 36.6      28 chunks 43.2 -> 35.3   40 chunks 60.2 -> 41.0*  79 chunks 116 -> 65.2*
+//   128 x 256  H8 B2     13 chunks 58.5 -> 57.0      18 chunks 78.0 -> 59.0   28 chunks 117 -> 58.9    40 chunks 165 -> 70.2*
+// The line is that of slower kernels on both sides.  Of these rows none that it cuts is slower for it by more than 1 %; what it leaves uncut would be
+// shorter cut from 18 chunks of 128-wide keys on in the forward (128 x 256, 28 chunks: by 16 us), from 28 (128 x 128), 18 (64 x 128) and 18
+// (128 x 256: by up to 58 us) in the backward.
 // `block`: a POP call, whose chunks end at its blocks and whose gradient passes share fewer launches (64 x 128, B4 H4 T1440
 // in blocks of 144, 30 chunks, with the suffix call and the launches between the two: 200 -> 166 us).
 bool cut_pays(const Shape& s, int n, int tokens, bool backward, int block = 0) {
@@ -467,13 +469,15 @@ int plan_backward(const Shape& s) {
 
 // Whether the bytes that a POP call cut at its blocks moves are worth the chain they replace: q, k, v, o, k and v a second time,
 // and per element of a block's state 18 bytes (fp32 written, read and written by the scan, read; bf16 out), where the uncut call
-// moves 2.  There are as many states as blocks, however many fill the chip, and the cut call streams them at 3.5 to 4.5 TB/s
-// while the uncut one walks, 1.4 to 2 us a chunk: 6.8 MB a step tell the two apart (three steps: the launches).  Uncut -> cut,
-// forward / backward, us:
-//   128 x 128  blocks of 64    B10 H4 T4096   131 -> 227 / 226 -> 355      B4 H4 T4096   130 -> 97 / 226 -> 148
-//   128 x 128  blocks of 144   B10 H4 T16384  589 -> 595 / 926 -> 1014     B4 H8 T4096   145 -> 119 / 237 -> 217
-//   64 x 128   blocks of 64    B6 H8 T4096     98 -> 144 / 193 -> 258      B6 H4 T2048    52 -> 52 / 163 -> 81
-//   64 x 64    blocks of 64    B10 H8 T4096    98 -> 123 / 160 -> 236      B6 H8 T16384  444 -> 432 / 665 -> 667
+// moves 2.  There are as many states as blocks, however many fill the chip, and the cut call streams them at 3.5 to 4.8 TB/s
+// while the uncut one walks, 1.2 to 1.3 us a chunk with 64-wide keys, 1.9 to 2.2 with 128: 6.8 MB a step tell the two apart (three steps:
+// the launches).  Uncut -> cut, forward / backward, us, launches in a row, *: the line cuts it:
+//   128 x 128  blocks of 64    B10 H4 T4096   130 -> 211 / 227 -> 332      B4 H4 T4096   130 -> 115* / 226 -> 154*
+//   128 x 128  blocks of 144   B10 H4 T16384  597 -> 559 / 933 -> 973      B4 H8 T4096   146 -> 117* / 238 -> 205*
+//   64 x 128   blocks of 64    B6 H8 T4096     80 -> 126 / 192 -> 245      B6 H4 T2048    42 -> 49* / 155 -> 83*
+//   64 x 64    blocks of 64    B10 H8 T4096    80 -> 116 / 158 -> 222      B6 H8 T16384  334 -> 382* / 541 -> 578*
+// The line is from when a chunk of 64-wide keys took 1.5 to 1.7 us: it now cuts some of those calls that walk as fast or faster (the
+// last two rows' right).
 bool block_states_pay(const Shape& s, int segments, int block) {
   if (fpk_launch_steps() <= 0) return true;   // (a device whose launches cost nothing)
   const double chunks = (double)segments * ((block + fpk::CH - 1) / fpk::CH);

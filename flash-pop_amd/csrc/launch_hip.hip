@@ -230,7 +230,8 @@ int fpk_stream_is_capturing(void* stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-// About 5 us (dispatch, ramp-up, first loads, the last workgroup's drain) against 1.1 to 1.4 us for a step.
+// About 5 us (dispatch, ramp-up, first loads, the last workgroup's drain) against 1.4 us for a step of 128-wide keys.  (Of 64-wide ones, 0.72
+// us, it is seven; the lines that count with it were drawn when a step of those took 1.1 us.)
 int fpk_launch_steps() { return 4; }
 
 // Compute units of the current device (cached per thread and device).

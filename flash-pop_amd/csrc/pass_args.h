@@ -130,15 +130,16 @@ struct ContribArgs {
 inline bool contrib_fits(long long T, int H, int dk, int dB) { return (T + CH) * H * (dk > dB ? dk : dB) * 2 < (1LL << 32); }
 // Whether that pass is the faster form of a state-only pass over `seqs` sequences, else it is the pass kernel's state-only walk, 64
 // columns of a state per workgroup of 512 threads, which go from sequence to sequence with the next one's rows on their way.
-// 128 x 128 of a state per workgroup: always (B16 T2048 H8 128 x 256: 44 us against 67; the least, B12 T448 H8, 12.0 against 11.0).
+// 128 x 128 of a state per workgroup: always (B16 T2048 H8 128 x 256: 43 us against 66; the least, B12 T448 H8, 11.1 against 11.3).
 // 64 x 64, with the same bits as the walk: but for many workgroups of short sequences.  Speed over the walk's at 256 units, inputs
-// not in a cache up to 768 workgroups, 64 x 64 / 64 x 128:
+// not in a cache, launches in a row, 64 x 64 / 64 x 128:
 //                   64 wg          160            256            320            768            1024           1296           2048           4096
-//   1 chunk         1.04 / 1.03    1.00 / 1.01    .98 / 1.00     1.10 / 1.09    .97 / .99      .90 / .96      .92 / .92      .85 / .85      .85 / .81
-//   2               1.08 / 1.07    1.05 / 1.04    1.01 / 1.03    1.13 / 1.16    .98 / 1.01     .92 / .99      1.01 / 1.07    .91 / .94      .91 / .95
-//   4               1.11 / 1.11    1.10 / 1.10    1.06 / 1.07    1.27 / 1.31    1.03 / 1.12    .96 / 1.00     1.11 / 1.15    .98 / 1.05     .95 / 1.05
-//   6               1.16 / 1.17    1.13 / 1.15    1.09 / 1.12    1.29 / 1.41    1.04 / 1.16    1.03 / 1.07    1.12 / 1.18    1.04 / 1.11    1.00 / 1.10
-//   12              1.25 / 1.25    1.17 / 1.21    1.16 / 1.18    1.42 / 1.57    1.11 / 1.23    1.07 / 1.14    1.18 / 1.29    1.08 / 1.18    1.05 / 1.00
+//   1 chunk         1.11 / 1.08    1.09 / 1.09    1.11 / 1.13    1.26 / 1.25    1.24 / 1.26    1.03 / 1.06    1.10 / 1.12    1.02 / 1.05    .96 / .99
+//   2               1.16 / 1.17    1.12 / 1.14    1.14 / 1.17    1.29 / 1.33    1.24 / 1.31    1.09 / 1.17    1.18 / 1.28    1.05 / 1.14    1.06 / 1.10
+//   4               1.18 / 1.14    1.14 / 1.15    1.15 / 1.16    1.39 / 1.42    1.24 / 1.35    1.14 / 1.20    1.21 / 1.29    1.15 / 1.23    1.12 / 1.22
+//   6               1.21 / 1.20    1.16 / 1.19    1.21 / 1.20    1.49 / 1.55    1.27 / 1.37    1.18 / 1.26    1.28 / 1.35    1.22 / 1.30    1.16 / 1.28
+//   12              1.29 / 1.28    1.19 / 1.23    1.32 / 1.29    1.50 / 1.71    1.27 / 1.42    1.19 / 1.30    1.30 / 1.43    1.21 / 1.32    1.17 / 1.11
+// (The line is from before its sums left in whole lines, when short sequences lost from 768 workgroups on, down to .81.)
 // 128 x 64 has no form of its own: one lost to the walk from 512 workgroups on (.75 to .93 times its speed).
 inline bool contrib_pays(long long seqs, int T, int H, int dk, int dB, int compute_units) {
   if (dk != 64) return dk == 128 && dB % 128 == 0;

@@ -14,8 +14,8 @@
 // 64 rows: 64 columns per workgroup of 256 threads (37 KB of LDS: several share a compute unit), bit for bit what the pass
 // kernel's state-only walk gives, which takes all other states and many short sequences of these (contrib_pays):
 // chunks are cut from where the walk starts, so that walking backward the short one is the first of the sequence, every weight is
-// a power of gamma of its own, and the tokens are summed in order (ContribTile::AS_WALK).  64 x 128, B20 T256 H12 11.1 us in the
-// walk, 9.4 here; B40 T144 H4 9.1, 7.3.  128 columns of a 64-row state per workgroup were slower.
+// a power of gamma of its own, and the tokens are summed in order (ContribTile::AS_WALK).  64 x 128, B20 T256 H12 11.5 us in the
+// walk, 8.8 here; B40 T128 H4 8.0, 6.2.  128 columns of a 64-row state per workgroup were slower.
 //
 // 128 rows: 128 columns per workgroup of 512 threads; chunks from the first token on in both directions, weights of a k-step
 // from those of the one before.
