@@ -604,21 +604,21 @@ FP_DEVICE void retention_pass_fill_dir(const PassArgs& p, const PassTensors& io,
     if (REV && L != CH) wread = io.s_read * fprt::exp2_approx((float)(i_row < L ? L - 1 - i_row : 0) * lg);
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] *= wread;
+    // In the order of retention_pass_ws.h, whose waves begin with the tile that they made themselves, those of the odd column blocks the other
+    // one: a call's o has the same bits whichever of the two kernels takes it
+    auto other_tile = [&]() {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) acc = fprt::mfma_32x32x16_bf16(z[REV ? 2 + k : k], pj[k], acc);   // (seen by the row block that walks later)
+    };
+    if (other && ns == 1) other_tile();
     if (ih == 0) {
 #pragma unroll
       for (int k = 0; k < 2; ++k) acc = fprt::mfma_32x32x16_bf16(z[k], pi[k], acc);
-      if (other) {
-#pragma unroll
-        for (int k = 0; k < 2; ++k) acc = fprt::mfma_32x32x16_bf16(z[2 + k], pj[k], acc);
-      }
     } else {
 #pragma unroll
       for (int k = 0; k < 2; ++k) acc = fprt::mfma_32x32x16_bf16(z[2 + k], pi[k], acc);
-      if (other) {
-#pragma unroll
-        for (int k = 0; k < 2; ++k) acc = fprt::mfma_32x32x16_bf16(z[k], pj[k], acc);
-      }
     }
+    if (other && ns == 0) other_tile();
     float gL = gL_full;
     if (L != CH) gL = fprt::exp2_approx((float)L * lg);
 #pragma unroll

@@ -803,3 +803,28 @@ def test_tensors_that_are_not_aligned(emu_lib, choose_backward, which, B, T, dk,
     assert emu_lib.emu_misaligned_fills() == 0
     for i, (g, r) in enumerate(zip(got, ref)):
         hp.assert_close(g, r, f"output {i}")
+
+
+@pytest.mark.parametrize("B,T,dk,dv,block", [
+    (1, 200, 64, 64, 0), (2, 130, 64, 128, 0),    # one sequence per workgroup
+    (20, 64, 64, 64, 0), (9, 100, 64, 128, 0),    # several
+    (1, 200, 64, 128, 64), (2, 130, 64, 64, 50),  # block states
+    (6, 200, 128, 128, 0), (3, 130, 128, 256, 0),  # 128 columns per workgroup: outputs and states (its walk backward adds half chunks in turn)
+])
+def test_outputs_do_not_depend_on_alignment(emu_lib, choose_backward, B, T, dk, dv, block):
+    """Aligned tensors are copied straight into LDS, others go through registers in another kernel, which a rule may choose for aligned ones,
+    too: outputs, states and gradients are the same bit for bit."""
+    choose_backward(PASSES)
+    decays = oracle.head_decays(1, (4, 9))
+    q, k, v, s = hp.make_inputs(B, T, 1, dk, dv, seed=T + B, state_std=0.5)
+    d_o, d_s = hp.make_cotangents([(B, T, 1, dv), (B, T // block, 1, dk, dv) if block else (B, 1, dk, dv)], seed=T)
+
+    def outputs(move):
+        q_, k_, v_, s_, do_, ds_ = (move(t) for t in (q, k, v, s, d_o, d_s))
+        if block:
+            return hp.raw_pop_fwd(emu_lib, q_, k_, v_, s_, decays, block) + hp.raw_pop_bwd(emu_lib, q_, k_, v_, s_, decays, block, do_, ds_)
+        forward = hp.raw_fwd(emu_lib, q_, k_, v_, s_, decays)
+        return forward if dk == 128 else forward + hp.raw_bwd(emu_lib, q_, k_, v_, s_, decays, do_, ds_)
+
+    for i, (a, b) in enumerate(zip(outputs(lambda t: t), outputs(_shifted))):
+        assert torch.equal(a, b), f"output {i}: {(a != b).sum().item()} elements differ"
