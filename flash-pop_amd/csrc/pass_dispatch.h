@@ -106,6 +106,21 @@ inline bool copies_aligned(const PassArgs& a) {
   return at % 16 == 0;
 }
 
+// Whether a pass of 64-wide keys over several sequences per workgroup, each of at most one chunk, takes the pass kernel's walk, whose rows go
+// through registers: with one step a sequence, a step here (rows, a state in, a state out) is longer than there.  Speed of that walk over
+// the kernel of retention_pass_fill.h, 256 units, by workgroups of 64 columns (sequences x heads x column tiles); inputs not in a cache /
+// written by the launches right before:
+//                     288            512            768            1024           1536           2048           4096
+//   64 x 64   T40     1.06 / .95     1.06 / .97    1.06 / 1.20     1.05 / 1.16    1.01 / 1.08    .98            .92
+//             T64     1.08 / 1.00    1.10 / 1.05   1.11 / 1.22     1.07 / 1.16    1.01 / 1.06    .98            .95
+//   64 x 128  T64     1.07 / 1.01    1.05 / 1.09   1.03 / 1.18     1.01 / 1.18    .96 / 1.05     .95            .88
+//   64 x 256  T64     1.05 / 1.01    1.06 / 1.01   1.04 / 1.15     1.02 / 1.12    .99 / 1.07     .93            .87
+// Two chunks: .99 to 1.03 / 1.04 to 1.07 (64 x 64, 384 and 512), less beyond and with wider values.  Several passes in a launch (the backward's): .93
+// to .98.
+inline bool pass_is_short(const PassArgs& a, int passes, int compute_units) {
+  return passes == 1 && a.T <= CH && (long long)a.B * a.H * (a.dB / BV) <= 6LL * compute_units;
+}
+
 // Calls run.template go<DA, MODE, NH>(slot), run.template fill<MODE>(slot) for the kernel of retention_pass_fill.h or run.wide(slot) for
 // that of retention_pass_wide.h, for the instantiation that a launch of the `n` planned passes needs; `slot` numbers the
 // instantiations 0 .. PASS_KERNELS - 1.
@@ -129,6 +144,7 @@ int dispatch_pass(const PassArgs* planned, int n, int compute_units, Run&& run) 
       return run.template go<64, WALK_PLAIN, 1>(26);
     }
     if (blocks) return run.template fill<FILL_BLOCKS>(1);
+    if (multi && pass_is_short(a, n, compute_units)) return run.template go<64, WALK_MULTI, 1>(25);
     if (multi) return run.template fill<FILL_MULTI>(3);
     return run.template fill<FILL_PLAIN>(4);
   }

@@ -1,6 +1,6 @@
 // Wave-specialised retention pass (see pass_args.h for the recurrence): dA = 64 or 128 per visit,
 // dA = 256 in two visits per chunk, dA = 192 in three (NH below).  (dA = 64 itself: state-only walks, those with suffixes that do not
-// fold, tensors that are not 16-byte aligned; its other walks: retention_pass_fill.h.  dA = 128 with columns enough: retention_pass_wide.h.)
+// fold, tensors that are not 16-byte aligned, many sequences of one chunk; its other walks: retention_pass_fill.h.  dA = 128 with columns enough: retention_pass_wide.h.)
 //
 // One workgroup of 8 wave64 owns one (batch, head) stream and one 64-column slice of
 // Z / Y / R.  Hardware places waves w and w + 4 on the same SIMD, so every SIMD runs one

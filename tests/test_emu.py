@@ -828,3 +828,26 @@ def test_outputs_do_not_depend_on_alignment(emu_lib, choose_backward, B, T, dk, 
 
     for i, (a, b) in enumerate(zip(outputs(lambda t: t), outputs(_shifted))):
         assert torch.equal(a, b), f"output {i}: {(a != b).sum().item()} elements differ"
+
+
+@pytest.mark.parametrize("kernel,passes,B,T,H,dv", [
+    (4, 1, 256, 64, 1, 64),       # one workgroup per sequence while they fit the device at once
+    (25, 1, 257, 64, 1, 64),
+    (25, 1, 43, 33, 12, 128),
+    (25, 1, 96, 1, 8, 128),
+    (3, 1, 97, 64, 8, 128),       # more than six per unit
+    (25, 1, 24, 64, 16, 256),
+    (3, 1, 257, 65, 1, 64),       # a second chunk
+    (3, 2, 257, 64, 1, 64),       # passes that share a launch
+])
+def test_rule_of_sequences_of_one_chunk(emu_lib, kernel, passes, B, T, H, dv):
+    """Which forwards of 64-wide keys and at most one chunk go through registers, at 256 units."""
+    assert emu_lib.emu_pass_kernel(passes, B, T, H, 64, dv, 0, 0, 0, 256) == kernel
+
+
+@pytest.mark.parametrize("B,T,dv", [(9, 64, 64), (48, 64, 64), (49, 40, 64), (13, 33, 128), (5, 50, 256)])
+def test_sequences_of_one_chunk(emu_lib, choose_backward, B, T, dv):
+    """Short sequences on more workgroups than the device has units (8), on both sides of the rule."""
+    assert (emu_lib.emu_pass_kernel(1, B, T, 1, 64, dv, 0, 0, 0, 8) == 25) == (B * dv // 64 <= 48)
+    choose_backward(PASSES)
+    test_plain_fwd_bwd(emu_lib, B, T, 1, 64, dv, 0.5)

@@ -515,6 +515,12 @@ def test_pass_of_128_columns_per_workgroup(hip_lib, B, T, H, dv, state_std):
             assert hip_lib.fp_set_backward_choice(0, -1) == 0
 
 
+@pytest.mark.parametrize("B,T,H,dv,state_std", [(36, 64, 8, 64, 0.1), (72, 33, 12, 128, None), (97, 64, 4, 256, 0.1)])
+def test_sequences_of_one_chunk(hip_lib, B, T, H, dv, state_std):
+    """64-wide keys and at most one chunk a sequence, on more workgroups than the device has units, on both sides of six per unit."""
+    run_plain(B, T, H, 64, dv, state_std, seed=T, oracle_batches=sorted({0, B // 2, B - 1}), oracle_device=DEV)
+
+
 @pytest.mark.parametrize("B,T,H,dk,dv,block,Ls", [
     (2, 193, 4, 64, 64, 0, 0), (75, 65, 4, 64, 64, 0, 0), (2, 300, 4, 64, 128, 64, 0), (2, 192, 4, 64, 128, 64, 16), (10, 97, 16, 128, 128, 0, 0),
 ])
